@@ -2,161 +2,10 @@
 // reverse-edge insertion and refinement.  One point per wavefront.
 // Reference: graph_kernel.cuh (build_kernel :249-316, build_boundary_kernel :318-376, reverse_graph_kernel
 // :378-414, insert_reverse_kernel :416-453, refine_kernel :580-673) as sequenced by glide_impl.cuh:77-316.
-#include "prune.hpp"
+#include "graph.hpp"
 #include "host_util.hpp"
 
 namespace glide {
-
-struct BuildArgs {
-    const float* reorder_data;
-    const uint32_t* knn_graph;
-    const uint32_t* map;
-    const uint32_t* segment_starts;
-    const uint32_t* segment_lengths;
-    const uint32_t* start_points;
-    uint32_t* graph;
-    unsigned long long* counters;
-    uint32_t first_point, point_count;   // reorder ids [first_point, first_point + point_count)
-    uint32_t segment_num, graph_degree;
-    uint32_t boundary_start;             // boundary kernel: segment start (= num); 0xffffffff for the regular kernel
-    uint32_t boundary_start_point;
-    float relaxant;
-    BeamParams p;                         // p.degree = knn_degree
-};
-
-template <int MAX_CAND, int MAX_BEAM, int DIMV>
-__global__ __launch_bounds__(64) void build_kernel(BuildArgs a) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    auto* lds = reinterpret_cast<BeamLds<MAX_CAND>*>(smem);
-    auto* pl = reinterpret_cast<PruneLds<MAX_BEAM>*>(smem + sizeof(BeamLds<MAX_CAND>));
-    uint32_t* hash = reinterpret_cast<uint32_t*>(smem + sizeof(BeamLds<MAX_CAND>) + sizeof(PruneLds<MAX_BEAM>));
-    if (blockIdx.x >= a.point_count) return;
-    const uint32_t point = a.first_point + blockIdx.x;
-    const bool boundary = a.boundary_start != kInvalid;
-
-    const bool segment_mode = a.map == nullptr;   // one staged partition: local ids in and out (build_for_large_kernel)
-    uint32_t seg_start, entry;
-    if (segment_mode) {
-        seg_start = 0;
-        entry = a.boundary_start_point;
-    } else if (boundary) {
-        seg_start = a.boundary_start;
-        entry = a.boundary_start_point;
-    } else {
-        uint32_t seg = 0;
-        for (; seg < a.segment_num; seg++)
-            if (point < a.segment_starts[seg] + a.segment_lengths[seg]) break;
-        seg_start = a.segment_starts[seg];
-        entry = a.start_points[seg];
-    }
-    const float* sdata = a.reorder_data + static_cast<size_t>(seg_start) * a.p.dim;
-    const uint32_t* sgraph = a.knn_graph + static_cast<size_t>(seg_start) * a.p.degree;
-
-    Beam<MAX_CAND, MAX_BEAM, DIMV> b;
-    b.init(lds, hash, a.p, a.reorder_data + static_cast<size_t>(point) * a.p.dim);
-    // get_init (search_kernel.cuh:336-360): all neighbours of the entry are hashed; the one whose *local* id equals
-    // this point's *reorder* id is left unscored (the reference compares across id spaces, graph_kernel.cuh:295-298)
-    b.expand(entry, sgraph, sdata, kInvalid, point);
-    b.run(sgraph, sdata, point - seg_start);
-
-    uint32_t pool = beam_to_pool(b, pl);
-    prune_pool<MAX_BEAM, DIMV>(pl, pool, a.reorder_data, a.p.dim, seg_start, a.graph_degree, a.relaxant, a.p.metric, b.lane,
-                               b.cnt.rows_scored);
-    wave_sync();
-    if (segment_mode) {   // map_to_graph (graph_kernel.cuh:145-150)
-        uint32_t* row = a.graph + static_cast<size_t>(point) * a.graph_degree;
-        for (uint32_t i = b.lane; i < a.graph_degree; i += 64) row[i] = pl->neighbor[i];
-        b.flush_counters(a.counters);
-        return;
-    }
-    uint32_t* row = a.graph + static_cast<size_t>(a.map[point]) * a.graph_degree;
-    if (boundary) {
-        merge_boundary_row<MAX_BEAM>(pl, row, a.map, a.graph_degree, b.lane);
-    } else {  // map_to_graph_sub (graph_kernel.cuh:152-158)
-        for (uint32_t i = b.lane; i < a.graph_degree; i += 64) {
-            const uint32_t nb = pl->neighbor[i];
-            row[i] = nb == kInvalid ? kInvalid : a.map[nb];
-        }
-    }
-    b.flush_counters(a.counters);
-}
-
-struct RefineArgs {
-    const float* data;
-    const uint32_t* graph_in;
-    uint32_t* graph_out;
-    const float* centroids;
-    const uint32_t* start_points;
-    unsigned long long* counters;
-    const uint32_t* order;   // nullable: workgroup i refines point order[i] (a permutation of the points)
-    uint32_t num, centroid_num, max_centroid, segment_start_point;
-    float relaxant;
-    BeamParams p;   // p.degree = graph_degree
-};
-
-template <int DIMV>
-__device__ __forceinline__ uint32_t pick_centroid_refine(uint32_t max_centroid, const RowRegs<DIMV>& q, const float* centroids,
-                                                         uint32_t centroid_num, uint32_t dim, int metric, float* scratch, int lane) {
-    switch (max_centroid) {
-        case 32: return nearest_centroid<32, DIMV>(q, centroids, centroid_num, dim, metric, scratch, lane);
-        case 64: return nearest_centroid<64, DIMV>(q, centroids, centroid_num, dim, metric, scratch, lane);
-        case 128: return nearest_centroid<128, DIMV>(q, centroids, centroid_num, dim, metric, scratch, lane);
-        default: return nearest_centroid<256, DIMV>(q, centroids, centroid_num, dim, metric, scratch, lane);
-    }
-}
-
-// Rows are read from graph_in and written to graph_out (every row is written: copied, with its empty slots
-// filled).  The reference refines in place while other blocks still traverse the rows.
-template <int MAX_CAND, int MAX_BEAM, int DIMV>
-__global__ __launch_bounds__(64) void refine_kernel(RefineArgs a) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    auto* lds = reinterpret_cast<BeamLds<MAX_CAND>*>(smem);
-    using Prune = PruneLds<MAX_BEAM, (MAX_CAND < 64 ? 64 : MAX_CAND)>;   // the row has at most MAX_CAND slots here
-    auto* pl = reinterpret_cast<Prune*>(smem + sizeof(BeamLds<MAX_CAND>));
-    float* cent = reinterpret_cast<float*>(smem + sizeof(BeamLds<MAX_CAND>) + sizeof(Prune));
-    uint32_t* hash = reinterpret_cast<uint32_t*>(cent + round_up32(a.centroid_num));
-    if (blockIdx.x >= a.num) return;
-    const uint32_t point = a.order ? a.order[blockIdx.x] : blockIdx.x;
-    if (point >= a.num) return;
-    const int lane = lane_id();
-    const uint32_t D = a.p.degree;
-    const uint32_t* in_row = a.graph_in + static_cast<size_t>(point) * D;
-    uint32_t* out_row = a.graph_out + static_cast<size_t>(point) * D;
-
-    uint32_t need = 0;
-    for (uint32_t base = 0; base < Prune::kCap; base += 64) {
-        const uint32_t i = base + lane;
-        const uint32_t g = i < D ? in_row[i] : kInvalid;
-        pl->s_graph[i] = g;
-        if (i < D) out_row[i] = g;
-        need += __popcll(ballot(i < D && g == kInvalid));
-    }
-    wave_sync();
-    if (need == 0) return;
-
-    Beam<MAX_CAND, MAX_BEAM, DIMV> b;
-    b.init(lds, hash, a.p, a.data + static_cast<size_t>(point) * a.p.dim);
-    if (a.centroids != nullptr) {
-        const uint32_t c0 = pick_centroid_refine<DIMV>(a.max_centroid, b.q, a.centroids, a.centroid_num, a.p.dim, a.p.metric, cent, lane);
-        b.expand(a.start_points[c0], a.graph_in, a.data, kInvalid, kInvalid);
-    } else {   // refine_for_large_kernel (graph_kernel.cuh:796-798): get_init from the segment's start point
-        b.expand(a.segment_start_point, a.graph_in, a.data, kInvalid, point);
-    }
-    b.run(a.graph_in, a.data, point);
-
-    uint32_t pool = beam_to_pool(b, pl);
-    prune_pool_refine<MAX_BEAM, DIMV>(pl, pool, a.data, a.p.dim, point, D, need, a.relaxant, a.p.metric, lane, b.cnt.rows_scored);
-    wave_sync();
-    uint32_t used = 0;
-    for (uint32_t base = 0; base < round_up32(D); base += 64) {  // holes in slot order (graph_kernel.cuh:659-671)
-        const uint32_t i = base + lane;
-        const bool hole = i < D && pl->s_graph[i] == kInvalid;
-        const uint64_t m = ballot(hole);
-        if (hole) out_row[i] = pl->neighbor[used + prefix_count(m)];
-        used += __popcll(m);
-    }
-    b.flush_counters(a.counters);
-}
 
 // ------------------------------------------------------------------------------------------ reverse edges
 // Reference order of arrival in a row's reverse list is whatever the atomics give; here the list is the D
@@ -286,42 +135,6 @@ __global__ __launch_bounds__(64) void merge_boundary_kernel(const uint32_t* boun
 }
 
 // ------------------------------------------------------------------------------------------ dispatch
-using build_fn = void (*)(BuildArgs);
-using refine_fn = void (*)(RefineArgs);
-
-template <int MAX_CAND, int MAX_BEAM>
-build_fn pick_build_dim(uint32_t dim) {
-    if (dim <= 128) return build_kernel<MAX_CAND, MAX_BEAM, 1>;
-    if (dim <= 256) return build_kernel<MAX_CAND, MAX_BEAM, 2>;
-    if (dim <= 512) return build_kernel<MAX_CAND, MAX_BEAM, 4>;
-    if (dim <= 1024) return build_kernel<MAX_CAND, MAX_BEAM, 8>;
-    if (dim <= 2048) return build_kernel<MAX_CAND, MAX_BEAM, 16>;
-    return build_kernel<MAX_CAND, MAX_BEAM, 32>;
-}
-template <int MAX_CAND>
-build_fn pick_build_beam(uint32_t beam, uint32_t dim) {
-    if (beam <= 64) return pick_build_dim<MAX_CAND, 64>(dim);
-    if (beam <= 128) return pick_build_dim<MAX_CAND, 128>(dim);
-    if (beam <= 256) return pick_build_dim<MAX_CAND, 256>(dim);
-    return pick_build_dim<MAX_CAND, 512>(dim);
-}
-template <int MAX_CAND, int MAX_BEAM>
-refine_fn pick_refine_dim(uint32_t dim) {
-    if (dim <= 128) return refine_kernel<MAX_CAND, MAX_BEAM, 1>;
-    if (dim <= 256) return refine_kernel<MAX_CAND, MAX_BEAM, 2>;
-    if (dim <= 512) return refine_kernel<MAX_CAND, MAX_BEAM, 4>;
-    if (dim <= 1024) return refine_kernel<MAX_CAND, MAX_BEAM, 8>;
-    if (dim <= 2048) return refine_kernel<MAX_CAND, MAX_BEAM, 16>;
-    return refine_kernel<MAX_CAND, MAX_BEAM, 32>;
-}
-template <int MAX_CAND>
-refine_fn pick_refine_beam(uint32_t beam, uint32_t dim) {
-    if (beam <= 64) return pick_refine_dim<MAX_CAND, 64>(dim);
-    if (beam <= 128) return pick_refine_dim<MAX_CAND, 128>(dim);
-    if (beam <= 256) return pick_refine_dim<MAX_CAND, 256>(dim);
-    return pick_refine_dim<MAX_CAND, 512>(dim);
-}
-
 size_t prune_lds_bytes(uint32_t beam) {
     return beam <= 64 ? sizeof(PruneLds<64>) : beam <= 128 ? sizeof(PruneLds<128>) : beam <= 256 ? sizeof(PruneLds<256>) : sizeof(PruneLds<512>);
 }
@@ -344,8 +157,7 @@ int check_beam_sizes(uint32_t degree, uint32_t graph_degree, uint32_t beam, uint
 }
 
 int launch_build(BuildArgs& a, hipStream_t stream) {
-    build_fn fn = a.p.degree <= 64 ? pick_build_beam<64>(a.p.beam, a.p.dim)
-                : a.p.degree <= 128 ? pick_build_beam<128>(a.p.beam, a.p.dim) : pick_build_beam<256>(a.p.beam, a.p.dim);
+    build_fn fn = pick_build(a.p.degree, a.p.beam, a.p.dim);
     const size_t lds_bytes = beam_lds_bytes(a.p.degree) + prune_lds_bytes(a.p.beam) + (size_t{1} << a.p.hash_bit) * sizeof(uint32_t);
     GLIDE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)));
     hipLaunchKernelGGL(fn, dim3(a.point_count), dim3(64), lds_bytes, stream, a);
@@ -473,8 +285,7 @@ int glide_hip_refine_segment(const float* segment_data, uint32_t num, uint32_t d
     a.segment_start_point = start_point;
     a.relaxant = relaxant;
     a.p = BeamParams{beam, graph_degree, dim, hash_bit, hash_reset_interval ? hash_reset_interval : 1, max_iterations, min_iterations, metric};
-    refine_fn fn = graph_degree <= 64 ? pick_refine_beam<64>(beam, dim)
-                 : graph_degree <= 128 ? pick_refine_beam<128>(beam, dim) : pick_refine_beam<256>(beam, dim);
+    refine_fn fn = pick_refine(graph_degree, beam, dim);
     const size_t lds_bytes = beam_lds_bytes(graph_degree) + prune_lds_bytes(beam) + (size_t{1} << hash_bit) * sizeof(uint32_t);
     GLIDE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)));
     hipLaunchKernelGGL(fn, dim3(num), dim3(64), lds_bytes, as_stream(stream), a);
@@ -574,8 +385,7 @@ int launch_refine(const float* data, uint32_t num, uint32_t dim, const uint32_t*
     a.segment_start_point = 0;
     a.relaxant = relaxant;
     a.p = BeamParams{beam, graph_degree, dim, hash_bit, hash_reset_interval ? hash_reset_interval : 1, max_iterations, min_iterations, metric};
-    refine_fn fn = graph_degree <= 64 ? pick_refine_beam<64>(beam, dim)
-                 : graph_degree <= 128 ? pick_refine_beam<128>(beam, dim) : pick_refine_beam<256>(beam, dim);
+    refine_fn fn = pick_refine(graph_degree, beam, dim);
     const size_t lds_bytes = beam_lds_bytes(graph_degree) + prune_lds_bytes_refine(beam, graph_degree) + round_up32(centroid_num) * sizeof(float) +
                              (size_t{1} << hash_bit) * sizeof(uint32_t);
     GLIDE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)));

@@ -1,0 +1,166 @@
+// Sub-graph build with pruning and refinement, one point per wavefront, for one degree bucket (GLIDE_CAND candidate slots).
+// Reference: graph_kernel.cuh (build_kernel :249-316, build_boundary_kernel :318-376, refine_kernel :580-673).
+#include "graph.hpp"
+
+namespace glide {
+
+template <int MAX_CAND, int MAX_BEAM, int DIMV>
+__global__ __launch_bounds__(64) void build_kernel(BuildArgs a) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    auto* lds = reinterpret_cast<BeamLds<MAX_CAND>*>(smem);
+    auto* pl = reinterpret_cast<PruneLds<MAX_BEAM>*>(smem + sizeof(BeamLds<MAX_CAND>));
+    uint32_t* hash = reinterpret_cast<uint32_t*>(smem + sizeof(BeamLds<MAX_CAND>) + sizeof(PruneLds<MAX_BEAM>));
+    if (blockIdx.x >= a.point_count) return;
+    const uint32_t point = a.first_point + blockIdx.x;
+    const bool boundary = a.boundary_start != kInvalid;
+
+    const bool segment_mode = a.map == nullptr;   // one staged partition: local ids in and out (build_for_large_kernel)
+    uint32_t seg_start, entry;
+    if (segment_mode) {
+        seg_start = 0;
+        entry = a.boundary_start_point;
+    } else if (boundary) {
+        seg_start = a.boundary_start;
+        entry = a.boundary_start_point;
+    } else {
+        uint32_t seg = 0;
+        for (; seg < a.segment_num; seg++)
+            if (point < a.segment_starts[seg] + a.segment_lengths[seg]) break;
+        seg_start = a.segment_starts[seg];
+        entry = a.start_points[seg];
+    }
+    const float* sdata = a.reorder_data + static_cast<size_t>(seg_start) * a.p.dim;
+    const uint32_t* sgraph = a.knn_graph + static_cast<size_t>(seg_start) * a.p.degree;
+
+    Beam<MAX_CAND, MAX_BEAM, DIMV> b;
+    b.init(lds, hash, a.p, a.reorder_data + static_cast<size_t>(point) * a.p.dim);
+    // get_init (search_kernel.cuh:336-360): all neighbours of the entry are hashed; the one whose *local* id equals
+    // this point's *reorder* id is left unscored (the reference compares across id spaces, graph_kernel.cuh:295-298)
+    b.expand(entry, sgraph, sdata, kInvalid, point);
+    b.run(sgraph, sdata, point - seg_start);
+
+    uint32_t pool = beam_to_pool(b, pl);
+    prune_pool<MAX_BEAM, DIMV>(pl, pool, a.reorder_data, a.p.dim, seg_start, a.graph_degree, a.relaxant, a.p.metric, b.lane,
+                               b.cnt.rows_scored);
+    wave_sync();
+    if (segment_mode) {   // map_to_graph (graph_kernel.cuh:145-150)
+        uint32_t* row = a.graph + static_cast<size_t>(point) * a.graph_degree;
+        for (uint32_t i = b.lane; i < a.graph_degree; i += 64) row[i] = pl->neighbor[i];
+        b.flush_counters(a.counters);
+        return;
+    }
+    uint32_t* row = a.graph + static_cast<size_t>(a.map[point]) * a.graph_degree;
+    if (boundary) {
+        merge_boundary_row<MAX_BEAM>(pl, row, a.map, a.graph_degree, b.lane);
+    } else {  // map_to_graph_sub (graph_kernel.cuh:152-158)
+        for (uint32_t i = b.lane; i < a.graph_degree; i += 64) {
+            const uint32_t nb = pl->neighbor[i];
+            row[i] = nb == kInvalid ? kInvalid : a.map[nb];
+        }
+    }
+    b.flush_counters(a.counters);
+}
+
+template <int DIMV>
+__device__ __forceinline__ uint32_t pick_centroid_refine(uint32_t max_centroid, const RowRegs<DIMV>& q, const float* centroids,
+                                                         uint32_t centroid_num, uint32_t dim, int metric, float* scratch, int lane) {
+    switch (max_centroid) {
+        case 32: return nearest_centroid<32, DIMV>(q, centroids, centroid_num, dim, metric, scratch, lane);
+        case 64: return nearest_centroid<64, DIMV>(q, centroids, centroid_num, dim, metric, scratch, lane);
+        case 128: return nearest_centroid<128, DIMV>(q, centroids, centroid_num, dim, metric, scratch, lane);
+        default: return nearest_centroid<256, DIMV>(q, centroids, centroid_num, dim, metric, scratch, lane);
+    }
+}
+
+// Rows are read from graph_in and written to graph_out (every row is written: copied, with its empty slots
+// filled).  The reference refines in place while other blocks still traverse the rows.
+template <int MAX_CAND, int MAX_BEAM, int DIMV>
+__global__ __launch_bounds__(64) void refine_kernel(RefineArgs a) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    auto* lds = reinterpret_cast<BeamLds<MAX_CAND>*>(smem);
+    using Prune = PruneLds<MAX_BEAM, (MAX_CAND < 64 ? 64 : MAX_CAND)>;   // the row has at most MAX_CAND slots here
+    auto* pl = reinterpret_cast<Prune*>(smem + sizeof(BeamLds<MAX_CAND>));
+    float* cent = reinterpret_cast<float*>(smem + sizeof(BeamLds<MAX_CAND>) + sizeof(Prune));
+    uint32_t* hash = reinterpret_cast<uint32_t*>(cent + round_up32(a.centroid_num));
+    if (blockIdx.x >= a.num) return;
+    const uint32_t point = a.order ? a.order[blockIdx.x] : blockIdx.x;
+    if (point >= a.num) return;
+    const int lane = lane_id();
+    const uint32_t D = a.p.degree;
+    const uint32_t* in_row = a.graph_in + static_cast<size_t>(point) * D;
+    uint32_t* out_row = a.graph_out + static_cast<size_t>(point) * D;
+
+    uint32_t need = 0;
+    for (uint32_t base = 0; base < Prune::kCap; base += 64) {
+        const uint32_t i = base + lane;
+        const uint32_t g = i < D ? in_row[i] : kInvalid;
+        pl->s_graph[i] = g;
+        if (i < D) out_row[i] = g;
+        need += __popcll(ballot(i < D && g == kInvalid));
+    }
+    wave_sync();
+    if (need == 0) return;
+
+    Beam<MAX_CAND, MAX_BEAM, DIMV> b;
+    b.init(lds, hash, a.p, a.data + static_cast<size_t>(point) * a.p.dim);
+    if (a.centroids != nullptr) {
+        const uint32_t c0 = pick_centroid_refine<DIMV>(a.max_centroid, b.q, a.centroids, a.centroid_num, a.p.dim, a.p.metric, cent, lane);
+        b.expand(a.start_points[c0], a.graph_in, a.data, kInvalid, kInvalid);
+    } else {   // refine_for_large_kernel (graph_kernel.cuh:796-798): get_init from the segment's start point
+        b.expand(a.segment_start_point, a.graph_in, a.data, kInvalid, point);
+    }
+    b.run(a.graph_in, a.data, point);
+
+    uint32_t pool = beam_to_pool(b, pl);
+    prune_pool_refine<MAX_BEAM, DIMV>(pl, pool, a.data, a.p.dim, point, D, need, a.relaxant, a.p.metric, lane, b.cnt.rows_scored);
+    wave_sync();
+    uint32_t used = 0;
+    for (uint32_t base = 0; base < round_up32(D); base += 64) {  // holes in slot order (graph_kernel.cuh:659-671)
+        const uint32_t i = base + lane;
+        const bool hole = i < D && pl->s_graph[i] == kInvalid;
+        const uint64_t m = ballot(hole);
+        if (hole) out_row[i] = pl->neighbor[used + prefix_count(m)];
+        used += __popcll(m);
+    }
+    b.flush_counters(a.counters);
+}
+
+template <int MAX_CAND, int MAX_BEAM>
+build_fn pick_build_dim(uint32_t dim) {
+    if (dim <= 128) return build_kernel<MAX_CAND, MAX_BEAM, 1>;
+    if (dim <= 256) return build_kernel<MAX_CAND, MAX_BEAM, 2>;
+    if (dim <= 512) return build_kernel<MAX_CAND, MAX_BEAM, 4>;
+    if (dim <= 1024) return build_kernel<MAX_CAND, MAX_BEAM, 8>;
+    if (dim <= 2048) return build_kernel<MAX_CAND, MAX_BEAM, 16>;
+    return build_kernel<MAX_CAND, MAX_BEAM, 32>;
+}
+template <int MAX_CAND>
+build_fn pick_build_beam(uint32_t beam, uint32_t dim) {
+    if (beam <= 64) return pick_build_dim<MAX_CAND, 64>(dim);
+    if (beam <= 128) return pick_build_dim<MAX_CAND, 128>(dim);
+    if (beam <= 256) return pick_build_dim<MAX_CAND, 256>(dim);
+    return pick_build_dim<MAX_CAND, 512>(dim);
+}
+template <int MAX_CAND, int MAX_BEAM>
+refine_fn pick_refine_dim(uint32_t dim) {
+    if (dim <= 128) return refine_kernel<MAX_CAND, MAX_BEAM, 1>;
+    if (dim <= 256) return refine_kernel<MAX_CAND, MAX_BEAM, 2>;
+    if (dim <= 512) return refine_kernel<MAX_CAND, MAX_BEAM, 4>;
+    if (dim <= 1024) return refine_kernel<MAX_CAND, MAX_BEAM, 8>;
+    if (dim <= 2048) return refine_kernel<MAX_CAND, MAX_BEAM, 16>;
+    return refine_kernel<MAX_CAND, MAX_BEAM, 32>;
+}
+template <int MAX_CAND>
+refine_fn pick_refine_beam(uint32_t beam, uint32_t dim) {
+    if (beam <= 64) return pick_refine_dim<MAX_CAND, 64>(dim);
+    if (beam <= 128) return pick_refine_dim<MAX_CAND, 128>(dim);
+    if (beam <= 256) return pick_refine_dim<MAX_CAND, 256>(dim);
+    return pick_refine_dim<MAX_CAND, 512>(dim);
+}
+
+#define GLIDE_PICK_NAME(kind, cand) pick_##kind##_##cand
+#define GLIDE_PICK(kind, cand) GLIDE_PICK_NAME(kind, cand)
+build_fn GLIDE_PICK(build, GLIDE_CAND)(uint32_t beam, uint32_t dim) { return pick_build_beam<GLIDE_CAND>(beam, dim); }
+refine_fn GLIDE_PICK(refine, GLIDE_CAND)(uint32_t beam, uint32_t dim) { return pick_refine_beam<GLIDE_CAND>(beam, dim); }
+
+}  // namespace glide

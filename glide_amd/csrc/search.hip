@@ -1,197 +1,9 @@
 // glide_hip_search: one query per wavefront beam search over the finished index.
 // Reference: search_kernel (search_kernel.cuh:393-490) launched by GLIDE::search (glide_impl.cuh:370-454).
-#include "beam.hpp"
+#include "search.hpp"
 #include "host_util.hpp"
 
 namespace glide {
-
-struct SearchArgs {
-    const float* data;
-    const uint32_t* graph;
-    const float* centroids;
-    const uint32_t* start_points;
-    const float* queries;
-    uint32_t* result_ids;
-    float* result_dists;
-    unsigned long long* counters;
-    uint32_t centroid_num, max_centroid, top_k, query_num;
-    BeamParams p;
-};
-
-template <int DIMV, bool TEAM = false>
-__device__ __forceinline__ uint32_t pick_centroid(uint32_t max_centroid, const RowRegs<DIMV>& q, const float* centroids,
-                                                  uint32_t centroid_num, uint32_t dim, int metric, float* scratch, int lane) {
-    switch (max_centroid) {  // bucket chosen like reference kernel_config.cuh:161-171
-        case 32: return nearest_centroid<32, DIMV, TEAM>(q, centroids, centroid_num, dim, metric, scratch, lane);
-        case 64: return nearest_centroid<64, DIMV, TEAM>(q, centroids, centroid_num, dim, metric, scratch, lane);
-        case 128: return nearest_centroid<128, DIMV, TEAM>(q, centroids, centroid_num, dim, metric, scratch, lane);
-        default: return nearest_centroid<256, DIMV, TEAM>(q, centroids, centroid_num, dim, metric, scratch, lane);
-    }
-}
-
-template <int MAX_CAND, int MAX_BEAM, int DIMV, bool WHOLE = false>
-__device__ __forceinline__ void search_body(const SearchArgs a) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    auto* lds = reinterpret_cast<BeamLds<MAX_CAND>*>(smem);
-    float* cent = reinterpret_cast<float*>(smem + sizeof(BeamLds<MAX_CAND>));
-    uint32_t* hash = reinterpret_cast<uint32_t*>(cent + round_up32(a.centroid_num));
-    // a wavefront takes queries blockIdx.x, blockIdx.x + gridDim.x, ... (the host sizes the grid)
-    for (uint32_t qid = blockIdx.x; qid < a.query_num; qid += gridDim.x) {
-        Beam<MAX_CAND, MAX_BEAM, DIMV, false, WHOLE> b;
-        b.init(lds, hash, a.p, a.queries + static_cast<size_t>(qid) * a.p.dim);
-        const uint32_t c0 = pick_centroid<DIMV>(a.max_centroid, b.q, a.centroids, a.centroid_num, a.p.dim, a.p.metric, cent, b.lane);
-        const uint32_t entry = a.start_points[c0];
-        b.expand(entry, a.graph, a.data, kInvalid, kInvalid);  // result_init: entry node itself is never scored
-        b.run(a.graph, a.data, kInvalid);
-
-        constexpr int NB = MAX_BEAM / 64;
-#pragma unroll
-        for (int r = 0; r < NB; r++) {
-            const uint32_t e = NB * b.lane + r;
-            if (e < a.top_k) {
-                a.result_ids[static_cast<size_t>(qid) * a.top_k + e] = b.bv[r] & kClean;
-                a.result_dists[static_cast<size_t>(qid) * a.top_k + e] = b.bk[r];
-            }
-        }
-        b.flush_counters(a.counters);
-        wave_sync();   // the next query reuses the LDS
-    }
-}
-
-// Beams above 256 on rows of up to 512 dims: held to the registers of four wavefronts per SIMD (the kernel asks for a
-// dozen more, which costs it the fourth wavefront and buys nothing: the vector ALU is the limit).
-template <int MAX_CAND, int MAX_BEAM, int DIMV, bool WHOLE = false>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MAX_BEAM > 256 && DIMV <= 4 ? 4 : 1)))
-void search_kernel(SearchArgs a) {
-    search_body<MAX_CAND, MAX_BEAM, DIMV, WHOLE>(a);
-}
-// The beam-256 kernels are bound by the vector ALU (sorting networks) and need 103 registers, one wavefront per SIMD
-// short of the next occupancy step: held to five wavefronts per SIMD (96 registers, five of them spilled) they run
-// 5 % faster.  Other beams are either already there or would spill much more.
-template <int MAX_CAND, int MAX_BEAM, int DIMV>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 5))) void search_kernel_dense(SearchArgs a) {
-    search_body<MAX_CAND, MAX_BEAM, DIMV>(a);
-}
-
-// Small batches of long rows (more than 256 dims): a team of kTeam wavefronts per query.  Wavefront 0 owns the search
-// (beam, visited set, sorting networks) exactly as in search_kernel; between two of its passes every wavefront of the
-// team scores a share of the expansion's candidate rows.  One wavefront can keep only a few 2-4 KB rows in flight in its
-// registers, and a search is a chain of dependent expansions: while the batch leaves SIMDs idle, a team gives a query
-// kTeam times the bytes on their way and an expansion takes one or two memory round trips instead of six (64 queries of
-// 960 dims: 1.9 times the throughput at beams up to 256, 1.3 times above).  Once a batch fills the chip on its own
-// (about two wavefronts per SIMD) the row gathers run at the rate the memory system sustains for scattered rows either
-// way and the team only adds its barriers, so larger batches keep one wavefront per query.  The query row sits in LDS
-// once per team (RefInLds) so that the registers hold rows in flight; every distance is summed in the order
-// search_kernel sums it, so results are identical.
-constexpr int kTeam = 4;
-
-template <int DIMV>
-struct TeamShape {
-    static constexpr int U = DIMV >= 16 ? 1 : (DIMV == 8 ? 2 : 4);   // row steps in flight per wavefront: 64 row registers either way
-    static constexpr size_t query_bytes = sizeof(float4) * RowShape<DIMV>::NV * RowShape<DIMV>::LPR;
-};
-
-template <int MAX_CAND, int MAX_BEAM, int DIMV, bool WHOLE = false>
-__global__ __launch_bounds__(64 * kTeam) void search_team_kernel(SearchArgs a) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    using Shape = RowShape<DIMV>;
-    auto* lds = reinterpret_cast<BeamLds<MAX_CAND>*>(smem);
-    float* cent = reinterpret_cast<float*>(smem + sizeof(BeamLds<MAX_CAND>));
-    float4* qlds = reinterpret_cast<float4*>(cent + round_up32(a.centroid_num));
-    uint32_t* ctl = reinterpret_cast<uint32_t*>(qlds + Shape::NV * Shape::LPR);   // [0] rows to score, [1] search over
-    uint32_t* hash = ctl + 4;
-    const uint32_t wave = threadIdx.x >> 6;
-    const int lane = lane_id();
-    for (uint32_t qid = blockIdx.x; qid < a.query_num; qid += gridDim.x) {
-        Beam<MAX_CAND, MAX_BEAM, DIMV, true, WHOLE> b;
-        uint32_t iter = 0;
-        bool terminate = false;
-        if (wave == 0) {
-            b.init(lds, hash, a.p, a.queries + static_cast<size_t>(qid) * a.p.dim);
-            if (Shape::row_of_lane(lane) == 0) {
-#pragma unroll
-                for (int c = 0; c < Shape::NV; c++) qlds[c * Shape::LPR + Shape::lane_in_row(lane)] = b.q.v[c];
-            }
-            const uint32_t c0 = pick_centroid<DIMV, true>(a.max_centroid, b.q, a.centroids, a.centroid_num, a.p.dim, a.p.metric, cent, lane);
-            const uint32_t nv = b.expand_list(a.start_points[c0], a.graph, kInvalid, kInvalid);   // result_init: the entry node itself is never scored
-            if (lane == 0) {
-                ctl[0] = nv;
-                ctl[1] = 0;
-            }
-        }
-        __syncthreads();
-        while (true) {
-            const uint32_t nv = ctl[0];
-            score_share<DIMV, TeamShape<DIMV>::U>(RefInLds<DIMV>{qlds}, a.data, a.p.dim, a.p.metric, 0, nv, lane, wave, kTeam,
-                                                  [lds](uint32_t idx) { return lds->cand_id[lds->vlist[idx]]; },
-                                                  [lds](uint32_t idx, float d) { lds->cand_dist[lds->vlist[idx]] = d; });
-            __syncthreads();
-            if (wave == 0) {
-                uint32_t next = 0;
-                const bool more = b.step_to_list(iter, terminate, a.graph, kInvalid, next);
-                if (lane == 0) {
-                    ctl[0] = next;
-                    ctl[1] = more ? 0u : 1u;
-                }
-            }
-            __syncthreads();
-            if (ctl[1] != 0) break;
-        }
-        if (wave == 0) {
-            constexpr int NB = MAX_BEAM / 64;
-#pragma unroll
-            for (int r = 0; r < NB; r++) {
-                const uint32_t e = NB * lane + r;
-                if (e < a.top_k) {
-                    a.result_ids[static_cast<size_t>(qid) * a.top_k + e] = b.bv[r] & kClean;
-                    a.result_dists[static_cast<size_t>(qid) * a.top_k + e] = b.bk[r];
-                }
-            }
-            b.flush_counters(a.counters);
-        }
-        __syncthreads();   // the next query reuses the LDS
-    }
-}
-
-using search_fn = void (*)(SearchArgs);
-
-template <int MAX_CAND, int MAX_BEAM, bool WHOLE = false>
-search_fn pick_dim(uint32_t dim) {
-    if constexpr (MAX_BEAM == 256 && MAX_CAND <= 128) {
-        if (dim <= 128) return search_kernel_dense<MAX_CAND, MAX_BEAM, 1>;
-        if (dim <= 256) return search_kernel_dense<MAX_CAND, MAX_BEAM, 2>;
-        if (dim <= 512) return search_kernel_dense<MAX_CAND, MAX_BEAM, 4>;
-    }
-    if (dim <= 128) return search_kernel<MAX_CAND, MAX_BEAM, 1, WHOLE>;
-    if (dim <= 256) return search_kernel<MAX_CAND, MAX_BEAM, 2, WHOLE>;
-    if (dim <= 512) return search_kernel<MAX_CAND, MAX_BEAM, 4, WHOLE>;
-    if (dim <= 1024) return search_kernel<MAX_CAND, MAX_BEAM, 8, WHOLE>;
-    if (dim <= 2048) return search_kernel<MAX_CAND, MAX_BEAM, 16, WHOLE>;
-    return search_kernel<MAX_CAND, MAX_BEAM, 32, WHOLE>;
-}
-template <int MAX_CAND, int MAX_BEAM, bool WHOLE = false>
-search_fn pick_team_dim(uint32_t dim) {
-    if (dim <= 512) return search_team_kernel<MAX_CAND, MAX_BEAM, 4, WHOLE>;
-    if (dim <= 1024) return search_team_kernel<MAX_CAND, MAX_BEAM, 8, WHOLE>;
-    if (dim <= 2048) return search_team_kernel<MAX_CAND, MAX_BEAM, 16, WHOLE>;
-    return search_team_kernel<MAX_CAND, MAX_BEAM, 32, WHOLE>;
-}
-template <int MAX_CAND>
-search_fn pick_team_beam(uint32_t beam, uint32_t dim) {
-    if (beam <= 64) return pick_team_dim<MAX_CAND, 64>(dim);
-    if (beam <= 128) return pick_team_dim<MAX_CAND, 128>(dim);
-    if (beam <= 256) return pick_team_dim<MAX_CAND, 256>(dim);
-    if (beam == 512) return pick_team_dim<MAX_CAND, 512, true>(dim);
-    return pick_team_dim<MAX_CAND, 512>(dim);
-}
-template <int MAX_CAND>
-search_fn pick_beam(uint32_t beam, uint32_t dim) {
-    if (beam <= 64) return pick_dim<MAX_CAND, 64>(dim);
-    if (beam <= 128) return pick_dim<MAX_CAND, 128>(dim);
-    if (beam <= 256) return pick_dim<MAX_CAND, 256>(dim);
-    if (beam == 512) return pick_dim<MAX_CAND, 512, true>(dim);
-    return pick_dim<MAX_CAND, 512>(dim);
-}
 
 // Grid size for the one-query-per-wavefront search kernel.  With small beams the kernel is bound by row gathers; when
 // the batch is a little larger than what the chip holds at once (10 000 queries against 8 192 wavefront slots),
@@ -263,9 +75,7 @@ int launch_search(const float* data, uint32_t num, uint32_t dim, const uint32_t*
     a.p.metric = metric;
 
     const bool team = dim > 256 && static_cast<size_t>(query_num) * kTeam <= 2 * simd_count();   // see search_team_kernel
-    search_fn fn;
-    if (team) fn = graph_degree <= 64 ? pick_team_beam<64>(beam, dim) : graph_degree <= 128 ? pick_team_beam<128>(beam, dim) : pick_team_beam<256>(beam, dim);
-    else fn = graph_degree <= 64 ? pick_beam<64>(beam, dim) : graph_degree <= 128 ? pick_beam<128>(beam, dim) : pick_beam<256>(beam, dim);
+    search_fn fn = graph_degree <= 64 ? pick_search_64(beam, dim, team) : graph_degree <= 128 ? pick_search_128(beam, dim, team) : pick_search_256(beam, dim, team);
     const size_t lds_bytes = beam_lds_bytes(graph_degree) + round_up32(centroid_num) * sizeof(float) +
                              (size_t{1} << hash_bit) * sizeof(uint32_t) +
                              (team ? (dim <= 512 ? TeamShape<4>::query_bytes : dim <= 1024 ? TeamShape<8>::query_bytes : dim <= 2048 ? TeamShape<16>::query_bytes : TeamShape<32>::query_bytes) + 16 : 0);

@@ -1,0 +1,144 @@
+// The beam search inside one partition of the large path, for one degree bucket (GLIDE_CAND candidate slots).
+// Reference: search_on_sub_kernel (search_kernel.cuh:653-765) with result_merge (:609-651).
+#include "search_sub.hpp"
+
+namespace glide {
+
+// result_merge (search_kernel.cuh:609-651): best top_k of (running result, this partition's beam head)
+template <int MAX_TOPK, int MAX_BEAM>
+__device__ __forceinline__ void merge_result(const float* beam_dist, const uint32_t* beam_id, const uint32_t* map, float* final_dists,
+                                             uint32_t* final_ids, uint32_t top_k, int lane) {
+    constexpr int NR = WaveNet<MAX_TOPK>::NR;
+    const bool live = MAX_TOPK >= 64 || lane < 32;
+    float k[NR];
+    uint32_t v[NR];
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+        const uint32_t e = NR * lane + r;
+        k[r] = (live && e < top_k) ? final_dists[e] : FLT_MAX;
+        v[r] = (live && e < top_k) ? final_ids[e] : kInvalid;
+        const uint32_t kk = MAX_TOPK - 1 - e;
+        if (live && kk < top_k) {
+            const float rk = beam_dist[kk];
+            if (k[r] > rk) {
+                k[r] = rk;
+                v[r] = map[beam_id[kk] & kClean];
+            }
+        }
+    }
+    WaveNet<MAX_TOPK>::merge(k, v, lane);
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+        const uint32_t e = NR * lane + r;
+        if (live && e < top_k) {
+            final_dists[e] = k[r];
+            final_ids[e] = v[r];
+        }
+    }
+}
+
+// search_on_sub_kernel (search_kernel.cuh:653-765)
+template <int MAX_CAND, int MAX_BEAM, int DIMV, bool WHOLE = false>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MAX_BEAM > 256 && DIMV <= 4 ? 4 : 1)))   // as search_kernel
+void search_sub_kernel(SubArgs a) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    auto* lds = reinterpret_cast<BeamLds<MAX_CAND>*>(smem);
+    float* head_dist = reinterpret_cast<float*>(smem + sizeof(BeamLds<MAX_CAND>));   // beam head staged for the merge (128 pairs)
+    uint32_t* head_id = reinterpret_cast<uint32_t*>(head_dist + 128);
+    uint32_t* hash = head_id + 128;
+    uint32_t qid = blockIdx.x;
+    const float* data = a.data;
+    const uint32_t* graph = a.graph;
+    const uint32_t* map = a.map;
+    uint32_t start_point = a.start_point;
+    if (a.pair_segment) {
+        if (qid >= a.list_len) return;
+        const uint32_t seg = a.pair_segment[qid];
+        const size_t start = a.segment_starts[seg];
+        data += start * a.p.dim;
+        graph += start * a.p.degree;
+        map += start;
+        start_point = a.segment_start_points[seg];
+        if (start_point == kInvalid) {   // an empty partition: nothing to find
+            for (uint32_t e = lane_id(); e < a.top_k; e += 64) {
+                a.pair_dists[static_cast<size_t>(blockIdx.x) * a.top_k + e] = FLT_MAX;
+                a.pair_ids[static_cast<size_t>(blockIdx.x) * a.top_k + e] = kInvalid;
+            }
+            return;
+        }
+        qid = a.query_list[qid];
+    } else if (a.query_list) {
+        if (qid >= a.list_len) return;
+        qid = a.query_list[qid];
+    } else {
+        if (qid >= a.query_num) return;
+        bool is_search = false;   // wave-uniform scan of this query's partition list
+        for (uint32_t i = 0; i < a.centroid_num; i++) {
+            const uint32_t s = a.segment_ids[static_cast<size_t>(qid) * a.centroid_num + i];
+            if (s == a.segment_id) { is_search = true; break; }
+            if (s == kInvalid) break;
+        }
+        if (!is_search) return;
+    }
+
+    Beam<MAX_CAND, MAX_BEAM, DIMV, false, WHOLE> b;
+    b.init(lds, hash, a.p, a.queries + static_cast<size_t>(qid) * a.p.dim);
+    b.expand(start_point, graph, data, kInvalid, kInvalid);   // get_init with point_id = 0xffffffff
+    b.run(graph, data, kInvalid);
+
+    constexpr int NB = MAX_BEAM / 64;
+    if (a.pair_segment) {   // the head of this pair's beam, ids already as input row numbers; merged per query afterwards
+#pragma unroll
+        for (int r = 0; r < NB; r++) {
+            const uint32_t e = NB * b.lane + r;
+            if (e < a.top_k) {
+                const float d = b.bk[r];
+                a.pair_dists[static_cast<size_t>(blockIdx.x) * a.top_k + e] = d;
+                a.pair_ids[static_cast<size_t>(blockIdx.x) * a.top_k + e] = d < FLT_MAX ? map[b.bv[r] & kClean] : kInvalid;
+            }
+        }
+        b.flush_counters(a.counters);
+        return;
+    }
+#pragma unroll
+    for (int r = 0; r < NB; r++) {
+        const uint32_t e = NB * b.lane + r;
+        if (e < 128) {
+            head_dist[e] = b.bk[r];
+            head_id[e] = b.bv[r];
+        }
+    }
+    wave_sync();
+    float* fd = a.final_dists + static_cast<size_t>(qid) * a.top_k;
+    uint32_t* fi = a.final_ids + static_cast<size_t>(qid) * a.top_k;
+    switch (a.max_topk) {   // kernel_config.cuh:312-323
+        case 32: merge_result<32, MAX_BEAM>(head_dist, head_id, map, fd, fi, a.top_k, b.lane); break;
+        case 64: merge_result<64, MAX_BEAM>(head_dist, head_id, map, fd, fi, a.top_k, b.lane); break;
+        default: merge_result<128, MAX_BEAM>(head_dist, head_id, map, fd, fi, a.top_k, b.lane); break;
+    }
+    b.flush_counters(a.counters);
+}
+
+template <int MAX_CAND, int MAX_BEAM, bool WHOLE = false>
+sub_fn pick_sub_dim(uint32_t dim) {
+    if (dim <= 128) return search_sub_kernel<MAX_CAND, MAX_BEAM, 1, WHOLE>;
+    if (dim <= 256) return search_sub_kernel<MAX_CAND, MAX_BEAM, 2, WHOLE>;
+    if (dim <= 512) return search_sub_kernel<MAX_CAND, MAX_BEAM, 4, WHOLE>;
+    if (dim <= 1024) return search_sub_kernel<MAX_CAND, MAX_BEAM, 8, WHOLE>;
+    if (dim <= 2048) return search_sub_kernel<MAX_CAND, MAX_BEAM, 16, WHOLE>;
+    return search_sub_kernel<MAX_CAND, MAX_BEAM, 32, WHOLE>;
+}
+template <int MAX_CAND>
+sub_fn pick_sub_beam(uint32_t beam, uint32_t dim) {
+    if (beam <= 64) return pick_sub_dim<MAX_CAND, 64>(dim);
+    if (beam <= 128) return pick_sub_dim<MAX_CAND, 128>(dim);
+    if (beam <= 256) return pick_sub_dim<MAX_CAND, 256>(dim);
+    if (beam == 512) return pick_sub_dim<MAX_CAND, 512, true>(dim);   // the whole of the widest beam: merged in the registers
+    return pick_sub_dim<MAX_CAND, 512>(dim);
+}
+
+#define GLIDE_PICK_NAME(cand) pick_sub_##cand
+#define GLIDE_PICK(cand) GLIDE_PICK_NAME(cand)
+sub_fn GLIDE_PICK(GLIDE_CAND)(uint32_t beam, uint32_t dim) { return pick_sub_beam<GLIDE_CAND>(beam, dim); }
+
+}  // namespace glide
