@@ -25,10 +25,10 @@ struct BeamCounters {  // wave-uniform tallies for traffic accounting
 };
 
 template <int MAX_CAND>
-struct BeamLds {  // per-wave LDS (the hash table follows, 1 << hash_bit words)
+struct alignas(16) BeamLds {  // per-wave LDS (the hash table follows, 1 << hash_bit words)
     uint32_t cand_id[MAX_CAND];
-    float cand_dist[MAX_CAND];
-    uint32_t vlist[MAX_CAND];
+    float cand_dist[MAX_CAND];   // squared distances of vlist's rows while an expansion is scored, then distances by slot or rank
+    uint32_t vlist[MAX_CAND];    // row ids to score, compacted
 };
 
 // Beams the kernels take: up to 512 (the reference's widest bucket, kernel_config.cuh:41-48); above 256 a multiple of 16, so
@@ -70,43 +70,73 @@ struct RefInLds {
     __device__ __forceinline__ float4 chunk(int c, int t) const { return q[c * RowShape<DIMV>::LPR + t]; }
 };
 
-// Distances from a reference row to `count` listed rows, RowShape<DIMV>::ROWS rows per step (one per lane group), U steps
-// in flight.  id_of(idx) -> row id of list entry idx; out(idx, dist) is called by one lane per scored row.  A team of
-// `members` wavefronts splits the list in runs of ROWS * U entries, member `member` taking every members-th run; the sum
-// of a row is formed in the same order whoever forms it.
-template <int DIMV, int U, class Ref, class IdFn, class OutFn>
-__device__ __forceinline__ void score_share(const Ref ref, const float* data, uint32_t dim, int metric, uint32_t first, uint32_t count,
-                                            int lane, uint32_t member, uint32_t members, IdFn id_of, OutFn out) {
+// U steps of RowShape<DIMV>::ROWS rows each (one row per lane group): entries base .. base + ROWS * U of the list.
+// FULL: the rows fill the row shape exactly, so no load needs a mask.
+template <int DIMV, int U, bool FULL, class Ref, class IdFn, class OutFn>
+__device__ __forceinline__ void score_step(const Ref ref, const float* data, uint32_t dim, uint32_t base, uint32_t count, int g, int t,
+                                           IdFn id_of, OutFn out) {
     using Shape = RowShape<DIMV>;
-    const int g = Shape::row_of_lane(lane), t = Shape::lane_in_row(lane);
-    for (uint32_t base = first + member * Shape::ROWS * U; base < count; base += Shape::ROWS * U * members) {
-        RowRegs<DIMV> rows[U];
+    RowRegs<DIMV> rows[U];
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            // lane groups past the end re-read the last listed row (same cache lines, no branch); their result is dropped
-            const uint32_t idx = base + Shape::ROWS * u + g;
-            load_row<DIMV>(rows[u], data + static_cast<size_t>(id_of(idx < count ? idx : count - 1)) * dim, dim, t);
-        }
+    for (int u = 0; u < U; u++) {
+        // lane groups past the end re-read the last listed row (same cache lines, no branch); their result is dropped
+        const uint32_t idx = base + Shape::ROWS * u + g;
+        load_row<DIMV, FULL>(rows[u], data + static_cast<size_t>(id_of(idx < count ? idx : count - 1)) * dim, dim, t);
+    }
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const uint32_t idx = base + Shape::ROWS * u + g;
-            float acc = 0.f;
+    for (int u = 0; u < U; u++) {
+        const uint32_t idx = base + Shape::ROWS * u + g;
+        float acc = 0.f;
 #pragma unroll
-            for (int c = 0; c < Shape::NV; c++) acc = sqdist4(ref.chunk(c, t), rows[u].v[c], acc);
-            const float d = finish_distance(row_sum<DIMV>(acc), metric);
-            if (t == 0 && idx < count) out(idx, d);
-        }
+        for (int c = 0; c < Shape::NV; c++) acc = sqdist4(ref.chunk(c, t), rows[u].v[c], acc);
+        const float sq = row_sum<DIMV>(acc);
+        if (t == 0 && idx < count) out(idx, sq);
     }
 }
 
+// Squared distances from a reference row to `count` listed rows, U steps in flight.  id_of(idx) -> row id of list entry
+// idx; out(idx, squared distance) is called by one lane per scored row (the root, some fifteen instructions, is left to
+// the pass that reads the results with one lane per row).  A team of `members` wavefronts splits the list in runs of
+// ROWS * U entries, member `member` taking every members-th run; the sum of a row is formed in the same order whoever
+// forms it.  A run with at most half its entries takes half the steps: an expansion scores a dozen rows on average, and
+// every step issues its loads and arithmetic whether its lane groups have rows or not.
+template <int DIMV, int U, bool FULL, class Ref, class IdFn, class OutFn>
+__device__ __forceinline__ void score_runs(const Ref ref, const float* data, uint32_t dim, uint32_t first, uint32_t count,
+                                           int lane, uint32_t member, uint32_t members, IdFn id_of, OutFn out) {
+    using Shape = RowShape<DIMV>;
+    const int g = Shape::row_of_lane(lane), t = Shape::lane_in_row(lane);
+    for (uint32_t base = first + member * Shape::ROWS * U; base < count; base += Shape::ROWS * U * members) {
+        if constexpr (U > 1) {
+            if (count - base <= Shape::ROWS * (U / 2)) {
+                score_step<DIMV, U / 2, FULL>(ref, data, dim, base, count, g, t, id_of, out);
+                continue;
+            }
+        }
+        score_step<DIMV, U, FULL>(ref, data, dim, base, count, g, t, id_of, out);
+    }
+}
+template <int DIMV, int U, class Ref, class IdFn, class OutFn>
+__device__ __forceinline__ void score_share(const Ref ref, const float* data, uint32_t dim, uint32_t first, uint32_t count,
+                                            int lane, uint32_t member, uint32_t members, IdFn id_of, OutFn out) {
+    // Rows of exactly 128 or 256 dims are the usual ones and their searches the ones the vector ALU bounds: no masks there.
+    // Longer rows are bound by their bytes, a second copy of the loop would buy them nothing.
+    if constexpr (DIMV <= 2) {
+        if (dim == RowShape<DIMV>::LPR * RowShape<DIMV>::NV * 4) {
+            score_runs<DIMV, U, true>(ref, data, dim, first, count, lane, member, members, id_of, out);
+            return;
+        }
+    }
+    score_runs<DIMV, U, false>(ref, data, dim, first, count, lane, member, members, id_of, out);
+}
+
 template <int DIMV, class IdFn, class OutFn>
-__device__ __forceinline__ void score_list(const RowRegs<DIMV>& ref, const float* data, uint32_t dim, int metric,
+__device__ __forceinline__ void score_list(const RowRegs<DIMV>& ref, const float* data, uint32_t dim,
                                            uint32_t first, uint32_t count, int lane, IdFn id_of, OutFn out) {
     // Steps in flight.  Rows of more than 512 dims are 2-4 KB each and a step holds only two of them: with one step in
     // flight a wavefront had 8 KB on its way, too little to cover the memory latency when a launch has about one
     // wavefront per SIMD (1 000 queries); four steps took the 960-dim beam-512 search from 16.8 to 13.2 ms.
     constexpr int U = DIMV == 8 ? 4 : 2;   // rows of more than 1024 dims (DIMV 16, 32) take 64 registers a lane each: two steps
-    score_share<DIMV, U>(RefInRegs<DIMV>{ref}, data, dim, metric, first, count, lane, 0u, 1u, id_of, out);
+    score_share<DIMV, U>(RefInRegs<DIMV>{ref}, data, dim, first, count, lane, 0u, 1u, id_of, out);
 }
 
 // TEAM: the beam's wavefront is one of several in its workgroup (the others only score rows, see search_team_kernel).
@@ -117,7 +147,7 @@ struct Beam {
     static_assert(!WHOLE || MAX_BEAM > 256, "beams up to 256 merge in the registers anyway");
     static __device__ __forceinline__ void wave_sync() { wave_sync_in<TEAM>(); }
     static constexpr int NB = MAX_BEAM / 64;
-    static constexpr int NC = MAX_CAND / 64;
+    static constexpr int NC = MAX_CAND / 64;   // candidate slots per lane: slot 64 * i + lane
     static constexpr int NC32 = MAX_CAND / 32;  // items per lane in the reference's 32-lane layout
 
     float bk[NB];
@@ -129,6 +159,9 @@ struct Beam {
     BeamCounters cnt;
     int lane;
     uint32_t last_scored;   // rows scored by the latest expansion (wave-uniform)
+    uint32_t until_reset;   // iterations left until the visited set is reset (a countdown: a remainder by a run-time divisor is two dozen instructions)
+    uint32_t cid;           // candidate id of this lane's slot (MAX_CAND == 64; larger buckets keep the ids in LDS)
+    uint32_t place[NC];     // where in vlist each of this lane's slots is; kInvalid: not scored
 
     __device__ __forceinline__ void init(BeamLds<MAX_CAND>* lds_, uint32_t* hash_, const BeamParams& p_, const float* query) {
         lds = lds_;
@@ -136,8 +169,16 @@ struct Beam {
         p = p_;
         lane = lane_id();
         load_row<DIMV>(q, query, p.dim, RowShape<DIMV>::lane_in_row(lane));
+        until_reset = p.reset_interval;
         hash_clear(hash, p.hash_bit, lane);
         wave_sync();
+    }
+
+    // whether this iteration ends with a reset of the visited set
+    __device__ __forceinline__ bool count_down() {
+        if (--until_reset != 0) return false;
+        until_reset = p.reset_interval;
+        return true;
     }
 
     // One pass of the main loop up to the next expansion's candidate list (what `run` does between two score phases).
@@ -145,7 +186,7 @@ struct Beam {
     __device__ __forceinline__ bool step_to_list(uint32_t& iter, bool& terminate, const uint32_t* graph, uint32_t self_id, uint32_t& nv) {
         absorb(iter == 0);
         cnt.iterations++;
-        const bool reset_now = ((iter + 1) % p.reset_interval) == 0;
+        const bool reset_now = count_down();
         if (reset_now) {
             hash_clear(hash, p.hash_bit, lane);
             wave_sync();
@@ -166,22 +207,24 @@ struct Beam {
     // Expansion of `parent` (reference compute_distance / get_init / result_init second half):
     // every neighbour not yet in the visited set becomes a candidate; `exclude_insert` is never inserted,
     // `exclude_score` is inserted and kept as a candidate id but gets distance FLT_MAX.
-    // First half: the candidate slots and the list of slots to score (returns its length).
+    // First half: the candidate slots and the list of rows to score (returns its length).  vlist holds the row ids
+    // themselves, one LDS read before the row loads instead of two that depend on each other.
     __device__ __forceinline__ uint32_t expand_list(uint32_t parent, const uint32_t* graph, uint32_t exclude_insert, uint32_t exclude_score) {
         uint32_t nv = 0;
         if (parent != kInvalid) cnt.graph_rows++;
 #pragma unroll
-        for (int s0 = 0; s0 < MAX_CAND; s0 += 64) {
-            const uint32_t s = s0 + lane;
+        for (int i = 0; i < NC; i++) {
+            const uint32_t s = 64 * i + lane;
             uint32_t nid = kInvalid;
             if (s < p.degree && parent != kInvalid) nid = graph[static_cast<size_t>(parent) * p.degree + s];
             const uint32_t flag = (nid != kInvalid && nid != exclude_insert) ? hash_insert(hash, p.hash_bit, nid) : 0;
-            const uint32_t cid = flag ? nid : kInvalid;
-            lds->cand_id[s] = cid;
-            lds->cand_dist[s] = FLT_MAX;
-            const bool score = cid != kInvalid && cid != exclude_score;
+            const uint32_t c = flag ? nid : kInvalid;
+            if constexpr (NC == 1) cid = c;
+            else lds->cand_id[s] = c;
+            const bool score = c != kInvalid && c != exclude_score;
             const uint64_t m = ballot(score);
-            if (score) lds->vlist[nv + prefix_count(m)] = s;
+            place[i] = score ? nv + prefix_count(m) : kInvalid;
+            if (score) lds->vlist[place[i]] = c;
             nv += __popcll(m);
         }
         wave_sync();
@@ -194,15 +237,32 @@ struct Beam {
                                            uint32_t exclude_insert, uint32_t exclude_score) {
         const uint32_t nv = expand_list(parent, graph, exclude_insert, exclude_score);
         BeamLds<MAX_CAND>* l = lds;
-        score_list<DIMV>(q, data, p.dim, p.metric, 0, nv, lane,
-                         [l](uint32_t idx) { return l->cand_id[l->vlist[idx]]; },
-                         [l](uint32_t idx, float d) { l->cand_dist[l->vlist[idx]] = d; });
+        score_list<DIMV>(q, data, p.dim, 0, nv, lane,
+                         [l](uint32_t idx) { return l->vlist[idx]; },
+                         [l](uint32_t idx, float sq) { l->cand_dist[idx] = sq; });
+        wave_sync();
+    }
+
+    // Distance of this lane's slot i of the latest expansion; FLT_MAX where nothing was scored.
+    __device__ __forceinline__ float slot_distance(int i) const {
+        const float d = finish_distance(lds->cand_dist[place[i] & (MAX_CAND - 1)], p.metric);
+        return place[i] != kInvalid ? d : FLT_MAX;
+    }
+    // Buckets of more than 64 slots: from the order of vlist to the slots.
+    __device__ __forceinline__ void distances_to_slots() {
+        float d[NC];
+#pragma unroll
+        for (int i = 0; i < NC; i++) d[i] = slot_distance(i);
+        wave_sync();
+#pragma unroll
+        for (int i = 0; i < NC; i++) lds->cand_dist[64 * i + lane] = d[i];
         wave_sync();
     }
 
     // Candidate sort, one network over the wavefront (reference sort_for_candidate, single-warp branch,
-    // search_kernel.cuh:9-37): strided load, sort, blocked store of every element.
-    __device__ __forceinline__ void sort_candidates_one() {
+    // search_kernel.cuh:9-37): strided load, sort, blocked store of every element.  `key` is the distance of this lane's
+    // slot (MAX_CAND == 64).
+    __device__ __forceinline__ void sort_candidates_one(float key) {
         if constexpr (MAX_CAND == 64) {
             // At most 32 slots in use: the strided load puts them on the even elements of the 64-element network and
             // +inf on the odd ones.  Every comparator of that network then meets at most one real key, or two real
@@ -211,21 +271,18 @@ struct Beam {
             // (the CPU tests compare the two networks on tie-rich inputs), in 15 stages instead of 21.
             // The one exception is a real id whose key is not below FLT_MAX (the build kernels leave the point itself
             // unscored): among the +inf keys its place does depend on the network, so that case takes the long way.
-            if (p.degree <= 32) {
-                float hk[1];
-                uint32_t hv[1];
-                const uint32_t slot = lane & 31;   // both halves of the wavefront sort the same 32 slots
-                hk[0] = slot < p.degree ? lds->cand_dist[slot] : FLT_MAX;
-                hv[0] = slot < p.degree ? lds->cand_id[slot] : kInvalid;
-                if (ballot(hv[0] != kInvalid && !(hk[0] < FLT_MAX)) == 0) {
-                    WaveNet<32>::sort(hk, hv, lane);
-                    wave_sync();
-                    lds->cand_dist[lane] = lane < 32 ? hk[0] : FLT_MAX;
-                    lds->cand_id[lane] = lane < 32 ? hv[0] : kInvalid;
-                    wave_sync();
-                    return;
-                }
+            if (p.degree <= 32 && ballot(cid != kInvalid && !(key < FLT_MAX)) == 0) {
+                float hk[1] = {key};
+                uint32_t hv[1] = {cid};   // the slots of the upper half of the wavefront are empty
+                WaveNet<32>::sort(hk, hv, lane);
+                lds->cand_dist[lane] = hk[0];
+                lds->cand_id[lane] = hv[0];
+                wave_sync();
+                return;
             }
+            lds->cand_dist[lane] = key;
+            lds->cand_id[lane] = cid;
+            wave_sync();
         }
         float ck[NC];
         uint32_t cv[NC];
@@ -430,8 +487,8 @@ struct Beam {
     // candidate, entry `beam - 1 - k` by the k-th smallest, so if even the smallest candidate is not below the largest
     // entry nothing is replaced, and the candidate sort in front of it only feeds that test.  Half of all iterations of
     // a wide beam end here (the further a search has come, the fewer neighbours of its frontier are nearer than the worst
-    // entry it holds), for one LDS read per lane.
-    __device__ __forceinline__ uint64_t entering(float& ck) {
+    // entry it holds), for one comparison per lane.
+    __device__ __forceinline__ uint64_t entering(float ck) const {
         static_assert(MAX_CAND == 64, "one candidate slot per lane");
         // The beam is ascending, so its last entry is the largest key of the lane that holds it among that lane's entries
         // below `beam` (written as a maximum: a chain of selects between the registers becomes a run-time index, which
@@ -446,7 +503,6 @@ struct Beam {
             for (int r = 1; r < NB; r++) mine = fmaxf(mine, NB * lane + r <= static_cast<int>(last) ? bk[r] : 0.f);
             tail = read_lane(mine, static_cast<int>(last / NB));
         }
-        ck = static_cast<uint32_t>(lane) < p.degree ? lds->cand_dist[lane] : FLT_MAX;
         return ballot(ck < tail);
     }
 
@@ -456,14 +512,15 @@ struct Beam {
         // exchanged) and no candidate can displace a beam entry, so the beam stays as it is.
         if (!first && last_scored == 0) return;
         if constexpr (MAX_CAND == 64) {
-            if (!first) {
-                float ck;
-                const uint64_t em = entering(ck);
-                if (em == 0) return;
-            }
+            const float ck = slot_distance(0);
+            if (!first && entering(ck) == 0) return;
+            wave_sync();
+            sort_candidates_one(ck);
+        } else {
+            distances_to_slots();
+            if constexpr (MAX_CAND > 128) sort_candidates_two();
+            else sort_candidates_one(0.f);
         }
-        if constexpr (MAX_CAND > 128) sort_candidates_two();
-        else sort_candidates_one();
         if (first) {
 #pragma unroll
             for (int r = 0; r < NB; r++) {
@@ -511,24 +568,27 @@ struct Beam {
 
     // first unexplored beam entry (reference select_current_point); marks it explored
     __device__ __forceinline__ uint32_t select_parent() {
-        // entries behind the beam are pads (kInvalid), which carry the explored bit like every unfilled entry
-        int rsel = NB;
-#pragma unroll
-        for (int r = NB - 1; r >= 0; r--)
-            if ((bv[r] & kExplored) == 0) rsel = r;
-        const uint64_t m = ballot(rsel < NB);
-        if (m == 0) return kInvalid;
-        const int src = __builtin_ctzll(m);
-        const int r_src = __builtin_amdgcn_readlane(rsel, src);
-        uint32_t mine = 0;
+        // Entries behind the beam are pads (kInvalid), which carry the explored bit like every unfilled entry.  One compare
+        // per register; the rest is scalar, and the chosen entry is read by its lane number and marked under a one-lane mask.
+        uint64_t open[NB], any = 0;
 #pragma unroll
         for (int r = 0; r < NB; r++) {
-            if (r == r_src) {
-                mine = bv[r];
-                if (lane == src) bv[r] |= kExplored;
+            open[r] = ballot(static_cast<int>(bv[r]) >= 0);
+            any |= open[r];
+        }
+        if (any == 0) return kInvalid;
+        const int src = __builtin_ctzll(any);
+        uint32_t mine = 0;
+        bool taken = false;
+#pragma unroll
+        for (int r = 0; r < NB; r++) {
+            if (!taken && ((open[r] >> src) & 1) != 0) {
+                mine = read_lane(bv[r], src);
+                bv[r] = select_by_mask(bv[r], bv[r] | kExplored, 1ull << src);
+                taken = true;
             }
         }
-        return read_lane(mine, src);
+        return mine;
     }
 
     __device__ __forceinline__ void restore_hash() {
@@ -546,7 +606,7 @@ struct Beam {
         while (true) {
             absorb(iter == 0);
             cnt.iterations++;
-            const bool reset_now = ((iter + 1) % p.reset_interval) == 0;
+            const bool reset_now = count_down();
             if (reset_now) {
                 hash_clear(hash, p.hash_bit, lane);
                 wave_sync();

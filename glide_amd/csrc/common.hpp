@@ -113,20 +113,24 @@ __device__ __forceinline__ uint32_t wave_exclusive_scan(uint32_t value, uint32_t
 
 // ---------------------------------------------------------------- LDS open-addressing hash set (reference hashmap.cuh:23-56)
 __device__ __forceinline__ void hash_clear(uint32_t* table, uint32_t bitlen, int lane) {
+    if (bitlen >= 8) {   // 16 bytes a lane (the tables of the beam kernels are 16-byte aligned)
+        const uint4 none = make_uint4(kInvalid, kInvalid, kInvalid, kInvalid);
+        for (uint32_t i = lane; i < (1u << (bitlen - 2)); i += kWave) reinterpret_cast<uint4*>(table)[i] = none;
+        return;
+    }
     for (uint32_t i = lane; i < (1u << bitlen); i += kWave) table[i] = kInvalid;
 }
-// returns 1 iff `key` was newly stored; 0 if present or the table is full
+// returns 1 iff `key` was newly stored; 0 if present or the table is full (one exit, the outcome read off the last slot
+// afterwards: a loop with three outcomes costs twice the mask bookkeeping per probe)
 __device__ __forceinline__ uint32_t hash_insert(uint32_t* table, uint32_t bitlen, uint32_t key) {
     const uint32_t size = 1u << bitlen;
     const uint32_t mask = size - 1;
-    uint32_t index = (key ^ (key >> bitlen)) & mask;
-    for (uint32_t i = 0; i < size; i++) {
-        const uint32_t old = atomicCAS(&table[index], kInvalid, key);
-        if (old == kInvalid) return 1;
-        if (old == key) return 0;
+    uint32_t index = (key ^ (key >> bitlen)) & mask, left = size, old;
+    do {
+        old = atomicCAS(&table[index], kInvalid, key);
         index = (index + 1) & mask;
-    }
-    return 0;
+    } while ((old != kInvalid) & (old != key) & (--left != 0));
+    return old == kInvalid ? 1u : 0u;
 }
 
 // ---------------------------------------------------------------- row distance, several rows per wave-wide load
@@ -153,12 +157,12 @@ struct RowRegs {
 };
 
 // t = RowShape<DIMV>::lane_in_row(lane)
-template <int DIMV>
+template <int DIMV, bool FULL = false>   // FULL: dim fills the shape exactly
 __device__ __forceinline__ void load_row(RowRegs<DIMV>& r, const float* row, uint32_t dim, int t) {
 #pragma unroll
     for (int c = 0; c < RowShape<DIMV>::NV; c++) {
         const uint32_t d0 = (c * RowShape<DIMV>::LPR + t) * 4;
-        r.v[c] = d0 < dim ? *reinterpret_cast<const float4*>(row + d0) : make_float4(0.f, 0.f, 0.f, 0.f);
+        r.v[c] = FULL || d0 < dim ? *reinterpret_cast<const float4*>(row + d0) : make_float4(0.f, 0.f, 0.f, 0.f);
     }
 }
 

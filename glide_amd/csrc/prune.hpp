@@ -12,12 +12,12 @@ constexpr uint32_t kMaxDegree = 256;   // largest graph / kNN degree (reference 
 // sizes it by its degree bucket (less LDS per wavefront, more wavefronts per CU); the build kernels, whose output
 // degree is independent of the degree bucket of the kNN graph they search, keep the maximum.
 template <int MAX_BEAM, int DCAP = static_cast<int>(kMaxDegree)>
-struct PruneLds {
+struct alignas(16) PruneLds {
     static_assert(DCAP % 64 == 0 && DCAP <= static_cast<int>(kMaxDegree), "row capacity");
     static constexpr uint32_t kCap = DCAP;
     uint32_t pool_id[MAX_BEAM];
     float pool_dist[MAX_BEAM];
-    uint32_t keep[MAX_BEAM];
+    float head_sq[MAX_BEAM];   // squared distance of each entry to the latest head
     uint32_t neighbor[DCAP];
     uint32_t s_graph[DCAP];
     uint32_t fresh[DCAP];
@@ -33,14 +33,14 @@ __device__ __forceinline__ uint32_t beam_to_pool(Beam<MAX_CAND, MAX_BEAM, DIMV>&
 #pragma unroll
     for (int r = 0; r < NB; r++) {
         const uint32_t e = NB * b.lane + r;
-        pl->keep[e] = b.bv[r] & kClean;                       // reuse `keep` as staging for ids
+        pl->head_sq[e] = __uint_as_float(b.bv[r] & kClean);   // `head_sq` stages the ids
         pl->pool_dist[e] = b.bk[r];
     }
     wave_sync();
     uint32_t n = 0;
     for (uint32_t base = 0; base < b.p.beam; base += 64) {
         const uint32_t i = base + b.lane;
-        const uint32_t id = i < b.p.beam ? pl->keep[i] : kClean;
+        const uint32_t id = i < b.p.beam ? __float_as_uint(pl->head_sq[i]) : kClean;
         const float d = i < b.p.beam ? pl->pool_dist[i] : FLT_MAX;
         const bool ok = id != kClean;
         const uint64_t m = ballot(ok);
@@ -56,15 +56,15 @@ __device__ __forceinline__ uint32_t beam_to_pool(Beam<MAX_CAND, MAX_BEAM, DIMV>&
     return n;
 }
 
-// stable compaction of the pool by the keep flags of entries [first, pool_size)
+// stable compaction of the pool: entries [first, pool_size) that the latest head does not occlude
 template <int MAX_BEAM, class PL>
-__device__ __forceinline__ uint32_t compact_pool(PL* pl, uint32_t first, uint32_t pool_size, int lane) {
+__device__ __forceinline__ uint32_t compact_pool(PL* pl, uint32_t first, uint32_t pool_size, float relaxant, int metric, int lane) {
     uint32_t n = 0;
     for (uint32_t base = 0; base < pool_size; base += 64) {
         const uint32_t i = base + lane;
-        const bool ok = i >= first && i < pool_size && pl->keep[i] != 0;
         const uint32_t id = i < pool_size ? pl->pool_id[i] : 0u;
         const float d = i < pool_size ? pl->pool_dist[i] : 0.f;
+        const bool ok = i >= first && i < pool_size && !(relaxant * finish_distance(pl->head_sq[i < pool_size ? i : 0u], metric) < d);
         const uint64_t m = ballot(ok);
         wave_sync();
         if (ok) {
@@ -93,11 +93,11 @@ __device__ __forceinline__ uint32_t prune_pool(PL* pl, uint32_t pool_size, const
         RowRegs<DIMV> hrow;
         load_row<DIMV>(hrow, data + static_cast<size_t>(head) * dim, dim, RowShape<DIMV>::lane_in_row(lane));
         rows_scored += pool_size - 1;
-        score_list<DIMV>(hrow, data, dim, metric, 1, pool_size, lane,
+        score_list<DIMV>(hrow, data, dim, 1, pool_size, lane,
                          [pl, segment_start](uint32_t idx) { return pl->pool_id[idx] + segment_start; },
-                         [pl, relaxant](uint32_t idx, float d) { pl->keep[idx] = (relaxant * d < pl->pool_dist[idx]) ? 0u : 1u; });
+                         [pl](uint32_t idx, float sq) { pl->head_sq[idx] = sq; });
         wave_sync();
-        pool_size = compact_pool<MAX_BEAM>(pl, 1, pool_size, lane);
+        pool_size = compact_pool<MAX_BEAM>(pl, 1, pool_size, relaxant, metric, lane);
     }
     return nsize;
 }
@@ -130,11 +130,11 @@ __device__ __forceinline__ uint32_t prune_pool_refine(PL* pl, uint32_t pool_size
         RowRegs<DIMV> hrow;
         load_row<DIMV>(hrow, data + static_cast<size_t>(head) * dim, dim, RowShape<DIMV>::lane_in_row(lane));
         rows_scored += pool_size - position;
-        score_list<DIMV>(hrow, data, dim, metric, position, pool_size, lane,
+        score_list<DIMV>(hrow, data, dim, position, pool_size, lane,
                          [pl](uint32_t idx) { return pl->pool_id[idx]; },
-                         [pl, relaxant](uint32_t idx, float d) { pl->keep[idx] = (relaxant * d < pl->pool_dist[idx]) ? 0u : 1u; });
+                         [pl](uint32_t idx, float sq) { pl->head_sq[idx] = sq; });
         wave_sync();
-        pool_size = compact_pool<MAX_BEAM>(pl, position, pool_size, lane);
+        pool_size = compact_pool<MAX_BEAM>(pl, position, pool_size, relaxant, metric, lane);
     }
     return nsize;
 }

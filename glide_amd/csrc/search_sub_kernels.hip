@@ -39,7 +39,7 @@ __device__ __forceinline__ void merge_result(const float* beam_dist, const uint3
 
 // search_on_sub_kernel (search_kernel.cuh:653-765)
 template <int MAX_CAND, int MAX_BEAM, int DIMV, bool WHOLE = false>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MAX_BEAM > 256 && DIMV <= 4 ? 4 : 1)))   // as search_kernel
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DIMV > 4 ? 1 : MAX_BEAM > 256 ? 4 : MAX_CAND <= 64 ? 5 : 1)))   // as search_kernel
 void search_sub_kernel(SubArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     auto* lds = reinterpret_cast<BeamLds<MAX_CAND>*>(smem);
