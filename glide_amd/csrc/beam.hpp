@@ -260,30 +260,38 @@ struct Beam {
     }
 
     // Candidate sort, one network over the wavefront (reference sort_for_candidate, single-warp branch,
-    // search_kernel.cuh:9-37): strided load, sort, blocked store of every element.  `key` is the distance of this lane's
-    // slot (MAX_CAND == 64).
-    __device__ __forceinline__ void sort_candidates_one(float key) {
-        if constexpr (MAX_CAND == 64) {
-            // At most 32 slots in use: the strided load puts them on the even elements of the 64-element network and
-            // +inf on the odd ones.  Every comparator of that network then meets at most one real key, or two real
-            // keys that the 32-element network compares at the same point of its own sequence and in the same
-            // direction, so sorting the 32 slots with the 32-element network gives the same sequence, ties included
-            // (the CPU tests compare the two networks on tie-rich inputs), in 15 stages instead of 21.
-            // The one exception is a real id whose key is not below FLT_MAX (the build kernels leave the point itself
-            // unscored): among the +inf keys its place does depend on the network, so that case takes the long way.
-            if (p.degree <= 32 && ballot(cid != kInvalid && !(key < FLT_MAX)) == 0) {
-                float hk[1] = {key};
-                uint32_t hv[1] = {cid};   // the slots of the upper half of the wavefront are empty
-                WaveNet<32>::sort(hk, hv, lane);
-                lds->cand_dist[lane] = hk[0];
-                lds->cand_id[lane] = hv[0];
-                wave_sync();
-                return;
-            }
+    // search_kernel.cuh:9-37): strided load, sort, blocked store of every element.  One candidate slot per lane: `key` is
+    // the distance of this lane's slot; `as_is` leaves out the network (see absorb).  What lies behind the slots in use or
+    // behind the beam gets an infinite distance, which replaces no beam entry.
+    __device__ __forceinline__ void sort_candidates_lane(float key, bool as_is) {
+        const uint32_t limit = p.degree < p.beam ? p.degree : p.beam;
+        // At most 32 slots in use: the strided load puts them on the even elements of the 64-element network and
+        // +inf on the odd ones.  Every comparator of that network then meets at most one real key, or two real
+        // keys that the 32-element network compares at the same point of its own sequence and in the same
+        // direction, so sorting the 32 slots with the 32-element network gives the same sequence, ties included
+        // (the CPU tests compare the two networks on tie-rich inputs), in 15 stages instead of 21.
+        // The one exception is a real id whose key is not below FLT_MAX (the build kernels leave the point itself
+        // unscored): among the +inf keys its place does depend on the network, so that case takes the long way.
+        uint32_t k[1] = {__float_as_uint(key)}, v[1] = {cid};   // few slots: those of the upper half of the wavefront are empty
+        if (p.degree <= 32 && ballot(cid != kInvalid && !(key < FLT_MAX)) == 0) {
+            KeyNet<32>::sort(k, v, lane);
+        } else {
             lds->cand_dist[lane] = key;
             lds->cand_id[lane] = cid;
             wave_sync();
+            const uint32_t slot = (lane >> 1) + 32 * (lane & 1);        // reference loads strided: j = lane + 32*i
+            k[0] = __float_as_uint(lds->cand_dist[slot]);
+            v[0] = lds->cand_id[slot];
+            if (!as_is) KeyNet<64>::sort(k, v, lane);
+            wave_sync();
         }
+        lds->cand_dist[lane] = static_cast<uint32_t>(lane) < limit ? __uint_as_float(k[0]) : __builtin_inff();
+        lds->cand_id[lane] = v[0];
+        wave_sync();
+    }
+
+    // ... with two slots per lane (MAX_CAND == 128)
+    __device__ __forceinline__ void sort_candidates_one() {
         float ck[NC];
         uint32_t cv[NC];
 #pragma unroll
@@ -493,11 +501,11 @@ struct Beam {
         // The beam is ascending, so its last entry is the largest key of the lane that holds it among that lane's entries
         // below `beam` (written as a maximum: a chain of selects between the registers becomes a run-time index, which
         // moves the beam out of the registers).  Keys are not negative.
-        const uint32_t last = p.beam - 1;
         float tail;
-        if (p.beam == MAX_BEAM) {   // a beam that fills its bucket ends in the last register of the last lane
-            tail = read_lane(bk[NB - 1], 63);
+        if (p.beam % NB == 0) {   // the last entry is the last register of a lane (beams are multiples of 32 as a rule)
+            tail = read_lane(bk[NB - 1], static_cast<int>(p.beam / NB) - 1);
         } else {
+            const uint32_t last = p.beam - 1;
             float mine = bk[0];
 #pragma unroll
             for (int r = 1; r < NB; r++) mine = fmaxf(mine, NB * lane + r <= static_cast<int>(last) ? bk[r] : 0.f);
@@ -506,20 +514,94 @@ struct Beam {
         return ballot(ck < tail);
     }
 
+    // Beam merge for beams of up to 256 entries (reference sort_for_beam, single-warp branch): the k-th smallest candidate
+    // displaces entry MAX_BEAM - 1 - k if that is larger, then the merge network runs.
+    __device__ __forceinline__ void merge_beam() {
+        bool replaced = false;
+        uint32_t k[NB];
+#pragma unroll
+        for (int r = 0; r < NB; r++) k[r] = __float_as_uint(bk[r]);
+        if constexpr (NC == 1) {
+            // a lane's candidates are NB neighbouring places, in reverse; behind those that count the distance is infinite
+            struct alignas(4 * NB) Keys { float d[NB]; };
+            struct alignas(4 * NB) Ids { uint32_t id[NB]; };
+            const int from = NB * (63 - lane);
+            if (from < MAX_CAND) {
+                const Keys c = *reinterpret_cast<const Keys*>(lds->cand_dist + from);
+                const Ids ci = *reinterpret_cast<const Ids*>(lds->cand_id + from);
+#pragma unroll
+                for (int r = 0; r < NB; r++) {
+                    const uint32_t o = __float_as_uint(c.d[NB - 1 - r]);
+                    const bool smaller = o < k[r];
+                    bv[r] = smaller ? ci.id[NB - 1 - r] : bv[r];
+                    k[r] = smaller ? o : k[r];
+                    replaced |= smaller;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < NB; r++) {
+                const uint32_t e = NB * lane + r;
+                const uint32_t j = MAX_BEAM - 1 - e;
+                if (j < p.beam && j < p.degree) {
+                    const uint32_t c = __float_as_uint(lds->cand_dist[j]);
+                    if (k[r] > c) {
+                        k[r] = c;
+                        bv[r] = lds->cand_id[j];
+                        replaced = true;
+                    }
+                }
+            }
+        }
+        // Nothing replaced: the beam is still the ascending sequence the previous merge left, and the merge
+        // network (strict comparisons) is the identity on it.
+        if (ballot(replaced) == 0) return;
+        KeyNet<MAX_BEAM>::merge(k, bv, lane);
+#pragma unroll
+        for (int r = 0; r < NB; r++) bk[r] = __uint_as_float(k[r]);
+        reset_pads();
+    }
+
+    // entries pushed past the end of the beam
+    __device__ __forceinline__ void reset_pads() {
+        if (p.beam == MAX_BEAM) return;   // a beam that fills its bucket has nothing behind it (and the lane masks of this loop are not held)
+#pragma unroll
+        for (int r = 0; r < NB; r++) {
+            const uint32_t e = NB * lane + r;
+            if (e >= p.beam) {
+                bk[r] = FLT_MAX;
+                bv[r] = kInvalid;
+            }
+        }
+    }
+
     // reference update_result_buffer: sort the candidates, then fold them into the beam
     __device__ __forceinline__ void absorb(bool first) {
         // No row scored: every candidate distance is FLT_MAX, the sort would not move anything (equal keys are never
         // exchanged) and no candidate can displace a beam entry, so the beam stays as it is.
         if (!first && last_scored == 0) return;
-        if constexpr (MAX_CAND == 64) {
-            const float ck = slot_distance(0);
-            if (!first && entering(ck) == 0) return;
+        if constexpr (NC == 1) {
+            float key = slot_distance(0);
+            bool as_is = false;
+            if (first) {
+                // Rows with a NaN compare with nothing.  Beside rows that do they are dropped; when there is nothing else (a
+                // query with a NaN) all keep their slots, and no later candidate will be below any of them.
+                if (ballot(key != key) != 0) {
+                    as_is = ballot(key < FLT_MAX) == 0;
+                    if (!as_is && key != key) {
+                        key = FLT_MAX;
+                        cid = kInvalid;
+                    }
+                }
+            } else if (entering(key) == 0) {
+                return;
+            }
             wave_sync();
-            sort_candidates_one(ck);
+            sort_candidates_lane(key, as_is);
         } else {
             distances_to_slots();
             if constexpr (MAX_CAND > 128) sort_candidates_two();
-            else sort_candidates_one(0.f);
+            else sort_candidates_one();
         }
         if (first) {
 #pragma unroll
@@ -533,35 +615,7 @@ struct Beam {
             if constexpr (WHOLE) merge_beam_full();
             else merge_beam_general();
         } else {
-            bool replaced = false;
-#pragma unroll
-            for (int r = 0; r < NB; r++) {
-                const uint32_t e = NB * lane + r;
-                const uint32_t k = MAX_BEAM - 1 - e;
-                if (k < p.beam && k < p.degree) {
-                    const float c = lds->cand_dist[k];
-                    if (bk[r] > c) {
-                        bk[r] = c;
-                        bv[r] = lds->cand_id[k];
-                        replaced = true;
-                    }
-                }
-            }
-            // Nothing replaced: the beam is still the ascending sequence the previous merge left, and the merge
-            // network (strict comparisons) is the identity on it.
-            if (ballot(replaced) != 0) {
-                WaveNet<MAX_BEAM>::merge(bk, bv, lane);
-                if (p.beam < MAX_BEAM) {   // a beam that fills its bucket has nothing behind it (and the lane masks of this loop are not held)
-#pragma unroll
-                    for (int r = 0; r < NB; r++) {
-                        const uint32_t e = NB * lane + r;
-                        if (e >= p.beam) {
-                            bk[r] = FLT_MAX;
-                            bv[r] = kInvalid;
-                        }
-                    }
-                }
-            }
+            merge_beam();
         }
         wave_sync();
     }
@@ -655,21 +709,21 @@ __device__ __forceinline__ uint32_t nearest_centroid(const RowRegs<DIMV>& q, con
         if (t == 0 && c < centroid_num) cent_dist[c] = d;
     }
     wave_sync_in<TEAM>();
-    constexpr int NR = WaveNet<MAX_CENTROID>::NR;
+    constexpr int NR = KeyNet<MAX_CENTROID>::NR;
     constexpr int N32 = MAX_CENTROID / 32;
-    float k[NR];
-    uint32_t v[NR];
+    uint32_t k[NR], v[NR];
 #pragma unroll
     for (int r = 0; r < NR; r++) {
         const uint32_t e = NR * lane + r;
         const uint32_t j = (e / N32) + 32 * (e % N32);
         const bool ok = (MAX_CENTROID >= 64 || lane < 32) && j < centroid_num;
-        k[r] = ok ? cent_dist[j] : FLT_MAX;
+        k[r] = __float_as_uint(ok ? cent_dist[j] : FLT_MAX);
         v[r] = ok ? j : kInvalid;
     }
-    WaveNet<MAX_CENTROID>::sort(k, v, lane);
+    KeyNet<MAX_CENTROID>::sort(k, v, lane);
     wave_sync_in<TEAM>();
-    return read_lane(v[0], 0);
+    const uint32_t nearest = read_lane(v[0], 0);
+    return nearest == kInvalid ? 0u : nearest;   // nothing below the padding: a query with a NaN
 }
 
 }  // namespace glide

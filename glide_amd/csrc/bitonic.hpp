@@ -92,4 +92,92 @@ struct WaveNet {
     static __device__ __forceinline__ void merge(float (&k)[NR], uint32_t (&v)[NR], int lane) { merge_from<M, M / 2>(k, v, lane); }
 };
 
+// The same networks with one register per element index e = NR * lane + r, for keys that order as unsigned integers (the
+// bits of a non-negative float do).  A compare-exchange across lanes is then a median: the lower partner keeps
+// med3(mine, other, 0), the upper one med3(mine, other, ~0), and the value follows if and only if the key changed --
+// equal keys stay, as in WaveNet.  That is five vector instructions a (key, value) pair (three where the exchange itself
+// runs in the LDS crossbar) instead of six to eight, no scalar ones instead of four, and no lane masks: the constants
+// of WaveNet's masks filled the scalar registers of the beam kernels, which spilled two hundred of them.  The four-lane
+// exchange, two masked DPP moves a register, goes through the crossbar as well, which these kernels leave idle.
+// Descending blocks are sorted ascending on complemented keys.  A lane's constants (one bit of its number, spread over a
+// register) are made where they are used, from a lane number the compiler cannot see through: seven of them held in
+// registers throughout a beam search would cost a wavefront per SIMD.
+template <int M>
+struct KeyNet {
+    static_assert(M >= 32 && M <= 256, "network size");
+    static constexpr int NR = M <= 64 ? 1 : M / 64;
+
+    static __device__ __forceinline__ int opaque(int lane) {
+        asm volatile("" : "+v"(lane));
+        return lane;
+    }
+    // ~0 in the lanes whose number has bit `bit` set, else 0
+    static __device__ __forceinline__ uint32_t lane_bit(int lane, int bit) { return static_cast<uint32_t>((lane << (31 - bit)) >> 31); }
+    static constexpr int log2_of(int x) { return x <= 1 ? 0 : 1 + log2_of(x / 2); }
+    template <int LM>
+    static __device__ __forceinline__ uint32_t partner(uint32_t x) {
+        if constexpr (LM == 4) return static_cast<uint32_t>(__builtin_amdgcn_ds_swizzle(static_cast<int>(x), 0x101F));   // and 0x1f, xor 4
+        else return lane_xor<LM>(x);
+    }
+    static __device__ __forceinline__ uint32_t med3(uint32_t a, uint32_t b, uint32_t c) {
+        const uint32_t lo = a < b ? a : b, hi = a < b ? b : a;
+        const uint32_t h = hi < c ? hi : c;
+        return lo > h ? lo : h;
+    }
+    template <int LM>
+    static __device__ __forceinline__ void exchange(uint32_t& k, uint32_t& v, uint32_t keeps_max) {
+        const uint32_t nk = med3(k, partner<LM>(k), keeps_max), ov = partner<LM>(v);
+        v = nk != k ? ov : v;
+        k = nk;
+    }
+    // stages J, J/2, .. 1, all ascending
+    template <int J>
+    static __device__ __forceinline__ void merge_from(uint32_t (&k)[NR], uint32_t (&v)[NR], int lane) {
+        if constexpr (J < NR) {
+#pragma unroll
+            for (int r = 0; r < NR; r++) {
+                if ((r & J) == 0) {
+                    const uint32_t a = k[r], b = k[r | J], va = v[r], vb = v[r | J];
+                    k[r] = a < b ? a : b;
+                    k[r | J] = a < b ? b : a;
+                    const bool moved = k[r] != a;
+                    v[r] = moved ? vb : va;
+                    v[r | J] = moved ? va : vb;
+                }
+            }
+        } else {
+            const uint32_t keeps_max = lane_bit(lane, log2_of(J / NR));
+#pragma unroll
+            for (int r = 0; r < NR; r++) exchange<J / NR>(k[r], v[r], keeps_max);
+        }
+        if constexpr (J > 1) merge_from<J / 2>(k, v, lane);
+    }
+    // final ascending merge of a bitonic sequence
+    static __device__ __forceinline__ void merge(uint32_t (&k)[NR], uint32_t (&v)[NR], int lane) { merge_from<M / 2>(k, v, opaque(lane)); }
+
+    // complements the keys of the descending blocks of level K (elements with bit K)
+    template <int K>
+    static __device__ __forceinline__ void turn(uint32_t (&k)[NR], int lane) {
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            if constexpr (K < NR) {
+                if (r & K) k[r] = ~k[r];
+            } else {
+                k[r] ^= lane_bit(lane, log2_of(K / NR));
+            }
+        }
+    }
+    template <int K>
+    static __device__ __forceinline__ void sort_from(uint32_t (&k)[NR], uint32_t (&v)[NR], int lane) {
+        if constexpr (K < M) turn<K>(k, lane);
+        merge_from<K / 2>(k, v, lane);
+        if constexpr (K < M) {
+            turn<K>(k, lane);
+            sort_from<K * 2>(k, v, lane);
+        }
+    }
+    // full ascending sort; M == 32 uses the two 32-lane halves of the wavefront as two networks
+    static __device__ __forceinline__ void sort(uint32_t (&k)[NR], uint32_t (&v)[NR], int lane) { sort_from<2>(k, v, opaque(lane)); }
+};
+
 }  // namespace glide

@@ -60,7 +60,21 @@ __global__ __launch_bounds__(64) void bitonic_kernel(float* keys, uint32_t* vals
         k[r] = live ? keys[static_cast<size_t>(b) * M + e] : FLT_MAX;
         v[r] = live ? vals[static_cast<size_t>(b) * M + e] : kInvalid;
     }
-    if (MERGE_ONLY) {
+    // keys that order like their bits take the networks the beam kernels run
+    bool plain = M <= 256;
+#pragma unroll
+    for (int r = 0; r < NR; r++) plain &= __float_as_uint(k[r]) <= 0x7f800000u;
+    if (ballot(!plain) == 0) {
+        if constexpr (M <= 256) {
+            uint32_t u[NR];
+#pragma unroll
+            for (int r = 0; r < NR; r++) u[r] = __float_as_uint(k[r]);
+            if (MERGE_ONLY) KeyNet<M>::merge(u, v, lane);
+            else KeyNet<M>::sort(u, v, lane);
+#pragma unroll
+            for (int r = 0; r < NR; r++) k[r] = __uint_as_float(u[r]);
+        }
+    } else if (MERGE_ONLY) {
         WaveNet<M>::merge(k, v, lane);
     } else {
         WaveNet<M>::sort(k, v, lane);
