@@ -160,6 +160,7 @@ struct Beam {
     int lane;
     uint32_t last_scored;   // rows scored by the latest expansion (wave-uniform)
     uint32_t until_reset;   // iterations left until the visited set is reset (a countdown: a remainder by a run-time divisor is two dozen instructions)
+    bool tied;              // some beam entries have equal keys (MAX_CAND == 64)
     uint32_t cid;           // candidate id of this lane's slot (MAX_CAND == 64; larger buckets keep the ids in LDS)
     uint32_t place[NC];     // where in vlist each of this lane's slots is; kInvalid: not scored
 
@@ -575,6 +576,90 @@ struct Beam {
         }
     }
 
+    // ---- few candidates below the last beam entry --------------------------------------------------------------------
+    // Where all keys involved are distinct there is one ascending order, whatever network makes it.  Then up to kInsertMost
+    // candidates are inserted one by one: with the beam ascending, entry e becomes the median of entry e - 1, the candidate
+    // and itself.  That is 4 NB + 5 vector instructions a candidate, and no LDS, against the candidate sort (70) and the
+    // beam merge (27 / 55 / 116 for NB = 1 / 2 / 4) of the general way.  Where keys are equal the networks decide the order
+    // (the reference's comparators), so an equal pair within the beam (`tied`, kept since the last merge: insertions make
+    // none) or with a candidate sends the expansion there.  Integer rows meet equal distances often in wide beams, float
+    // rows next to never.
+    static constexpr uint32_t kInsertMost = 8;
+    // Up to kRankMost candidates that differ from each other are ranked by counting (4 instructions each), more are sorted.
+    static constexpr uint32_t kRankMost = 14;
+
+    // whether two beam entries have equal keys, or an entry orders like the padding without being padding
+    __device__ __forceinline__ bool has_ties() const {
+        uint64_t any = 0;
+        const uint32_t pad = __float_as_uint(FLT_MAX);
+#pragma unroll
+        for (int r = 0; r < NB; r++) {
+            const uint32_t k = __float_as_uint(bk[r]);
+            const uint32_t next = r + 1 < NB ? __float_as_uint(bk[r + 1 < NB ? r + 1 : 0])
+                                             : static_cast<uint32_t>(__builtin_amdgcn_update_dpp(-1, static_cast<int>(__float_as_uint(bk[0])), 0x130, 0xf, 0xf, false));   // wave_shl:1
+            const uint64_t real = ballot(k < pad);
+            any |= (ballot(k == next) & real) | (ballot(bv[r] != kInvalid) & ~real);
+        }
+        return any != 0;
+    }
+    __device__ __forceinline__ bool meets_equal(float key, uint64_t em) const {
+        uint64_t equal = 0;
+        for (uint64_t rest = em; rest; rest &= rest - 1) {
+            const int j = __builtin_ctzll(rest);
+            const float c = read_lane(key, j);
+            equal |= ballot(key == c) & (rest & (rest - 1));   // a later candidate with this key
+#pragma unroll
+            for (int r = 0; r < NB; r++) equal |= ballot(bk[r] == c);
+        }
+        return equal != 0;
+    }
+    // the value one lane below (lane 0: zero)
+    template <class T>
+    static __device__ __forceinline__ T lane_below(T x) {
+        return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x138, 0xf, 0xf, true));   // wave_shr:1
+    }
+    __device__ __forceinline__ void insert(float key, uint64_t em) {
+        for (uint64_t rest = em; rest; rest &= rest - 1) {
+            const int j = __builtin_ctzll(rest);
+            const float c = read_lane(key, j);
+            const uint32_t id = read_lane(cid, j);
+            const float pk = lane_below(bk[NB - 1]);
+            const uint32_t pv = lane_below(bv[NB - 1]);
+            uint64_t below[NB];   // lanes whose entry r comes behind the candidate
+#pragma unroll
+            for (int r = 0; r < NB; r++) below[r] = ballot(c < bk[r]);
+            const uint64_t below_first = below[NB - 1] << 1;   // ... whose entry -1, the last one of the lane below, does
+#pragma unroll
+            for (int r = NB - 1; r >= 0; r--) {
+                const float prev_k = r ? bk[r ? r - 1 : 0] : pk;
+                const uint32_t prev_v = r ? bv[r ? r - 1 : 0] : pv;
+                const uint64_t prev_below = r ? below[r ? r - 1 : 0] : below_first;
+                bk[r] = __builtin_amdgcn_fmed3f(prev_k, c, bk[r]);
+                bv[r] = select_by_mask(bv[r], select_by_mask(id, prev_v, prev_below), below[r]);
+            }
+        }
+        reset_pads();
+    }
+    // The entering candidates in ascending order at the front of the candidate lists; false if two have the same key.
+    __device__ __forceinline__ bool rank_candidates(float key, uint64_t em) {
+        uint32_t rank = 0;
+        uint64_t equal = 0;
+        for (uint64_t rest = em; rest; rest &= rest - 1) {
+            const float c = read_lane(key, __builtin_ctzll(rest));
+            equal |= ballot(key == c) & (rest & (rest - 1));
+            rank += c < key ? 1u : 0u;
+        }
+        if (equal != 0) return false;
+        lds->cand_dist[lane] = __builtin_inff();
+        wave_sync();
+        if (((em >> lane) & 1) != 0 && rank < p.beam) {
+            lds->cand_dist[rank] = key;
+            lds->cand_id[rank] = cid;
+        }
+        wave_sync();
+        return true;
+    }
+
     // reference update_result_buffer: sort the candidates, then fold them into the beam
     __device__ __forceinline__ void absorb(bool first) {
         // No row scored: every candidate distance is FLT_MAX, the sort would not move anything (equal keys are never
@@ -593,11 +678,19 @@ struct Beam {
                         cid = kInvalid;
                     }
                 }
-            } else if (entering(key) == 0) {
-                return;
+                wave_sync();
+                sort_candidates_lane(key, as_is);
+            } else {
+                const uint64_t em = entering(key);
+                if (em == 0) return;
+                const uint32_t m = __popcll(em);
+                if (m <= kInsertMost && !tied && !meets_equal(key, em)) {
+                    insert(key, em);
+                    return;
+                }
+                wave_sync();
+                if (m > kRankMost || !rank_candidates(key, em)) sort_candidates_lane(key, false);
             }
-            wave_sync();
-            sort_candidates_lane(key, as_is);
         } else {
             distances_to_slots();
             if constexpr (MAX_CAND > 128) sort_candidates_two();
@@ -618,6 +711,7 @@ struct Beam {
             merge_beam();
         }
         wave_sync();
+        if constexpr (NC == 1) tied = has_ties();
     }
 
     // first unexplored beam entry (reference select_current_point); marks it explored
