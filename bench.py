@@ -113,8 +113,6 @@ def search_kernel_name(dim, degree, beam, queries, compute_units):
     whole = "true" if beam == 512 else "false"      # the whole of the widest beam: merged in the registers
     if dim > 256 and queries * 4 <= 2 * 4 * compute_units:
         return "search_team_kernel<%s,%s>" % (shape, whole)
-    if 128 < beam <= 256 and degree <= 128 and dim <= 512:
-        return "search_kernel_dense<%s>" % shape
     return "search_kernel<%s,%s>" % (shape, whole)
 
 

@@ -169,6 +169,7 @@ struct Beam {
         hash = hash_;
         p = p_;
         lane = lane_id();
+        asm volatile("" : "+v"(lane));   // as in run: nothing made from it is to be kept from one query to the next
         load_row<DIMV>(q, query, p.dim, RowShape<DIMV>::lane_in_row(lane));
         until_reset = p.reset_interval;
         hash_clear(hash, p.hash_bit, lane);
@@ -752,6 +753,7 @@ struct Beam {
         uint32_t iter = 0;
         bool terminate = false;
         while (true) {
+            asm volatile("" : "+v"(lane));   // a dozen addresses and masks made from the lane number are cheaper made anew in an iteration than held (and spilled) across it
             absorb(iter == 0);
             cnt.iterations++;
             const bool reset_now = count_down();

@@ -4,10 +4,10 @@
 
 namespace glide {
 
-// Up to 64 slots and beams of up to 128 on rows of up to 512 dims, here and in refine_kernel: held to six wavefronts per
-// SIMD (80 registers where the kernels would take 86-89, up to eight of them spilled outside the beam loop).
+// Up to 64 slots on rows of up to 512 dims, here and in refine_kernel: six wavefronts per SIMD (80 registers; beams up to
+// 128 need no more anyway, beam 256 would take up to 84), five above beam 256 (96).
 template <int MAX_CAND, int MAX_BEAM, int DIMV>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MAX_CAND <= 64 && MAX_BEAM <= 128 && DIMV <= 4 ? 6 : 1))) void build_kernel(BuildArgs a) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DIMV > 4 || MAX_CAND > 64 ? 1 : MAX_BEAM > 256 ? 5 : 6))) void build_kernel(BuildArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     auto* lds = reinterpret_cast<BeamLds<MAX_CAND>*>(smem);
     auto* pl = reinterpret_cast<PruneLds<MAX_BEAM>*>(smem + sizeof(BeamLds<MAX_CAND>));
@@ -77,7 +77,7 @@ __device__ __forceinline__ uint32_t pick_centroid_refine(uint32_t max_centroid, 
 // Rows are read from graph_in and written to graph_out (every row is written: copied, with its empty slots
 // filled).  The reference refines in place while other blocks still traverse the rows.
 template <int MAX_CAND, int MAX_BEAM, int DIMV>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MAX_CAND <= 64 && MAX_BEAM <= 128 && DIMV <= 4 ? 6 : 1))) void refine_kernel(RefineArgs a) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DIMV > 4 || MAX_CAND > 64 ? 1 : MAX_BEAM > 256 ? 5 : 6))) void refine_kernel(RefineArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     auto* lds = reinterpret_cast<BeamLds<MAX_CAND>*>(smem);
     using Prune = PruneLds<MAX_BEAM, (MAX_CAND < 64 ? 64 : MAX_CAND)>;   // the row has at most MAX_CAND slots here

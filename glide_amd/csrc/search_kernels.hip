@@ -44,22 +44,19 @@ __device__ __forceinline__ void search_body(const SearchArgs a) {
     }
 }
 
-// Beams above 256 on rows of up to 512 dims: held to the registers of four wavefronts per SIMD (the kernel asks for a
-// dozen more, which costs it the fourth wavefront and buys nothing: the vector ALU is the limit).
-// Narrower beams over up to 64 slots: five wavefronts per SIMD (96 registers, where the kernel would take 101).  These
-// searches wait for their gathers, and a wavefront more is worth it: 10 000 queries at beam 64 on a million 128-dim rows
-// 1.66 ms with four, 1.35 with five.
+// Rows of up to 512 dims and up to 64 slots: six wavefronts per SIMD (80 registers; beams up to 128 need no more anyway,
+// beam 256 would take 84), above beam 256 five (96 of 97).  These searches wait for their gathers and their own dependent
+// steps, and a wavefront more is worth it.  Wider buckets hold several slots a lane and keep the bounds they were measured at.
+template <int MAX_CAND, int MAX_BEAM, int DIMV>
+constexpr int search_waves() {
+    if (DIMV > 4) return 1;
+    if (MAX_CAND <= 64) return MAX_BEAM > 256 ? 5 : 6;
+    return MAX_BEAM > 256 ? 4 : MAX_BEAM == 256 && MAX_CAND <= 128 ? 5 : 1;
+}
 template <int MAX_CAND, int MAX_BEAM, int DIMV, bool WHOLE = false>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DIMV > 4 ? 1 : MAX_BEAM > 256 ? 4 : MAX_CAND <= 64 ? 5 : 1)))
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(search_waves<MAX_CAND, MAX_BEAM, DIMV>())))
 void search_kernel(SearchArgs a) {
     search_body<MAX_CAND, MAX_BEAM, DIMV, WHOLE>(a);
-}
-// The beam-256 kernels are bound by the vector ALU (sorting networks) and need 103 registers, one wavefront per SIMD
-// short of the next occupancy step: held to five wavefronts per SIMD (96 registers, five of them spilled) they run
-// 5 % faster.  Other beams are either already there or would spill much more.
-template <int MAX_CAND, int MAX_BEAM, int DIMV>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 5))) void search_kernel_dense(SearchArgs a) {
-    search_body<MAX_CAND, MAX_BEAM, DIMV>(a);
 }
 
 // Small batches of long rows (more than 256 dims): a team of kTeam wavefronts per query.  Wavefront 0 owns the search
@@ -136,11 +133,6 @@ __global__ __launch_bounds__(64 * kTeam) void search_team_kernel(SearchArgs a) {
 
 template <int MAX_CAND, int MAX_BEAM, bool WHOLE = false>
 search_fn pick_dim(uint32_t dim) {
-    if constexpr (MAX_BEAM == 256 && MAX_CAND <= 128) {
-        if (dim <= 128) return search_kernel_dense<MAX_CAND, MAX_BEAM, 1>;
-        if (dim <= 256) return search_kernel_dense<MAX_CAND, MAX_BEAM, 2>;
-        if (dim <= 512) return search_kernel_dense<MAX_CAND, MAX_BEAM, 4>;
-    }
     if (dim <= 128) return search_kernel<MAX_CAND, MAX_BEAM, 1, WHOLE>;
     if (dim <= 256) return search_kernel<MAX_CAND, MAX_BEAM, 2, WHOLE>;
     if (dim <= 512) return search_kernel<MAX_CAND, MAX_BEAM, 4, WHOLE>;
