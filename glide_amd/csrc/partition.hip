@@ -653,17 +653,12 @@ __device__ __forceinline__ uint32_t wave_locate(Load load, uint32_t len, double 
     return static_cast<uint32_t>(__shfl(static_cast<int>(last), src));
 }
 
-// one workgroup of 16 wavefronts: chunk sums of min_dist, then wavefront j draws candidate j
-__global__ __launch_bounds__(1024) void kmeanspp_pick_kernel(uint32_t n, const float* min_dist, uint32_t seed, uint32_t step, uint32_t trials,
-                                                            uint32_t* candidates) {
-    __shared__ double part[1024];
+// one workgroup of 16 wavefronts: chunk sums of min_dist (in global memory or LDS), then wavefront j draws candidate j
+__device__ __forceinline__ void draw_candidates(double* part, uint32_t n, const float* min_dist, uint32_t seed, uint32_t step, uint32_t trials,
+                                                uint32_t* candidates) {
     const uint32_t t = threadIdx.x;
     const int lane = lane_id();
     const uint32_t wave = t >> 6;
-    if (step == 0) {
-        if (t < trials) candidates[t] = seed_hash(seed, 0) % n;
-        return;
-    }
     const uint32_t chunk = (n + 1023) / 1024;
     {
         const uint32_t lo = t * chunk < n ? t * chunk : n, hi = lo + chunk < n ? lo + chunk : n;
@@ -689,74 +684,141 @@ __global__ __launch_bounds__(1024) void kmeanspp_pick_kernel(uint32_t n, const f
     }
     if (lane == 0) candidates[wave] = cand;
 }
+__global__ __launch_bounds__(1024) void kmeanspp_pick_kernel(uint32_t n, const float* min_dist, uint32_t seed, uint32_t step, uint32_t trials,
+                                                            uint32_t* candidates) {
+    __shared__ double part[1024];
+    if (step == 0) {
+        if (threadIdx.x < trials) candidates[threadIdx.x] = seed_hash(seed, 0) % n;
+        return;
+    }
+    draw_candidates(part, n, min_dist, seed, step, trials, candidates);
+}
 
-// 64 sample rows per workgroup, 16 per wavefront: potential of every candidate over these rows, in double
-__global__ __launch_bounds__(256) void kmeanspp_trial_kernel(const float* sample, uint32_t n, uint32_t dim, const float* min_dist,
-                                                             const uint32_t* candidates, uint32_t trials, double* partial) {
-    __shared__ double wave_pot[4][kSeedTrials];
-    const int lane = lane_id();
-    const uint32_t wave = threadIdx.x >> 6;
-    double pot[kSeedTrials];
+// 64 sample rows per workgroup, LANES lanes a row: squared distance of every row to every candidate (kept for the next
+// kernel, which lowers min_dist by the winner's) and the candidates' potentials over these rows, in double, summed row after
+// row in four runs of 16 whatever the layout.  Rows of up to 128 dims take half a wavefront and four rows a group, with the
+// candidates in registers: the kernel is a few memory round trips long, so what counts is to have them all under way at once
+// (20 000 rows of 128 dims, 7 candidates: 30 us with one wavefront going through 16 rows).
+constexpr uint32_t kTrialThreads = 512;
+template <int LANES>
+__global__ __launch_bounds__(kTrialThreads) void kmeanspp_trial_kernel(const float* sample, uint32_t n, uint32_t dim, const float* min_dist,
+                                                                      const uint32_t* candidates, uint32_t trials, double* partial, float* trial_dist) {
+    static_assert(kSeedPoints * kSeedTrials == kTrialThreads, "one distance a thread");
+    constexpr uint32_t kGroups = kTrialThreads / LANES, kRows = kSeedPoints / kGroups;
+    __shared__ float dist[kSeedTrials][kSeedPoints];
+    __shared__ double run_pot[4][kSeedTrials];
+    const uint32_t group = threadIdx.x / LANES, t = threadIdx.x % LANES, first = blockIdx.x * kSeedPoints;
+    if constexpr (LANES == 32) {
+        const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+        const bool in = t * 4 < dim;
+        float4 c[kSeedTrials], x[kRows];
 #pragma unroll
-    for (uint32_t j = 0; j < kSeedTrials; j++) pot[j] = 0.0;
-    for (uint32_t r = 0; r < kSeedPoints / 4; r++) {
-        const uint32_t i = blockIdx.x * kSeedPoints + wave * (kSeedPoints / 4) + r;
-        if (i >= n) break;
-        const float* x = sample + static_cast<size_t>(i) * dim;
-        const float md = min_dist[i];
+        for (uint32_t r = 0; r < kRows; r++) {
+            const uint32_t i = first + group * kRows + r;
+            x[r] = in ? *reinterpret_cast<const float4*>(sample + static_cast<size_t>(i < n ? i : n - 1) * dim + t * 4) : zero;
+        }
 #pragma unroll
-        for (uint32_t j = 0; j < kSeedTrials; j++) {
-            if (j >= trials) break;
-            const float* c = sample + static_cast<size_t>(candidates[j]) * dim;
-            float acc = 0.f;
-            for (uint32_t d0 = lane * 4; d0 < dim; d0 += 256) {
-                const float4 a = *reinterpret_cast<const float4*>(x + d0);
-                const float4 b = *reinterpret_cast<const float4*>(c + d0);
-                const float dx = a.x - b.x, dy = a.y - b.y, dz = a.z - b.z, dw = a.w - b.w;
-                acc = fmaf(dx, dx, acc);
-                acc = fmaf(dy, dy, acc);
-                acc = fmaf(dz, dz, acc);
-                acc = fmaf(dw, dw, acc);
+        for (uint32_t j = 0; j < kSeedTrials; j++)
+            c[j] = in ? *reinterpret_cast<const float4*>(sample + static_cast<size_t>(candidates[j < trials ? j : 0]) * dim + t * 4) : zero;
+#pragma unroll
+        for (uint32_t r = 0; r < kRows; r++)
+#pragma unroll
+            for (uint32_t j = 0; j < kSeedTrials; j++) {
+                if (j >= trials) break;
+                const float d = half_wave_sum(sqdist4(x[r], c[j], 0.f));
+                if (t == 0) dist[j][group * kRows + r] = d;
             }
-            acc = wave_sum(acc);
-            pot[j] += static_cast<double>(fminf(md, acc));
+    } else {
+        for (uint32_t r = 0; r < kRows; r++) {
+            const uint32_t i = first + group * kRows + r;
+            const float* x = sample + static_cast<size_t>(i < n ? i : n - 1) * dim;
+            for (uint32_t j = 0; j < trials; j++) {
+                const float* c = sample + static_cast<size_t>(candidates[j]) * dim;
+                float acc = 0.f;
+                for (uint32_t d0 = t * 4; d0 < dim; d0 += 256)
+                    acc = sqdist4(*reinterpret_cast<const float4*>(x + d0), *reinterpret_cast<const float4*>(c + d0), acc);
+                acc = wave_sum(acc);
+                if (t == 0) dist[j][group * kRows + r] = acc;
+            }
         }
     }
-    if (lane == 0)
-        for (uint32_t j = 0; j < kSeedTrials; j++) wave_pot[wave][j] = pot[j];
+    __syncthreads();
+    {
+        const uint32_t j = threadIdx.x / kSeedPoints, i = first + threadIdx.x % kSeedPoints;
+        if (j < trials && i < n) trial_dist[static_cast<size_t>(j) * n + i] = dist[j][threadIdx.x % kSeedPoints];
+    }
+    if (threadIdx.x < 4 * kSeedTrials) {
+        const uint32_t run = threadIdx.x / kSeedTrials, j = threadIdx.x % kSeedTrials;
+        double pot = 0.0;
+        if (j < trials)
+            for (uint32_t r = run * 16; r < run * 16 + 16 && first + r < n; r++) pot += static_cast<double>(fminf(min_dist[first + r], dist[j][r]));
+        run_pot[run][j] = pot;
+    }
     __syncthreads();
     if (threadIdx.x < kSeedTrials)
         partial[static_cast<size_t>(blockIdx.x) * kSeedTrials + threadIdx.x] =
-            wave_pot[0][threadIdx.x] + wave_pot[1][threadIdx.x] + wave_pot[2][threadIdx.x] + wave_pot[3][threadIdx.x];
+            run_pot[0][threadIdx.x] + run_pot[1][threadIdx.x] + run_pot[2][threadIdx.x] + run_pot[3][threadIdx.x];
 }
 
-// one workgroup: potentials summed over the trial kernel's workgroups, the smallest wins (the first on a tie); its row
-// becomes centroid `step`
+// Potentials summed over the trial kernel's workgroups, the smallest wins (the first on a tie); its row becomes centroid
+// `step`.  256 threads at least; returns which candidate won, to every thread.
+__device__ __forceinline__ uint32_t choose_winner(const float* sample, uint32_t dim, const double* partial, uint32_t blocks, const uint32_t* candidates,
+                                                  uint32_t trials, uint32_t step, float* centroids, uint32_t* chosen_rows) {
+    __shared__ double slice[kSeedTrials][32];
+    __shared__ double total[kSeedTrials];
+    __shared__ uint32_t best;
+    if (threadIdx.x < 32 * kSeedTrials) {
+        const uint32_t j = threadIdx.x >> 5, sl = threadIdx.x & 31;
+        double acc = 0.0;
+        if (step > 0 && j < trials)
+            for (uint32_t b = sl; b < blocks; b += 32) acc += partial[static_cast<size_t>(b) * kSeedTrials + j];
+        slice[j][sl] = acc;
+    }
+    __syncthreads();
+    if (threadIdx.x < kSeedTrials) {
+        double p = 0.0;
+        for (uint32_t q = 0; q < 32; q++) p += slice[threadIdx.x][q];
+        total[threadIdx.x] = p;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t b = 0;
+        for (uint32_t c = 1; c < (step > 0 ? trials : 1u); c++)
+            if (total[c] < total[b]) b = c;
+        best = b;
+        if (chosen_rows) chosen_rows[step] = candidates[b];
+    }
+    __syncthreads();
+    const uint32_t won = best;
+    const float* src = sample + static_cast<size_t>(candidates[won]) * dim;
+    for (uint32_t d = threadIdx.x; d < dim; d += blockDim.x) centroids[static_cast<size_t>(step) * dim + d] = src[d];
+    return won;
+}
 __global__ __launch_bounds__(256) void kmeanspp_choose_kernel(const float* sample, uint32_t dim, const double* partial, uint32_t blocks,
                                                               const uint32_t* candidates, uint32_t trials, uint32_t step, float* centroids,
                                                               uint32_t* chosen_rows) {
-    __shared__ double slice[kSeedTrials][32];
-    __shared__ uint32_t winner;
-    const uint32_t j = threadIdx.x >> 5, sl = threadIdx.x & 31;
-    double acc = 0.0;
-    if (step > 0 && j < trials)
-        for (uint32_t b = sl; b < blocks; b += 32) acc += partial[static_cast<size_t>(b) * kSeedTrials + j];
-    slice[j][sl] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t best = 0;
-        double best_pot = 0.0;
-        for (uint32_t c = 0; c < (step > 0 ? trials : 1u); c++) {
-            double p = 0.0;
-            for (uint32_t q = 0; q < 32; q++) p += slice[c][q];
-            if (c == 0 || p < best_pot) { best_pot = p; best = c; }
-        }
-        winner = candidates[best];
-        if (chosen_rows) chosen_rows[step] = winner;
+    choose_winner(sample, dim, partial, blocks, candidates, trials, step, centroids, chosen_rows);
+}
+
+// Between two trials, in one workgroup: the winner of `step`, min_dist lowered by its distances, and the candidates of the
+// next step.  min_dist passes through LDS, which is what limits it to kSeedLdsRows rows (128 KB); a larger sample takes the
+// kernels above one after another.  20 000 rows, 256 clusters: a step was four launches and 54 us of kernels.
+constexpr uint32_t kSeedLdsRows = 32768;
+__global__ __launch_bounds__(1024) void kmeanspp_next_kernel(const float* sample, uint32_t n, uint32_t dim, const double* partial, uint32_t blocks,
+                                                             const float* trial_dist, uint32_t trials, uint32_t seed, uint32_t step, uint32_t last,
+                                                             float* min_dist, uint32_t* candidates, float* centroids, uint32_t* chosen_rows) {
+    extern __shared__ __align__(16) float md[];   // n values
+    __shared__ double part[1024];
+    const uint32_t won = choose_winner(sample, dim, partial, blocks, candidates, trials, step, centroids, chosen_rows);
+    if (last) return;
+    const float* d = trial_dist + static_cast<size_t>(won) * n;
+    for (uint32_t i = threadIdx.x; i < n; i += 1024) {
+        const float m = fminf(min_dist[i], d[i]);
+        md[i] = m;
+        min_dist[i] = m;
     }
-    __syncthreads();
-    const float* src = sample + static_cast<size_t>(winner) * dim;
-    for (uint32_t d = threadIdx.x; d < dim; d += 256) centroids[static_cast<size_t>(step) * dim + d] = src[d];
+    __syncthreads();   // every thread has read the old candidates by now
+    draw_candidates(part, n, md, seed, step + 1, trials, candidates);
 }
 
 // one wavefront per sample row: min_dist[i] = min(min_dist[i], |x_i - c|^2) (set on the first step)
@@ -833,6 +895,78 @@ __global__ __launch_bounds__(256) void kmeans_accumulate_kernel(const float* sam
         atomicAdd(reinterpret_cast<unsigned long long*>(&sums[static_cast<size_t>(bc) * dim + d]),
                   static_cast<unsigned long long>(__float2ll_rn(x[d] * scale)));   // two's complement: the wrap-around sum is the signed sum
     if (lane == 0) atomicAdd(&counts[bc], 1u);
+}
+
+// Rows of up to 128 dims: half a wavefront keeps four points and goes through the centroids once for all of them (a
+// centroid row is read by one half-wavefront in eight points' place, not by every point: 256 centroids and 20 000 points
+// were 2.6 GB of reads a step).  With few clusters the sums are hot -- every point adds to one of k x dim places -- so a
+// workgroup collects them in LDS and adds them up once; the sums are integers, the order does not matter.
+constexpr uint32_t kSumPoints = 4;             // points of a half-wavefront
+constexpr uint32_t kLdsSums = 4096;            // 32 KB of 64-bit sums
+__global__ __launch_bounds__(256) void kmeans_accumulate_narrow_kernel(const float* sample, uint32_t n, uint32_t dim, const float* centroids,
+                                                                       uint32_t k, long long* sums, uint32_t* counts, const uint32_t* max_bits,
+                                                                       uint32_t in_lds) {
+    extern __shared__ __align__(16) unsigned long long local[];   // in_lds: k x dim sums, then k counts
+    uint32_t* local_counts = reinterpret_cast<uint32_t*>(local + (in_lds ? k * dim : 0u));
+    const uint32_t t = threadIdx.x & 31, group = threadIdx.x >> 5;
+    const bool in = t * 4 < dim;
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (in_lds) {
+        for (uint32_t i = threadIdx.x; i < k * dim; i += 256) local[i] = 0;
+        for (uint32_t i = threadIdx.x; i < k; i += 256) local_counts[i] = 0;
+        __syncthreads();
+    }
+    const float scale = kmeans_scale(*max_bits, n);
+    for (uint32_t first = (blockIdx.x * 8 + group) * kSumPoints; first < n; first += gridDim.x * 8 * kSumPoints) {
+        float4 x[kSumPoints];
+        float best[kSumPoints];
+        uint32_t nearest[kSumPoints];
+#pragma unroll
+        for (uint32_t p = 0; p < kSumPoints; p++) {
+            const uint32_t i = first + p < n ? first + p : n - 1;
+            x[p] = in ? *reinterpret_cast<const float4*>(sample + static_cast<size_t>(i) * dim + t * 4) : zero;
+            best[p] = FLT_MAX;
+            nearest[p] = 0;
+        }
+        float4 next = in ? *reinterpret_cast<const float4*>(centroids + t * 4) : zero;
+        for (uint32_t c = 0; c < k; c++) {
+            const float4 row = next;
+            if (in && c + 1 < k) next = *reinterpret_cast<const float4*>(centroids + static_cast<size_t>(c + 1) * dim + t * 4);
+#pragma unroll
+            for (uint32_t p = 0; p < kSumPoints; p++) {
+                const float d = half_wave_sum(sqdist4(x[p], row, 0.f));
+                if (d < best[p]) {
+                    best[p] = d;
+                    nearest[p] = c;
+                }
+            }
+        }
+#pragma unroll
+        for (uint32_t p = 0; p < kSumPoints; p++) {
+            if (first + p >= n) break;
+            if (in) {
+                const size_t at = static_cast<size_t>(nearest[p]) * dim + t * 4;
+                const float v[4] = {x[p].x, x[p].y, x[p].z, x[p].w};
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const auto fixed = static_cast<unsigned long long>(__float2ll_rn(v[e] * scale));   // two's complement: the wrap-around sum is the signed sum
+                    if (in_lds) atomicAdd(&local[at + e], fixed);
+                    else atomicAdd(reinterpret_cast<unsigned long long*>(sums) + at + e, fixed);
+                }
+            }
+            if (t == 0) {
+                if (in_lds) atomicAdd(&local_counts[nearest[p]], 1u);
+                else atomicAdd(&counts[nearest[p]], 1u);
+            }
+        }
+    }
+    if (in_lds) {
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < k * dim; i += 256)
+            if (local[i]) atomicAdd(reinterpret_cast<unsigned long long*>(&sums[i]), local[i]);
+        for (uint32_t i = threadIdx.x; i < k; i += 256)
+            if (local_counts[i]) atomicAdd(&counts[i], local_counts[i]);
+    }
 }
 
 __global__ void kmeans_update_kernel(float* centroids, const long long* sums, const uint32_t* counts, uint32_t k, uint32_t dim, uint32_t n,
@@ -1000,7 +1134,9 @@ size_t glide_hip_kmeans_workspace_bytes(uint32_t cluster_num, uint32_t dim) {
 
 size_t glide_hip_kmeans_seed_workspace_bytes(uint32_t sample_num) {
     // min_dist (f32 per row) | candidates (8 u32) | per-workgroup potentials of the trial kernel (8 f64 each)
-    return align_up(static_cast<size_t>(sample_num) * 4, 256) + 256 + static_cast<size_t>(ceil_div(sample_num, kSeedPoints)) * kSeedTrials * 8;
+    // | distances of every row to the candidates (8 f32 per row)
+    return align_up(static_cast<size_t>(sample_num) * 4, 256) + 256 + static_cast<size_t>(ceil_div(sample_num, kSeedPoints)) * kSeedTrials * 8 +
+           static_cast<size_t>(sample_num) * kSeedTrials * 4;
 }
 
 int glide_hip_kmeans_seed(const float* sample, uint32_t sample_num, uint32_t dim, uint32_t cluster_num, uint32_t seed, float* centroids,
@@ -1016,10 +1152,23 @@ int glide_hip_kmeans_seed(const float* sample, uint32_t sample_num, uint32_t dim
     uint32_t* candidates = reinterpret_cast<uint32_t*>(w + align_up(static_cast<size_t>(sample_num) * 4, 256));
     double* partial = reinterpret_cast<double*>(w + align_up(static_cast<size_t>(sample_num) * 4, 256) + 256);
     const uint32_t trials = seed_trials(cluster_num), blocks = ceil_div(sample_num, kSeedPoints);
+    float* trial_dist = reinterpret_cast<float*>(partial + static_cast<size_t>(blocks) * kSeedTrials);
+    const bool in_lds = sample_num <= kSeedLdsRows;
+    const size_t lds = static_cast<size_t>(sample_num) * sizeof(float);
+    if (in_lds && cluster_num > 1)
+        GLIDE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&kmeanspp_next_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          static_cast<int>(lds)));
+    auto trial = dim <= 128 ? kmeanspp_trial_kernel<32> : kmeanspp_trial_kernel<64>;
     for (uint32_t step = 0; step < cluster_num; step++) {
-        hipLaunchKernelGGL(kmeanspp_pick_kernel, dim3(1), dim3(1024), 0, s, sample_num, min_dist, seed, step, trials, candidates);
+        if (step <= 1 || !in_lds)
+            hipLaunchKernelGGL(kmeanspp_pick_kernel, dim3(1), dim3(1024), 0, s, sample_num, min_dist, seed, step, trials, candidates);
         if (step > 0)
-            hipLaunchKernelGGL(kmeanspp_trial_kernel, dim3(blocks), dim3(256), 0, s, sample, sample_num, dim, min_dist, candidates, trials, partial);
+            hipLaunchKernelGGL(trial, dim3(blocks), dim3(kTrialThreads), 0, s, sample, sample_num, dim, min_dist, candidates, trials, partial, trial_dist);
+        if (step > 0 && in_lds) {
+            hipLaunchKernelGGL(kmeanspp_next_kernel, dim3(1), dim3(1024), lds, s, sample, sample_num, dim, partial, blocks, trial_dist, trials, seed, step,
+                               step + 1 == cluster_num ? 1u : 0u, min_dist, candidates, centroids, chosen_rows);
+            continue;
+        }
         hipLaunchKernelGGL(kmeanspp_choose_kernel, dim3(1), dim3(256), 0, s, sample, dim, partial, blocks, candidates, trials, step, centroids,
                            chosen_rows);
         if (step + 1 < cluster_num)
@@ -1045,11 +1194,20 @@ int glide_hip_kmeans_fit(const float* sample, uint32_t sample_num, uint32_t dim,
     const size_t values = static_cast<size_t>(sample_num) * dim;
     hipLaunchKernelGGL(kmeans_range_kernel, dim3(static_cast<uint32_t>(values / 256 < 4096 ? values / 256 + 1 : 4096)), dim3(256), 0, s, sample,
                        values, max_bits);
+    const bool narrow = dim <= 128 && reinterpret_cast<uintptr_t>(sample) % 16 == 0 && reinterpret_cast<uintptr_t>(centroids) % 16 == 0;
+    const bool in_lds = static_cast<size_t>(cluster_num) * dim <= kLdsSums;
+    // with sums in LDS every workgroup adds k x dim of them up at its end, so it takes 128 points at least
+    const uint32_t sum_blocks = ceil_div(sample_num, in_lds ? 128 : 8 * kSumPoints);
+    const size_t sum_lds = in_lds ? static_cast<size_t>(cluster_num) * dim * 8 + static_cast<size_t>(cluster_num) * 4 : 0;
     for (uint32_t it = 0; it < iterations; it++) {
         rc = glide_hip_fill_u32(reinterpret_cast<uint32_t*>(sums), 0u, words, stream);
         if (rc != GLIDE_OK) return rc;
-        hipLaunchKernelGGL(kmeans_accumulate_kernel, dim3(ceil_div(sample_num, 4)), dim3(256), 0, s, sample, sample_num, dim, centroids,
-                           cluster_num, sums, counts, max_bits);
+        if (narrow)
+            hipLaunchKernelGGL(kmeans_accumulate_narrow_kernel, dim3(sum_blocks), dim3(256), sum_lds, s, sample, sample_num, dim, centroids,
+                               cluster_num, sums, counts, max_bits, in_lds ? 1u : 0u);
+        else
+            hipLaunchKernelGGL(kmeans_accumulate_kernel, dim3(ceil_div(sample_num, 4)), dim3(256), 0, s, sample, sample_num, dim, centroids,
+                               cluster_num, sums, counts, max_bits);
         hipLaunchKernelGGL(kmeans_update_kernel, dim3(ceil_div(cluster_num * dim, 256)), dim3(256), 0, s, centroids, sums, counts,
                            cluster_num, dim, sample_num, max_bits);
     }

@@ -1,0 +1,46 @@
+"""k-means kernels at the sizes where their layouts change: rows of up to 128 dims (half a wavefront a row) and beyond,
+samples that pass through LDS while seeding (32768 rows) and one row more, sums in LDS (4096 values) and in memory, and
+samples that do not fill a workgroup.  Integer rows: every distance and every sum is exact, so the outcome is one."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def rows_of(n, dim, seed):
+    return np.random.default_rng(seed).integers(0, 16, (n, dim)).astype(np.float32)
+
+
+@pytest.mark.parametrize("n, dim, k", [(1, 4, 1), (63, 128, 3), (65, 132, 5), (1000, 256, 9), (200, 260, 4), (32768, 8, 3), (32769, 8, 3)])
+def test_seeding_rows(n, dim, k):
+    from glide_amd import capi as hip
+    from oracle import oracle as O
+    hip.set_device(0)
+    x = rows_of(n, dim, n)
+    e_cent, e_rows = O.kmeans_seed(x, k, 5)
+    cent, rows = hip.DeviceArray((k, dim), np.float32), hip.DeviceArray(k, np.uint32)
+    sb = hip.kmeans_seed_workspace_bytes(n)
+    ws = hip.DeviceArray(sb // 8 + 1, np.uint64)
+    hip.kmeans_seed(hip.DeviceArray.from_numpy(x), n, dim, k, 5, cent, ws, sb, chosen_rows=rows)
+    hip.synchronize()
+    assert np.array_equal(rows.numpy(), e_rows)
+    assert np.array_equal(cent.numpy(), e_cent)
+
+
+@pytest.mark.parametrize("n, dim, k", [(1, 4, 1), (31, 128, 32), (129, 128, 32), (300, 128, 33), (257, 100, 5), (1000, 4, 256), (900, 132, 7)])
+def test_one_lloyd_step(n, dim, k):
+    from glide_amd import capi as hip
+    hip.set_device(0)
+    x = rows_of(n, dim, 3 * n + k)
+    start = rows_of(k, dim, k)          # equal distances are common: the first centroid wins
+    cent = hip.DeviceArray.from_numpy(start)
+    wb = hip.kmeans_workspace_bytes(k, dim)
+    ws = hip.DeviceArray(wb // 8 + 1, np.uint64)
+    hip.kmeans_fit(hip.DeviceArray.from_numpy(x), n, dim, k, 1, cent, ws, wb)
+    hip.synchronize()
+    nearest = ((x[:, None].astype(np.float64) - start[None]) ** 2).sum(-1).argmin(1)
+    expect = start.copy()
+    for c in range(k):
+        if (nearest == c).any():
+            expect[c] = (x[nearest == c].sum(0, dtype=np.float64) / (nearest == c).sum()).astype(np.float32)
+    assert np.array_equal(cent.numpy(), expect)
