@@ -366,7 +366,11 @@ class GLIDE:
         if d_query.shape[1] != self.dim():
             raise ValueError("queries of %d values for points of %d" % (d_query.shape[1], self.dim()))
         nq = d_query.shape[0]
-        d_ids, d_dists = out if out is not None else (capi.DeviceArray((nq, param.top_k), np.uint32), capi.DeviceArray((nq, param.top_k), np.float32))
+        if out is not None:
+            d_ids, d_dists = out
+        else:      # ids and distances in one allocation: one to make and free, and one copy back
+            d_both = capi.DeviceArray((2, nq, param.top_k), np.uint32)
+            d_ids, d_dists = d_both.ptr, d_both.ptr + d_both.nbytes // 2
         with _Timer() as t:
             capi.search(self.d_data, self.num(), self.dim(), self.d_graph, self._graph_degree, self.d_centroids, self.centroid_num(),
                         self.d_start_points, d_query, nq, param.top_k, param.beam, param.max_iterations, param.min_iterations,
@@ -376,4 +380,5 @@ class GLIDE:
             result["QPS"] = nq / t.seconds if t.seconds > 0 else float("inf")
         if out is not None:
             return None
-        return d_ids.numpy(), d_dists.numpy()
+        both = d_both.numpy()
+        return both[0], both[1].view(np.float32)
