@@ -19,7 +19,7 @@ struct alignas(16) PruneLds {
     float pool_dist[MAX_BEAM];
     float head_sq[MAX_BEAM];   // squared distance of each entry to the latest head
     uint32_t neighbor[DCAP];
-    uint32_t s_graph[DCAP];
+    alignas(16) uint32_t s_graph[DCAP];
     uint32_t fresh[DCAP];
     uint32_t dup_mask[DCAP / 32];
 };
@@ -108,19 +108,25 @@ __device__ __forceinline__ uint32_t prune_pool_refine(PL* pl, uint32_t pool_size
                                                       uint32_t self, uint32_t graph_degree, uint32_t need, float relaxant,
                                                       int metric, int lane, uint32_t& rows_scored) {
     for (uint32_t i = lane; i < PL::kCap; i += 64) pl->neighbor[i] = kInvalid;
+    // Which entries are admissible does not change while the pool shrinks: settled once, the others marked in the top bit of
+    // their id (ids are below 2^31), which moves with them.
+    for (uint32_t base = 0; base < pool_size; base += 64) {
+        const uint32_t i = base + lane;
+        const uint32_t id = i < pool_size ? pl->pool_id[i] : self;
+        bool bad = id == self;
+        for (uint32_t j = 0; j < PL::kCap && j < graph_degree; j += 4) {   // slots behind the row are empty
+            const uint4 g = *reinterpret_cast<const uint4*>(pl->s_graph + j);
+            bad |= (g.x == id) | (g.y == id) | (g.z == id) | (g.w == id);
+        }
+        if (bad && i < pool_size) pl->pool_id[i] = id | kExplored;
+    }
     wave_sync();
     uint32_t nsize = 0;
     while (nsize < need && pool_size > 0) {
         uint32_t position = kInvalid;  // select_point: first admissible pool entry
         for (uint32_t base = 0; base < pool_size && position == kInvalid; base += 64) {
             const uint32_t i = base + lane;
-            bool ok = false;
-            if (i < pool_size) {
-                const uint32_t id = pl->pool_id[i];
-                ok = id != kInvalid && id != self;
-                for (uint32_t j = 0; ok && j < graph_degree; j++) ok = pl->s_graph[j] != id;
-            }
-            const uint64_t m = ballot(ok);
+            const uint64_t m = ballot(i < pool_size && (pl->pool_id[i < pool_size ? i : 0u] & kExplored) == 0);
             if (m) position = base + __builtin_ctzll(m);
         }
         if (position == kInvalid) break;
@@ -131,7 +137,7 @@ __device__ __forceinline__ uint32_t prune_pool_refine(PL* pl, uint32_t pool_size
         load_row<DIMV>(hrow, data + static_cast<size_t>(head) * dim, dim, RowShape<DIMV>::lane_in_row(lane));
         rows_scored += pool_size - position;
         score_list<DIMV>(hrow, data, dim, position, pool_size, lane,
-                         [pl](uint32_t idx) { return pl->pool_id[idx]; },
+                         [pl](uint32_t idx) { return pl->pool_id[idx] & kClean; },
                          [pl](uint32_t idx, float sq) { pl->head_sq[idx] = sq; });
         wave_sync();
         pool_size = compact_pool<MAX_BEAM>(pl, position, pool_size, relaxant, metric, lane);
