@@ -161,6 +161,8 @@ struct Beam {
     uint32_t last_scored;   // rows scored by the latest expansion (wave-uniform)
     uint32_t until_reset;   // iterations left until the visited set is reset (a countdown: a remainder by a run-time divisor is two dozen instructions)
     bool tied;              // some beam entries have equal keys (MAX_CAND == 64)
+    bool beyond;            // some beam entries are rows whose key is not below the padding's: infinite, or the unscored point of a build (MAX_CAND == 64)
+    bool unordered;         // the beam holds rows that compare with nothing, and no others (see absorb)
     uint32_t cid;           // candidate id of this lane's slot (MAX_CAND == 64; larger buckets keep the ids in LDS)
     uint32_t place[NC];     // where in vlist each of this lane's slots is; kInvalid: not scored
 
@@ -172,6 +174,7 @@ struct Beam {
         asm volatile("" : "+v"(lane));   // as in run: nothing made from it is to be kept from one query to the next
         load_row<DIMV>(q, query, p.dim, RowShape<DIMV>::lane_in_row(lane));
         until_reset = p.reset_interval;
+        unordered = false;
         hash_clear(hash, p.hash_bit, lane);
         wave_sync();
     }
@@ -250,15 +253,27 @@ struct Beam {
         const float d = finish_distance(lds->cand_dist[place[i] & (MAX_CAND - 1)], p.metric);
         return place[i] != kInvalid ? d : FLT_MAX;
     }
-    // Buckets of more than 64 slots: from the order of vlist to the slots.
-    __device__ __forceinline__ void distances_to_slots() {
+    // Buckets of more than 64 slots: from the order of vlist to the slots.  Slots that are not candidates (see absorb) become
+    // empty; returns false if the expansion leaves the beam as it is.
+    __device__ __forceinline__ bool distances_to_slots(bool& fresh) {
         float d[NC];
+        uint64_t some = 0, nans = 0;
 #pragma unroll
-        for (int i = 0; i < NC; i++) d[i] = slot_distance(i);
+        for (int i = 0; i < NC; i++) {
+            d[i] = slot_distance(i);
+            some |= ballot(d[i] < FLT_MAX);
+            nans |= ballot(d[i] != d[i]);
+        }
+        if (!admit(fresh, some != 0, nans != 0)) return false;
         wave_sync();
 #pragma unroll
-        for (int i = 0; i < NC; i++) lds->cand_dist[64 * i + lane] = d[i];
+        for (int i = 0; i < NC; i++) {
+            const bool drop = !unordered && d[i] != d[i];
+            lds->cand_dist[64 * i + lane] = drop ? FLT_MAX : d[i];
+            if (drop) lds->cand_id[64 * i + lane] = kInvalid;
+        }
         wave_sync();
+        return true;
     }
 
     // Candidate sort, one network over the wavefront (reference sort_for_candidate, single-warp branch,
@@ -589,9 +604,10 @@ struct Beam {
     // Up to kRankMost candidates that differ from each other are ranked by counting (4 instructions each), more are sorted.
     static constexpr uint32_t kRankMost = 14;
 
-    // whether two beam entries have equal keys, or an entry orders like the padding without being padding
-    __device__ __forceinline__ bool has_ties() const {
-        uint64_t any = 0;
+    // After a merge: whether two beam entries have equal keys, and whether an entry orders like the padding or behind it
+    // without being padding.
+    __device__ __forceinline__ void note_order() {
+        uint64_t equal = 0, behind = 0;
         const uint32_t pad = __float_as_uint(FLT_MAX);
 #pragma unroll
         for (int r = 0; r < NB; r++) {
@@ -599,9 +615,11 @@ struct Beam {
             const uint32_t next = r + 1 < NB ? __float_as_uint(bk[r + 1 < NB ? r + 1 : 0])
                                              : static_cast<uint32_t>(__builtin_amdgcn_update_dpp(-1, static_cast<int>(__float_as_uint(bk[0])), 0x130, 0xf, 0xf, false));   // wave_shl:1
             const uint64_t real = ballot(k < pad);
-            any |= (ballot(k == next) & real) | (ballot(bv[r] != kInvalid) & ~real);
+            equal |= ballot(k == next) & real;
+            behind |= ballot(bv[r] != kInvalid) & ~real;
         }
-        return any != 0;
+        tied = equal != 0;
+        beyond = behind != 0;
     }
     __device__ __forceinline__ bool meets_equal(float key, uint64_t em) const {
         uint64_t equal = 0;
@@ -641,7 +659,8 @@ struct Beam {
         }
         reset_pads();
     }
-    // The entering candidates in ascending order at the front of the candidate lists; false if two have the same key.
+    // The entering candidates in ascending order at the front of the candidate lists; false if two have the same key.  Not for
+    // a beam with entries behind the padding: there the sorted list's empty slots, left out here, displace them.
     __device__ __forceinline__ bool rank_candidates(float key, uint64_t em) {
         uint32_t rank = 0;
         uint64_t equal = 0;
@@ -661,43 +680,53 @@ struct Beam {
         return true;
     }
 
+    // Rows at a distance that is not a number (a NaN in the row or in the query) compare with nothing, and a network that
+    // meets one leaves its other keys unsorted.  They are no candidates, except while there are no others: the entry's
+    // neighbours then make up the beam unsorted and are expanded like any entry (a query with a NaN ends with them), until an
+    // expansion finds a row at a finite distance and a new beam starts with that expansion's candidates.
+    // `fresh`: whether the beam is to start with this expansion; false if the beam stays as it is.
+    __device__ __forceinline__ bool admit(bool& fresh, bool some_finite, bool some_nan) {
+        if (fresh || unordered) {
+            if (!fresh && !some_finite) return false;
+            unordered = some_nan && !some_finite;
+            fresh = true;
+        }
+        return true;
+    }
+
     // reference update_result_buffer: sort the candidates, then fold them into the beam
     __device__ __forceinline__ void absorb(bool first) {
         // No row scored: every candidate distance is FLT_MAX, the sort would not move anything (equal keys are never
         // exchanged) and no candidate can displace a beam entry, so the beam stays as it is.
         if (!first && last_scored == 0) return;
+        bool fresh = first;
         if constexpr (NC == 1) {
             float key = slot_distance(0);
-            bool as_is = false;
-            if (first) {
-                // Rows with a NaN compare with nothing.  Beside rows that do they are dropped; when there is nothing else (a
-                // query with a NaN) all keep their slots, and no later candidate will be below any of them.
-                if (ballot(key != key) != 0) {
-                    as_is = ballot(key < FLT_MAX) == 0;
-                    if (!as_is && key != key) {
-                        key = FLT_MAX;
-                        cid = kInvalid;
-                    }
+            if (first || unordered) {
+                if (!admit(fresh, ballot(key < FLT_MAX) != 0, ballot(key != key) != 0)) return;
+                if (!unordered && key != key) {
+                    key = FLT_MAX;
+                    cid = kInvalid;
                 }
                 wave_sync();
-                sort_candidates_lane(key, as_is);
+                sort_candidates_lane(key, unordered);
             } else {
-                const uint64_t em = entering(key);
+                const uint64_t em = entering(key);   // without those that are not a number; a sorted list has them behind all others
                 if (em == 0) return;
                 const uint32_t m = __popcll(em);
-                if (m <= kInsertMost && !tied && !meets_equal(key, em)) {
+                if (m <= kInsertMost && !tied && !beyond && !meets_equal(key, em)) {
                     insert(key, em);
                     return;
                 }
                 wave_sync();
-                if (m > kRankMost || !rank_candidates(key, em)) sort_candidates_lane(key, false);
+                if (m > kRankMost || beyond || !rank_candidates(key, em)) sort_candidates_lane(key, false);
             }
         } else {
-            distances_to_slots();
+            if (!distances_to_slots(fresh)) return;
             if constexpr (MAX_CAND > 128) sort_candidates_two();
             else sort_candidates_one();
         }
-        if (first) {
+        if (fresh) {
 #pragma unroll
             for (int r = 0; r < NB; r++) {
                 const uint32_t e = NB * lane + r;
@@ -712,7 +741,7 @@ struct Beam {
             merge_beam();
         }
         wave_sync();
-        if constexpr (NC == 1) tied = has_ties();
+        if constexpr (NC == 1) note_order();
     }
 
     // first unexplored beam entry (reference select_current_point); marks it explored
