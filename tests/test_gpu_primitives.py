@@ -51,6 +51,37 @@ def test_bitonic_merge_bit_exact(hip, m):
         assert np.array_equal(gk[b], ek) and np.array_equal(gv[b], ev), (m, b)
 
 
+@pytest.mark.parametrize("shift", [0, 6], ids=["keys >= 0", "keys of either sign"])
+@pytest.mark.parametrize("m", [32, 64, 128, 256])
+def test_both_network_forms_with_ties(hip, m, shift):
+    """Up to 256 elements there are two forms of the networks, one for keys that order like their bits and one for any keys:
+    a row with a negative key takes the second.  Tie-rich rows through the sort and the merge of each."""
+    from oracle import oracle as O
+    rng = np.random.default_rng(1000 + m)
+    batch = 48
+    keys = rng.integers(0, 12, (batch, m)).astype(np.float32)
+    keys[:8] = rng.integers(0, 3, (8, m))
+    keys[8:16, ::2] = np.float32(3.4e38)
+    keys[16:20] = np.inf
+    keys[16:20, 1::3] = 5.0
+    ordered = keys.copy()
+    ordered[:, : m // 2].sort(axis=1)
+    ordered[:, m // 2 :] = -np.sort(-ordered[:, m // 2 :], axis=1)
+    ordered[40:] = keys[40:]                                          # not bitonic: still a fixed function of the input
+    vals = rng.permutation(batch * m).reshape(batch, m).astype(np.uint32)
+    for given, on_gpu, on_cpu in ((keys, hip.bitonic_sort_kv, O.bitonic_warp_sort), (ordered, hip.bitonic_merge_kv, lambda k, v: O.bitonic_warp_merge(k, v, 32))):
+        given = given - np.float32(shift)
+        if shift:
+            given[:, 0] = -6.0
+        assert (given.min(axis=1) < 0).all() == (shift > 0)
+        dk, dv = hip.DeviceArray.from_numpy(given), hip.DeviceArray.from_numpy(vals)
+        on_gpu(dk, dv, m, batch)
+        gk, gv = dk.numpy(), dv.numpy()
+        for b in range(batch):
+            ek, ev = on_cpu(given[b], vals[b])
+            assert np.array_equal(gk[b], ek) and np.array_equal(gv[b], ev), (m, shift, b)
+
+
 @pytest.mark.parametrize("bitlen", [8, 10, 13])
 def test_hashmap_bit_exact(hip, bitlen):
     from oracle import oracle as O
