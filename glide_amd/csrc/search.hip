@@ -5,28 +5,18 @@
 
 namespace glide {
 
-// Grid size for the one-query-per-wavefront search kernel.  With small beams the kernel is bound by row gathers; when
-// the batch is a little larger than what the chip holds at once (10 000 queries against 8 192 wavefront slots),
-// hardware dispatch runs one full round and a thin, latency-bound tail.  Equal rounds are faster: the grid is the
-// batch divided by the number of rounds and every wavefront loops over its share.  Larger beams are bound by the
-// sorting networks and keep one workgroup per query.
 size_t simd_count() {
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) return 0;
     return static_cast<size_t>(cus) * 4;
 }
 
-uint32_t balanced_grid(uint32_t items, uint32_t beam, size_t lds_bytes) {
-    if (beam > 64) return items;
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-        return items;
-    const size_t by_lds = lds_bytes ? (160 * 1024) / lds_bytes : 32;
-    const size_t slots = static_cast<size_t>(cus) * (by_lds < 32 ? by_lds : 32);   // 4 SIMDs x 8 wavefronts per CU
-    if (slots == 0 || items <= slots) return items;
-    const size_t rounds = (items + slots - 1) / slots;
-    return static_cast<uint32_t>((items + rounds - 1) / rounds);
-}
+// One workgroup per query, up to half of what a launch can hold (2^32 threads); beyond that a wavefront takes several.
+// Batches above what the chip holds at once are left to the hardware's dispatch.  Dividing them into equal rounds, several
+// queries a wavefront, helps while rows come from memory and the rounds just fit what is resident (7 000 queries at beam
+// 64: 743 against 633 us on unit rows), but rows that stay in cache make queries unequally long and lose by it (same batch
+// on the mixture: 439 against 512 us; 25 000 queries in rounds of 6 250: 1.40 times the time there, 1.20 on rows from memory).
+constexpr uint32_t kMostWorkgroups = 1u << 25;
 
 }  // namespace glide
 
@@ -81,7 +71,7 @@ int launch_search(const float* data, uint32_t num, uint32_t dim, const uint32_t*
                              (team ? (dim <= 512 ? TeamShape<4>::query_bytes : dim <= 1024 ? TeamShape<8>::query_bytes : dim <= 2048 ? TeamShape<16>::query_bytes : TeamShape<32>::query_bytes) + 16 : 0);
     GLIDE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)));
     if (team) hipLaunchKernelGGL(fn, dim3(query_num), dim3(64 * kTeam), lds_bytes, as_stream(stream), a);
-    else hipLaunchKernelGGL(fn, dim3(balanced_grid(query_num, beam, lds_bytes)), dim3(64), lds_bytes, as_stream(stream), a);
+    else hipLaunchKernelGGL(fn, dim3(query_num < kMostWorkgroups ? query_num : kMostWorkgroups), dim3(64), lds_bytes, as_stream(stream), a);
     return launch_status();
 }
 }  // namespace

@@ -21,7 +21,7 @@ __device__ __forceinline__ void search_body(const SearchArgs a) {
     auto* lds = reinterpret_cast<BeamLds<MAX_CAND>*>(smem);
     float* cent = reinterpret_cast<float*>(smem + sizeof(BeamLds<MAX_CAND>));
     uint32_t* hash = reinterpret_cast<uint32_t*>(cent + round_up32(a.centroid_num));
-    // a wavefront takes queries blockIdx.x, blockIdx.x + gridDim.x, ... (the host sizes the grid)
+    // one query a workgroup, as far as a launch has workgroups
     for (uint32_t qid = blockIdx.x; qid < a.query_num; qid += gridDim.x) {
         Beam<MAX_CAND, MAX_BEAM, DIMV, false, WHOLE> b;
         b.init(lds, hash, a.p, a.queries + static_cast<size_t>(qid) * a.p.dim);

@@ -184,6 +184,21 @@ def test_search_degree_above_128(hip, deg):
         assert gcnt == [est["iterations"], est["rows_scored"], est["graph_rows"]]
 
 
+def test_more_queries_than_workgroups(hip):
+    """Above 2^25 queries a workgroup takes more than one."""
+    rng = np.random.default_rng(5)
+    nq, n = (1 << 25) + 77, 64
+    data = rng.integers(0, 9, (n, 4)).astype(np.float32)
+    graph = rng.integers(0, n, (n, 8)).astype(np.uint32)
+    few = rng.integers(0, 9, (101, 4)).astype(np.float32)
+    sp = dict(beam=32, max_iterations=3, min_iterations=0, hash_bit=8, hash_reset_interval=4)
+    index = (data, graph, data[:2].copy(), np.array([5, 9], np.uint32))
+    eids, edists, _ = run_gpu_search(hip, *index, few, 1, sp)
+    reps = -(-nq // few.shape[0])
+    gids, gdists, _ = run_gpu_search(hip, *index, np.tile(few, (reps, 1))[:nq], 1, sp)
+    assert np.array_equal(gids, np.tile(eids, (reps, 1))[:nq]) and np.array_equal(gdists, np.tile(edists, (reps, 1))[:nq])
+
+
 def test_search_rejects_unsupported_sizes(hip):
     d = hip.DeviceArray(4096, np.float32)
     base = dict(data=d, num=8, dim=128, graph=d, graph_degree=32, centroids=d, centroid_num=2, start_points=d, queries=d,
