@@ -245,10 +245,11 @@ int launch_search_sub(const float* segment_data, uint32_t dim, const uint32_t* s
     a.top_k = top_k;
     a.max_topk = top_k <= 32 ? 32 : (top_k <= 64 ? 64 : 128);
     a.p = BeamParams{beam, graph_degree, dim, hash_bit, hash_reset_interval ? hash_reset_interval : 1, max_iterations, min_iterations, metric};
-    sub_fn fn = pick_sub(graph_degree, beam, dim);
+    const uint32_t wavefronts = query_list ? list_len : query_num;
+    sub_fn fn = pick_sub(graph_degree, beam, dim, wavefronts);
     const size_t lds_bytes = beam_lds_bytes(graph_degree) + 128 * 8 + (size_t{1} << hash_bit) * sizeof(uint32_t);
     GLIDE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)));
-    hipLaunchKernelGGL(fn, dim3(query_list ? list_len : query_num), dim3(64), lds_bytes, as_stream(stream), a);
+    hipLaunchKernelGGL(fn, dim3(wavefronts), dim3(64), lds_bytes, as_stream(stream), a);
     return launch_status();
 }
 }  // namespace
@@ -380,7 +381,7 @@ extern "C" int glide_hip_search_partitions(const float* data, uint32_t dim, cons
         a.max_topk = top_k <= 32 ? 32 : (top_k <= 64 ? 64 : 128);
         a.list_len = pairs;
         a.p = BeamParams{beam, graph_degree, dim, hash_bit, hash_reset_interval ? hash_reset_interval : 1, max_iterations, min_iterations, metric};
-        sub_fn fn = pick_sub(graph_degree, beam, dim);
+        sub_fn fn = pick_sub(graph_degree, beam, dim, pairs);
         const size_t lds_bytes = beam_lds_bytes(graph_degree) + 128 * 8 + (size_t{1} << hash_bit) * sizeof(uint32_t);
         GLIDE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)));
         hipLaunchKernelGGL(fn, dim3(pairs), dim3(64), lds_bytes, s, a);

@@ -38,10 +38,10 @@ __device__ __forceinline__ void merge_result(const float* beam_dist, const uint3
 }
 
 // search_on_sub_kernel (search_kernel.cuh:653-765)
-// Up to 64 slots: five wavefronts per SIMD and no more.  A batch searches many partitions side by side and is bound by its
-// gathers; six wavefronts (the kernel would fit) cost 5 000 queries over 64 partitions 2.50 ms instead of 2.37.
-template <int MAX_CAND, int MAX_BEAM, int DIMV, bool WHOLE = false>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DIMV > 4 ? 1 : MAX_CAND <= 64 ? 5 : MAX_BEAM > 256 ? 4 : 1, DIMV > 4 || MAX_CAND > 64 ? 8 : 5)))
+// Up to 64 slots on rows of up to 512 dims: five wavefronts per SIMD, for beams up to 64 five or SIX (75 registers allow it;
+// which one is decided per launch, see six_resident).
+template <int MAX_CAND, int MAX_BEAM, int DIMV, bool WHOLE = false, bool SIX = false>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DIMV > 4 ? 1 : MAX_CAND <= 64 ? (SIX ? 6 : 5) : MAX_BEAM > 256 ? 4 : 1, DIMV > 4 || MAX_CAND > 64 ? 8 : (SIX ? 6 : 5))))
 void search_sub_kernel(SubArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     auto* lds = reinterpret_cast<BeamLds<MAX_CAND>*>(smem);
@@ -131,7 +131,10 @@ sub_fn pick_sub_dim(uint32_t dim) {
     return search_sub_kernel<MAX_CAND, MAX_BEAM, 32, WHOLE>;
 }
 template <int MAX_CAND>
-sub_fn pick_sub_beam(uint32_t beam, uint32_t dim) {
+sub_fn pick_sub_beam(uint32_t beam, uint32_t dim, bool six) {
+    if constexpr (MAX_CAND <= 64) {
+        if (beam <= 64 && dim <= 512 && six) return dim <= 128 ? search_sub_kernel<MAX_CAND, 64, 1, false, true> : dim <= 256 ? search_sub_kernel<MAX_CAND, 64, 2, false, true> : search_sub_kernel<MAX_CAND, 64, 4, false, true>;
+    }
     if (beam <= 64) return pick_sub_dim<MAX_CAND, 64>(dim);
     if (beam <= 128) return pick_sub_dim<MAX_CAND, 128>(dim);
     if (beam <= 256) return pick_sub_dim<MAX_CAND, 256>(dim);
@@ -141,6 +144,6 @@ sub_fn pick_sub_beam(uint32_t beam, uint32_t dim) {
 
 #define GLIDE_PICK_NAME(cand) pick_sub_##cand
 #define GLIDE_PICK(cand) GLIDE_PICK_NAME(cand)
-sub_fn GLIDE_PICK(GLIDE_CAND)(uint32_t beam, uint32_t dim) { return pick_sub_beam<GLIDE_CAND>(beam, dim); }
+sub_fn GLIDE_PICK(GLIDE_CAND)(uint32_t beam, uint32_t dim, bool six) { return pick_sub_beam<GLIDE_CAND>(beam, dim, six); }
 
 }  // namespace glide

@@ -129,6 +129,49 @@ def test_search_over_partitions_bit_exact(hip, large_index, top_k, beam):
     assert hip.read_counters(cnt)[0] > 0
 
 
+@pytest.mark.parametrize("dim", [32, 200, 512])
+def test_search_over_partitions_many_pairs(hip, dim):
+    """Beams up to 64 run with five or six wavefronts per SIMD, by how many (query, partition) pairs there are: counts on
+    both sides of a full round of five and of six, in the three-launch form and partition by partition."""
+    from oracle import oracle as O
+    rng = np.random.default_rng(dim)
+    per, c, top_k = 300, 2, 5
+    data = rng.integers(0, 5, (c * per, dim)).astype(np.float32)
+    graph = rng.integers(0, per, (c * per, 16)).astype(np.uint32)
+    graph[rng.random(graph.shape) < 0.1] = INV
+    ids = rng.permutation(c * per).astype(np.uint32)
+    entries = np.array([7, 250], np.uint32)
+    starts = np.array([0, per], np.uint32)
+    lane = hip.device_info()["compute_units"] * 4
+    queries = rng.integers(0, 5, (6 * lane // 2 + 1, dim)).astype(np.float32)
+    for beam, pairs in ((32, 5 * lane), (32, 5 * lane + 2), (64, 6 * lane), (64, 6 * lane + 2)):
+        nq = pairs // c
+        q, sp = queries[:nq], O.search_params(beam, 16)
+        seg = np.tile(np.arange(c, dtype=np.uint32), (nq, 1))
+        e_ids, e_d = np.full((nq, top_k), INV, np.uint32), np.full((nq, top_k), np.finfo(np.float32).max, np.float32)
+        for s in range(c):
+            sl = slice(s * per, (s + 1) * per)
+            O.search_sub(data[sl], graph[sl], ids[sl], q, seg, s, int(entries[s]), top_k, sp, e_ids, e_d)
+        args = (sp["beam"], sp["max_iterations"], sp["min_iterations"], sp["hash_bit"], sp["hash_reset_interval"], 0)
+        d_data, d_graph, d_ids, d_q, d_seg = (hip.DeviceArray.from_numpy(np.ascontiguousarray(x)) for x in (data, graph, ids, q, seg))
+        g_ids, g_d = hip.DeviceArray((nq, top_k), np.uint32), hip.DeviceArray((nq, top_k), np.float32)
+        print("dim", dim, "beam", beam, "pairs", pairs, flush=True)
+        hip.search_partitions(d_data, dim, d_graph, 16, d_ids, hip.DeviceArray.from_numpy(starts), hip.DeviceArray.from_numpy(entries), c, d_q, nq, d_seg,
+                              top_k, *args, g_ids, g_d)
+        assert np.array_equal(g_ids.numpy(), e_ids) and np.array_equal(g_d.numpy(), e_d)
+    # 5 * lane + 2 queries of one partition at a time
+    q = np.tile(queries, (2, 1))[: 5 * lane + 2]
+    nq, sp = q.shape[0], O.search_params(64, 16)
+    seg = np.zeros((nq, 1), np.uint32)
+    e_ids, e_d = np.full((nq, top_k), INV, np.uint32), np.full((nq, top_k), np.finfo(np.float32).max, np.float32)
+    g_ids, g_d = hip.DeviceArray.from_numpy(e_ids), hip.DeviceArray.from_numpy(e_d)
+    O.search_sub(data[:per], graph[:per], ids[:per], q, seg, 0, 7, top_k, sp, e_ids, e_d)
+    hip.search_sub(d_data, dim, d_graph, 16, d_ids, hip.DeviceArray.from_numpy(q), nq, hip.DeviceArray.from_numpy(seg), 1, 0, 7, top_k, sp["beam"],
+                   sp["max_iterations"], sp["min_iterations"], sp["hash_bit"], sp["hash_reset_interval"], 0, g_ids, g_d)
+    hip.synchronize()
+    assert np.array_equal(g_ids.numpy(), e_ids) and np.array_equal(g_d.numpy(), e_d)
+
+
 def test_place_and_merge_boundary_bit_exact(hip):
     """The two passes of the merged large build against the oracle's row merge, on rows that take both of its
     branches (at least half of the copy's neighbours already present / fewer) and on rows with empty slots."""
