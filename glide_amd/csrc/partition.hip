@@ -694,11 +694,11 @@ __global__ __launch_bounds__(1024) void kmeanspp_pick_kernel(uint32_t n, const f
     draw_candidates(part, n, min_dist, seed, step, trials, candidates);
 }
 
-// 64 sample rows per workgroup, LANES lanes a row: squared distance of every row to every candidate (kept for the next
-// kernel, which lowers min_dist by the winner's) and the candidates' potentials over these rows, in double, summed row after
-// row in four runs of 16 whatever the layout.  Rows of up to 128 dims take half a wavefront and four rows a group, with the
-// candidates in registers: the kernel is a few memory round trips long, so what counts is to have them all under way at once
-// (20 000 rows of 128 dims, 7 candidates: 30 us with one wavefront going through 16 rows).
+// 64 sample rows per workgroup, LANES lanes a row: squared distance of every row to every candidate (kept in trial_dist,
+// nullable, for kmeanspp_next_kernel, which lowers min_dist by the winner's) and the candidates' potentials over these rows,
+// in double, summed row after row in four runs of 16 whatever the layout.  Rows of up to 128 dims take half a wavefront and
+// four rows a group, with the candidates in registers: the kernel is a few memory round trips long, so what counts is to have
+// them all under way at once (20 000 rows of 128 dims, 7 candidates: 30 us with one wavefront going through 16 rows).
 constexpr uint32_t kTrialThreads = 512;
 template <int LANES>
 __global__ __launch_bounds__(kTrialThreads) void kmeanspp_trial_kernel(const float* sample, uint32_t n, uint32_t dim, const float* min_dist,
@@ -743,7 +743,7 @@ __global__ __launch_bounds__(kTrialThreads) void kmeanspp_trial_kernel(const flo
         }
     }
     __syncthreads();
-    {
+    if (trial_dist) {
         const uint32_t j = threadIdx.x / kSeedPoints, i = first + threadIdx.x % kSeedPoints;
         if (j < trials && i < n) trial_dist[static_cast<size_t>(j) * n + i] = dist[j][threadIdx.x % kSeedPoints];
     }
@@ -1134,9 +1134,9 @@ size_t glide_hip_kmeans_workspace_bytes(uint32_t cluster_num, uint32_t dim) {
 
 size_t glide_hip_kmeans_seed_workspace_bytes(uint32_t sample_num) {
     // min_dist (f32 per row) | candidates (8 u32) | per-workgroup potentials of the trial kernel (8 f64 each)
-    // | distances of every row to the candidates (8 f32 per row)
+    // | distances of every row to the candidates (8 f32 per row), for samples whose steps pass through LDS
     return align_up(static_cast<size_t>(sample_num) * 4, 256) + 256 + static_cast<size_t>(ceil_div(sample_num, kSeedPoints)) * kSeedTrials * 8 +
-           static_cast<size_t>(sample_num) * kSeedTrials * 4;
+           (sample_num <= kSeedLdsRows ? static_cast<size_t>(sample_num) * kSeedTrials * 4 : 0);
 }
 
 int glide_hip_kmeans_seed(const float* sample, uint32_t sample_num, uint32_t dim, uint32_t cluster_num, uint32_t seed, float* centroids,
@@ -1152,8 +1152,8 @@ int glide_hip_kmeans_seed(const float* sample, uint32_t sample_num, uint32_t dim
     uint32_t* candidates = reinterpret_cast<uint32_t*>(w + align_up(static_cast<size_t>(sample_num) * 4, 256));
     double* partial = reinterpret_cast<double*>(w + align_up(static_cast<size_t>(sample_num) * 4, 256) + 256);
     const uint32_t trials = seed_trials(cluster_num), blocks = ceil_div(sample_num, kSeedPoints);
-    float* trial_dist = reinterpret_cast<float*>(partial + static_cast<size_t>(blocks) * kSeedTrials);
     const bool in_lds = sample_num <= kSeedLdsRows;
+    float* trial_dist = in_lds ? reinterpret_cast<float*>(partial + static_cast<size_t>(blocks) * kSeedTrials) : nullptr;
     const size_t lds = static_cast<size_t>(sample_num) * sizeof(float);
     if (in_lds && cluster_num > 1)
         GLIDE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&kmeanspp_next_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,

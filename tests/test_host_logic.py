@@ -34,6 +34,16 @@ def test_unsupported_sizes_raise_like_the_reference():
         G._check_sizes(64, 257)
 
 
+def test_seeding_workspace_holds_what_is_used():
+    """Distances to the candidates (32 bytes a row) are kept for samples whose steps pass through LDS, 32768 rows; a larger
+    sample needs its smallest distances and 8 potentials per 64 rows."""
+    from glide_amd import capi
+    size = capi.kmeans_seed_workspace_bytes
+    assert size(32768) >= 36 * 32768
+    for n in (32769, 50_000, 1_000_001):
+        assert 4 * n + 64 * (n // 64) <= size(n) <= 4 * n + 64 * (n // 64 + 1) + 512
+
+
 def test_file_formats_round_trip(tmp_path):
     rng = np.random.default_rng(0)
     m = rng.standard_normal((7, 5)).astype(np.float32)
