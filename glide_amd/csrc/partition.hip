@@ -653,6 +653,9 @@ __device__ __forceinline__ uint32_t wave_locate(Load load, uint32_t len, double 
     return static_cast<uint32_t>(__shfl(static_cast<int>(last), src));
 }
 
+// four values of a row, zeros in the lanes behind its end
+__device__ __forceinline__ float4 load4(const float* p, bool in) { return in ? *reinterpret_cast<const float4*>(p) : make_float4(0.f, 0.f, 0.f, 0.f); }
+
 // one workgroup of 16 wavefronts: chunk sums of min_dist (in global memory or LDS), then wavefront j draws candidate j
 __device__ __forceinline__ void draw_candidates(double* part, uint32_t n, const float* min_dist, uint32_t seed, uint32_t step, uint32_t trials,
                                                 uint32_t* candidates) {
@@ -699,8 +702,15 @@ __global__ __launch_bounds__(1024) void kmeanspp_pick_kernel(uint32_t n, const f
 // in double, summed row after row in four runs of 16 whatever the layout.  Rows of up to 128 dims take half a wavefront and
 // four rows a group, with the candidates in registers: the kernel is a few memory round trips long, so what counts is to have
 // them all under way at once (20 000 rows of 128 dims, 7 candidates: 30 us with one wavefront going through 16 rows).
+// The candidates' ids are read before the first row, so that no row load waits for them, and the masked loads choose between
+// values: choosing between a row in memory and zeros held in a variable selects an address, which put the zeros into private
+// memory, made the loads flat ones and every wait for an id a wait for all rows (a step of 20 000 rows of 128 dims and 7
+// candidates, next kernel included: 28.8 -> 26.3 us; a sample of 200 rows 14.4 -> 13.5 us).  Rows of 129 to 256 dims go four at
+// a time (one at a time 2.5 % slower on 200 000 rows than a wavefront that keeps the sums of all candidates, four 4-15 %
+// faster); longer ones one at a time, so that a workgroup's rows stay in the L1 from candidate to candidate (960 dims, 50 000
+// rows: four at a time 1.36 times the time).
 constexpr uint32_t kTrialThreads = 512;
-template <int LANES>
+template <int LANES, uint32_t TOGETHER = 1>   // TOGETHER: rows of more than 128 dims under way at once
 __global__ __launch_bounds__(kTrialThreads) void kmeanspp_trial_kernel(const float* sample, uint32_t n, uint32_t dim, const float* min_dist,
                                                                       const uint32_t* candidates, uint32_t trials, double* partial, float* trial_dist) {
     static_assert(kSeedPoints * kSeedTrials == kTrialThreads, "one distance a thread");
@@ -709,17 +719,18 @@ __global__ __launch_bounds__(kTrialThreads) void kmeanspp_trial_kernel(const flo
     __shared__ double run_pot[4][kSeedTrials];
     const uint32_t group = threadIdx.x / LANES, t = threadIdx.x % LANES, first = blockIdx.x * kSeedPoints;
     if constexpr (LANES == 32) {
-        const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+        uint32_t id[kSeedTrials];
+#pragma unroll
+        for (uint32_t j = 0; j < kSeedTrials; j++) id[j] = candidates[j < trials ? j : 0];
         const bool in = t * 4 < dim;
         float4 c[kSeedTrials], x[kRows];
 #pragma unroll
         for (uint32_t r = 0; r < kRows; r++) {
             const uint32_t i = first + group * kRows + r;
-            x[r] = in ? *reinterpret_cast<const float4*>(sample + static_cast<size_t>(i < n ? i : n - 1) * dim + t * 4) : zero;
+            x[r] = load4(sample + static_cast<size_t>(i < n ? i : n - 1) * dim + t * 4, in);
         }
 #pragma unroll
-        for (uint32_t j = 0; j < kSeedTrials; j++)
-            c[j] = in ? *reinterpret_cast<const float4*>(sample + static_cast<size_t>(candidates[j < trials ? j : 0]) * dim + t * 4) : zero;
+        for (uint32_t j = 0; j < kSeedTrials; j++) c[j] = load4(sample + static_cast<size_t>(id[j]) * dim + t * 4, in);
 #pragma unroll
         for (uint32_t r = 0; r < kRows; r++)
 #pragma unroll
@@ -729,16 +740,22 @@ __global__ __launch_bounds__(kTrialThreads) void kmeanspp_trial_kernel(const flo
                 if (t == 0) dist[j][group * kRows + r] = d;
             }
     } else {
-        for (uint32_t r = 0; r < kRows; r++) {
+        for (uint32_t r = 0; r < kRows; r += TOGETHER) {
             const uint32_t i = first + group * kRows + r;
-            const float* x = sample + static_cast<size_t>(i < n ? i : n - 1) * dim;
             for (uint32_t j = 0; j < trials; j++) {
                 const float* c = sample + static_cast<size_t>(candidates[j]) * dim;
-                float acc = 0.f;
-                for (uint32_t d0 = t * 4; d0 < dim; d0 += 256)
-                    acc = sqdist4(*reinterpret_cast<const float4*>(x + d0), *reinterpret_cast<const float4*>(c + d0), acc);
-                acc = wave_sum(acc);
-                if (t == 0) dist[j][group * kRows + r] = acc;
+                float acc[TOGETHER] = {};
+                for (uint32_t d0 = t * 4; d0 < dim; d0 += 256) {
+                    const float4 b = *reinterpret_cast<const float4*>(c + d0);
+#pragma unroll
+                    for (uint32_t p = 0; p < TOGETHER; p++)
+                        acc[p] = sqdist4(*reinterpret_cast<const float4*>(sample + static_cast<size_t>(i + p < n ? i + p : n - 1) * dim + d0), b, acc[p]);
+                }
+#pragma unroll
+                for (uint32_t p = 0; p < TOGETHER; p++) {
+                    const float d = wave_sum(acc[p]);
+                    if (t == 0) dist[j][group * kRows + r + p] = d;
+                }
             }
         }
     }
@@ -1158,7 +1175,7 @@ int glide_hip_kmeans_seed(const float* sample, uint32_t sample_num, uint32_t dim
     if (in_lds && cluster_num > 1)
         GLIDE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&kmeanspp_next_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                           static_cast<int>(lds)));
-    auto trial = dim <= 128 ? kmeanspp_trial_kernel<32> : kmeanspp_trial_kernel<64>;
+    auto trial = dim <= 128 ? kmeanspp_trial_kernel<32> : dim <= 256 ? kmeanspp_trial_kernel<64, 4> : kmeanspp_trial_kernel<64>;
     for (uint32_t step = 0; step < cluster_num; step++) {
         if (step <= 1 || !in_lds)
             hipLaunchKernelGGL(kmeanspp_pick_kernel, dim3(1), dim3(1024), 0, s, sample_num, min_dist, seed, step, trials, candidates);
