@@ -927,7 +927,6 @@ __global__ __launch_bounds__(256) void kmeans_accumulate_narrow_kernel(const flo
     uint32_t* local_counts = reinterpret_cast<uint32_t*>(local + (in_lds ? k * dim : 0u));
     const uint32_t t = threadIdx.x & 31, group = threadIdx.x >> 5;
     const bool in = t * 4 < dim;
-    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
     if (in_lds) {
         for (uint32_t i = threadIdx.x; i < k * dim; i += 256) local[i] = 0;
         for (uint32_t i = threadIdx.x; i < k; i += 256) local_counts[i] = 0;
@@ -941,11 +940,11 @@ __global__ __launch_bounds__(256) void kmeans_accumulate_narrow_kernel(const flo
 #pragma unroll
         for (uint32_t p = 0; p < kSumPoints; p++) {
             const uint32_t i = first + p < n ? first + p : n - 1;
-            x[p] = in ? *reinterpret_cast<const float4*>(sample + static_cast<size_t>(i) * dim + t * 4) : zero;
+            x[p] = load4(sample + static_cast<size_t>(i) * dim + t * 4, in);
             best[p] = FLT_MAX;
             nearest[p] = 0;
         }
-        float4 next = in ? *reinterpret_cast<const float4*>(centroids + t * 4) : zero;
+        float4 next = load4(centroids + t * 4, in);
         for (uint32_t c = 0; c < k; c++) {
             const float4 row = next;
             if (in && c + 1 < k) next = *reinterpret_cast<const float4*>(centroids + static_cast<size_t>(c + 1) * dim + t * 4);
@@ -961,19 +960,21 @@ __global__ __launch_bounds__(256) void kmeans_accumulate_narrow_kernel(const flo
 #pragma unroll
         for (uint32_t p = 0; p < kSumPoints; p++) {
             if (first + p >= n) break;
-            if (in) {
-                const size_t at = static_cast<size_t>(nearest[p]) * dim + t * 4;
+            // the fixed-point values in two's complement: the wrap-around sum is the signed sum
+            const size_t at = static_cast<size_t>(nearest[p]) * dim;
+            if (in_lds) {
                 const float v[4] = {x[p].x, x[p].y, x[p].z, x[p].w};
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const auto fixed = static_cast<unsigned long long>(__float2ll_rn(v[e] * scale));   // two's complement: the wrap-around sum is the signed sum
-                    if (in_lds) atomicAdd(&local[at + e], fixed);
-                    else atomicAdd(reinterpret_cast<unsigned long long*>(sums) + at + e, fixed);
-                }
-            }
-            if (t == 0) {
-                if (in_lds) atomicAdd(&local_counts[nearest[p]], 1u);
-                else atomicAdd(&counts[nearest[p]], 1u);
+                for (int e = 0; e < 4; e++)
+                    if (in) atomicAdd(&local[at + t * 4 + e], static_cast<unsigned long long>(__float2ll_rn(v[e] * scale)));
+                if (t == 0) atomicAdd(&local_counts[nearest[p]], 1u);
+            } else {
+                // adjacent lanes on adjacent sums, the row read once more for it: in the order of the registers an instruction
+                // reached four sums of a 128-byte line instead of sixteen (64 clusters of 128 dims 1.27 times the time)
+                const float* values = sample + static_cast<size_t>(first + p) * dim;
+                for (uint32_t d = t; d < dim; d += 32)
+                    atomicAdd(reinterpret_cast<unsigned long long*>(sums) + at + d, static_cast<unsigned long long>(__float2ll_rn(values[d] * scale)));
+                if (t == 0) atomicAdd(&counts[nearest[p]], 1u);
             }
         }
     }
@@ -984,6 +985,18 @@ __global__ __launch_bounds__(256) void kmeans_accumulate_narrow_kernel(const flo
         for (uint32_t i = threadIdx.x; i < k; i += 256)
             if (local_counts[i]) atomicAdd(&counts[i], local_counts[i]);
     }
+}
+
+// Where the narrow kernel is ahead of a wavefront per point.  A half-wavefront goes through all centroids for four points at a
+// time, a long chain of its own, so it takes a sample that fills the chip all the same: 12 000 points with sums in memory (a
+// step at 256 clusters of 128 dims, narrow : wide, is 1.43 : 1 with 8 000 points, 1 : 1.05 with 12 000, 1 : 1.31 with 20 000).
+// With sums in LDS the points also have to outweigh the k x dim sums that every workgroup adds up at its end, but few clusters
+// make hot sums of the wide kernel's atomics.  The lines are where the two met, within a tenth, on rows of 28, 64, 100 and 128
+// dims: 550 points for 2 clusters, 1 150 for 8, 2 000 for 16, 7 500 for 32, 16 000 for 64, 42 000 for 128 (twice as many
+// points: 1 : 1.65 for 16 clusters, 1 : 1.75 for 64; half as many: 1.5 : 1 and 1.7 : 1).
+inline bool narrow_pays(uint32_t points, uint32_t clusters, bool in_lds) {
+    if (!in_lds) return points >= 12000;
+    return points >= (clusters <= 16 ? 400 + 100 * clusters : clusters <= 64 ? 250 * clusters : 340 * clusters);
 }
 
 __global__ void kmeans_update_kernel(float* centroids, const long long* sums, const uint32_t* counts, uint32_t k, uint32_t dim, uint32_t n,
@@ -1211,8 +1224,9 @@ int glide_hip_kmeans_fit(const float* sample, uint32_t sample_num, uint32_t dim,
     const size_t values = static_cast<size_t>(sample_num) * dim;
     hipLaunchKernelGGL(kmeans_range_kernel, dim3(static_cast<uint32_t>(values / 256 < 4096 ? values / 256 + 1 : 4096)), dim3(256), 0, s, sample,
                        values, max_bits);
-    const bool narrow = dim <= 128 && reinterpret_cast<uintptr_t>(sample) % 16 == 0 && reinterpret_cast<uintptr_t>(centroids) % 16 == 0;
     const bool in_lds = static_cast<size_t>(cluster_num) * dim <= kLdsSums;
+    const bool narrow = dim <= 128 && narrow_pays(sample_num, cluster_num, in_lds) && reinterpret_cast<uintptr_t>(sample) % 16 == 0 &&
+                        reinterpret_cast<uintptr_t>(centroids) % 16 == 0;
     // with sums in LDS every workgroup adds k x dim of them up at its end, so it takes 128 points at least
     const uint32_t sum_blocks = ceil_div(sample_num, in_lds ? 128 : 8 * kSumPoints);
     const size_t sum_lds = in_lds ? static_cast<size_t>(cluster_num) * dim * 8 + static_cast<size_t>(cluster_num) * 4 : 0;

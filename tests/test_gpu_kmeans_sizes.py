@@ -44,3 +44,25 @@ def test_one_lloyd_step(n, dim, k):
         if (nearest == c).any():
             expect[c] = (x[nearest == c].sum(0, dtype=np.float64) / (nearest == c).sum()).astype(np.float32)
     assert np.array_equal(cent.numpy(), expect)
+
+
+# one side and the other of every line between the two kernels of a Lloyd step: sums in LDS (up to 16, 64 and 1024 clusters)
+# and in memory
+@pytest.mark.parametrize("n, dim, k", [(499, 4, 1), (500, 4, 1), (1199, 128, 8), (1201, 100, 8), (2000, 28, 16), (4250, 128, 17), (4249, 128, 17),
+                                       (16001, 64, 64), (22100, 60, 65), (22099, 60, 65), (348160, 4, 1024), (11999, 128, 33), (12000, 128, 33),
+                                       (12003, 100, 256)])
+def test_one_lloyd_step_by_either_kernel(n, dim, k):
+    from glide_amd import capi as hip
+    hip.set_device(0)
+    x, start = rows_of(n, dim, n + k), rows_of(k, dim, k)
+    cent = hip.DeviceArray.from_numpy(start)
+    wb = hip.kmeans_workspace_bytes(k, dim)
+    ws = hip.DeviceArray(wb // 8 + 1, np.uint64)
+    hip.kmeans_fit(hip.DeviceArray.from_numpy(x), n, dim, k, 1, cent, ws, wb)
+    hip.synchronize()
+    half = (start ** 2).sum(1) / 2                                       # integers and halves below 2^24: exact
+    nearest = np.concatenate([(half - x[i:i + 4096] @ start.T).argmin(1) for i in range(0, n, 4096)])
+    sums, counts = np.zeros((k, dim)), np.bincount(nearest, minlength=k)
+    np.add.at(sums, nearest, x)
+    expect = np.where(counts[:, None] > 0, sums / np.maximum(counts, 1)[:, None], start).astype(np.float32)
+    assert np.array_equal(cent.numpy(), expect)
