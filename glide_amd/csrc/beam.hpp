@@ -161,8 +161,10 @@ struct Beam {
     uint32_t last_scored;   // rows scored by the latest expansion (wave-uniform)
     uint32_t until_reset;   // iterations left until the visited set is reset (a countdown: a remainder by a run-time divisor is two dozen instructions)
     bool tied;              // some beam entries have equal keys (MAX_CAND == 64)
-    bool beyond;            // some beam entries are rows whose key is not below the padding's: infinite, or the unscored point of a build (MAX_CAND == 64)
-    bool unordered;         // the beam holds rows that compare with nothing, and no others (see absorb)
+    // Entering candidates that are ranked rather than sorted (MAX_CAND == 64), or kUnordered: the beam holds rows that compare
+    // with nothing, and no others (see absorb).  One number, so that the loop carries no second flag: that costs 1-2 %.
+    static constexpr int kUnordered = -1;
+    int rank_most;
     uint32_t cid;           // candidate id of this lane's slot (MAX_CAND == 64; larger buckets keep the ids in LDS)
     uint32_t place[NC];     // where in vlist each of this lane's slots is; kInvalid: not scored
 
@@ -174,7 +176,6 @@ struct Beam {
         asm volatile("" : "+v"(lane));   // as in run: nothing made from it is to be kept from one query to the next
         load_row<DIMV>(q, query, p.dim, RowShape<DIMV>::lane_in_row(lane));
         until_reset = p.reset_interval;
-        unordered = false;
         hash_clear(hash, p.hash_bit, lane);
         wave_sync();
     }
@@ -253,25 +254,43 @@ struct Beam {
         const float d = finish_distance(lds->cand_dist[place[i] & (MAX_CAND - 1)], p.metric);
         return place[i] != kInvalid ? d : FLT_MAX;
     }
-    // Buckets of more than 64 slots: from the order of vlist to the slots.  Slots that are not candidates (see absorb) become
-    // empty; returns false if the expansion leaves the beam as it is.
-    __device__ __forceinline__ bool distances_to_slots(bool& fresh) {
+    // Buckets of more than 64 slots: from the order of vlist to the slots.  What is not a number is dropped where a beam starts
+    // (see absorb) and orders last after that: its bits are above those of infinity.  Returns false if the beam stays as it is;
+    // `first` becomes true if the expansion starts a new one.
+    __device__ __forceinline__ bool distances_to_slots(bool& first) {
         float d[NC];
-        uint64_t some = 0, nans = 0;
 #pragma unroll
-        for (int i = 0; i < NC; i++) {
-            d[i] = slot_distance(i);
-            some |= ballot(d[i] < FLT_MAX);
-            nans |= ballot(d[i] != d[i]);
+        for (int i = 0; i < NC; i++) d[i] = slot_distance(i);
+        if (first || rank_most == kUnordered) {
+            bool some = false, nan = false;
+#pragma unroll
+            for (int i = 0; i < NC; i++) {
+                some |= d[i] < FLT_MAX;
+                nan |= d[i] != d[i];
+            }
+            const uint64_t finite = ballot(some), nans = ballot(nan);
+            if (!first && finite == 0) return false;
+            first = true;
+            rank_most = nans != 0 && finite == 0 ? kUnordered : kRankMost;
+            if (finite != 0) {
+#pragma unroll
+                for (int i = 0; i < NC; i++) {
+                    if (d[i] != d[i]) {
+                        d[i] = FLT_MAX;
+                        lds->cand_id[64 * i + lane] = kInvalid;
+                    }
+                }
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < NC; i++) {
+                const uint32_t bits = __float_as_uint(d[i]);
+                d[i] = __uint_as_float(bits < 0x7f800000u ? bits : 0x7f800000u);
+            }
         }
-        if (!admit(fresh, some != 0, nans != 0)) return false;
         wave_sync();
 #pragma unroll
-        for (int i = 0; i < NC; i++) {
-            const bool drop = !unordered && d[i] != d[i];
-            lds->cand_dist[64 * i + lane] = drop ? FLT_MAX : d[i];
-            if (drop) lds->cand_id[64 * i + lane] = kInvalid;
-        }
+        for (int i = 0; i < NC; i++) lds->cand_dist[64 * i + lane] = d[i];
         wave_sync();
         return true;
     }
@@ -517,18 +536,22 @@ struct Beam {
         static_assert(MAX_CAND == 64, "one candidate slot per lane");
         // The beam is ascending, so its last entry is the largest key of the lane that holds it among that lane's entries
         // below `beam` (written as a maximum: a chain of selects between the registers becomes a run-time index, which
-        // moves the beam out of the registers).  Keys are not negative.
-        float tail;
+        // moves the beam out of the registers).  Keys are not negative, so they compare as their bits; what is not a number is
+        // above everything else and enters nowhere.
+        uint32_t tail;
         if (p.beam % NB == 0) {   // the last entry is the last register of a lane (beams are multiples of 32 as a rule)
-            tail = read_lane(bk[NB - 1], static_cast<int>(p.beam / NB) - 1);
+            tail = read_lane(__float_as_uint(bk[NB - 1]), static_cast<int>(p.beam / NB) - 1);
         } else {
             const uint32_t last = p.beam - 1;
-            float mine = bk[0];
+            uint32_t mine = __float_as_uint(bk[0]);
 #pragma unroll
-            for (int r = 1; r < NB; r++) mine = fmaxf(mine, NB * lane + r <= static_cast<int>(last) ? bk[r] : 0.f);
+            for (int r = 1; r < NB; r++) {
+                const uint32_t k = NB * lane + r <= static_cast<int>(last) ? __float_as_uint(bk[r]) : 0u;
+                mine = mine > k ? mine : k;
+            }
             tail = read_lane(mine, static_cast<int>(last / NB));
         }
-        return ballot(ck < tail);
+        return ballot(__float_as_uint(ck) < tail);
     }
 
     // Beam merge for beams of up to 256 entries (reference sort_for_beam, single-warp branch): the k-th smallest candidate
@@ -602,12 +625,13 @@ struct Beam {
     // rows next to never.
     static constexpr uint32_t kInsertMost = 8;
     // Up to kRankMost candidates that differ from each other are ranked by counting (4 instructions each), more are sorted.
-    static constexpr uint32_t kRankMost = 14;
+    // A beam that starts with rows at an infinite distance has all of them sorted: the empty slots of the sorted list, left out
+    // of the ranked one, displace such rows, which only come in at the start.
+    static constexpr int kRankMost = 14;
 
-    // After a merge: whether two beam entries have equal keys, and whether an entry orders like the padding or behind it
-    // without being padding.
-    __device__ __forceinline__ void note_order() {
-        uint64_t equal = 0, behind = 0;
+    // whether two beam entries have equal keys, or an entry orders like the padding without being padding
+    __device__ __forceinline__ bool has_ties() const {
+        uint64_t any = 0;
         const uint32_t pad = __float_as_uint(FLT_MAX);
 #pragma unroll
         for (int r = 0; r < NB; r++) {
@@ -615,11 +639,9 @@ struct Beam {
             const uint32_t next = r + 1 < NB ? __float_as_uint(bk[r + 1 < NB ? r + 1 : 0])
                                              : static_cast<uint32_t>(__builtin_amdgcn_update_dpp(-1, static_cast<int>(__float_as_uint(bk[0])), 0x130, 0xf, 0xf, false));   // wave_shl:1
             const uint64_t real = ballot(k < pad);
-            equal |= ballot(k == next) & real;
-            behind |= ballot(bv[r] != kInvalid) & ~real;
+            any |= (ballot(k == next) & real) | (ballot(bv[r] != kInvalid) & ~real);
         }
-        tied = equal != 0;
-        beyond = behind != 0;
+        return any != 0;
     }
     __device__ __forceinline__ bool meets_equal(float key, uint64_t em) const {
         uint64_t equal = 0;
@@ -659,8 +681,7 @@ struct Beam {
         }
         reset_pads();
     }
-    // The entering candidates in ascending order at the front of the candidate lists; false if two have the same key.  Not for
-    // a beam with entries behind the padding: there the sorted list's empty slots, left out here, displace them.
+    // The entering candidates in ascending order at the front of the candidate lists; false if two have the same key.
     __device__ __forceinline__ bool rank_candidates(float key, uint64_t em) {
         uint32_t rank = 0;
         uint64_t equal = 0;
@@ -680,53 +701,58 @@ struct Beam {
         return true;
     }
 
+    // What the first candidates of a beam say about it; beside rows at a finite distance those at none are dropped.
+    __device__ __forceinline__ void start_beam(float& key) {
+        const uint64_t finite = ballot(key < FLT_MAX), nans = ballot(key != key);
+        rank_most = finite == 0 && nans != 0 ? kUnordered : ballot(key > FLT_MAX) != 0 ? 0 : kRankMost;
+        if (finite != 0 && key != key) {
+            key = FLT_MAX;
+            cid = kInvalid;
+        }
+    }
+
+    // reference update_result_buffer: sort the candidates, then fold them into the beam
+    //
     // Rows at a distance that is not a number (a NaN in the row or in the query) compare with nothing, and a network that
     // meets one leaves its other keys unsorted.  They are no candidates, except while there are no others: the entry's
     // neighbours then make up the beam unsorted and are expanded like any entry (a query with a NaN ends with them), until an
     // expansion finds a row at a finite distance and a new beam starts with that expansion's candidates.
-    // `fresh`: whether the beam is to start with this expansion; false if the beam stays as it is.
-    __device__ __forceinline__ bool admit(bool& fresh, bool some_finite, bool some_nan) {
-        if (fresh || unordered) {
-            if (!fresh && !some_finite) return false;
-            unordered = some_nan && !some_finite;
-            fresh = true;
-        }
-        return true;
-    }
-
-    // reference update_result_buffer: sort the candidates, then fold them into the beam
     __device__ __forceinline__ void absorb(bool first) {
         // No row scored: every candidate distance is FLT_MAX, the sort would not move anything (equal keys are never
         // exchanged) and no candidate can displace a beam entry, so the beam stays as it is.
         if (!first && last_scored == 0) return;
-        bool fresh = first;
         if constexpr (NC == 1) {
             float key = slot_distance(0);
-            if (first || unordered) {
-                if (!admit(fresh, ballot(key < FLT_MAX) != 0, ballot(key != key) != 0)) return;
-                if (!unordered && key != key) {
-                    key = FLT_MAX;
-                    cid = kInvalid;
-                }
+            if (first) {
+                start_beam(key);
                 wave_sync();
-                sort_candidates_lane(key, unordered);
+                sort_candidates_lane(key, rank_most == kUnordered);
             } else {
-                const uint64_t em = entering(key);   // without those that are not a number; a sorted list has them behind all others
+                const uint64_t em = entering(key);
                 if (em == 0) return;
                 const uint32_t m = __popcll(em);
-                if (m <= kInsertMost && !tied && !beyond && !meets_equal(key, em)) {
+                if (m <= kInsertMost && !tied && !meets_equal(key, em)) {
                     insert(key, em);
                     return;
                 }
                 wave_sync();
-                if (m > kRankMost || beyond || !rank_candidates(key, em)) sort_candidates_lane(key, false);
+                if (static_cast<int>(m) > rank_most || !rank_candidates(key, em)) {
+                    // An unordered beam's keys are above all others and count as tied, so every candidate that enters one comes here
+                    // (one that took none of its rows in has none to expand either, and no candidates follow).
+                    if (rank_most == kUnordered) {
+                        if (ballot(key < FLT_MAX) == 0) return;
+                        start_beam(key);
+                        first = true;
+                    }
+                    sort_candidates_lane(key, false);
+                }
             }
         } else {
-            if (!distances_to_slots(fresh)) return;
+            if (!distances_to_slots(first)) return;
             if constexpr (MAX_CAND > 128) sort_candidates_two();
             else sort_candidates_one();
         }
-        if (fresh) {
+        if (first) {
 #pragma unroll
             for (int r = 0; r < NB; r++) {
                 const uint32_t e = NB * lane + r;
@@ -741,7 +767,7 @@ struct Beam {
             merge_beam();
         }
         wave_sync();
-        if constexpr (NC == 1) note_order();
+        if constexpr (NC == 1) tied = has_ties();
     }
 
     // first unexplored beam entry (reference select_current_point); marks it explored
