@@ -141,7 +141,7 @@ __device__ __forceinline__ void score_list(const RowRegs<DIMV>& ref, const float
 
 // TEAM: the beam's wavefront is one of several in its workgroup (the others only score rows, see search_team_kernel).
 // WHOLE: the host promises beam == MAX_BEAM (asked for beams above 256 only, i.e. beam 512): the two-half merge of such a
-// beam needs no lane permutations (merge_beam_full), and the kernel 112 registers instead of 128.
+// beam needs no lane permutations and tracks no turning points (merge_beam_full).
 template <int MAX_CAND, int MAX_BEAM, int DIMV, bool TEAM = false, bool WHOLE = false>
 struct Beam {
     static_assert(!WHOLE || MAX_BEAM > 256, "beams up to 256 merge in the registers anyway");

@@ -110,7 +110,7 @@ __device__ __forceinline__ uint32_t prune_pool_refine(PL* pl, uint32_t pool_size
     for (uint32_t i = lane; i < PL::kCap; i += 64) pl->neighbor[i] = kInvalid;
     // Which entries are admissible does not change while the pool shrinks: settled once, the others marked in the top bit of
     // their id (ids are below 2^31), which moves with them.  Compared slot by slot in every round, they were some
-    // 160 instructions and as many LDS reads a round (cosine build of 235k rows 63.5 -> 62.6 ms).
+    // 160 instructions and as many LDS reads a round.  What that takes off a build is below the spread of its runs (1 %).
     for (uint32_t base = 0; base < pool_size; base += 64) {
         const uint32_t i = base + lane;
         const uint32_t id = i < pool_size ? pl->pool_id[i] : self;
