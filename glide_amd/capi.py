@@ -61,7 +61,11 @@ def device_info():
 
 
 class DeviceArray:
-    """A typed device allocation owned through glide_hip_malloc / glide_hip_free."""
+    """A typed device allocation owned through glide_hip_malloc / glide_hip_free.
+
+    `writes` counts the calls of this module that wrote into it.  Reading `ptr` hands out its address, and with it the means
+    to write unseen: the array counts as `shared` from then on.  What is derived from an array's contents and kept (the
+    index's rows as bytes) holds while the array is not shared and its `writes` have not moved."""
 
     def __init__(self, shape, dtype):
         self.shape = tuple(int(s) for s in (shape if isinstance(shape, (tuple, list)) else (shape,)))
@@ -69,7 +73,13 @@ class DeviceArray:
         self.nbytes = int(np.prod(self.shape, dtype=np.int64)) * self.dtype.itemsize
         p = vp()
         check(lib().glide_hip_malloc(C.byref(p), C.c_size_t(self.nbytes)), "glide_hip_malloc")
-        self.ptr = p.value
+        self._address = p.value
+        self.writes, self.shared = 0, False
+
+    @property
+    def ptr(self):
+        self.shared = True
+        return self._address
 
     @classmethod
     def from_numpy(cls, arr, dtype=None):
@@ -83,25 +93,27 @@ class DeviceArray:
         d = cls(shape, dtype)
         assert d.dtype.itemsize == 4
         v = int(np.array([value], dtype=d.dtype).view(np.uint32)[0])
-        check(lib().glide_hip_fill_u32(vp(d.ptr), u32(v), C.c_size_t(d.nbytes // 4), None), "glide_hip_fill_u32")
+        check(lib().glide_hip_fill_u32(vp(d._address), u32(v), C.c_size_t(d.nbytes // 4), None), "glide_hip_fill_u32")
         return d
 
     def upload(self, arr):
         arr = np.ascontiguousarray(arr, dtype=self.dtype)
         assert arr.nbytes == self.nbytes
-        check(lib().glide_hip_memcpy_h2d(vp(self.ptr), arr.ctypes.data_as(vp), C.c_size_t(self.nbytes), None),
+        self.writes += 1
+        check(lib().glide_hip_memcpy_h2d(vp(self._address), arr.ctypes.data_as(vp), C.c_size_t(self.nbytes), None),
               "glide_hip_memcpy_h2d")
 
     def numpy(self):
         out = np.empty(self.shape, dtype=self.dtype)
-        check(lib().glide_hip_memcpy_d2h(out.ctypes.data_as(vp), vp(self.ptr), C.c_size_t(self.nbytes), None),
+        check(lib().glide_hip_memcpy_d2h(out.ctypes.data_as(vp), vp(self._address), C.c_size_t(self.nbytes), None),
               "glide_hip_memcpy_d2h")
         return out
 
     def free(self):
-        if self.ptr:
-            lib().glide_hip_free(vp(self.ptr))
-            self.ptr = None
+        if self._address:
+            lib().glide_hip_free(vp(self._address))
+            self._address = None
+            self.writes += 1
 
     def __del__(self):
         try:
@@ -128,12 +140,20 @@ def _ptr(x):
     if x is None:
         return vp(None)
     if isinstance(x, DeviceArray):
-        return vp(x.ptr)
+        return vp(x._address)
     if isinstance(x, int):
         return vp(x)
     if hasattr(x, "data_ptr"):
         return vp(x.data_ptr())
     raise TypeError("not a device buffer: %r" % type(x))
+
+
+def _out(x, stream=None):
+    """_ptr of a buffer that the call writes; on a stream of the caller's, at a time that is not known here."""
+    if isinstance(x, DeviceArray):
+        x.writes += 1
+        x.shared |= stream is not None
+    return _ptr(x)
 
 
 def synchronize(stream=None):
@@ -165,12 +185,12 @@ class Event:
 # ------------------------------------------------------------------------------------------- entry points
 def search(data, num, dim, graph, graph_degree, centroids, centroid_num, start_points, queries, query_num, top_k,
            beam, max_iterations, min_iterations, hash_bit, hash_reset_interval, metric, result_ids, result_dists,
-           counters=None, stream=None):
-    check(lib().glide_hip_search(_ptr(data), u32(num), u32(dim), _ptr(graph), u32(graph_degree), _ptr(centroids),
-                                 u32(centroid_num), _ptr(start_points), _ptr(queries), u32(query_num), u32(top_k),
-                                 u32(beam), u32(max_iterations), u32(min_iterations), u32(hash_bit),
-                                 u32(hash_reset_interval), C.c_int(metric), _ptr(result_ids), _ptr(result_dists),
-                                 _ptr(counters), vp(stream)), "glide_hip_search")
+           counters=None, stream=None, byte_rows=None):
+    check(lib().glide_hip_search_bytes(_ptr(data), _ptr(byte_rows), u32(num), u32(dim), _ptr(graph), u32(graph_degree), _ptr(centroids),
+                                       u32(centroid_num), _ptr(start_points), _ptr(queries), u32(query_num), u32(top_k),
+                                       u32(beam), u32(max_iterations), u32(min_iterations), u32(hash_bit),
+                                       u32(hash_reset_interval), C.c_int(metric), _out(result_ids), _out(result_dists),
+                                       _out(counters), vp(stream)), "glide_hip_search")
 
 
 def search_merged(data, num, dim, graph, graph_degree, centroids, centroid_num, start_points, queries, query_num, top_k,
@@ -179,49 +199,49 @@ def search_merged(data, num, dim, graph, graph_degree, centroids, centroid_num, 
     check(lib().glide_hip_search_merged(_ptr(data), u32(num), u32(dim), _ptr(graph), u32(graph_degree), _ptr(centroids),
                                         u32(centroid_num), _ptr(start_points), _ptr(queries), u32(query_num), u32(top_k),
                                         u32(beam), u32(max_iterations), u32(min_iterations), u32(hash_bit),
-                                        u32(hash_reset_interval), C.c_int(metric), _ptr(result_ids), _ptr(result_dists),
-                                        _ptr(counters), vp(stream)), "glide_hip_search_merged")
+                                        u32(hash_reset_interval), C.c_int(metric), _out(result_ids), _out(result_dists),
+                                        _out(counters), vp(stream)), "glide_hip_search_merged")
 
 
 def distance_batch(a, b, n, dim, metric, out, stream=None):
-    check(lib().glide_hip_distance_batch(_ptr(a), _ptr(b), u32(n), u32(dim), C.c_int(metric), _ptr(out), vp(stream)),
+    check(lib().glide_hip_distance_batch(_ptr(a), _ptr(b), u32(n), u32(dim), C.c_int(metric), _out(out), vp(stream)),
           "glide_hip_distance_batch")
 
 
 def bitonic_sort_kv(keys, vals, m, batch, stream=None):
-    check(lib().glide_hip_bitonic_sort_kv(_ptr(keys), _ptr(vals), u32(m), u32(batch), vp(stream)),
+    check(lib().glide_hip_bitonic_sort_kv(_out(keys), _out(vals), u32(m), u32(batch), vp(stream)),
           "glide_hip_bitonic_sort_kv")
 
 
 def bitonic_merge_kv(keys, vals, m, batch, stream=None):
-    check(lib().glide_hip_bitonic_merge_kv(_ptr(keys), _ptr(vals), u32(m), u32(batch), vp(stream)),
+    check(lib().glide_hip_bitonic_merge_kv(_out(keys), _out(vals), u32(m), u32(batch), vp(stream)),
           "glide_hip_bitonic_merge_kv")
 
 
 def hashmap_insert_seq(table, bitlen, keys, n, flags, stream=None):
-    check(lib().glide_hip_hashmap_insert_seq(_ptr(table), u32(bitlen), _ptr(keys), u32(n), _ptr(flags), vp(stream)),
+    check(lib().glide_hip_hashmap_insert_seq(_out(table), u32(bitlen), _ptr(keys), u32(n), _out(flags), vp(stream)),
           "glide_hip_hashmap_insert_seq")
 
 
 def build_subgraph(reorder_data, num, dim, knn_graph, knn_degree, mp, segment_starts, segment_lengths, segment_num,
                    start_points, graph_degree, beam, max_iterations, min_iterations, hash_bit, hash_reset_interval,
-                   relaxant, metric, graph, counters=None, stream=None):
-    check(lib().glide_hip_build_subgraph(_ptr(reorder_data), u32(num), u32(dim), _ptr(knn_graph), u32(knn_degree),
-                                         _ptr(mp), _ptr(segment_starts), _ptr(segment_lengths), u32(segment_num),
-                                         _ptr(start_points), u32(graph_degree), u32(beam), u32(max_iterations),
-                                         u32(min_iterations), u32(hash_bit), u32(hash_reset_interval), f32(relaxant),
-                                         C.c_int(metric), _ptr(graph), _ptr(counters), vp(stream)),
+                   relaxant, metric, graph, counters=None, stream=None, byte_rows=None):
+    check(lib().glide_hip_build_subgraph_bytes(_ptr(reorder_data), _ptr(byte_rows), u32(num), u32(dim), _ptr(knn_graph), u32(knn_degree),
+                                               _ptr(mp), _ptr(segment_starts), _ptr(segment_lengths), u32(segment_num),
+                                               _ptr(start_points), u32(graph_degree), u32(beam), u32(max_iterations),
+                                               u32(min_iterations), u32(hash_bit), u32(hash_reset_interval), f32(relaxant),
+                                               C.c_int(metric), _out(graph), _out(counters), vp(stream)),
           "glide_hip_build_subgraph")
 
 
 def build_boundary(reorder_data, num, reorder_num, dim, knn_graph, knn_degree, mp, start_point, graph_degree, beam,
                    max_iterations, min_iterations, hash_bit, hash_reset_interval, relaxant, metric, graph,
-                   counters=None, stream=None):
-    check(lib().glide_hip_build_boundary(_ptr(reorder_data), u32(num), u32(reorder_num), u32(dim), _ptr(knn_graph),
-                                         u32(knn_degree), _ptr(mp), u32(start_point), u32(graph_degree), u32(beam),
-                                         u32(max_iterations), u32(min_iterations), u32(hash_bit),
-                                         u32(hash_reset_interval), f32(relaxant), C.c_int(metric), _ptr(graph),
-                                         _ptr(counters), vp(stream)), "glide_hip_build_boundary")
+                   counters=None, stream=None, byte_rows=None):
+    check(lib().glide_hip_build_boundary_bytes(_ptr(reorder_data), _ptr(byte_rows), u32(num), u32(reorder_num), u32(dim), _ptr(knn_graph),
+                                               u32(knn_degree), _ptr(mp), u32(start_point), u32(graph_degree), u32(beam),
+                                               u32(max_iterations), u32(min_iterations), u32(hash_bit),
+                                               u32(hash_reset_interval), f32(relaxant), C.c_int(metric), _out(graph),
+                                               _out(counters), vp(stream)), "glide_hip_build_boundary")
 
 
 def reverse_edges_workspace_bytes(num, graph_degree):
@@ -231,32 +251,32 @@ def reverse_edges_workspace_bytes(num, graph_degree):
 
 
 def reverse_edges(graph, num, graph_degree, reverse_graph, reverse_counts, workspace, workspace_bytes, stream=None):
-    check(lib().glide_hip_reverse_edges(_ptr(graph), u32(num), u32(graph_degree), _ptr(reverse_graph),
-                                        _ptr(reverse_counts), _ptr(workspace), C.c_size_t(workspace_bytes),
+    check(lib().glide_hip_reverse_edges(_ptr(graph), u32(num), u32(graph_degree), _out(reverse_graph),
+                                        _out(reverse_counts), _out(workspace), C.c_size_t(workspace_bytes),
                                         vp(stream)), "glide_hip_reverse_edges")
 
 
 def insert_reverse(graph, reverse_graph, reverse_counts, num, graph_degree, stream=None):
-    check(lib().glide_hip_insert_reverse(_ptr(graph), _ptr(reverse_graph), _ptr(reverse_counts), u32(num),
+    check(lib().glide_hip_insert_reverse(_out(graph), _ptr(reverse_graph), _ptr(reverse_counts), u32(num),
                                          u32(graph_degree), vp(stream)), "glide_hip_insert_reverse")
 
 
 def refine(data, num, dim, graph_in, graph_out, graph_degree, centroids, centroid_num, start_points, beam,
            max_iterations, min_iterations, hash_bit, hash_reset_interval, relaxant, metric, counters=None,
-           stream=None, order=None):
-    check(lib().glide_hip_refine(_ptr(data), u32(num), u32(dim), _ptr(graph_in), _ptr(graph_out), u32(graph_degree),
-                                 _ptr(centroids), u32(centroid_num), _ptr(start_points), u32(beam),
-                                 u32(max_iterations), u32(min_iterations), u32(hash_bit), u32(hash_reset_interval),
-                                 f32(relaxant), C.c_int(metric), _ptr(order), _ptr(counters), vp(stream)), "glide_hip_refine")
+           stream=None, order=None, byte_rows=None):
+    check(lib().glide_hip_refine_bytes(_ptr(data), _ptr(byte_rows), u32(num), u32(dim), _ptr(graph_in), _out(graph_out), u32(graph_degree),
+                                       _ptr(centroids), u32(centroid_num), _ptr(start_points), u32(beam),
+                                       u32(max_iterations), u32(min_iterations), u32(hash_bit), u32(hash_reset_interval),
+                                       f32(relaxant), C.c_int(metric), _ptr(order), _out(counters), vp(stream)), "glide_hip_refine")
 
 
 def refine_merged(data, num, dim, graph_in, graph_out, graph_degree, centroids, centroid_num, start_points, beam,
            max_iterations, min_iterations, hash_bit, hash_reset_interval, relaxant, metric, counters=None,
            stream=None, order=None):
-    check(lib().glide_hip_refine_merged(_ptr(data), u32(num), u32(dim), _ptr(graph_in), _ptr(graph_out), u32(graph_degree),
+    check(lib().glide_hip_refine_merged(_ptr(data), u32(num), u32(dim), _ptr(graph_in), _out(graph_out), u32(graph_degree),
                                  _ptr(centroids), u32(centroid_num), _ptr(start_points), u32(beam),
                                  u32(max_iterations), u32(min_iterations), u32(hash_bit), u32(hash_reset_interval),
-                                 f32(relaxant), C.c_int(metric), _ptr(order), _ptr(counters), vp(stream)), "glide_hip_refine_merged")
+                                 f32(relaxant), C.c_int(metric), _ptr(order), _out(counters), vp(stream)), "glide_hip_refine_merged")
 
 
 def _size_fn(name):
@@ -272,8 +292,8 @@ def partition_assign_workspace_bytes(num, centroid_num):
 def partition_assign(data, num, dim, centroids, centroid_num, boundary_factor, metric, segment_indexes,
                      segment_lengths, nearest_dists, workspace, workspace_bytes, stream=None):
     check(lib().glide_hip_partition_assign(_ptr(data), u32(num), u32(dim), _ptr(centroids), u32(centroid_num),
-                                           f32(boundary_factor), C.c_int(metric), _ptr(segment_indexes),
-                                           _ptr(segment_lengths), _ptr(nearest_dists), _ptr(workspace),
+                                           f32(boundary_factor), C.c_int(metric), _out(segment_indexes),
+                                           _out(segment_lengths), _out(nearest_dists), _out(workspace),
                                            C.c_size_t(workspace_bytes), vp(stream)), "glide_hip_partition_assign")
 
 
@@ -293,8 +313,8 @@ def partition_assign_fixed_max_points():
 def partition_assign_fixed(data, num, dim, centroids, centroid_num, boundary_factor, metric, segment_indexes,
                            segment_lengths, nearest_dists, stream=None, check_status=True):
     rc = lib().glide_hip_partition_assign_fixed(_ptr(data), u32(num), u32(dim), _ptr(centroids), u32(centroid_num),
-                                                f32(boundary_factor), C.c_int(metric), _ptr(segment_indexes),
-                                                _ptr(segment_lengths), _ptr(nearest_dists), vp(stream))
+                                                f32(boundary_factor), C.c_int(metric), _out(segment_indexes),
+                                                _out(segment_lengths), _out(nearest_dists), vp(stream))
     if check_status:
         check(rc, "glide_hip_partition_assign_fixed")
     return rc
@@ -302,11 +322,11 @@ def partition_assign_fixed(data, num, dim, centroids, centroid_num, boundary_fac
 
 def reorder(data, num, dim, segment_indexes, segment_starts, reorder_data, mp, stream=None):
     check(lib().glide_hip_reorder(_ptr(data), u32(num), u32(dim), _ptr(segment_indexes), _ptr(segment_starts),
-                                  _ptr(reorder_data), _ptr(mp), vp(stream)), "glide_hip_reorder")
+                                  _out(reorder_data, stream), _out(mp), vp(stream)), "glide_hip_reorder")
 
 
 def sample_rows(data, dim, sample_ids, sample_num, sample, stream=None):
-    check(lib().glide_hip_sample_rows(_ptr(data), u32(dim), _ptr(sample_ids), u32(sample_num), _ptr(sample),
+    check(lib().glide_hip_sample_rows(_ptr(data), u32(dim), _ptr(sample_ids), u32(sample_num), _out(sample, stream),
                                       vp(stream)), "glide_hip_sample_rows")
 
 
@@ -319,13 +339,13 @@ def kmeans_seed_workspace_bytes(sample_num):
 
 
 def kmeans_seed(sample, sample_num, dim, cluster_num, seed, centroids, workspace, workspace_bytes, chosen_rows=None, stream=None):
-    check(lib().glide_hip_kmeans_seed(_ptr(sample), u32(sample_num), u32(dim), u32(cluster_num), u32(seed), _ptr(centroids),
-                                      _ptr(chosen_rows), _ptr(workspace), C.c_size_t(workspace_bytes), vp(stream)), "glide_hip_kmeans_seed")
+    check(lib().glide_hip_kmeans_seed(_ptr(sample), u32(sample_num), u32(dim), u32(cluster_num), u32(seed), _out(centroids),
+                                      _out(chosen_rows), _out(workspace), C.c_size_t(workspace_bytes), vp(stream)), "glide_hip_kmeans_seed")
 
 
 def kmeans_fit(sample, sample_num, dim, cluster_num, iterations, centroids, workspace, workspace_bytes, stream=None):
     check(lib().glide_hip_kmeans_fit(_ptr(sample), u32(sample_num), u32(dim), u32(cluster_num), u32(iterations),
-                                     _ptr(centroids), _ptr(workspace), C.c_size_t(workspace_bytes), vp(stream)),
+                                     _out(centroids), _out(workspace), C.c_size_t(workspace_bytes), vp(stream)),
           "glide_hip_kmeans_fit")
 
 
@@ -337,8 +357,8 @@ def nnd_build(reorder_data, reorder_num, dim, segment_starts, segment_lengths, s
               termination_threshold, seed, knn_graph, workspace, workspace_bytes, stats=None, stream=None):
     check(lib().glide_hip_nnd_build(_ptr(reorder_data), u32(reorder_num), u32(dim), _ptr(segment_starts),
                                     _ptr(segment_lengths), u32(segment_num), u32(knn_degree), u32(iterations),
-                                    f32(termination_threshold), u32(seed), _ptr(knn_graph), _ptr(workspace),
-                                    C.c_size_t(workspace_bytes), _ptr(stats), vp(stream)), "glide_hip_nnd_build")
+                                    f32(termination_threshold), u32(seed), _out(knn_graph), _out(workspace),
+                                    C.c_size_t(workspace_bytes), _out(stats), vp(stream)), "glide_hip_nnd_build")
 
 
 class NndLayout(C.Structure):
@@ -356,13 +376,13 @@ def nnd_layout(reorder_num, dim, knn_degree):
 
 def _nnd_stage(name, reorder_num, dim, segment_starts, segment_lengths, segment_num, knn_degree, workspace, workspace_bytes, stream):
     check(getattr(lib(), name)(u32(reorder_num), u32(dim), _ptr(segment_starts), _ptr(segment_lengths), u32(segment_num),
-                               u32(knn_degree), _ptr(workspace), C.c_size_t(workspace_bytes), vp(stream)), name)
+                               u32(knn_degree), _out(workspace), C.c_size_t(workspace_bytes), vp(stream)), name)
 
 
 def nnd_prepare(reorder_data, reorder_num, dim, segment_starts, segment_lengths, segment_num, knn_degree, seed, workspace,
                 workspace_bytes, stream=None):
     check(lib().glide_hip_nnd_prepare(_ptr(reorder_data), u32(reorder_num), u32(dim), _ptr(segment_starts), _ptr(segment_lengths),
-                                      u32(segment_num), u32(knn_degree), u32(seed), _ptr(workspace), C.c_size_t(workspace_bytes),
+                                      u32(segment_num), u32(knn_degree), u32(seed), _out(workspace), C.c_size_t(workspace_bytes),
                                       vp(stream)), "glide_hip_nnd_prepare")
 
 
@@ -385,23 +405,32 @@ def nnd_merge(*args, stream=None):
 def nnd_converge(reorder_num, dim, segment_starts, segment_lengths, segment_num, knn_degree, termination_threshold, workspace,
                  workspace_bytes, stream=None):
     check(lib().glide_hip_nnd_converge(u32(reorder_num), u32(dim), _ptr(segment_starts), _ptr(segment_lengths), u32(segment_num),
-                                       u32(knn_degree), f32(termination_threshold), _ptr(workspace), C.c_size_t(workspace_bytes),
+                                       u32(knn_degree), f32(termination_threshold), _out(workspace), C.c_size_t(workspace_bytes),
                                        vp(stream)), "glide_hip_nnd_converge")
 
 
 def nnd_finalize(reorder_num, dim, segment_starts, segment_lengths, segment_num, knn_degree, knn_graph, stats, workspace,
                  workspace_bytes, stream=None):
     check(lib().glide_hip_nnd_finalize(u32(reorder_num), u32(dim), _ptr(segment_starts), _ptr(segment_lengths), u32(segment_num),
-                                       u32(knn_degree), _ptr(knn_graph), _ptr(stats), _ptr(workspace), C.c_size_t(workspace_bytes),
+                                       u32(knn_degree), _out(knn_graph), _out(stats), _out(workspace), C.c_size_t(workspace_bytes),
                                        vp(stream)), "glide_hip_nnd_finalize")
 
 
 def widen_u8(src, count, dst, stream=None):
-    check(lib().glide_hip_widen_u8(_ptr(src), C.c_size_t(count), _ptr(dst), vp(stream)), "glide_hip_widen_u8")
+    check(lib().glide_hip_widen_u8(_ptr(src), C.c_size_t(count), _out(dst, stream), vp(stream)), "glide_hip_widen_u8")
+
+
+def byte_rows_bytes(num, dim):
+    return int(_size_fn("glide_hip_byte_rows_bytes")(u32(num), u32(dim)))
+
+
+def pack_byte_rows(rows, num, dim, byte_rows, other_values, stream=None):
+    check(lib().glide_hip_pack_byte_rows(_ptr(rows), u32(num), u32(dim), _out(byte_rows), _out(other_values), vp(stream)),
+          "glide_hip_pack_byte_rows")
 
 
 def copy_rows(src, num, src_dim, dst, dst_dim, stream=None):
-    check(lib().glide_hip_copy_rows(_ptr(src), C.c_uint64(num), C.c_uint32(src_dim), _ptr(dst), C.c_uint32(dst_dim), vp(stream)),
+    check(lib().glide_hip_copy_rows(_ptr(src), C.c_uint64(num), C.c_uint32(src_dim), _out(dst, stream), C.c_uint32(dst_dim), vp(stream)),
           "glide_hip_copy_rows")
 
 
@@ -410,38 +439,38 @@ def build_segment(segment_data, num, dim, knn_graph, knn_degree, start_point, gr
     check(lib().glide_hip_build_segment(_ptr(segment_data), u32(num), u32(dim), _ptr(knn_graph), u32(knn_degree),
                                         u32(start_point), u32(graph_degree), u32(beam), u32(max_iterations),
                                         u32(min_iterations), u32(hash_bit), u32(hash_reset_interval), f32(relaxant),
-                                        C.c_int(metric), _ptr(graph), _ptr(counters), vp(stream)), "glide_hip_build_segment")
+                                        C.c_int(metric), _out(graph), _out(counters), vp(stream)), "glide_hip_build_segment")
 
 
 def place_segment_graph(segment_graph, segment_length, graph_degree, segment_start, merged_graph, stream=None):
     check(lib().glide_hip_place_segment_graph(_ptr(segment_graph), u32(segment_length), u32(graph_degree), u32(segment_start),
-                                              _ptr(merged_graph), vp(stream)), "glide_hip_place_segment_graph")
+                                              _out(merged_graph), vp(stream)), "glide_hip_place_segment_graph")
 
 
 def merge_boundary_graph(boundary_graph, boundary_num, graph_degree, home_rows, merged_graph, stream=None):
     check(lib().glide_hip_merge_boundary_graph(_ptr(boundary_graph), u32(boundary_num), u32(graph_degree), _ptr(home_rows),
-                                               _ptr(merged_graph), vp(stream)), "glide_hip_merge_boundary_graph")
+                                               _out(merged_graph), vp(stream)), "glide_hip_merge_boundary_graph")
 
 
 def refine_segment(segment_data, num, dim, graph_in, graph_out, graph_degree, start_point, beam, max_iterations,
                    min_iterations, hash_bit, hash_reset_interval, relaxant, metric, counters=None, stream=None):
-    check(lib().glide_hip_refine_segment(_ptr(segment_data), u32(num), u32(dim), _ptr(graph_in), _ptr(graph_out),
+    check(lib().glide_hip_refine_segment(_ptr(segment_data), u32(num), u32(dim), _ptr(graph_in), _out(graph_out),
                                          u32(graph_degree), u32(start_point), u32(beam), u32(max_iterations),
                                          u32(min_iterations), u32(hash_bit), u32(hash_reset_interval), f32(relaxant),
-                                         C.c_int(metric), _ptr(counters), vp(stream)), "glide_hip_refine_segment")
+                                         C.c_int(metric), _out(counters), vp(stream)), "glide_hip_refine_segment")
 
 
 def select_segments(queries, query_num, dim, centroids, centroid_num, min_segment_num, boundary_factor, metric,
                     segment_ids, stream=None):
     check(lib().glide_hip_select_segments(_ptr(queries), u32(query_num), u32(dim), _ptr(centroids), u32(centroid_num),
                                           u32(min_segment_num), f32(boundary_factor), C.c_int(metric),
-                                          _ptr(segment_ids), vp(stream)), "glide_hip_select_segments")
+                                          _out(segment_ids), vp(stream)), "glide_hip_select_segments")
 
 
 def group_queries(segment_ids, query_num, centroid_num, counts, offsets, lists, stream=None):
     wb = int(_size_fn("glide_hip_group_queries_workspace_bytes")(u32(centroid_num)))
     ws = DeviceArray(wb // 4 + 1, np.uint32)
-    check(lib().glide_hip_group_queries(_ptr(segment_ids), u32(query_num), u32(centroid_num), _ptr(counts), _ptr(offsets), _ptr(lists),
+    check(lib().glide_hip_group_queries(_ptr(segment_ids), u32(query_num), u32(centroid_num), _out(counts), _out(offsets), _out(lists),
                                         _ptr(ws), C.c_size_t(wb), vp(stream)), "glide_hip_group_queries")
     synchronize(stream)      # the workspace is released on return
 
@@ -452,8 +481,8 @@ def search_sub_listed(segment_data, dim, segment_graph, graph_degree, segment_ma
     check(lib().glide_hip_search_sub_listed(_ptr(segment_data), u32(dim), _ptr(segment_graph), u32(graph_degree), _ptr(segment_map),
                                             _ptr(queries), u32(query_num), _ptr(query_list), u32(list_len), u32(segment_id),
                                             u32(start_point), u32(top_k), u32(beam), u32(max_iterations), u32(min_iterations),
-                                            u32(hash_bit), u32(hash_reset_interval), C.c_int(metric), _ptr(final_ids), _ptr(final_dists),
-                                            _ptr(counters), vp(stream)), "glide_hip_search_sub_listed")
+                                            u32(hash_bit), u32(hash_reset_interval), C.c_int(metric), _out(final_ids), _out(final_dists),
+                                            _out(counters), vp(stream)), "glide_hip_search_sub_listed")
 
 
 def search_partitions(data, dim, graph, graph_degree, mp, segment_starts, segment_start_points, segment_num, queries, query_num,
@@ -464,8 +493,8 @@ def search_partitions(data, dim, graph, graph_degree, mp, segment_starts, segmen
     check(lib().glide_hip_search_partitions(_ptr(data), u32(dim), _ptr(graph), u32(graph_degree), _ptr(mp), _ptr(segment_starts),
                                             _ptr(segment_start_points), u32(segment_num), _ptr(queries), u32(query_num), _ptr(segment_ids),
                                             u32(top_k), u32(beam), u32(max_iterations), u32(min_iterations), u32(hash_bit),
-                                            u32(hash_reset_interval), C.c_int(metric), _ptr(final_ids), _ptr(final_dists), _ptr(ws),
-                                            C.c_size_t(wb), _ptr(counters), vp(stream)), "glide_hip_search_partitions")
+                                            u32(hash_reset_interval), C.c_int(metric), _out(final_ids), _out(final_dists), _ptr(ws),
+                                            C.c_size_t(wb), _out(counters), vp(stream)), "glide_hip_search_partitions")
     synchronize(stream)      # the workspace is released on return
 
 
@@ -476,5 +505,5 @@ def search_sub(segment_data, dim, segment_graph, graph_degree, segment_map, quer
                                      _ptr(segment_map), _ptr(queries), u32(query_num), _ptr(segment_ids),
                                      u32(centroid_num), u32(segment_id), u32(start_point), u32(top_k), u32(beam),
                                      u32(max_iterations), u32(min_iterations), u32(hash_bit), u32(hash_reset_interval),
-                                     C.c_int(metric), _ptr(final_ids), _ptr(final_dists), _ptr(counters), vp(stream)),
+                                     C.c_int(metric), _out(final_ids), _out(final_dists), _out(counters), vp(stream)),
           "glide_hip_search_sub")

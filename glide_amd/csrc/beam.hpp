@@ -59,7 +59,10 @@ __device__ __forceinline__ void wave_sync_in() {
 template <int DIMV>
 struct RefInRegs {
     const RowRegs<DIMV>& r;
-    __device__ __forceinline__ float4 chunk(int c, int) const { return r.v[c]; }
+    __device__ __forceinline__ float sqdist(const RowRegs<DIMV>& row, int) const {
+        if constexpr (RowShape<DIMV>::BYTES) return byte_sqdist<DIMV>(r, row.v);
+        else return row_sum<DIMV>(partial_sqdist<DIMV>(r, row));
+    }
 };
 // ... or LDS, laid out as the loads of one lane group would hold it (chunk c of lane t at [c * LPR + t]): the wavefronts
 // of a team share one copy and keep their registers for rows in flight.  The two lane groups of a wide row read the same
@@ -67,13 +70,18 @@ struct RefInRegs {
 template <int DIMV>
 struct RefInLds {
     const float4* q;
-    __device__ __forceinline__ float4 chunk(int c, int t) const { return q[c * RowShape<DIMV>::LPR + t]; }
+    __device__ __forceinline__ float sqdist(const RowRegs<DIMV>& row, int t) const {
+        float acc = 0.f;
+#pragma unroll
+        for (int c = 0; c < RowShape<DIMV>::NV; c++) acc = sqdist4(q[c * RowShape<DIMV>::LPR + t], row.v[c], acc);
+        return row_sum<DIMV>(acc);
+    }
 };
 
 // U steps of RowShape<DIMV>::ROWS rows each (one row per lane group): entries base .. base + ROWS * U of the list.
 // FULL: the rows fill the row shape exactly, so no load needs a mask.
 template <int DIMV, int U, bool FULL, class Ref, class IdFn, class OutFn>
-__device__ __forceinline__ void score_step(const Ref ref, const float* data, uint32_t dim, uint32_t base, uint32_t count, int g, int t,
+__device__ __forceinline__ void score_step(const Ref ref, row_data<DIMV> data, uint32_t dim, uint32_t base, uint32_t count, int g, int t,
                                            IdFn id_of, OutFn out) {
     using Shape = RowShape<DIMV>;
     RowRegs<DIMV> rows[U];
@@ -81,15 +89,12 @@ __device__ __forceinline__ void score_step(const Ref ref, const float* data, uin
     for (int u = 0; u < U; u++) {
         // lane groups past the end re-read the last listed row (same cache lines, no branch); their result is dropped
         const uint32_t idx = base + Shape::ROWS * u + g;
-        load_row<DIMV, FULL>(rows[u], data + static_cast<size_t>(id_of(idx < count ? idx : count - 1)) * dim, dim, t);
+        load_row<DIMV, FULL>(rows[u], row_at<DIMV>(data, id_of(idx < count ? idx : count - 1), dim), dim, t);
     }
 #pragma unroll
     for (int u = 0; u < U; u++) {
         const uint32_t idx = base + Shape::ROWS * u + g;
-        float acc = 0.f;
-#pragma unroll
-        for (int c = 0; c < Shape::NV; c++) acc = sqdist4(ref.chunk(c, t), rows[u].v[c], acc);
-        const float sq = row_sum<DIMV>(acc);
+        const float sq = ref.sqdist(rows[u], t);
         if (t == 0 && idx < count) out(idx, sq);
     }
 }
@@ -101,11 +106,17 @@ __device__ __forceinline__ void score_step(const Ref ref, const float* data, uin
 // forms it.  A run with at most half its entries takes half the steps: an expansion scores a dozen rows on average, and
 // every step issues its loads and arithmetic whether its lane groups have rows or not.
 template <int DIMV, int U, bool FULL, class Ref, class IdFn, class OutFn>
-__device__ __forceinline__ void score_runs(const Ref ref, const float* data, uint32_t dim, uint32_t first, uint32_t count,
+__device__ __forceinline__ void score_runs(const Ref ref, row_data<DIMV> data, uint32_t dim, uint32_t first, uint32_t count,
                                            int lane, uint32_t member, uint32_t members, IdFn id_of, OutFn out) {
     using Shape = RowShape<DIMV>;
     const int g = Shape::row_of_lane(lane), t = Shape::lane_in_row(lane);
     for (uint32_t base = first + member * Shape::ROWS * U; base < count; base += Shape::ROWS * U * members) {
+        if constexpr (U > 2 && Shape::BYTES) {
+            if (count - base <= Shape::ROWS) {
+                score_step<DIMV, 1, FULL>(ref, data, dim, base, count, g, t, id_of, out);
+                continue;
+            }
+        }
         if constexpr (U > 1) {
             if (count - base <= Shape::ROWS * (U / 2)) {
                 score_step<DIMV, U / 2, FULL>(ref, data, dim, base, count, g, t, id_of, out);
@@ -116,11 +127,11 @@ __device__ __forceinline__ void score_runs(const Ref ref, const float* data, uin
     }
 }
 template <int DIMV, int U, class Ref, class IdFn, class OutFn>
-__device__ __forceinline__ void score_share(const Ref ref, const float* data, uint32_t dim, uint32_t first, uint32_t count,
+__device__ __forceinline__ void score_share(const Ref ref, row_data<DIMV> data, uint32_t dim, uint32_t first, uint32_t count,
                                             int lane, uint32_t member, uint32_t members, IdFn id_of, OutFn out) {
     // Rows of exactly 128 or 256 dims are the usual ones and their searches the ones the vector ALU bounds: no masks there.
     // Longer rows are bound by their bytes, a second copy of the loop would buy them nothing.
-    if constexpr (DIMV <= 2) {
+    if constexpr (DIMV == 1 || DIMV == 2) {
         if (dim == RowShape<DIMV>::LPR * RowShape<DIMV>::NV * 4) {
             score_runs<DIMV, U, true>(ref, data, dim, first, count, lane, member, members, id_of, out);
             return;
@@ -130,12 +141,13 @@ __device__ __forceinline__ void score_share(const Ref ref, const float* data, ui
 }
 
 template <int DIMV, class IdFn, class OutFn>
-__device__ __forceinline__ void score_list(const RowRegs<DIMV>& ref, const float* data, uint32_t dim,
+__device__ __forceinline__ void score_list(const RowRegs<DIMV>& ref, row_data<DIMV> data, uint32_t dim,
                                            uint32_t first, uint32_t count, int lane, IdFn id_of, OutFn out) {
     // Steps in flight.  Rows of more than 512 dims are 2-4 KB each and a step holds only two of them: with one step in
     // flight a wavefront had 8 KB on its way, too little to cover the memory latency when a launch has about one
     // wavefront per SIMD (1 000 queries); four steps took the 960-dim beam-512 search from 16.8 to 13.2 ms.
-    constexpr int U = DIMV == 8 ? 4 : 2;   // rows of more than 1024 dims (DIMV 16, 32) take 64 registers a lane each: two steps
+    // A step of byte rows is one load: four of them (32 or 16 rows) on their way at once.
+    constexpr int U = DIMV == 8 || RowShape<DIMV>::BYTES ? 4 : 2;   // rows of more than 1024 dims (DIMV 16, 32) take 64 registers a lane each: two steps
     score_share<DIMV, U>(RefInRegs<DIMV>{ref}, data, dim, first, count, lane, 0u, 1u, id_of, out);
 }
 
@@ -168,16 +180,30 @@ struct Beam {
     uint32_t cid;           // candidate id of this lane's slot (MAX_CAND == 64; larger buckets keep the ids in LDS)
     uint32_t place[NC];     // where in vlist each of this lane's slots is; kInvalid: not scored
 
-    __device__ __forceinline__ void init(BeamLds<MAX_CAND>* lds_, uint32_t* hash_, const BeamParams& p_, const float* query) {
+    __device__ __forceinline__ void begin(BeamLds<MAX_CAND>* lds_, uint32_t* hash_, const BeamParams& p_) {
         lds = lds_;
         hash = hash_;
         p = p_;
         lane = lane_id();
         asm volatile("" : "+v"(lane));   // as in run: nothing made from it is to be kept from one query to the next
-        load_row<DIMV>(q, query, p.dim, RowShape<DIMV>::lane_in_row(lane));
         until_reset = p.reset_interval;
+    }
+    __device__ __forceinline__ void init(BeamLds<MAX_CAND>* lds_, uint32_t* hash_, const BeamParams& p_, row_data<DIMV> query) {
+        begin(lds_, hash_, p_);
+        load_reference<DIMV>(q, query, p.dim, RowShape<DIMV>::lane_in_row(lane));
         hash_clear(hash, p.hash_bit, lane);
         wave_sync();
+    }
+    // An fp32 query against rows of bytes; false if it is not of bytes itself.
+    __device__ __forceinline__ bool init_packing(BeamLds<MAX_CAND>* lds_, uint32_t* hash_, const BeamParams& p_, const float* query) {
+        static_assert(RowShape<DIMV>::BYTES, "rows of bytes");
+        begin(lds_, hash_, p_);
+        const bool exact = pack_bytes(query, 16 * RowShape<DIMV>::lane_in_row(lane), p.dim, q.v);
+        if (ballot(!exact) != 0) return false;
+        q.sq = dot_bytes(q.v, q.v, 0u);
+        hash_clear(hash, p.hash_bit, lane);
+        wave_sync();
+        return true;
     }
 
     // whether this iteration ends with a reset of the visited set
@@ -239,7 +265,7 @@ struct Beam {
         return nv;
     }
 
-    __device__ __forceinline__ void expand(uint32_t parent, const uint32_t* graph, const float* data,
+    __device__ __forceinline__ void expand(uint32_t parent, const uint32_t* graph, row_data<DIMV> data,
                                            uint32_t exclude_insert, uint32_t exclude_score) {
         const uint32_t nv = expand_list(parent, graph, exclude_insert, exclude_score);
         BeamLds<MAX_CAND>* l = lds;
@@ -804,7 +830,7 @@ struct Beam {
     }
 
     // main loop; candidates of the entry expansion must already be in LDS
-    __device__ __forceinline__ void run(const uint32_t* graph, const float* data, uint32_t self_id) {
+    __device__ __forceinline__ void run(const uint32_t* graph, row_data<DIMV> data, uint32_t self_id) {
         uint32_t iter = 0;
         bool terminate = false;
         while (true) {

@@ -141,29 +141,98 @@ __device__ __forceinline__ uint32_t hash_insert(uint32_t* table, uint32_t bitlen
 //   DIMV 1: 8 lanes x 4 loads (8 rows per wavefront)    DIMV 2: 16 lanes x 4 loads (4 rows)
 //   DIMV 4: 32 lanes x 4 loads (2 rows)                 DIMV 8 / 16: 32 lanes x 8 / 16 loads (2 rows)
 //   DIMV 32: 64 lanes x 16 loads (1 row; up to 4096 dims)
+//   DIMV -1: rows of bytes, 8 lanes x 1 load (8 rows, up to 128 dims)    DIMV -2: 16 lanes x 1 load (4 rows, up to 256 dims)
 template <int DIMV>
 struct RowShape {
-    static_assert(DIMV == 1 || DIMV == 2 || DIMV == 4 || DIMV == 8 || DIMV == 16 || DIMV == 32, "row shape");
-    static constexpr int LPR = DIMV == 1 ? 8 : (DIMV == 2 ? 16 : (DIMV == 32 ? 64 : 32));
-    static constexpr int NV = DIMV >= 16 ? 16 : (DIMV == 8 ? 8 : 4);
+    static_assert(DIMV == 1 || DIMV == 2 || DIMV == 4 || DIMV == 8 || DIMV == 16 || DIMV == 32 || DIMV == -1 || DIMV == -2, "row shape");
+    static constexpr bool BYTES = DIMV < 0;
+    static constexpr int LPR = DIMV == 1 || DIMV == -1 ? 8 : (DIMV == 2 || DIMV == -2 ? 16 : (DIMV == 32 ? 64 : 32));
+    static constexpr int NV = BYTES ? 1 : DIMV >= 16 ? 16 : (DIMV == 8 ? 8 : 4);
     static constexpr int ROWS = 64 / LPR;
+    static constexpr int STRIDE = LPR * 16;   // bytes from row to row, where rows are bytes
     static __device__ __forceinline__ int lane_in_row(int lane) { return lane & (LPR - 1); }
     static __device__ __forceinline__ int row_of_lane(int lane) { return lane / LPR; }
 };
 
-template <int DIMV>
+// Rows of whole numbers 0 .. 255 (image descriptors, quantised embeddings) are searched as bytes: a quarter of the memory
+// traffic, and |x - q|^2 = x.x - 2 x.q + q.q takes eight dot products of four bytes for sixteen dims in place of 32 fp32
+// instructions.  All of it is integer arithmetic and exact; with at most kMostByteDims dims every sum the fp32 form makes
+// stays below 2^24 and is exact as well, so both give the same distances to the bit.  Measured on 128 dims, fp32 : bytes:
+// 10 000 searches of a million rows at beam 64 1 347 : 500 us (rows from memory; 1 query 124 : 110), at beam 256 on the mixture,
+// whose rows come from the caches, 2 320 : 1 710; refinement of a million points 71 : 55 ms (40.6 : 30.6 thousand vector
+// instructions a point, 0.95 of their issue rate), sub-graphs 44 : 33 ms.
+constexpr uint32_t kMostByteDims = 256;   // 256 * 255^2 < 2^24
+constexpr uint32_t kMostByteDegree = 64;  // the searches over rows of bytes are built for one candidate slot a lane
+
+// a lane's share of a row
+template <int DIMV, bool BYTES = RowShape<DIMV>::BYTES>
 struct RowRegs {
     float4 v[RowShape<DIMV>::NV];
 };
+template <int DIMV>
+struct RowRegs<DIMV, true> {
+    uint4 v;
+    uint32_t sq;   // the share's own squared length: set where the row is what others are measured against
+};
+
+template <bool BYTES> struct RowData { using type = const float*; };
+template <> struct RowData<true> { using type = const unsigned char*; };
+template <int DIMV>
+using row_data = typename RowData<RowShape<DIMV>::BYTES>::type;   // where rows are read from
+
+template <int DIMV>
+__device__ __forceinline__ row_data<DIMV> row_at(row_data<DIMV> rows, uint32_t id, uint32_t dim) {
+    if constexpr (RowShape<DIMV>::BYTES) return rows + static_cast<size_t>(id) * RowShape<DIMV>::STRIDE;
+    else return rows + static_cast<size_t>(id) * dim;
+}
 
 // t = RowShape<DIMV>::lane_in_row(lane)
-template <int DIMV, bool FULL = false>   // FULL: dim fills the shape exactly
-__device__ __forceinline__ void load_row(RowRegs<DIMV>& r, const float* row, uint32_t dim, int t) {
+template <int DIMV, bool FULL = false>   // FULL: dim fills the shape exactly (rows of bytes always do: zeros behind them)
+__device__ __forceinline__ void load_row(RowRegs<DIMV>& r, row_data<DIMV> row, uint32_t dim, int t) {
+    if constexpr (RowShape<DIMV>::BYTES) {
+        r.v = *reinterpret_cast<const uint4*>(row + t * 16);
+    } else {
 #pragma unroll
-    for (int c = 0; c < RowShape<DIMV>::NV; c++) {
-        const uint32_t d0 = (c * RowShape<DIMV>::LPR + t) * 4;
-        r.v[c] = FULL || d0 < dim ? *reinterpret_cast<const float4*>(row + d0) : make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int c = 0; c < RowShape<DIMV>::NV; c++) {
+            const uint32_t d0 = (c * RowShape<DIMV>::LPR + t) * 4;
+            r.v[c] = FULL || d0 < dim ? *reinterpret_cast<const float4*>(row + d0) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
     }
+}
+
+__device__ __forceinline__ uint32_t dot_bytes(const uint4& a, const uint4& b, uint32_t acc) {
+    acc = __builtin_amdgcn_udot4(a.x, b.x, acc, false);
+    acc = __builtin_amdgcn_udot4(a.y, b.y, acc, false);
+    acc = __builtin_amdgcn_udot4(a.z, b.z, acc, false);
+    return __builtin_amdgcn_udot4(a.w, b.w, acc, false);
+}
+// a row that others are measured against
+template <int DIMV>
+__device__ __forceinline__ void load_reference(RowRegs<DIMV>& r, row_data<DIMV> row, uint32_t dim, int t) {
+    load_row<DIMV>(r, row, dim, t);
+    if constexpr (RowShape<DIMV>::BYTES) r.sq = dot_bytes(r.v, r.v, 0u);
+}
+
+// Sixteen fp32 values from `row + first` on as bytes; values behind `dim` are zeros.  False: one is no whole number 0 .. 255.
+__device__ __forceinline__ bool pack_bytes(const float* row, uint32_t first, uint32_t dim, uint4& out) {
+    uint32_t word[4];
+    bool exact = true;
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+        const uint32_t d0 = first + 4 * w;
+        const float4 x = d0 < dim ? *reinterpret_cast<const float4*>(row + d0) : make_float4(0.f, 0.f, 0.f, 0.f);
+        const float v[4] = {x.x, x.y, x.z, x.w};
+        word[w] = 0;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const bool in_range = v[e] >= 0.f && v[e] <= 255.f;   // false for what is not a number
+            const uint32_t b = in_range ? static_cast<uint32_t>(v[e]) : 0u;
+            exact &= in_range && static_cast<float>(b) == v[e];
+            word[w] |= b << (8 * e);
+        }
+    }
+    out = make_uint4(word[0], word[1], word[2], word[3]);
+    return exact;
 }
 
 __device__ __forceinline__ float sqdist4(const float4& a, const float4& b, float acc) {
@@ -194,6 +263,18 @@ __device__ __forceinline__ float row_sum(float v) {
     if constexpr (RowShape<DIMV>::LPR >= 32) v += lane_xor<16>(v);
     if constexpr (RowShape<DIMV>::LPR >= 64) v += lane_xor<32>(v);
     return v;
+}
+
+// Squared distance of a row to a reference row, both spread over a group of lanes; every lane of a group ends with it.
+template <int DIMV>
+__device__ __forceinline__ float byte_sqdist(const RowRegs<DIMV>& ref, const uint4& x) {
+    static_assert(RowShape<DIMV>::BYTES, "rows of bytes");
+    int v = static_cast<int>(dot_bytes(x, x, ref.sq)) - 2 * static_cast<int>(dot_bytes(ref.v, x, 0u));
+    v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, false);   // row_half_mirror
+    if constexpr (RowShape<DIMV>::LPR >= 16) v += __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, false);   // row_mirror
+    return static_cast<float>(v);
 }
 
 // reference distance.cuh:22-26: Euclidean reports sqrt, Cosine the squared L2 of pre-normalised rows

@@ -109,6 +109,26 @@ __global__ __launch_bounds__(256) void insert_reverse_kernel(uint32_t* graph, co
     }
 }
 
+// ------------------------------------------------------------------------------------------ rows as bytes
+// fp32 rows -> bytes, zeros behind them, sixteen dims a thread; *other is set if a value is no whole number 0 .. 255.  Bound by
+// reading the rows (1M x 128: 0.11 ms, 5.9 TB/s with what it writes).  The first workgroups are a launch of their own: rows
+// of fractions end there, and the others find the word set and leave (in one launch every wavefront reads its rows before
+// the word says anything, and all of them write it: 0.36 ms for 300k x 96 fractions).
+constexpr uint32_t kPackProbe = 64;
+__global__ __launch_bounds__(256) void pack_bytes_kernel(const float* rows, uint32_t num, uint32_t dim, uint32_t lanes, uint32_t first_block, uint4* bytes,
+                                                         uint32_t* other) {
+    if (*other != 0) return;
+    const size_t i = static_cast<size_t>(first_block + blockIdx.x) * 256 + threadIdx.x;
+    const size_t row = i / lanes;
+    bool exact = true;
+    if (row < num) {
+        uint4 out;
+        exact = pack_bytes(rows + row * dim, 16 * static_cast<uint32_t>(i % lanes), dim, out);
+        bytes[i] = out;
+    }
+    if (ballot(!exact) != 0 && lane_id() == 0) *other = 1u;
+}
+
 // ------------------------------------------------------------------------------------------ merged large build
 // A staged partition's sub-graph holds partition-local ids.  Its rows go to rows segment_start .. of the merged graph
 // with segment_start added to every id (what map_to_graph does through `map` on the small path,
@@ -156,8 +176,11 @@ int check_beam_sizes(uint32_t degree, uint32_t graph_degree, uint32_t beam, uint
     return GLIDE_OK;
 }
 
+bool byte_rows_serve(const unsigned char* bytes, uint32_t degree, uint32_t dim) { return bytes && degree <= kMostByteDegree && dim <= kMostByteDims; }
+
 int launch_build(BuildArgs& a, hipStream_t stream) {
-    build_fn fn = pick_build(a.p.degree, a.p.beam, a.p.dim);
+    if (reinterpret_cast<uintptr_t>(a.bytes) % 16) return GLIDE_ERR_BAD_ARGUMENT;
+    build_fn fn = byte_rows_serve(a.bytes, a.p.degree, a.p.dim) ? pick_build_bytes(a.p.beam, a.p.dim) : pick_build(a.p.degree, a.p.beam, a.p.dim);
     const size_t lds_bytes = beam_lds_bytes(a.p.degree) + prune_lds_bytes(a.p.beam) + (size_t{1} << a.p.hash_bit) * sizeof(uint32_t);
     GLIDE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)));
     hipLaunchKernelGGL(fn, dim3(a.point_count), dim3(64), lds_bytes, stream, a);
@@ -175,6 +198,16 @@ int glide_hip_build_subgraph(const float* reorder_data, uint32_t num, uint32_t d
                              uint32_t segment_num, const uint32_t* start_points, uint32_t graph_degree, uint32_t beam,
                              uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit, uint32_t hash_reset_interval,
                              float relaxant, int metric, uint32_t* graph, unsigned long long* counters, void* stream) {
+    return glide_hip_build_subgraph_bytes(reorder_data, nullptr, num, dim, knn_graph, knn_degree, map, segment_starts, segment_lengths, segment_num,
+                                          start_points, graph_degree, beam, max_iterations, min_iterations, hash_bit, hash_reset_interval, relaxant,
+                                          metric, graph, counters, stream);
+}
+
+int glide_hip_build_subgraph_bytes(const float* reorder_data, const void* byte_rows, uint32_t num, uint32_t dim, const uint32_t* knn_graph,
+                                   uint32_t knn_degree, const uint32_t* map, const uint32_t* segment_starts, const uint32_t* segment_lengths,
+                                   uint32_t segment_num, const uint32_t* start_points, uint32_t graph_degree, uint32_t beam,
+                                   uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit, uint32_t hash_reset_interval,
+                                   float relaxant, int metric, uint32_t* graph, unsigned long long* counters, void* stream) {
     if (!reorder_data || !knn_graph || !map || !segment_starts || !segment_lengths || !start_points || !graph)
         return GLIDE_ERR_BAD_ARGUMENT;
     if (max_iterations == 0 || segment_num == 0) return GLIDE_ERR_BAD_ARGUMENT;
@@ -183,6 +216,7 @@ int glide_hip_build_subgraph(const float* reorder_data, uint32_t num, uint32_t d
     if (num == 0) return GLIDE_OK;
     BuildArgs a;
     a.reorder_data = reorder_data;
+    a.bytes = static_cast<const unsigned char*>(byte_rows);
     a.knn_graph = knn_graph;
     a.map = map;
     a.segment_starts = segment_starts;
@@ -205,6 +239,15 @@ int glide_hip_build_boundary(const float* reorder_data, uint32_t num, uint32_t r
                              uint32_t knn_degree, const uint32_t* map, uint32_t start_point, uint32_t graph_degree, uint32_t beam,
                              uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit, uint32_t hash_reset_interval,
                              float relaxant, int metric, uint32_t* graph, unsigned long long* counters, void* stream) {
+    return glide_hip_build_boundary_bytes(reorder_data, nullptr, num, reorder_num, dim, knn_graph, knn_degree, map, start_point, graph_degree, beam,
+                                          max_iterations, min_iterations, hash_bit, hash_reset_interval, relaxant, metric, graph, counters, stream);
+}
+
+int glide_hip_build_boundary_bytes(const float* reorder_data, const void* byte_rows, uint32_t num, uint32_t reorder_num, uint32_t dim,
+                                   const uint32_t* knn_graph, uint32_t knn_degree, const uint32_t* map, uint32_t start_point,
+                                   uint32_t graph_degree, uint32_t beam, uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit,
+                                   uint32_t hash_reset_interval, float relaxant, int metric, uint32_t* graph, unsigned long long* counters,
+                                   void* stream) {
     if (!reorder_data || !knn_graph || !map || !graph) return GLIDE_ERR_BAD_ARGUMENT;
     if (max_iterations == 0 || reorder_num < num) return GLIDE_ERR_BAD_ARGUMENT;
     int rc = check_beam_sizes(knn_degree, graph_degree, beam, dim, hash_bit, metric);
@@ -213,6 +256,7 @@ int glide_hip_build_boundary(const float* reorder_data, uint32_t num, uint32_t r
     if (start_point >= reorder_num - num) return GLIDE_ERR_BAD_ARGUMENT;
     BuildArgs a;
     a.reorder_data = reorder_data;
+    a.bytes = static_cast<const unsigned char*>(byte_rows);
     a.knn_graph = knn_graph;
     a.map = map;
     a.segment_starts = nullptr;
@@ -243,6 +287,7 @@ int glide_hip_build_segment(const float* segment_data, uint32_t num, uint32_t di
     if (start_point >= num) return GLIDE_ERR_BAD_ARGUMENT;
     BuildArgs a;
     a.reorder_data = segment_data;
+    a.bytes = nullptr;
     a.knn_graph = knn_graph;
     a.map = nullptr;
     a.segment_starts = nullptr;
@@ -274,6 +319,7 @@ int glide_hip_refine_segment(const float* segment_data, uint32_t num, uint32_t d
     RefineArgs a;
     a.order = nullptr;
     a.data = segment_data;
+    a.bytes = nullptr;
     a.graph_in = graph_in;
     a.graph_out = graph_out;
     a.centroids = nullptr;
@@ -336,6 +382,29 @@ int glide_hip_insert_reverse(uint32_t* graph, const uint32_t* reverse_graph, con
     return launch_status();
 }
 
+size_t glide_hip_byte_rows_bytes(uint32_t num, uint32_t dim) {
+    if (dim == 0 || dim > kMostByteDims || dim % 4 != 0) return 0;
+    return static_cast<size_t>(num) * (dim <= 128 ? RowShape<-1>::STRIDE : RowShape<-2>::STRIDE);
+}
+
+int glide_hip_pack_byte_rows(const float* rows, uint32_t num, uint32_t dim, void* byte_rows, uint32_t* other_values, void* stream) {
+    if (!rows || !byte_rows || !other_values || dim == 0) return GLIDE_ERR_BAD_ARGUMENT;
+    if (dim > kMostByteDims || dim % 4 != 0) return GLIDE_ERR_UNSUPPORTED;
+    if (reinterpret_cast<uintptr_t>(rows) % 16 || reinterpret_cast<uintptr_t>(byte_rows) % 16) return GLIDE_ERR_BAD_ARGUMENT;
+    const int rc = glide_hip_fill_u32(other_values, 0u, 1, stream);
+    if (rc != GLIDE_OK || num == 0) return rc;
+    const uint32_t lanes = dim <= 128 ? RowShape<-1>::LPR : RowShape<-2>::LPR;   // sixteen dims each
+    const size_t blocks = (static_cast<size_t>(num) * lanes + 255) / 256;
+    if (blocks > (1u << 24)) return GLIDE_ERR_UNSUPPORTED;   // 2^32 threads; over 2^28 rows
+    const uint32_t probe = blocks < kPackProbe ? static_cast<uint32_t>(blocks) : kPackProbe;
+    hipLaunchKernelGGL(pack_bytes_kernel, dim3(probe), dim3(256), 0, as_stream(stream), rows, num, dim, lanes, 0u, static_cast<uint4*>(byte_rows),
+                       other_values);
+    if (blocks > probe)
+        hipLaunchKernelGGL(pack_bytes_kernel, dim3(static_cast<uint32_t>(blocks) - probe), dim3(256), 0, as_stream(stream), rows, num, dim, lanes, probe,
+                           static_cast<uint4*>(byte_rows), other_values);
+    return launch_status();
+}
+
 int glide_hip_place_segment_graph(const uint32_t* segment_graph, uint32_t segment_length, uint32_t graph_degree, uint32_t segment_start,
                                   uint32_t* merged_graph, void* stream) {
     if (!segment_graph || !merged_graph || graph_degree == 0) return GLIDE_ERR_BAD_ARGUMENT;
@@ -360,7 +429,7 @@ int glide_hip_merge_boundary_graph(const uint32_t* boundary_graph, uint32_t boun
 }  // extern "C"
 
 namespace {
-int launch_refine(const float* data, uint32_t num, uint32_t dim, const uint32_t* graph_in, uint32_t* graph_out, uint32_t graph_degree,
+int launch_refine(const float* data, const unsigned char* bytes, uint32_t num, uint32_t dim, const uint32_t* graph_in, uint32_t* graph_out, uint32_t graph_degree,
                   const float* centroids, uint32_t centroid_num, bool rank_all_centroids, const uint32_t* start_points, uint32_t beam,
                   uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit, uint32_t hash_reset_interval, float relaxant, int metric,
                   const uint32_t* order, unsigned long long* counters, void* stream) {
@@ -369,9 +438,11 @@ int launch_refine(const float* data, uint32_t num, uint32_t dim, const uint32_t*
     int rc = check_beam_sizes(graph_degree, graph_degree, beam, dim, hash_bit, metric);
     if (rc != GLIDE_OK) return rc;
     if (centroid_num > 256) return GLIDE_ERR_UNSUPPORTED;
+    if (reinterpret_cast<uintptr_t>(bytes) % 16) return GLIDE_ERR_BAD_ARGUMENT;
     if (num == 0) return GLIDE_OK;
     RefineArgs a;
     a.data = data;
+    a.bytes = bytes;
     a.graph_in = graph_in;
     a.graph_out = graph_out;
     a.centroids = centroids;
@@ -385,7 +456,7 @@ int launch_refine(const float* data, uint32_t num, uint32_t dim, const uint32_t*
     a.segment_start_point = 0;
     a.relaxant = relaxant;
     a.p = BeamParams{beam, graph_degree, dim, hash_bit, hash_reset_interval ? hash_reset_interval : 1, max_iterations, min_iterations, metric};
-    refine_fn fn = pick_refine(graph_degree, beam, dim);
+    refine_fn fn = byte_rows_serve(bytes, graph_degree, dim) ? pick_refine_bytes(beam, dim) : pick_refine(graph_degree, beam, dim);
     const size_t lds_bytes = beam_lds_bytes(graph_degree) + prune_lds_bytes_refine(beam, graph_degree) + round_up32(centroid_num) * sizeof(float) +
                              (size_t{1} << hash_bit) * sizeof(uint32_t);
     GLIDE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)));
@@ -399,8 +470,17 @@ extern "C" int glide_hip_refine(const float* data, uint32_t num, uint32_t dim, c
                                 uint32_t beam, uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit,
                                 uint32_t hash_reset_interval, float relaxant, int metric, const uint32_t* order,
                                 unsigned long long* counters, void* stream) {
-    return launch_refine(data, num, dim, graph_in, graph_out, graph_degree, centroids, centroid_num, false, start_points, beam, max_iterations,
+    return launch_refine(data, nullptr, num, dim, graph_in, graph_out, graph_degree, centroids, centroid_num, false, start_points, beam, max_iterations,
                          min_iterations, hash_bit, hash_reset_interval, relaxant, metric, order, counters, stream);
+}
+
+extern "C" int glide_hip_refine_bytes(const float* data, const void* byte_rows, uint32_t num, uint32_t dim, const uint32_t* graph_in,
+                                      uint32_t* graph_out, uint32_t graph_degree, const float* centroids, uint32_t centroid_num,
+                                      const uint32_t* start_points, uint32_t beam, uint32_t max_iterations, uint32_t min_iterations,
+                                      uint32_t hash_bit, uint32_t hash_reset_interval, float relaxant, int metric, const uint32_t* order,
+                                      unsigned long long* counters, void* stream) {
+    return launch_refine(data, static_cast<const unsigned char*>(byte_rows), num, dim, graph_in, graph_out, graph_degree, centroids, centroid_num, false,
+                         start_points, beam, max_iterations, min_iterations, hash_bit, hash_reset_interval, relaxant, metric, order, counters, stream);
 }
 
 extern "C" int glide_hip_refine_merged(const float* data, uint32_t num, uint32_t dim, const uint32_t* graph_in, uint32_t* graph_out,
@@ -408,6 +488,6 @@ extern "C" int glide_hip_refine_merged(const float* data, uint32_t num, uint32_t
                                        uint32_t beam, uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit,
                                        uint32_t hash_reset_interval, float relaxant, int metric, const uint32_t* order,
                                        unsigned long long* counters, void* stream) {
-    return launch_refine(data, num, dim, graph_in, graph_out, graph_degree, centroids, centroid_num, true, start_points, beam, max_iterations,
+    return launch_refine(data, nullptr, num, dim, graph_in, graph_out, graph_degree, centroids, centroid_num, true, start_points, beam, max_iterations,
                          min_iterations, hash_bit, hash_reset_interval, relaxant, metric, order, counters, stream);
 }

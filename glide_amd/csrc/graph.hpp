@@ -20,6 +20,7 @@ struct BuildArgs {
     uint32_t boundary_start_point;
     float relaxant;
     BeamParams p;                         // p.degree = knn_degree
+    const unsigned char* bytes;           // the same rows as bytes; the kernels for rows of bytes read nothing else
 };
 
 struct RefineArgs {
@@ -33,6 +34,7 @@ struct RefineArgs {
     uint32_t num, centroid_num, max_centroid, segment_start_point;
     float relaxant;
     BeamParams p;   // p.degree = graph_degree
+    const unsigned char* bytes;   // the same rows as bytes, for the kernels for rows of bytes
 };
 
 using build_fn = void (*)(BuildArgs);
@@ -44,6 +46,9 @@ build_fn pick_build_256(uint32_t beam, uint32_t dim);
 refine_fn pick_refine_64(uint32_t beam, uint32_t dim);
 refine_fn pick_refine_128(uint32_t beam, uint32_t dim);
 refine_fn pick_refine_256(uint32_t beam, uint32_t dim);
+// rows of bytes: up to 64 slots (kNN degree; graph degree) and kMostByteDims dims
+build_fn pick_build_bytes(uint32_t beam, uint32_t dim);
+refine_fn pick_refine_bytes(uint32_t beam, uint32_t dim);
 inline build_fn pick_build(uint32_t degree, uint32_t beam, uint32_t dim) {
     return degree <= 64 ? pick_build_64(beam, dim) : degree <= 128 ? pick_build_128(beam, dim) : pick_build_256(beam, dim);
 }

@@ -31,18 +31,21 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DIMV > 4 || 
         seg_start = a.segment_starts[seg];
         entry = a.start_points[seg];
     }
-    const float* sdata = a.reorder_data + static_cast<size_t>(seg_start) * a.p.dim;
+    row_data<DIMV> rows;
+    if constexpr (RowShape<DIMV>::BYTES) rows = a.bytes;
+    else rows = a.reorder_data;
+    const row_data<DIMV> sdata = row_at<DIMV>(rows, seg_start, a.p.dim);
     const uint32_t* sgraph = a.knn_graph + static_cast<size_t>(seg_start) * a.p.degree;
 
     Beam<MAX_CAND, MAX_BEAM, DIMV> b;
-    b.init(lds, hash, a.p, a.reorder_data + static_cast<size_t>(point) * a.p.dim);
+    b.init(lds, hash, a.p, row_at<DIMV>(rows, point, a.p.dim));
     // get_init (search_kernel.cuh:336-360): all neighbours of the entry are hashed; the one whose *local* id equals
     // this point's *reorder* id is left unscored (the reference compares across id spaces, graph_kernel.cuh:295-298)
     b.expand(entry, sgraph, sdata, kInvalid, point);
     b.run(sgraph, sdata, point - seg_start);
 
     uint32_t pool = beam_to_pool(b, pl);
-    prune_pool<MAX_BEAM, DIMV>(pl, pool, a.reorder_data, a.p.dim, seg_start, a.graph_degree, a.relaxant, a.p.metric, b.lane,
+    prune_pool<MAX_BEAM, DIMV>(pl, pool, rows, a.p.dim, seg_start, a.graph_degree, a.relaxant, a.p.metric, b.lane,
                                b.cnt.rows_scored);
     wave_sync();
     if (segment_mode) {   // map_to_graph (graph_kernel.cuh:145-150)
@@ -104,17 +107,28 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DIMV > 4 || 
     if (need == 0) return;
 
     Beam<MAX_CAND, MAX_BEAM, DIMV> b;
-    b.init(lds, hash, a.p, a.data + static_cast<size_t>(point) * a.p.dim);
+    row_data<DIMV> rows;
+    if constexpr (RowShape<DIMV>::BYTES) rows = a.bytes;
+    else rows = a.data;
+    b.init(lds, hash, a.p, row_at<DIMV>(rows, point, a.p.dim));
     if (a.centroids != nullptr) {
-        const uint32_t c0 = pick_centroid_refine<DIMV>(a.max_centroid, b.q, a.centroids, a.centroid_num, a.p.dim, a.p.metric, cent, lane);
-        b.expand(a.start_points[c0], a.graph_in, a.data, kInvalid, kInvalid);
+        uint32_t c0;
+        if constexpr (RowShape<DIMV>::BYTES) {
+            constexpr int F = -DIMV;   // centroids are fp32: the shape of an fp32 row of this length
+            RowRegs<F> q;
+            load_row<F>(q, a.data + static_cast<size_t>(point) * a.p.dim, a.p.dim, RowShape<F>::lane_in_row(lane));
+            c0 = pick_centroid_refine<F>(a.max_centroid, q, a.centroids, a.centroid_num, a.p.dim, a.p.metric, cent, lane);
+        } else {
+            c0 = pick_centroid_refine<DIMV>(a.max_centroid, b.q, a.centroids, a.centroid_num, a.p.dim, a.p.metric, cent, lane);
+        }
+        b.expand(a.start_points[c0], a.graph_in, rows, kInvalid, kInvalid);
     } else {   // refine_for_large_kernel (graph_kernel.cuh:796-798): get_init from the segment's start point
-        b.expand(a.segment_start_point, a.graph_in, a.data, kInvalid, point);
+        b.expand(a.segment_start_point, a.graph_in, rows, kInvalid, point);
     }
-    b.run(a.graph_in, a.data, point);
+    b.run(a.graph_in, rows, point);
 
     uint32_t pool = beam_to_pool(b, pl);
-    prune_pool_refine<MAX_BEAM, DIMV>(pl, pool, a.data, a.p.dim, point, D, need, a.relaxant, a.p.metric, lane, b.cnt.rows_scored);
+    prune_pool_refine<MAX_BEAM, DIMV>(pl, pool, rows, a.p.dim, point, D, need, a.relaxant, a.p.metric, lane, b.cnt.rows_scored);
     wave_sync();
     uint32_t used = 0;
     for (uint32_t base = 0; base < round_up32(D); base += 64) {  // holes in slot order (graph_kernel.cuh:659-671)
@@ -159,6 +173,25 @@ refine_fn pick_refine_beam(uint32_t beam, uint32_t dim) {
     if (beam <= 256) return pick_refine_dim<MAX_CAND, 256>(dim);
     return pick_refine_dim<MAX_CAND, 512>(dim);
 }
+
+#if GLIDE_CAND == 64
+template <int DIMV>
+build_fn pick_build_bytes_beam(uint32_t beam) {
+    if (beam <= 64) return build_kernel<64, 64, DIMV>;
+    if (beam <= 128) return build_kernel<64, 128, DIMV>;
+    if (beam <= 256) return build_kernel<64, 256, DIMV>;
+    return build_kernel<64, 512, DIMV>;
+}
+template <int DIMV>
+refine_fn pick_refine_bytes_beam(uint32_t beam) {
+    if (beam <= 64) return refine_kernel<64, 64, DIMV>;
+    if (beam <= 128) return refine_kernel<64, 128, DIMV>;
+    if (beam <= 256) return refine_kernel<64, 256, DIMV>;
+    return refine_kernel<64, 512, DIMV>;
+}
+build_fn pick_build_bytes(uint32_t beam, uint32_t dim) { return dim <= 128 ? pick_build_bytes_beam<-1>(beam) : pick_build_bytes_beam<-2>(beam); }
+refine_fn pick_refine_bytes(uint32_t beam, uint32_t dim) { return dim <= 128 ? pick_refine_bytes_beam<-1>(beam) : pick_refine_bytes_beam<-2>(beam); }
+#endif
 
 #define GLIDE_PICK_NAME(kind, cand) pick_##kind##_##cand
 #define GLIDE_PICK(kind, cand) GLIDE_PICK_NAME(kind, cand)

@@ -80,7 +80,7 @@ __device__ __forceinline__ uint32_t compact_pool(PL* pl, uint32_t first, uint32_
 
 // sync_prune: returns the neighbour count; pl->neighbor[0..round_up32(D)) holds ids (+segment_start) or invalid
 template <int MAX_BEAM, int DIMV, class PL>
-__device__ __forceinline__ uint32_t prune_pool(PL* pl, uint32_t pool_size, const float* data, uint32_t dim,
+__device__ __forceinline__ uint32_t prune_pool(PL* pl, uint32_t pool_size, row_data<DIMV> data, uint32_t dim,
                                                uint32_t segment_start, uint32_t graph_degree, float relaxant, int metric,
                                                int lane, uint32_t& rows_scored) {
     for (uint32_t i = lane; i < PL::kCap; i += 64) pl->neighbor[i] = kInvalid;
@@ -91,7 +91,7 @@ __device__ __forceinline__ uint32_t prune_pool(PL* pl, uint32_t pool_size, const
         if (lane == 0) pl->neighbor[nsize] = head;
         nsize++;
         RowRegs<DIMV> hrow;
-        load_row<DIMV>(hrow, data + static_cast<size_t>(head) * dim, dim, RowShape<DIMV>::lane_in_row(lane));
+        load_reference<DIMV>(hrow, row_at<DIMV>(data, head, dim), dim, RowShape<DIMV>::lane_in_row(lane));
         rows_scored += pool_size - 1;
         score_list<DIMV>(hrow, data, dim, 1, pool_size, lane,
                          [pl, segment_start](uint32_t idx) { return pl->pool_id[idx] + segment_start; },
@@ -104,7 +104,7 @@ __device__ __forceinline__ uint32_t prune_pool(PL* pl, uint32_t pool_size, const
 
 // sync_prune_refine: heads must be valid, differ from `self` and not already be in the row (pl->s_graph)
 template <int MAX_BEAM, int DIMV, class PL>
-__device__ __forceinline__ uint32_t prune_pool_refine(PL* pl, uint32_t pool_size, const float* data, uint32_t dim,
+__device__ __forceinline__ uint32_t prune_pool_refine(PL* pl, uint32_t pool_size, row_data<DIMV> data, uint32_t dim,
                                                       uint32_t self, uint32_t graph_degree, uint32_t need, float relaxant,
                                                       int metric, int lane, uint32_t& rows_scored) {
     for (uint32_t i = lane; i < PL::kCap; i += 64) pl->neighbor[i] = kInvalid;
@@ -135,7 +135,7 @@ __device__ __forceinline__ uint32_t prune_pool_refine(PL* pl, uint32_t pool_size
         if (lane == 0) pl->neighbor[nsize] = head;
         nsize++;
         RowRegs<DIMV> hrow;
-        load_row<DIMV>(hrow, data + static_cast<size_t>(head) * dim, dim, RowShape<DIMV>::lane_in_row(lane));
+        load_reference<DIMV>(hrow, row_at<DIMV>(data, head, dim), dim, RowShape<DIMV>::lane_in_row(lane));
         rows_scored += pool_size - position;
         score_list<DIMV>(hrow, data, dim, position, pool_size, lane,
                          [pl](uint32_t idx) { return pl->pool_id[idx] & kClean; },

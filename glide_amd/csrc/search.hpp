@@ -16,7 +16,11 @@ struct SearchArgs {
     unsigned long long* counters;
     uint32_t centroid_num, max_centroid, top_k, query_num;
     BeamParams p;
+    const unsigned char* bytes;   // the rows as bytes, for the kernels for rows of bytes
 };
+
+// First result id of a query that the kernel for rows of bytes leaves to the fp32 kernel (result ids are below 2^31).
+constexpr uint32_t kLeftOver = 0xfffffffeu;
 
 // Wavefronts of a team (search_team_kernel) and what one needs.
 constexpr int kTeam = 4;
@@ -33,5 +37,8 @@ using search_fn = void (*)(SearchArgs);
 search_fn pick_search_64(uint32_t beam, uint32_t dim, bool team);
 search_fn pick_search_128(uint32_t beam, uint32_t dim, bool team);
 search_fn pick_search_256(uint32_t beam, uint32_t dim, bool team);
+// Rows of bytes, up to 64 slots and kMostByteDims dims: the queries of bytes, and the fp32 kernel for those left over.
+search_fn pick_search_bytes(uint32_t beam, uint32_t dim);
+search_fn pick_search_left_over(uint32_t beam, uint32_t dim);
 
 }  // namespace glide

@@ -15,7 +15,8 @@ __device__ __forceinline__ uint32_t pick_centroid(uint32_t max_centroid, const R
     }
 }
 
-template <int MAX_CAND, int MAX_BEAM, int DIMV, bool WHOLE = false>
+// LEFT: only the queries that the kernel for rows of bytes has left over.
+template <int MAX_CAND, int MAX_BEAM, int DIMV, bool WHOLE, bool LEFT>
 __device__ __forceinline__ void search_body(const SearchArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     auto* lds = reinterpret_cast<BeamLds<MAX_CAND>*>(smem);
@@ -24,11 +25,28 @@ __device__ __forceinline__ void search_body(const SearchArgs a) {
     // one query a workgroup, as far as a launch has workgroups
     for (uint32_t qid = blockIdx.x; qid < a.query_num; qid += gridDim.x) {
         Beam<MAX_CAND, MAX_BEAM, DIMV, false, WHOLE> b;
-        b.init(lds, hash, a.p, a.queries + static_cast<size_t>(qid) * a.p.dim);
-        const uint32_t c0 = pick_centroid<DIMV>(a.max_centroid, b.q, a.centroids, a.centroid_num, a.p.dim, a.p.metric, cent, b.lane);
+        const float* query = a.queries + static_cast<size_t>(qid) * a.p.dim;
+        row_data<DIMV> rows;
+        uint32_t c0;
+        if constexpr (RowShape<DIMV>::BYTES) {
+            constexpr int F = -DIMV;   // centroids are fp32: the shape of an fp32 row of this length
+            if (!b.init_packing(lds, hash, a.p, query)) {   // not of bytes: left to the fp32 kernel behind this one
+                if (b.lane == 0) a.result_ids[static_cast<size_t>(qid) * a.top_k] = kLeftOver;
+                continue;
+            }
+            rows = a.bytes;
+            RowRegs<F> q;
+            load_row<F>(q, query, a.p.dim, RowShape<F>::lane_in_row(b.lane));
+            c0 = pick_centroid<F>(a.max_centroid, q, a.centroids, a.centroid_num, a.p.dim, a.p.metric, cent, b.lane);
+        } else {
+            if (LEFT && a.result_ids[static_cast<size_t>(qid) * a.top_k] != kLeftOver) continue;   // done on rows of bytes
+            b.init(lds, hash, a.p, query);
+            rows = a.data;
+            c0 = pick_centroid<DIMV>(a.max_centroid, b.q, a.centroids, a.centroid_num, a.p.dim, a.p.metric, cent, b.lane);
+        }
         const uint32_t entry = a.start_points[c0];
-        b.expand(entry, a.graph, a.data, kInvalid, kInvalid);  // result_init: entry node itself is never scored
-        b.run(a.graph, a.data, kInvalid);
+        b.expand(entry, a.graph, rows, kInvalid, kInvalid);  // result_init: entry node itself is never scored
+        b.run(a.graph, rows, kInvalid);
 
         constexpr int NB = MAX_BEAM / 64;
 #pragma unroll
@@ -53,10 +71,10 @@ constexpr int search_waves() {
     if (MAX_CAND <= 64) return MAX_BEAM > 256 ? 5 : 6;
     return MAX_BEAM > 256 ? 4 : MAX_BEAM == 256 && MAX_CAND <= 128 ? 5 : 1;
 }
-template <int MAX_CAND, int MAX_BEAM, int DIMV, bool WHOLE = false>
+template <int MAX_CAND, int MAX_BEAM, int DIMV, bool WHOLE = false, bool LEFT = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(search_waves<MAX_CAND, MAX_BEAM, DIMV>())))
 void search_kernel(SearchArgs a) {
-    search_body<MAX_CAND, MAX_BEAM, DIMV, WHOLE>(a);
+    search_body<MAX_CAND, MAX_BEAM, DIMV, WHOLE, LEFT>(a);
 }
 
 // Small batches of long rows (more than 256 dims): a team of kTeam wavefronts per query.  Wavefront 0 owns the search
@@ -163,6 +181,19 @@ search_fn pick_beam(uint32_t beam, uint32_t dim) {
     if (beam == 512) return pick_dim<MAX_CAND, 512, true>(dim);
     return pick_dim<MAX_CAND, 512>(dim);
 }
+
+#if GLIDE_CAND == 64
+template <int DIMV, bool LEFT = false>
+search_fn pick_bytes_beam(uint32_t beam) {
+    if (beam <= 64) return search_kernel<64, 64, DIMV, false, LEFT>;
+    if (beam <= 128) return search_kernel<64, 128, DIMV, false, LEFT>;
+    if (beam <= 256) return search_kernel<64, 256, DIMV, false, LEFT>;
+    if (beam == 512) return search_kernel<64, 512, DIMV, true, LEFT>;
+    return search_kernel<64, 512, DIMV, false, LEFT>;
+}
+search_fn pick_search_bytes(uint32_t beam, uint32_t dim) { return dim <= 128 ? pick_bytes_beam<-1>(beam) : pick_bytes_beam<-2>(beam); }
+search_fn pick_search_left_over(uint32_t beam, uint32_t dim) { return dim <= 128 ? pick_bytes_beam<1, true>(beam) : pick_bytes_beam<2, true>(beam); }
+#endif
 
 #define GLIDE_PICK_NAME(cand) pick_search_##cand
 #define GLIDE_PICK(cand) GLIDE_PICK_NAME(cand)

@@ -18,6 +18,7 @@ import numpy as np
 from . import capi
 
 INVALID = 0xFFFFFFFF
+BYTE_ROWS_DEGREE = 64      # the searches over rows of bytes take graphs of up to this degree
 
 
 class Metric:
@@ -171,6 +172,24 @@ def cut_rows(d_rows, dim):
     return h
 
 
+def byte_rows(d_rows):
+    """The rows of a DeviceArray once more as bytes, for the searches over rows of whole numbers 0..255, as a DeviceArray;
+    None where a value is none of those or rows of that length are not held so."""
+    num, dim = d_rows.shape
+    nbytes = capi.byte_rows_bytes(num, dim)
+    if nbytes == 0:
+        return None
+    d_other = capi.DeviceArray(1, np.uint32)
+    for rows in (min(num, 2048), num):      # the first ones alone: rows of fractions end there
+        d_bytes = capi.DeviceArray(capi.byte_rows_bytes(rows, dim), np.uint8)
+        capi.pack_byte_rows(d_rows, rows, dim, d_bytes, d_other)
+        if d_other.numpy()[0]:
+            d_bytes.free()
+            return None
+        if rows == num:
+            return d_bytes
+
+
 def preprocess(param, d_data, result=None):
     """partition.cuh:159-193.  d_data: DeviceArray (num, dim) float32; rows of a length that is no multiple of four are
     padded (pad_rows), and the reordered rows and centroids returned then have the padded length (cut_rows gives them
@@ -263,6 +282,7 @@ class GLIDE:
         self._graph_degree = int(graph_degree)
         self.d_graph = capi.DeviceArray((self.num(), self._graph_degree), np.uint32)
         self.d_start_points = None
+        self._bytes = None      # (rows as bytes, the array they were made from, its write count)
 
     # accessors (glide.cuh:81-125)
     def dim(self): return self.d_data.shape[1]
@@ -275,9 +295,26 @@ class GLIDE:
     def centroid_view(self): return self.d_centroids
     def start_point_view(self): return self.d_start_points
 
+    def _hold_byte_rows(self):
+        """The index's rows as bytes, made anew (load, build): where they are whole numbers 0..255 its searches read a quarter
+        of the memory and measure distances in integer arithmetic, with the same results to the bit."""
+        self._bytes = None
+        writes = self.d_data.writes
+        d_bytes = byte_rows(self.d_data) if self._graph_degree <= BYTE_ROWS_DEGREE else None
+        if d_bytes is not None:
+            self._bytes = d_bytes, self.d_data, writes
+
+    def _byte_rows(self):
+        """The rows as bytes, or None: there are none, or the rows may have been written since (a search then reads the rows)."""
+        if self._bytes is None:
+            return None
+        d_bytes, made_from, writes = self._bytes
+        return d_bytes if made_from is self.d_data and writes == made_from.writes and not made_from.shared else None
+
     def load(self, h_graph, h_start_points):                                   # glide_impl.cuh:32-41
         self.d_graph.upload(np.ascontiguousarray(h_graph, dtype=np.uint32))
         self.d_start_points = capi.DeviceArray.from_numpy(np.ascontiguousarray(h_start_points, dtype=np.uint32))
+        self._hold_byte_rows()
 
     def start_point_select(self, h_segment_start, h_segment_length, h_map, seed):   # glide_impl.cuh:43-75
         rng = np.random.default_rng(seed)
@@ -309,22 +346,25 @@ class GLIDE:
         times = {}
         p = search_param_knn
         with _Timer() as t:
+            d_bytes = byte_rows(d_reorder_data) if knn_degree <= BYTE_ROWS_DEGREE else None
             capi.build_subgraph(d_reorder_data, num, dim, d_knn_graph, knn_degree, d_map, d_ss, d_sl, len(h_segment_start), d_rsp,
                                 deg, p.beam, p.max_iterations, p.min_iterations, p.hash_bit, p.hash_reset_interval,
-                                build_param.relaxant_factor, self.metric, self.d_graph, cnt)
+                                build_param.relaxant_factor, self.metric, self.d_graph, cnt, byte_rows=d_bytes)
         times["subgraph"] = t.seconds
         with _Timer() as t:
             if reorder_num > num:
                 capi.build_boundary(d_reorder_data, num, reorder_num, dim, d_knn_graph, knn_degree, d_map,
                                     int(reorder_sp[self.centroid_num()]), deg, p.beam, p.max_iterations, p.min_iterations,
-                                    p.hash_bit, p.hash_reset_interval, build_param.relaxant_factor, self.metric, self.d_graph, cnt)
+                                    p.hash_bit, p.hash_reset_interval, build_param.relaxant_factor, self.metric, self.d_graph, cnt,
+                                    byte_rows=d_bytes)
         times["boundary"] = t.seconds
         if counters and result is not None:
             capi.synchronize()
             result["build_counters"] = capi.read_counters(cnt)
-        for consumed in (d_knn_graph, d_reorder_data):     # d_map is kept until the refine stage, which uses it as its order
-            capi.synchronize()
-            consumed.free()
+        capi.synchronize()
+        for consumed in (d_knn_graph, d_reorder_data, d_bytes):     # d_map is kept until the refine stage, which uses it as its order
+            if consumed is not None:
+                consumed.free()
         self.d_start_points = capi.DeviceArray.from_numpy(sp)
         # reverse_graph (glide_impl.cuh:194-256)
         d_rev = capi.DeviceArray((num, deg), np.uint32)
@@ -343,13 +383,17 @@ class GLIDE:
             p = search_param_refine
             cnt2 = capi.new_counters() if counters else None
             with _Timer() as t:
+                self._hold_byte_rows()
                 capi.refine(self.d_data, num, dim, self.d_graph, d_rev, deg, self.d_centroids, self.centroid_num(),
                             self.d_start_points, p.beam, p.max_iterations, p.min_iterations, p.hash_bit, p.hash_reset_interval,
-                            build_param.relaxant_factor, self.metric, cnt2, order=d_map)
+                            build_param.relaxant_factor, self.metric, cnt2, order=d_map,
+                            byte_rows=self._bytes[0] if self._bytes else None)
             times["refine"] = t.seconds
             self.d_graph, d_rev = d_rev, self.d_graph
             if counters and result is not None:
                 result["refine_counters"] = capi.read_counters(cnt2)
+        else:
+            self._hold_byte_rows()
         d_rev.free()
         d_map.free()
         if result is not None:
@@ -374,7 +418,7 @@ class GLIDE:
         with _Timer() as t:
             capi.search(self.d_data, self.num(), self.dim(), self.d_graph, self._graph_degree, self.d_centroids, self.centroid_num(),
                         self.d_start_points, d_query, nq, param.top_k, param.beam, param.max_iterations, param.min_iterations,
-                        param.hash_bit, param.hash_reset_interval, self.metric, d_ids, d_dists, counters, stream)
+                        param.hash_bit, param.hash_reset_interval, self.metric, d_ids, d_dists, counters, stream, byte_rows=self._byte_rows())
         if result is not None:
             result["search_time"] = t.seconds
             result["QPS"] = nq / t.seconds if t.seconds > 0 else float("inf")

@@ -1,0 +1,162 @@
+"""Searches, sub-graph builds and refinement over rows held as bytes against the same calls on the fp32 rows: sums of squares
+of up to 256 whole numbers 0..255 are exact in fp32 and in integers, so ids, distances, graphs and counters must agree to the
+bit.  Rows and queries reach both ends of the range (256 dims of 0 against 255 give the largest sum there is)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+INV = 0xFFFFFFFF
+
+
+@pytest.fixture(scope="module")
+def hip():
+    from glide_amd import capi
+    capi.set_device(0)
+    return capi
+
+
+def rows_of(rng, n, dim):
+    """Clustered bytes, a fifth of the values at the ends of the range, some rows equal, one all 0 and one all 255."""
+    x = rng.integers(0, 256, (8, dim))[rng.integers(0, 8, n)] + rng.integers(-20, 21, (n, dim))
+    x = np.clip(x, 0, 255)
+    x[rng.random((n, dim)) < 0.1] = 0
+    x[rng.random((n, dim)) < 0.1] = 255
+    x[n // 2: n // 2 + 5] = x[3]
+    x[0], x[1] = 0, 255
+    return x.astype(np.float32)
+
+
+def packed(hip, rows):
+    d = hip.DeviceArray.from_numpy(rows)
+    n, dim = rows.shape
+    d_bytes, d_other = hip.DeviceArray.full(hip.byte_rows_bytes(n, dim) // 4, 0xDEADBEEF), hip.DeviceArray.full(1, 7)
+    hip.pack_byte_rows(d, n, dim, d_bytes, d_other)
+    return d, d_bytes, int(d_other.numpy()[0])
+
+
+@pytest.mark.parametrize("n,dim", [(1, 4), (33, 100), (700, 128), (2049, 132), (5000, 256)])
+def test_packed_rows(hip, n, dim):
+    rows = rows_of(np.random.default_rng(n), max(n, 8), dim)[:n]
+    _, d_bytes, other = packed(hip, rows)
+    held = d_bytes.numpy().view(np.uint8).reshape(n, 128 if dim <= 128 else 256)
+    assert other == 0 and np.array_equal(held[:, :dim], rows) and not held[:, dim:].any()
+    for value, at in ((0.5, (n - 1, dim - 1)), (-1.0, (n // 2, 0)), (256.0, (0, dim // 2)), (np.nan, (n - 1, 3)), (np.inf, (0, 0)), (254.99998, (n // 3, 1))):
+        bad = rows.copy()
+        bad[at] = value
+        assert packed(hip, bad)[2] == 1, (value, at)
+    rows[n - 1, 0] = -0.0      # the same number as 0
+    assert packed(hip, rows)[2] == 0
+
+
+def test_lengths_that_are_not_held(hip):
+    assert hip.byte_rows_bytes(100, 260) == 0 and hip.byte_rows_bytes(100, 6) == 0 and hip.byte_rows_bytes(100, 256) == 25600
+    d = hip.DeviceArray((4, 260), np.float32)
+    with pytest.raises(hip.GlideHipError):
+        hip.pack_byte_rows(d, 4, 260, hip.DeviceArray(4096, np.uint8), hip.DeviceArray(1, np.uint32))
+
+
+CASES = [(dim, degree, beam, metric) for i, (dim, degree) in enumerate([(4, 8), (16, 32), (100, 24), (128, 32), (128, 64), (132, 40), (200, 64), (256, 32)])
+         for beam, metric in [((32, 64, 128, 256)[i % 4], i % 2), ((512, 288, 160, 96)[i % 4], 1 - i % 2)]]
+
+
+@pytest.mark.parametrize("dim,degree,beam,metric", CASES)
+def test_search(hip, dim, degree, beam, metric):
+    from oracle import oracle as O
+    rng = np.random.default_rng(dim + degree + beam)
+    n, nq, c = 900, 70, 3
+    rows = rows_of(rng, n, dim)
+    knn, _ = O.bruteforce_knn(rows, rows, degree, exclude_self=True)
+    knn[rng.random(knn.shape) < 0.05] = INV
+    queries = rows_of(rng, nq, dim)
+    queries[2] = rows[7]
+    odd = {5: 0.25, 11: -3.0, 30: 300.0, 41: 127.00001, nq - 1: 1e-30}       # queries that are not of bytes
+    for q, v in odd.items():
+        queries[q, dim - 1] = v
+    queries[50, 0] = np.nan
+    queries[51, 0] = -0.0
+    d, d_bytes, other = packed(hip, rows)
+    assert other == 0
+    sp = O.search_params(beam, degree)
+    d_g, d_q = hip.DeviceArray.from_numpy(knn), hip.DeviceArray.from_numpy(queries)
+    d_c, d_sp = hip.DeviceArray.from_numpy(rows[[10, 400, 800]] + 0.5), hip.DeviceArray.from_numpy(np.array([1, 0, 77], np.uint32))
+    got = []
+    for b in (None, d_bytes):
+        ids, dists, cnt = hip.DeviceArray.full((nq, 10), 0xDEADBEEF), hip.DeviceArray.full((nq, 10), 0xDEADBEEF), hip.new_counters()
+        hip.search(d, n, dim, d_g, degree, d_c, c, d_sp, d_q, nq, 10, sp["beam"], sp["max_iterations"], sp["min_iterations"], sp["hash_bit"],
+                   sp["hash_reset_interval"], metric, ids, dists, cnt, byte_rows=b)
+        hip.synchronize()
+        got.append((ids.numpy(), dists.numpy(), hip.read_counters(cnt)))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1]) and got[0][2] == got[1][2]
+
+
+@pytest.mark.parametrize("dim,knn_degree,degree,build_beam,refine_beam,metric",
+                         [(4, 16, 8, 32, 64, 0), (100, 32, 32, 64, 128, 0), (128, 64, 32, 128, 256, 1), (128, 32, 64, 256, 512, 0), (132, 24, 40, 64, 128, 1),
+                          (256, 64, 64, 320, 288, 0), (256, 32, 24, 64, 64, 1)])
+def test_build_and_refine(hip, dim, knn_degree, degree, build_beam, refine_beam, metric):
+    from oracle import oracle as O
+    rng = np.random.default_rng(dim + degree)
+    lengths, boundary = (400, 300), 120
+    n = sum(lengths)
+    rows = rows_of(rng, n, dim)
+    reorder = np.concatenate([rows, rows[rng.permutation(n)[:boundary]]])
+    mp = np.concatenate([rng.permutation(n), rng.permutation(n)[:boundary]]).astype(np.uint32)
+    starts, lens = np.array([0, lengths[0], n], np.uint32), np.array([*lengths, boundary], np.uint32)
+    knn = np.concatenate([O.bruteforce_knn(reorder[s:s + m], reorder[s:s + m], knn_degree, metric, exclude_self=True)[0] for s, m in zip(starts, lens)])
+    knn[rng.random(knn.shape) < 0.05] = INV
+    b, r = O.search_params(build_beam, knn_degree), O.search_params(refine_beam, max(knn_degree, degree))
+    d_re, d_re_bytes, other = packed(hip, reorder)
+    d_rows, d_rows_bytes, other2 = packed(hip, rows)
+    assert other == 0 and other2 == 0
+    up = hip.DeviceArray.from_numpy
+    d_knn, d_map, d_s, d_l = up(knn), up(mp), up(starts), up(lens)
+    d_sp, d_c, d_gsp = up(np.array([5, 9, 2], np.uint32)), up(rows[[20, 600]] + 0.25), up(np.array([3, 500], np.uint32))
+    got = []
+    for re_bytes, row_bytes in ((None, None), (d_re_bytes, d_rows_bytes)):
+        g, out, cnt = hip.DeviceArray.full((n, degree), INV), hip.DeviceArray.full((n, degree), 0xDEADBEEF), hip.new_counters()
+        args = (b["beam"], b["max_iterations"], b["min_iterations"], b["hash_bit"], b["hash_reset_interval"], 1.05, metric, g, cnt)
+        hip.build_subgraph(d_re, n, dim, d_knn, knn_degree, d_map, d_s, d_l, 3, d_sp, degree, *args, byte_rows=re_bytes)
+        hip.build_boundary(d_re, n, n + boundary, dim, d_knn, knn_degree, d_map, 2, degree, *args, byte_rows=re_bytes)
+        hip.refine(d_rows, n, dim, g, out, degree, d_c, 2, d_gsp, r["beam"], r["max_iterations"], r["min_iterations"], r["hash_bit"],
+                   r["hash_reset_interval"], 1.05, metric, cnt, order=d_map, byte_rows=row_bytes)
+        hip.synchronize()
+        got.append((g.numpy(), out.numpy(), hip.read_counters(cnt)))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1]) and got[0][2] == got[1][2]
+    assert (got[0][1] != INV).any()
+
+
+def test_index_follows_its_rows(hip):
+    """Rows written after load() are the rows that are searched, whoever writes them."""
+    from glide_amd import index as G
+    from oracle import oracle as O
+    rng = np.random.default_rng(3)
+    n, dim, degree = 600, 64, 16
+    first, second = rows_of(rng, n, dim), rows_of(rng, n, dim)
+    knn, _ = O.bruteforce_knn(first, first, degree, exclude_self=True)
+    sp, queries = G.make_search_parameter(64, degree), hip.DeviceArray.from_numpy(rows_of(rng, 20, dim))
+    d = hip.DeviceArray.from_numpy(first)
+    index = G.GLIDE(degree, d, first[:2], G.Metric.Euclidean)
+
+    def fresh(rows):
+        other = G.GLIDE(degree, rows + 0.0, first[:2], G.Metric.Euclidean)
+        other.load(knn, np.array([4, 9], np.uint32))
+        other._bytes = None
+        return other.search(sp, queries)
+
+    def agree(rows):
+        return all(np.array_equal(a, b) for a, b in zip(index.search(sp, queries), fresh(rows)))
+
+    index.load(knn, np.array([4, 9], np.uint32))
+    assert index._byte_rows() is not None and agree(first)
+    d.upload(second)
+    assert index._byte_rows() is None and agree(second)
+    index.load(knn, np.array([4, 9], np.uint32))
+    assert index._byte_rows() is not None and agree(second)
+    hip.copy_rows(hip.DeviceArray.from_numpy(first), n, dim, d, dim)
+    assert index._byte_rows() is None and agree(first)
+    index.load(knn, np.array([4, 9], np.uint32))
+    assert index._byte_rows() is not None and agree(first)
+    hip.copy_rows(hip.DeviceArray.from_numpy(second), n, dim, d.ptr, dim)     # by address: not seen as a write to `d`
+    assert index._byte_rows() is None and agree(second)
+    fractions = G.GLIDE(degree, first + 0.5, first[:2], G.Metric.Euclidean)
+    fractions.load(knn, np.array([4, 9], np.uint32))
+    assert fractions._byte_rows() is None
