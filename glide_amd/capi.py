@@ -325,6 +325,18 @@ def reorder(data, num, dim, segment_indexes, segment_starts, reorder_data, mp, s
                                   _out(reorder_data, stream), _out(mp), vp(stream)), "glide_hip_reorder")
 
 
+def sample_ids_workspace_bytes(num):
+    return int(_size_fn("glide_hip_sample_ids_workspace_bytes")(u32(num)))
+
+
+def sample_ids(num, count, seed, ids, workspace, workspace_bytes, stream=None):
+    """The first `count` entries of np.random.default_rng(seed).permutation(num), on the device."""
+    state = np.random.PCG64(seed).state["state"]
+    words = [v >> shift & 0xFFFFFFFFFFFFFFFF for v in (state["state"], state["inc"]) for shift in (64, 0)]
+    check(lib().glide_hip_sample_ids(u32(num), u32(count), (C.c_uint64 * 4)(*words), _out(ids), _out(workspace), C.c_size_t(workspace_bytes),
+                                     vp(stream)), "glide_hip_sample_ids")
+
+
 def sample_rows(data, dim, sample_ids, sample_num, sample, stream=None):
     check(lib().glide_hip_sample_rows(_ptr(data), u32(dim), _ptr(sample_ids), u32(sample_num), _out(sample, stream),
                                       vp(stream)), "glide_hip_sample_rows")

@@ -204,15 +204,16 @@ def preprocess(param, d_data, result=None):
     times = {}
     # get_centroids (partition.cuh:10-59): shuffle, sample, k-means on the sample
     sample_num = max(int(num * param.sample_factor), min(num, c))
-    rng = np.random.default_rng(param.seed)
-    ids = rng.permutation(num)[:sample_num].astype(np.uint32)
-    d_ids = capi.DeviceArray.from_numpy(ids)
+    d_ids = capi.DeviceArray(sample_num, np.uint32)
     d_sample = capi.DeviceArray((sample_num, dim), np.float32)
     d_centroids = capi.DeviceArray((c, dim), np.float32)
     wb = capi.kmeans_workspace_bytes(c, dim)
     ws = capi.DeviceArray(wb // 4 + 1, np.uint32)
     sb = capi.kmeans_seed_workspace_bytes(sample_num)
     seed_ws = capi.DeviceArray(sb // 8 + 1, np.uint64)
+    wb = capi.sample_ids_workspace_bytes(num)
+    ids_ws = capi.DeviceArray(wb // 16 + 1, np.dtype("V16"))
+    capi.sample_ids(num, sample_num, param.seed, d_ids, ids_ws, wb)
     with _Timer() as t:
         capi.sample_rows(d_data, dim, d_ids, sample_num, d_sample)
         capi.kmeans_seed(d_sample, sample_num, dim, c, param.seed, d_centroids, seed_ws, sb)
