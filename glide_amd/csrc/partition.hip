@@ -70,6 +70,75 @@ __device__ __forceinline__ void nearest_two(float dk, uint32_t ck, float& d0, ui
     }
 }
 
+// Chunks of kChunk dims go global -> registers -> LDS; the loads of chunk k+1 are issued before the matrix instructions of
+// chunk k, so their latency is covered by the MFMA work.  The squared norms of the points (for the error band of the ranking)
+// are summed on the way, those of the centroids too where they are asked for.  xw: the wavefront's part of x_tile.
+template <int CB, bool NORMS>
+__device__ __forceinline__ void centroid_products(const float* data, uint32_t num, uint32_t dim, const float* centroids, uint32_t centroid_num,
+                                                  uint32_t wave_base, int lane, float* cent_tile, float* xw, float16v (&acc)[CB], float (&xsq)[4],
+                                                  float (&csq)[CB]) {
+    const int half = lane >> 5, t = lane & 31;
+#pragma unroll
+    for (int cb = 0; cb < CB; cb++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[cb][r] = 0.f;
+    float4 cpre[CB], xpre[4];
+#pragma unroll
+    for (int it = 0; it < 4; it++) xsq[it] = 0.f;
+    if constexpr (NORMS) {
+#pragma unroll
+        for (int it = 0; it < CB; it++) csq[it] = 0.f;
+    }
+    auto prefetch = [&](uint32_t k0) {
+#pragma unroll
+        for (int it = 0; it < CB; it++) {   // centroid chunk: 8 lanes x float4 per row, 32*CB rows over 256 threads
+            const uint32_t idx = threadIdx.x + 256 * it;
+            const uint32_t row = idx >> 3, d0 = k0 + (idx & 7) * 4;
+            cpre[it] = (row < centroid_num && d0 < dim) ? *reinterpret_cast<const float4*>(centroids + static_cast<size_t>(row) * dim + d0)
+                                                           : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+#pragma unroll
+        for (int it = 0; it < 4; it++) {    // this wave's 32 points
+            const uint32_t row = it * 8 + (lane >> 3);
+            const uint32_t p = wave_base + row, d0 = k0 + (lane & 7) * 4;
+            xpre[it] = (p < num && d0 < dim) ? *reinterpret_cast<const float4*>(data + static_cast<size_t>(p) * dim + d0)
+                                                 : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    };
+    prefetch(0);
+    for (uint32_t k0 = 0; k0 < dim; k0 += kChunk) {
+        __syncthreads();   // every wave is done with the previous chunk
+#pragma unroll
+        for (int it = 0; it < CB; it++) {
+            const uint32_t idx = threadIdx.x + 256 * it;
+            *reinterpret_cast<float4*>(cent_tile + (idx >> 3) * kLdsStride + (idx & 7) * 4) = cpre[it];
+            if constexpr (NORMS)
+                csq[it] = fmaf(cpre[it].x, cpre[it].x, fmaf(cpre[it].y, cpre[it].y, fmaf(cpre[it].z, cpre[it].z, fmaf(cpre[it].w, cpre[it].w, csq[it]))));
+        }
+#pragma unroll
+        for (int it = 0; it < 4; it++) {
+            *reinterpret_cast<float4*>(xw + (it * 8 + (lane >> 3)) * kLdsStride + (lane & 7) * 4) = xpre[it];
+            xsq[it] = fmaf(xpre[it].x, xpre[it].x, fmaf(xpre[it].y, xpre[it].y, fmaf(xpre[it].z, xpre[it].z, fmaf(xpre[it].w, xpre[it].w, xsq[it]))));
+        }
+        __syncthreads();
+        if (k0 + kChunk < dim) prefetch(k0 + kChunk);
+        // v_mfma_f32_32x32x2_f32: lane supplies A[i = lane%32][k-slot = lane/32] and B[k-slot][j = lane%32].
+        // A k-slot pair is fed from one float4 per half (dims kk+4*half .. +3), component by component.
+#pragma unroll
+        for (int kk = 0; kk < kChunk; kk += 8) {
+            const float4 xv = *reinterpret_cast<const float4*>(xw + t * kLdsStride + kk + 4 * half);
+#pragma unroll
+            for (int cb = 0; cb < CB; cb++) {
+                const float4 cv = *reinterpret_cast<const float4*>(cent_tile + (cb * 32 + t) * kLdsStride + kk + 4 * half);
+                acc[cb] = __builtin_amdgcn_mfma_f32_32x32x2f32(cv.x, xv.x, acc[cb], 0, 0, 0);
+                acc[cb] = __builtin_amdgcn_mfma_f32_32x32x2f32(cv.y, xv.y, acc[cb], 0, 0, 0);
+                acc[cb] = __builtin_amdgcn_mfma_f32_32x32x2f32(cv.z, xv.z, acc[cb], 0, 0, 0);
+                acc[cb] = __builtin_amdgcn_mfma_f32_32x32x2f32(cv.w, xv.w, acc[cb], 0, 0, 0);
+            }
+        }
+    }
+}
+
 // CB = number of 32-centroid row blocks held in accumulators (centroid_num <= 32*CB).
 // One wavefront owns 32 points.  The matrix instruction takes the centroids as its A operand and the points as B, so
 // lane (t, half) ends with the scores of point t against 16 centroids of every block in its own registers and ranks
@@ -95,62 +164,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
     for (uint32_t i = threadIdx.x; i < 32 * CB; i += 256) cnorm[i] = i < a.centroid_num ? a.centroid_norms[i] : __builtin_inff();
 
     float16v acc[CB];
-#pragma unroll
-    for (int cb = 0; cb < CB; cb++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[cb][r] = 0.f;
-
-    // Chunks of kChunk dims go global -> registers -> LDS; the loads of chunk k+1 are issued before the matrix
-    // instructions of chunk k, so their latency is covered by the MFMA work.  The squared norms of the points (for the
-    // error band of the ranking) are summed on the way.
-    float4 cpre[CB], xpre[4];
-    float xsq[4] = {0.f, 0.f, 0.f, 0.f};
-    auto prefetch = [&](uint32_t k0) {
-#pragma unroll
-        for (int it = 0; it < CB; it++) {   // centroid chunk: 8 lanes x float4 per row, 32*CB rows over 256 threads
-            const uint32_t idx = threadIdx.x + 256 * it;
-            const uint32_t row = idx >> 3, d0 = k0 + (idx & 7) * 4;
-            cpre[it] = (row < a.centroid_num && d0 < a.dim) ? *reinterpret_cast<const float4*>(a.centroids + static_cast<size_t>(row) * a.dim + d0)
-                                                           : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-#pragma unroll
-        for (int it = 0; it < 4; it++) {    // this wave's 32 points
-            const uint32_t row = it * 8 + (lane >> 3);
-            const uint32_t p = wave_base + row, d0 = k0 + (lane & 7) * 4;
-            xpre[it] = (p < a.num && d0 < a.dim) ? *reinterpret_cast<const float4*>(a.data + static_cast<size_t>(p) * a.dim + d0)
-                                                 : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-    };
-    prefetch(0);
-    for (uint32_t k0 = 0; k0 < a.dim; k0 += kChunk) {
-        __syncthreads();   // every wave is done with the previous chunk
-#pragma unroll
-        for (int it = 0; it < CB; it++) {
-            const uint32_t idx = threadIdx.x + 256 * it;
-            *reinterpret_cast<float4*>(cent_tile + (idx >> 3) * kLdsStride + (idx & 7) * 4) = cpre[it];
-        }
-#pragma unroll
-        for (int it = 0; it < 4; it++) {
-            *reinterpret_cast<float4*>(xw + (it * 8 + (lane >> 3)) * kLdsStride + (lane & 7) * 4) = xpre[it];
-            xsq[it] = fmaf(xpre[it].x, xpre[it].x, fmaf(xpre[it].y, xpre[it].y, fmaf(xpre[it].z, xpre[it].z, fmaf(xpre[it].w, xpre[it].w, xsq[it]))));
-        }
-        __syncthreads();
-        if (k0 + kChunk < a.dim) prefetch(k0 + kChunk);
-        // v_mfma_f32_32x32x2_f32: lane supplies A[i = lane%32][k-slot = lane/32] and B[k-slot][j = lane%32].
-        // A k-slot pair is fed from one float4 per half (dims kk+4*half .. +3), component by component.
-#pragma unroll
-        for (int kk = 0; kk < kChunk; kk += 8) {
-            const float4 xv = *reinterpret_cast<const float4*>(xw + t * kLdsStride + kk + 4 * half);
-#pragma unroll
-            for (int cb = 0; cb < CB; cb++) {
-                const float4 cv = *reinterpret_cast<const float4*>(cent_tile + (cb * 32 + t) * kLdsStride + kk + 4 * half);
-                acc[cb] = __builtin_amdgcn_mfma_f32_32x32x2f32(cv.x, xv.x, acc[cb], 0, 0, 0);
-                acc[cb] = __builtin_amdgcn_mfma_f32_32x32x2f32(cv.y, xv.y, acc[cb], 0, 0, 0);
-                acc[cb] = __builtin_amdgcn_mfma_f32_32x32x2f32(cv.z, xv.z, acc[cb], 0, 0, 0);
-                acc[cb] = __builtin_amdgcn_mfma_f32_32x32x2f32(cv.w, xv.w, acc[cb], 0, 0, 0);
-            }
-        }
-    }
+    float xsq[4], unused_norms[CB];
+    centroid_products<CB, false>(a.data, a.num, a.dim, a.centroids, a.centroid_num, wave_base, lane, cent_tile, xw, acc, xsq, unused_norms);
 
     // From here on the wavefront is on its own.  Its x tile is free (LDS operations of one wavefront complete in order,
     // and the last matrix pass has read it) and becomes its scratch:
@@ -865,7 +880,9 @@ __global__ __launch_bounds__(256) void kmeanspp_distance_kernel(const float* sam
 // the largest magnitude still fit (2^35 for 500 000 rows of 0..255 data: every value exact; on unit-norm data values
 // below 2^-19 are rounded to 2^-43).
 
-// largest |value| of the sample, as the bit pattern of a non-negative float (which orders like the unsigned integer)
+// largest |value| of the sample, as the bit pattern of a non-negative float (which orders like the unsigned integer).  One
+// atomic a workgroup and few workgroups: with one for each of 16 000 wavefronts the kernel was those atomics, 188 us.
+constexpr uint32_t kRangeBlocks = 512;
 __global__ __launch_bounds__(256) void kmeans_range_kernel(const float* sample, size_t count, uint32_t* max_bits) {
     uint32_t m = 0;
     for (size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x; i < count; i += static_cast<size_t>(gridDim.x) * 256) {
@@ -877,7 +894,14 @@ __global__ __launch_bounds__(256) void kmeans_range_kernel(const float* sample, 
         const uint32_t o = static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), off));
         m = o > m ? o : m;
     }
-    if (lane_id() == 0 && m) atomicMax(max_bits, m);
+    __shared__ uint32_t of_wave[4];
+    if (lane_id() == 0) of_wave[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int w = 1; w < 4; w++) m = of_wave[w] > m ? of_wave[w] : m;
+        if (m) atomicMax(max_bits, m);
+    }
 }
 
 // scale = 2^e with max|x| * n * 2^e < 2^62
@@ -998,6 +1022,154 @@ __global__ __launch_bounds__(256) void kmeans_accumulate_narrow_kernel(const flo
 inline bool narrow_pays(uint32_t points, uint32_t clusters, bool in_lds) {
     if (!in_lds) return points >= 12000;
     return points >= (clusters <= 16 ? 400 + 100 * clusters : clusters <= 64 ? 250 * clusters : 340 * clusters);
+}
+
+// Many clusters: the nearest centroid by the matrix cores, ranked like assign_kernel's (see assign_band; one centroid is looked
+// for here, so the ones within the band of the smallest score are the only ones that can be it).  A point with one such
+// centroid needs no distance; for the few with more they are measured with exact_distance_half, the sum the kernels above
+// make, so all three choose the same centroid for every point.  What cannot be ranked -- a band that is not finite, a score
+// that is not a number, more than kKeep centroids in it -- is measured against every centroid, as the wide kernel does.
+// 20 000 points of 128 dims, 256 clusters: a step was 132 us with the narrow kernel, 64 vector instructions a point and
+// centroid and two and a half rounds of wavefronts; the matrix instructions here take 14 us.
+constexpr uint32_t kRankedRows = 16;
+template <int CB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void kmeans_accumulate_ranked_kernel(const float* sample, uint32_t n, uint32_t dim,
+                                                                                                              const float* centroids, uint32_t k, long long* sums,
+                                                                                                              uint32_t* counts, const uint32_t* max_bits) {
+    extern __shared__ __align__(16) float smem[];
+    float* cent_tile = smem;                                   // [32*CB][kLdsStride]
+    float* x_tile = cent_tile + 32 * CB * kLdsStride;          // [4 waves][32][kLdsStride]
+    float* cnorm = x_tile + 4 * 32 * kLdsStride;               // [32*CB]: |c|^2, +inf beyond k
+    const int lane = lane_id();
+    const int wave = threadIdx.x >> 6;
+    const int half = lane >> 5, t = lane & 31;
+    const uint32_t wave_base = blockIdx.x * kTilePoints + wave * 32;
+    float* xw = x_tile + wave * 32 * kLdsStride;
+    float16v acc[CB];
+    float xsq[4], csq[CB];
+    centroid_products<CB, true>(sample, n, dim, centroids, k, wave_base, lane, cent_tile, xw, acc, xsq, csq);
+#pragma unroll
+    for (int it = 0; it < CB; it++) {
+        const float total = row_sum<1>(csq[it]);   // the 8 lanes that staged a row
+        const uint32_t row = (threadIdx.x + 256 * it) >> 3;
+        if ((threadIdx.x & 7) == 0) cnorm[row] = row < k ? total : __builtin_inff();
+    }
+    __syncthreads();
+    if (wave_base >= n) return;
+    // the wavefront's x tile is free: its scratch
+    uint32_t* cand = reinterpret_cast<uint32_t*>(xw);          // [64][kKeep] centroids within the band, per lane
+    float* x_norm = xw + 64 * kKeep;                           // [32]
+    uint32_t* nearest = reinterpret_cast<uint32_t*>(x_norm + 32);   // [32]
+#pragma unroll
+    for (int it = 0; it < 4; it++) {
+        const float total = row_sum<1>(xsq[it]);
+        if ((lane & 7) == 0) x_norm[it * 8 + (lane >> 3)] = total;
+    }
+    float max_cn = 0.f;
+    for (uint32_t i = lane; i < k; i += 64) max_cn = fmaxf(max_cn, cnorm[i]);
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) max_cn = fmaxf(max_cn, __shfl_xor(max_cn, m));
+    __builtin_amdgcn_wave_barrier();
+    float smallest = __builtin_inff();
+#pragma unroll
+    for (int cb = 0; cb < CB; cb++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const float4 c4 = *reinterpret_cast<const float4*>(cnorm + cb * 32 + 8 * q + 4 * half);
+            const float cn[4] = {c4.x, c4.y, c4.z, c4.w};
+#pragma unroll
+            for (int m = 0; m < 4; m++) smallest = fminf(smallest, fmaf(-2.f, acc[cb][4 * q + m], cn[m]));
+        }
+    smallest = fminf(smallest, lane_xor<32>(smallest));
+    const float limit = smallest + assign_band(dim, x_norm[t], max_cn);
+    uint32_t found = 0;
+#pragma unroll
+    for (int cb = 0; cb < CB; cb++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const float4 c4 = *reinterpret_cast<const float4*>(cnorm + cb * 32 + 8 * q + 4 * half);
+            const float cn[4] = {c4.x, c4.y, c4.z, c4.w};
+            bool in[4];   // a score that is no number counts: its point is measured
+#pragma unroll
+            for (int m = 0; m < 4; m++) in[m] = !(fmaf(-2.f, acc[cb][4 * q + m], cn[m]) > limit);
+            if (in[0] | in[1] | in[2] | in[3]) {
+                const uint32_t c = cb * 32 + 8 * q + 4 * half;
+#pragma unroll
+                for (int m = 0; m < 4; m++) {
+                    if (in[m] && c + m < k) {
+                        if (found < kKeep) cand[lane * kKeep + found] = c + m;
+                        found++;
+                    }
+                }
+            }
+        }
+    const uint32_t of_other = lane_xor<32>(found);
+    const bool finite = limit < 1e37f;   // neither the norms nor the products have come near overflow
+    const bool all = !finite || found > kKeep || of_other > kKeep || found + of_other == 0;
+    const bool some = !all && found + of_other > 1;
+    if (!all && !some && found == 1) nearest[t] = cand[lane * kKeep];
+    __builtin_amdgcn_wave_barrier();
+    uint64_t measure = ballot((all || some) && wave_base + t < n) & 0xffffffffull;
+    const uint64_t in_full = ballot(all);
+    while (measure) {
+        const int p = __builtin_ctzll(measure);
+        measure &= measure - 1;
+        const uint32_t point = wave_base + p < n ? wave_base + p : n - 1;
+        const float* x = sample + static_cast<size_t>(point) * dim;
+        float best = FLT_MAX;
+        uint32_t bc = 0;
+        if ((in_full >> p) & 1) {
+            for (uint32_t c0 = 0; c0 < k; c0 += 2) {
+                const uint32_t c = c0 + half < k ? c0 + half : c0;
+                const float sq = exact_distance_half(x, centroids + static_cast<size_t>(c) * dim, dim, t);
+                const float da = read_lane(sq, 0), db = read_lane(sq, 32);
+                if (da < best) { best = da; bc = c0; }
+                if (c0 + 1 < k && db < best) { best = db; bc = c0 + 1; }
+            }
+        } else {   // each half of the wavefront goes through the centroids that lane p of it has found
+            const uint32_t mine = half ? read_lane(found, p + 32) : read_lane(found, p);
+            uint32_t hc = kInvalid;
+            for (uint32_t f = 0; f < mine; f++) {
+                const uint32_t c = cand[(p + 32 * half) * kKeep + f];
+                const float sq = exact_distance_half(x, centroids + static_cast<size_t>(c) * dim, dim, t);
+                if (sq < best) { best = sq; hc = c; }   // ascending ids: the first of equal ones stays
+            }
+            const float ob = lane_xor<32>(best);
+            const uint32_t oc = lane_xor<32>(hc);
+            bc = ob < best || (ob == best && oc < hc) ? oc : hc;
+            bc = read_lane(bc, 0);
+            if (bc == kInvalid) bc = 0;
+        }
+        if (lane == 0) nearest[p] = bc;
+    }
+    __builtin_amdgcn_wave_barrier();
+    const float scale = kmeans_scale(*max_bits, n);
+    const uint32_t points = n - wave_base < 32 ? n - wave_base : 32;
+    if (static_cast<uint32_t>(lane) < points) atomicAdd(&counts[nearest[lane]], 1u);
+    for (uint32_t d = lane; d < dim; d += 64) {
+        for (uint32_t p0 = 0; p0 < points; p0 += kRankedRows) {   // that many values under way: one after another they were half of the kernel
+            float x[kRankedRows];
+#pragma unroll
+            for (uint32_t p = 0; p < kRankedRows; p++) x[p] = sample[static_cast<size_t>(wave_base + (p0 + p < points ? p0 + p : 0u)) * dim + d];
+#pragma unroll
+            for (uint32_t p = 0; p < kRankedRows; p++)
+                if (p0 + p < points)   // two's complement, adjacent lanes on adjacent sums
+                    atomicAdd(reinterpret_cast<unsigned long long*>(sums) + static_cast<size_t>(nearest[p0 + p]) * dim + d,
+                              static_cast<unsigned long long>(__float2ll_rn(x[p] * scale)));
+        }
+    }
+}
+size_t ranked_lds_bytes(int cb) { return (static_cast<size_t>(32) * cb * kLdsStride + 4 * 32 * kLdsStride + 32 * cb) * sizeof(float); }
+
+// Where ranking is ahead, from both sides measured (a step, ranked : the better of the others).  Up to 128 dims the narrow
+// kernel with its sums in LDS keeps what it serves (20 000 points of 128 dims, 32 clusters 78 : 66 us); with sums in memory it
+// is 1.0 : 1 at 1 500 points and 2 000 on 128 dims 30 : 32 us for 64 clusters, 52 : 62 for 256, 20 000 points 75 : 134 and 78 :
+// 139.  Longer rows: 5 000 points of 960 dims 188 : 209 for 128 clusters, 156 : 146 for 64; 12 000 points 206 : 226 for 16
+// clusters, 356 : 845 for 256, but 309 : 222 for 4, whose few sums take the atomics of every point.
+inline bool ranking_pays(uint32_t points, uint32_t clusters, uint32_t dim, bool in_lds) {
+    if (clusters > 256) return false;
+    if (dim <= 128) return !in_lds && points >= 2000;
+    return clusters >= 16 && points >= (clusters >= 128 ? 2000 : 6000);
 }
 
 __global__ void kmeans_update_kernel(float* centroids, const long long* sums, const uint32_t* counts, uint32_t k, uint32_t dim, uint32_t n,
@@ -1223,7 +1395,7 @@ int glide_hip_kmeans_fit(const float* sample, uint32_t sample_num, uint32_t dim,
     int rc = glide_hip_fill_u32(max_bits, 0u, 1, stream);
     if (rc != GLIDE_OK) return rc;
     const size_t values = static_cast<size_t>(sample_num) * dim;
-    hipLaunchKernelGGL(kmeans_range_kernel, dim3(static_cast<uint32_t>(values / 256 < 4096 ? values / 256 + 1 : 4096)), dim3(256), 0, s, sample,
+    hipLaunchKernelGGL(kmeans_range_kernel, dim3(static_cast<uint32_t>(values / 256 < kRangeBlocks ? values / 256 + 1 : kRangeBlocks)), dim3(256), 0, s, sample,
                        values, max_bits);
     const bool in_lds = static_cast<size_t>(cluster_num) * dim <= kLdsSums;
     const bool narrow = dim <= 128 && narrow_pays(sample_num, cluster_num, in_lds) && reinterpret_cast<uintptr_t>(sample) % 16 == 0 &&
@@ -1231,10 +1403,18 @@ int glide_hip_kmeans_fit(const float* sample, uint32_t sample_num, uint32_t dim,
     // with sums in LDS every workgroup adds k x dim of them up at its end, so it takes 128 points at least
     const uint32_t sum_blocks = ceil_div(sample_num, in_lds ? 128 : 8 * kSumPoints);
     const size_t sum_lds = in_lds ? static_cast<size_t>(cluster_num) * dim * 8 + static_cast<size_t>(cluster_num) * 4 : 0;
+    auto ranked_kernel = cluster_num <= 32 ? kmeans_accumulate_ranked_kernel<1> : cluster_num <= 64 ? kmeans_accumulate_ranked_kernel<2>
+                         : cluster_num <= 128 ? kmeans_accumulate_ranked_kernel<4> : kmeans_accumulate_ranked_kernel<8>;
+    const size_t ranked_lds = ranked_lds_bytes(cluster_num <= 32 ? 1 : cluster_num <= 64 ? 2 : cluster_num <= 128 ? 4 : 8);
+    const bool ranked = ranking_pays(sample_num, cluster_num, dim, in_lds) && reinterpret_cast<uintptr_t>(sample) % 16 == 0 &&
+                        reinterpret_cast<uintptr_t>(centroids) % 16 == 0;
     for (uint32_t it = 0; it < iterations; it++) {
         rc = glide_hip_fill_u32(reinterpret_cast<uint32_t*>(sums), 0u, words, stream);
         if (rc != GLIDE_OK) return rc;
-        if (narrow)
+        if (ranked)
+            hipLaunchKernelGGL(ranked_kernel, dim3(ceil_div(sample_num, kTilePoints)), dim3(256), ranked_lds, s, sample, sample_num, dim, centroids,
+                               cluster_num, sums, counts, max_bits);
+        else if (narrow)
             hipLaunchKernelGGL(kmeans_accumulate_narrow_kernel, dim3(sum_blocks), dim3(256), sum_lds, s, sample, sample_num, dim, centroids,
                                cluster_num, sums, counts, max_bits, in_lds ? 1u : 0u);
         else
