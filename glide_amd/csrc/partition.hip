@@ -671,50 +671,9 @@ __device__ __forceinline__ uint32_t wave_locate(Load load, uint32_t len, double 
 // four values of a row, zeros in the lanes behind its end
 __device__ __forceinline__ float4 load4(const float* p, bool in) { return in ? *reinterpret_cast<const float4*>(p) : make_float4(0.f, 0.f, 0.f, 0.f); }
 
-// one workgroup of 16 wavefronts: chunk sums of min_dist (in global memory or LDS), then wavefront j draws candidate j
-__device__ __forceinline__ void draw_candidates(double* part, uint32_t n, const float* min_dist, uint32_t seed, uint32_t step, uint32_t trials,
-                                                uint32_t* candidates) {
-    const uint32_t t = threadIdx.x;
-    const int lane = lane_id();
-    const uint32_t wave = t >> 6;
-    const uint32_t chunk = (n + 1023) / 1024;
-    {
-        const uint32_t lo = t * chunk < n ? t * chunk : n, hi = lo + chunk < n ? lo + chunk : n;
-        double acc = 0.0;
-        for (uint32_t i = lo; i < hi; i++) acc += static_cast<double>(min_dist[i]);
-        part[t] = acc;
-    }
-    __syncthreads();
-    if (wave >= trials) return;
-    double total = 0.0;
-    for (uint32_t i = lane * 16; i < lane * 16 + 16; i++) total += part[i];
-    for (int off = 32; off >= 1; off >>= 1) total += __shfl_xor(total, off);
-    uint32_t cand = seed_hash(seed, 16 * step) % n;      // every row already coincides with a centroid
-    if (total > 0.0) {
-        const uint32_t h = seed_hash(seed, 16 * step + wave);
-        const double target = static_cast<double>(h >> 8) * (1.0 / 16777216.0) * total;
-        double before = 0.0, unused = 0.0;
-        const double* pp = part;
-        const uint32_t c = wave_locate([pp](uint32_t i) { return pp[i]; }, 1024, target, before, lane);
-        const uint32_t base = c * chunk, len = (base + chunk < n ? base + chunk : n) - base;
-        const float* md = min_dist + base;
-        cand = base + wave_locate([md](uint32_t i) { return static_cast<double>(md[i]); }, len, target - before, unused, lane);
-    }
-    if (lane == 0) candidates[wave] = cand;
-}
-__global__ __launch_bounds__(1024) void kmeanspp_pick_kernel(uint32_t n, const float* min_dist, uint32_t seed, uint32_t step, uint32_t trials,
-                                                            uint32_t* candidates) {
-    __shared__ double part[1024];
-    if (step == 0) {
-        if (threadIdx.x < trials) candidates[threadIdx.x] = seed_hash(seed, 0) % n;
-        return;
-    }
-    draw_candidates(part, n, min_dist, seed, step, trials, candidates);
-}
-
-// 64 sample rows per workgroup, LANES lanes a row: squared distance of every row to every candidate (kept in trial_dist,
-// nullable, for kmeanspp_next_kernel, which lowers min_dist by the winner's) and the candidates' potentials over these rows,
-// in double, summed row after row in four runs of 16 whatever the layout.  Rows of up to 128 dims take half a wavefront and
+// 64 sample rows per workgroup, LANES lanes a row: min_dist lowered by the distances to the last step's winner (`winner`, null
+// in the first step, says which of its candidates' trial_dist that are), the squared distance of every row to every candidate
+// (trial_dist, for the step after) and the candidates' potentials over these rows, in double, summed row after row in four runs of 16 whatever the layout.  Rows of up to 128 dims take half a wavefront and
 // four rows a group, with the candidates in registers: the kernel is a few memory round trips long, so what counts is to have
 // them all under way at once (20 000 rows of 128 dims, 7 candidates: 30 us with one wavefront going through 16 rows).
 // The candidates' ids are read before the first row, so that no row load waits for them, and the masked loads choose between
@@ -726,13 +685,21 @@ __global__ __launch_bounds__(1024) void kmeanspp_pick_kernel(uint32_t n, const f
 // rows: four at a time 1.36 times the time).
 constexpr uint32_t kTrialThreads = 512;
 template <int LANES, uint32_t TOGETHER = 1>   // TOGETHER: rows of more than 128 dims under way at once
-__global__ __launch_bounds__(kTrialThreads) void kmeanspp_trial_kernel(const float* sample, uint32_t n, uint32_t dim, const float* min_dist,
-                                                                      const uint32_t* candidates, uint32_t trials, double* partial, float* trial_dist) {
+__global__ __launch_bounds__(kTrialThreads) void kmeanspp_trial_kernel(const float* sample, uint32_t n, uint32_t dim, float* min_dist,
+                                                                      const uint32_t* candidates, uint32_t trials, const uint32_t* winner, double* partial,
+                                                                      float* trial_dist) {
     static_assert(kSeedPoints * kSeedTrials == kTrialThreads, "one distance a thread");
     constexpr uint32_t kGroups = kTrialThreads / LANES, kRows = kSeedPoints / kGroups;
     __shared__ float dist[kSeedTrials][kSeedPoints];
     __shared__ double run_pot[4][kSeedTrials];
+    __shared__ float lowered[kSeedPoints];
     const uint32_t group = threadIdx.x / LANES, t = threadIdx.x % LANES, first = blockIdx.x * kSeedPoints;
+    const uint32_t last = threadIdx.x < kSeedPoints && winner ? *winner : 0u;
+    float so_far = 0.f, to_winner = 0.f;
+    if (threadIdx.x < kSeedPoints && first + threadIdx.x < n) {
+        so_far = min_dist[first + threadIdx.x];
+        to_winner = winner ? trial_dist[static_cast<size_t>(last) * n + first + threadIdx.x] : so_far;
+    }
     if constexpr (LANES == 32) {
         uint32_t id[kSeedTrials];
 #pragma unroll
@@ -774,8 +741,13 @@ __global__ __launch_bounds__(kTrialThreads) void kmeanspp_trial_kernel(const flo
             }
         }
     }
+    if (threadIdx.x < kSeedPoints) {
+        const float low = fminf(so_far, to_winner);
+        lowered[threadIdx.x] = low;
+        if (winner && first + threadIdx.x < n) min_dist[first + threadIdx.x] = low;
+    }
     __syncthreads();
-    if (trial_dist) {
+    {
         const uint32_t j = threadIdx.x / kSeedPoints, i = first + threadIdx.x % kSeedPoints;
         if (j < trials && i < n) trial_dist[static_cast<size_t>(j) * n + i] = dist[j][threadIdx.x % kSeedPoints];
     }
@@ -783,7 +755,7 @@ __global__ __launch_bounds__(kTrialThreads) void kmeanspp_trial_kernel(const flo
         const uint32_t run = threadIdx.x / kSeedTrials, j = threadIdx.x % kSeedTrials;
         double pot = 0.0;
         if (j < trials)
-            for (uint32_t r = run * 16; r < run * 16 + 16 && first + r < n; r++) pot += static_cast<double>(fminf(min_dist[first + r], dist[j][r]));
+            for (uint32_t r = run * 16; r < run * 16 + 16 && first + r < n; r++) pot += static_cast<double>(fminf(lowered[r], dist[j][r]));
         run_pot[run][j] = pot;
     }
     __syncthreads();
@@ -793,7 +765,8 @@ __global__ __launch_bounds__(kTrialThreads) void kmeanspp_trial_kernel(const flo
 }
 
 // Potentials summed over the trial kernel's workgroups, the smallest wins (the first on a tie); its row becomes centroid
-// `step`.  256 threads at least; returns which candidate won, to every thread.
+// `step`.  256 threads at least; returns which candidate won, to every thread.  Sums are asked for eight at a time: one after
+// another they were most of a step.
 __device__ __forceinline__ uint32_t choose_winner(const float* sample, uint32_t dim, const double* partial, uint32_t blocks, const uint32_t* candidates,
                                                   uint32_t trials, uint32_t step, float* centroids, uint32_t* chosen_rows) {
     __shared__ double slice[kSeedTrials][32];
@@ -802,8 +775,15 @@ __device__ __forceinline__ uint32_t choose_winner(const float* sample, uint32_t 
     if (threadIdx.x < 32 * kSeedTrials) {
         const uint32_t j = threadIdx.x >> 5, sl = threadIdx.x & 31;
         double acc = 0.0;
-        if (step > 0 && j < trials)
-            for (uint32_t b = sl; b < blocks; b += 32) acc += partial[static_cast<size_t>(b) * kSeedTrials + j];
+        if (trials > 1 && j < trials) {
+            for (uint32_t b = sl; b < blocks; b += 32 * 8) {
+                double v[8];
+#pragma unroll
+                for (uint32_t u = 0; u < 8; u++) v[u] = b + 32 * u < blocks ? partial[static_cast<size_t>(b + 32 * u) * kSeedTrials + j] : 0.0;
+#pragma unroll
+                for (uint32_t u = 0; u < 8; u++) acc += v[u];
+            }
+        }
         slice[j][sl] = acc;
     }
     __syncthreads();
@@ -815,7 +795,7 @@ __device__ __forceinline__ uint32_t choose_winner(const float* sample, uint32_t 
     __syncthreads();
     if (threadIdx.x == 0) {
         uint32_t b = 0;
-        for (uint32_t c = 1; c < (step > 0 ? trials : 1u); c++)
+        for (uint32_t c = 1; c < trials; c++)
             if (total[c] < total[b]) b = c;
         best = b;
         if (chosen_rows) chosen_rows[step] = candidates[b];
@@ -826,52 +806,54 @@ __device__ __forceinline__ uint32_t choose_winner(const float* sample, uint32_t 
     for (uint32_t d = threadIdx.x; d < dim; d += blockDim.x) centroids[static_cast<size_t>(step) * dim + d] = src[d];
     return won;
 }
-__global__ __launch_bounds__(256) void kmeanspp_choose_kernel(const float* sample, uint32_t dim, const double* partial, uint32_t blocks,
-                                                              const uint32_t* candidates, uint32_t trials, uint32_t step, float* centroids,
-                                                              uint32_t* chosen_rows) {
-    choose_winner(sample, dim, partial, blocks, candidates, trials, step, centroids, chosen_rows);
-}
-
-// Between two trials, in one workgroup: the winner of `step`, min_dist lowered by its distances, and the candidates of the
-// next step.  min_dist passes through LDS, which is what limits it to kSeedLdsRows rows (128 KB); a larger sample takes the
-// kernels above one after another.  20 000 rows, 256 clusters: a step was four launches and 54 us of kernels.
-constexpr uint32_t kSeedLdsRows = 32768;
+// Between two trials, in one workgroup: the winner of `step` and the candidates of the next one, from the potentials alone --
+// a workgroup's potential for the winner is the sum of its rows' min_dist once lowered, so a draw looks for its place among
+// the workgroups' sums and then among the 64 rows of one of them.  min_dist itself is lowered by the trial that follows, each
+// workgroup its own rows.  (Going through min_dist here, 20 000 rows took 18 us a step, most of them loads one after another.)
 __global__ __launch_bounds__(1024) void kmeanspp_next_kernel(const float* sample, uint32_t n, uint32_t dim, const double* partial, uint32_t blocks,
-                                                             const float* trial_dist, uint32_t trials, uint32_t seed, uint32_t step, uint32_t last,
-                                                             float* min_dist, uint32_t* candidates, float* centroids, uint32_t* chosen_rows) {
-    extern __shared__ __align__(16) float md[];   // n values
-    __shared__ double part[1024];
+                                                             const float* min_dist, const float* trial_dist, uint32_t trials, uint32_t next_trials,
+                                                             uint32_t seed, uint32_t step, uint32_t* candidates, uint32_t* winner, float* centroids,
+                                                             uint32_t* chosen_rows) {
+    __shared__ double part[1024];   // sums of `chunk` workgroups each
     const uint32_t won = choose_winner(sample, dim, partial, blocks, candidates, trials, step, centroids, chosen_rows);
-    if (last) return;
-    const float* d = trial_dist + static_cast<size_t>(won) * n;
-    for (uint32_t i = threadIdx.x; i < n; i += 1024) {
-        const float m = fminf(min_dist[i], d[i]);
-        md[i] = m;
-        min_dist[i] = m;
+    if (next_trials == 0) return;   // that was the last one
+    if (threadIdx.x == 0) *winner = won;
+    const int lane = lane_id();
+    const uint32_t wave = threadIdx.x >> 6, chunk = (blocks + 1023) / 1024, parts = (blocks + chunk - 1) / chunk;
+    if (threadIdx.x < parts) {
+        const uint32_t lo = threadIdx.x * chunk, hi = lo + chunk < blocks ? lo + chunk : blocks;
+        double acc = 0.0;
+        for (uint32_t i = lo; i < hi; i++) acc += partial[static_cast<size_t>(i) * kSeedTrials + won];
+        part[threadIdx.x] = acc;
     }
     __syncthreads();   // every thread has read the old candidates by now
-    draw_candidates(part, n, md, seed, step + 1, trials, candidates);
+    if (wave >= next_trials) return;
+    double total = 0.0;
+    for (uint32_t i = lane; i < parts; i += 64) total += part[i];
+    for (int off = 32; off >= 1; off >>= 1) total += __shfl_xor(total, off);
+    uint32_t cand = seed_hash(seed, 16 * (step + 1)) % n;      // every row already coincides with a centroid
+    if (total > 0.0) {
+        const uint32_t h = seed_hash(seed, 16 * (step + 1) + wave);
+        const double target = static_cast<double>(h >> 8) * (1.0 / 16777216.0) * total;
+        double before = 0.0, before_block = 0.0, unused = 0.0;
+        const uint32_t c = wave_locate([&](uint32_t i) { return part[i]; }, parts, target, before, lane);
+        const uint32_t base = c * chunk, len = (base + chunk < blocks ? base + chunk : blocks) - base;
+        const double* sums = partial + static_cast<size_t>(base) * kSeedTrials + won;
+        const uint32_t block = base + wave_locate([&](uint32_t i) { return sums[static_cast<size_t>(i) * kSeedTrials]; }, len, target - before, before_block, lane);
+        const uint32_t first = block * kSeedPoints, rows = n - first < kSeedPoints ? n - first : kSeedPoints;
+        const float* md = min_dist + first;
+        const float* td = trial_dist + static_cast<size_t>(won) * n + first;
+        const double value = static_cast<uint32_t>(lane) < rows ? static_cast<double>(fminf(md[lane], td[lane])) : 0.0;   // a row a lane
+        cand = first + wave_locate([&](uint32_t) { return value; }, rows, target - before - before_block, unused, lane);
+    }
+    if (lane == 0) candidates[wave] = cand;
 }
 
-// one wavefront per sample row: min_dist[i] = min(min_dist[i], |x_i - c|^2) (set on the first step)
-__global__ __launch_bounds__(256) void kmeanspp_distance_kernel(const float* sample, uint32_t n, uint32_t dim, const float* centroid, float* min_dist,
-                                                                int first) {
-    const int lane = lane_id();
-    const uint32_t i = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (i >= n) return;
-    const float* x = sample + static_cast<size_t>(i) * dim;
-    float acc = 0.f;
-    for (uint32_t d0 = lane * 4; d0 < dim; d0 += 256) {
-        const float4 a = *reinterpret_cast<const float4*>(x + d0);
-        const float4 b = *reinterpret_cast<const float4*>(centroid + d0);
-        const float dx = a.x - b.x, dy = a.y - b.y, dz = a.z - b.z, dw = a.w - b.w;
-        acc = fmaf(dx, dx, acc);
-        acc = fmaf(dy, dy, acc);
-        acc = fmaf(dz, dz, acc);
-        acc = fmaf(dw, dw, acc);
-    }
-    acc = wave_sum(acc);
-    if (lane == 0) min_dist[i] = first ? acc : fminf(min_dist[i], acc);
+// Before the first step: one candidate, drawn uniformly, and no distances yet (the smaller of NaN and a distance is the distance).
+__global__ __launch_bounds__(256) void kmeanspp_begin_kernel(uint32_t n, uint32_t seed, float* min_dist, uint32_t* candidates) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) min_dist[i] = __builtin_nanf("");
+    if (i == 0) candidates[0] = seed_hash(seed, 0) % n;
 }
 
 // ---- Lloyd k-means on a sample (stand-in for cuvs::cluster::kmeans::fit, reference partition.cuh:48-54) ----
@@ -1336,10 +1318,10 @@ size_t glide_hip_kmeans_workspace_bytes(uint32_t cluster_num, uint32_t dim) {
 }
 
 size_t glide_hip_kmeans_seed_workspace_bytes(uint32_t sample_num) {
-    // min_dist (f32 per row) | candidates (8 u32) | per-workgroup potentials of the trial kernel (8 f64 each)
-    // | distances of every row to the candidates (8 f32 per row), for samples whose steps pass through LDS
+    // min_dist (f32 per row) | candidates (8 u32), winner (u32) | per-workgroup potentials of the trial kernel (8 f64 each)
+    // | distances of every row to the candidates (8 f32 per row)
     return align_up(static_cast<size_t>(sample_num) * 4, 256) + 256 + static_cast<size_t>(ceil_div(sample_num, kSeedPoints)) * kSeedTrials * 8 +
-           (sample_num <= kSeedLdsRows ? static_cast<size_t>(sample_num) * kSeedTrials * 4 : 0);
+           static_cast<size_t>(sample_num) * kSeedTrials * 4;
 }
 
 int glide_hip_kmeans_seed(const float* sample, uint32_t sample_num, uint32_t dim, uint32_t cluster_num, uint32_t seed, float* centroids,
@@ -1355,28 +1337,16 @@ int glide_hip_kmeans_seed(const float* sample, uint32_t sample_num, uint32_t dim
     uint32_t* candidates = reinterpret_cast<uint32_t*>(w + align_up(static_cast<size_t>(sample_num) * 4, 256));
     double* partial = reinterpret_cast<double*>(w + align_up(static_cast<size_t>(sample_num) * 4, 256) + 256);
     const uint32_t trials = seed_trials(cluster_num), blocks = ceil_div(sample_num, kSeedPoints);
-    const bool in_lds = sample_num <= kSeedLdsRows;
-    float* trial_dist = in_lds ? reinterpret_cast<float*>(partial + static_cast<size_t>(blocks) * kSeedTrials) : nullptr;
-    const size_t lds = static_cast<size_t>(sample_num) * sizeof(float);
-    if (in_lds && cluster_num > 1)
-        GLIDE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&kmeanspp_next_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          static_cast<int>(lds)));
+    uint32_t* winner = candidates + kSeedTrials;
+    float* trial_dist = reinterpret_cast<float*>(partial + static_cast<size_t>(blocks) * kSeedTrials);
     auto trial = dim <= 128 ? kmeanspp_trial_kernel<32> : dim <= 256 ? kmeanspp_trial_kernel<64, 4> : kmeanspp_trial_kernel<64>;
+    hipLaunchKernelGGL(kmeanspp_begin_kernel, dim3(ceil_div(sample_num, 256)), dim3(256), 0, s, sample_num, seed, min_dist, candidates);
     for (uint32_t step = 0; step < cluster_num; step++) {
-        if (step <= 1 || !in_lds)
-            hipLaunchKernelGGL(kmeanspp_pick_kernel, dim3(1), dim3(1024), 0, s, sample_num, min_dist, seed, step, trials, candidates);
-        if (step > 0)
-            hipLaunchKernelGGL(trial, dim3(blocks), dim3(kTrialThreads), 0, s, sample, sample_num, dim, min_dist, candidates, trials, partial, trial_dist);
-        if (step > 0 && in_lds) {
-            hipLaunchKernelGGL(kmeanspp_next_kernel, dim3(1), dim3(1024), lds, s, sample, sample_num, dim, partial, blocks, trial_dist, trials, seed, step,
-                               step + 1 == cluster_num ? 1u : 0u, min_dist, candidates, centroids, chosen_rows);
-            continue;
-        }
-        hipLaunchKernelGGL(kmeanspp_choose_kernel, dim3(1), dim3(256), 0, s, sample, dim, partial, blocks, candidates, trials, step, centroids,
-                           chosen_rows);
-        if (step + 1 < cluster_num)
-            hipLaunchKernelGGL(kmeanspp_distance_kernel, dim3(ceil_div(sample_num, 4)), dim3(256), 0, s, sample, sample_num, dim,
-                               centroids + static_cast<size_t>(step) * dim, min_dist, step == 0 ? 1 : 0);
+        const uint32_t now = step == 0 ? 1u : trials, next = step + 1 < cluster_num ? trials : 0u;
+        hipLaunchKernelGGL(trial, dim3(blocks), dim3(kTrialThreads), 0, s, sample, sample_num, dim, min_dist, candidates, now,
+                           step == 0 ? static_cast<const uint32_t*>(nullptr) : winner, partial, trial_dist);
+        hipLaunchKernelGGL(kmeanspp_next_kernel, dim3(1), dim3(1024), 0, s, sample, sample_num, dim, partial, blocks, min_dist, trial_dist, now, next, seed,
+                           step, candidates, winner, centroids, chosen_rows);
     }
     return launch_status();
 }
