@@ -72,11 +72,12 @@ __device__ __forceinline__ void nearest_two(float dk, uint32_t ck, float& d0, ui
 
 // Chunks of kChunk dims go global -> registers -> LDS; the loads of chunk k+1 are issued before the matrix instructions of
 // chunk k, so their latency is covered by the MFMA work.  The squared norms of the points (for the error band of the ranking)
-// are summed on the way, those of the centroids too where they are asked for.  xw: the wavefront's part of x_tile.
+// are summed on the way; where they are asked for, those of the centroids too, a centroid a thread from the staged chunk (a
+// register instead of eight).  xw: the wavefront's part of x_tile.
 template <int CB, bool NORMS>
 __device__ __forceinline__ void centroid_products(const float* data, uint32_t num, uint32_t dim, const float* centroids, uint32_t centroid_num,
                                                   uint32_t wave_base, int lane, float* cent_tile, float* xw, float16v (&acc)[CB], float (&xsq)[4],
-                                                  float (&csq)[CB]) {
+                                                  float& csq) {
     const int half = lane >> 5, t = lane & 31;
 #pragma unroll
     for (int cb = 0; cb < CB; cb++)
@@ -85,10 +86,7 @@ __device__ __forceinline__ void centroid_products(const float* data, uint32_t nu
     float4 cpre[CB], xpre[4];
 #pragma unroll
     for (int it = 0; it < 4; it++) xsq[it] = 0.f;
-    if constexpr (NORMS) {
-#pragma unroll
-        for (int it = 0; it < CB; it++) csq[it] = 0.f;
-    }
+    csq = 0.f;
     auto prefetch = [&](uint32_t k0) {
 #pragma unroll
         for (int it = 0; it < CB; it++) {   // centroid chunk: 8 lanes x float4 per row, 32*CB rows over 256 threads
@@ -112,8 +110,6 @@ __device__ __forceinline__ void centroid_products(const float* data, uint32_t nu
         for (int it = 0; it < CB; it++) {
             const uint32_t idx = threadIdx.x + 256 * it;
             *reinterpret_cast<float4*>(cent_tile + (idx >> 3) * kLdsStride + (idx & 7) * 4) = cpre[it];
-            if constexpr (NORMS)
-                csq[it] = fmaf(cpre[it].x, cpre[it].x, fmaf(cpre[it].y, cpre[it].y, fmaf(cpre[it].z, cpre[it].z, fmaf(cpre[it].w, cpre[it].w, csq[it]))));
         }
 #pragma unroll
         for (int it = 0; it < 4; it++) {
@@ -122,6 +118,15 @@ __device__ __forceinline__ void centroid_products(const float* data, uint32_t nu
         }
         __syncthreads();
         if (k0 + kChunk < dim) prefetch(k0 + kChunk);
+        if constexpr (NORMS) {
+            if (threadIdx.x < 32 * CB) {
+#pragma unroll 2
+                for (int d = 0; d < kChunk; d += 4) {
+                    const float4 c = *reinterpret_cast<const float4*>(cent_tile + threadIdx.x * kLdsStride + d);
+                    csq = fmaf(c.x, c.x, fmaf(c.y, c.y, fmaf(c.z, c.z, fmaf(c.w, c.w, csq))));
+                }
+            }
+        }
         // v_mfma_f32_32x32x2_f32: lane supplies A[i = lane%32][k-slot = lane/32] and B[k-slot][j = lane%32].
         // A k-slot pair is fed from one float4 per half (dims kk+4*half .. +3), component by component.
 #pragma unroll
@@ -164,8 +169,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
     for (uint32_t i = threadIdx.x; i < 32 * CB; i += 256) cnorm[i] = i < a.centroid_num ? a.centroid_norms[i] : __builtin_inff();
 
     float16v acc[CB];
-    float xsq[4], unused_norms[CB];
-    centroid_products<CB, false>(a.data, a.num, a.dim, a.centroids, a.centroid_num, wave_base, lane, cent_tile, xw, acc, xsq, unused_norms);
+    float xsq[4], unused_norm;
+    centroid_products<CB, false>(a.data, a.num, a.dim, a.centroids, a.centroid_num, wave_base, lane, cent_tile, xw, acc, xsq, unused_norm);
 
     // From here on the wavefront is on its own.  Its x tile is free (LDS operations of one wavefront complete in order,
     // and the last matrix pass has read it) and becomes its scratch:
@@ -1028,14 +1033,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     const uint32_t wave_base = blockIdx.x * kTilePoints + wave * 32;
     float* xw = x_tile + wave * 32 * kLdsStride;
     float16v acc[CB];
-    float xsq[4], csq[CB];
+    float xsq[4], csq;
     centroid_products<CB, true>(sample, n, dim, centroids, k, wave_base, lane, cent_tile, xw, acc, xsq, csq);
-#pragma unroll
-    for (int it = 0; it < CB; it++) {
-        const float total = row_sum<1>(csq[it]);   // the 8 lanes that staged a row
-        const uint32_t row = (threadIdx.x + 256 * it) >> 3;
-        if ((threadIdx.x & 7) == 0) cnorm[row] = row < k ? total : __builtin_inff();
-    }
+    if (threadIdx.x < 32 * CB) cnorm[threadIdx.x] = threadIdx.x < k ? csq : __builtin_inff();
     __syncthreads();
     if (wave_base >= n) return;
     // the wavefront's x tile is free: its scratch
