@@ -297,6 +297,11 @@ def partition_assign(data, num, dim, centroids, centroid_num, boundary_factor, m
                                            C.c_size_t(workspace_bytes), vp(stream)), "glide_hip_partition_assign")
 
 
+def release_memory():
+    """Gives device memory that freed arrays have left for later ones back to the device."""
+    check(lib().glide_hip_release_memory(), "glide_hip_release_memory")
+
+
 def mem_info():
     """(free, total) bytes of device memory on the current device."""
     free, total = C.c_size_t(0), C.c_size_t(0)

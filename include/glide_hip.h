@@ -46,6 +46,9 @@ int glide_hip_mem_info(size_t *free_bytes, size_t *total_bytes);
  * (replace raft::make_device_matrix / raft::copy / rmm stream pool / cudaEvent use, glide_impl.cuh:15-41,53-72) */
 int glide_hip_malloc(void **ptr, size_t bytes);
 int glide_hip_free(void *ptr);
+/* glide_hip_free keeps up to 2 GiB a device for later glide_hip_malloc calls (it returns, like hipFree, when all work of the
+ * device has ended).  glide_hip_release_memory gives that memory back to the device. */
+int glide_hip_release_memory(void);
 int glide_hip_host_alloc_pinned(void **ptr, size_t bytes);
 int glide_hip_host_free_pinned(void *ptr);
 int glide_hip_memcpy_h2d(void *dst, const void *src, size_t bytes, void *stream);
