@@ -277,7 +277,7 @@ struct Beam {
 
     // Distance of this lane's slot i of the latest expansion; FLT_MAX where nothing was scored.
     __device__ __forceinline__ float slot_distance(int i) const {
-        const float d = finish_distance(lds->cand_dist[place[i] & (MAX_CAND - 1)], p.metric);
+        const float d = finish_row_distance<DIMV>(lds->cand_dist[place[i] & (MAX_CAND - 1)], p.metric);
         return place[i] != kInvalid ? d : FLT_MAX;
     }
     // Buckets of more than 64 slots: from the order of vlist to the slots.  What is not a number is dropped where a beam starts

@@ -120,16 +120,21 @@ __device__ __forceinline__ void hash_clear(uint32_t* table, uint32_t bitlen, int
     }
     for (uint32_t i = lane; i < (1u << bitlen); i += kWave) table[i] = kInvalid;
 }
-// returns 1 iff `key` was newly stored; 0 if present or the table is full (one exit, the outcome read off the last slot
-// afterwards: a loop with three outcomes costs twice the mask bookkeeping per probe)
+// returns 1 iff `key` was newly stored; 0 if present or the table is full.  One exit, the outcome read off the last slot
+// afterwards (a loop with three outcomes costs twice the mask bookkeeping per probe, and so does an outcome that the loop
+// carries along as a mask: hence the opaque copy).  Four vector instructions a probe: the slot is a byte offset, wrapped by a
+// mask, and the count of probes is the same in every lane still probing, so it is kept on the scalar unit.  An expansion
+// probes four times or so, restoring a beam after a reset as often for each of its registers: with eight instructions a probe
+// they were a fifth of what a beam search issues.
 __device__ __forceinline__ uint32_t hash_insert(uint32_t* table, uint32_t bitlen, uint32_t key) {
-    const uint32_t size = 1u << bitlen;
-    const uint32_t mask = size - 1;
-    uint32_t index = (key ^ (key >> bitlen)) & mask, left = size, old;
+    const uint32_t mask = (4u << bitlen) - 4u;
+    uint32_t at = ((key ^ (key >> bitlen)) << 2) & mask, left = 1u << bitlen, old;
     do {
-        old = atomicCAS(&table[index], kInvalid, key);
-        index = (index + 1) & mask;
-    } while ((old != kInvalid) & (old != key) & (--left != 0));
+        old = atomicCAS(reinterpret_cast<uint32_t*>(reinterpret_cast<unsigned char*>(table) + at), kInvalid, key);
+        at = (at + 4u) & mask;
+        left = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(left))) - 1u;
+    } while ((old != kInvalid) & (old != key) & (left != 0));
+    asm("" : "+v"(old));
     return old == kInvalid ? 1u : 0u;
 }
 
@@ -274,10 +279,29 @@ __device__ __forceinline__ float byte_sqdist(const RowRegs<DIMV>& ref, const uin
     v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, false);
     v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, false);   // row_half_mirror
     if constexpr (RowShape<DIMV>::LPR >= 16) v += __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, false);   // row_mirror
+    asm("" : "+v"(v));   // the last addition stays with its lane move (in the one lane that writes the sum it would be three instructions)
     return static_cast<float>(v);
 }
 
 // reference distance.cuh:22-26: Euclidean reports sqrt, Cosine the squared L2 of pre-normalised rows
 __device__ __forceinline__ float finish_distance(float sq, int metric) { return metric == kEuclidean ? sqrtf(sq) : sq; }
+
+// The same for a whole number below 2^24, the squared distance of rows of bytes: sqrtf without the scaling it needs for very
+// small arguments and without the cases of infinity and NaN, half of its fourteen instructions.  The hardware root is off by
+// one place at most; with neighbours l and h of it, l * root >= sq says that it is too large, h * root < sq that it is too small
+// (both exact in the sign of one rounded multiply-add).
+__device__ __forceinline__ float finish_byte_distance(float sq, int metric) {
+    if (metric != kEuclidean) return sq;
+    const float root = __builtin_amdgcn_sqrtf(sq);
+    const float l = __uint_as_float(__float_as_uint(root) - 1u), h = __uint_as_float(__float_as_uint(root) + 1u);   // l of 0 is no number: neither test holds
+    const float below = fmaf(-l, root, sq), above = fmaf(-h, root, sq);
+    const float r = below <= 0.f ? l : root;
+    return above > 0.f ? h : r;
+}
+template <int DIMV>
+__device__ __forceinline__ float finish_row_distance(float sq, int metric) {
+    if constexpr (RowShape<DIMV>::BYTES) return finish_byte_distance(sq, metric);
+    else return finish_distance(sq, metric);
+}
 
 }  // namespace glide

@@ -85,8 +85,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DIMV > 4 || 
     auto* lds = reinterpret_cast<BeamLds<MAX_CAND>*>(smem);
     using Prune = PruneLds<MAX_BEAM, (MAX_CAND < 64 ? 64 : MAX_CAND)>;   // the row has at most MAX_CAND slots here
     auto* pl = reinterpret_cast<Prune*>(smem + sizeof(BeamLds<MAX_CAND>));
-    float* cent = reinterpret_cast<float*>(smem + sizeof(BeamLds<MAX_CAND>) + sizeof(Prune));
-    uint32_t* hash = reinterpret_cast<uint32_t*>(cent + round_up32(a.centroid_num));
+    uint32_t* hash = reinterpret_cast<uint32_t*>(smem + sizeof(BeamLds<MAX_CAND>) + sizeof(Prune));   // at a constant offset: no addition a probe
+    float* cent = reinterpret_cast<float*>(hash + (1u << a.p.hash_bit));
     if (blockIdx.x >= a.num) return;
     const uint32_t point = a.order ? a.order[blockIdx.x] : blockIdx.x;
     if (point >= a.num) return;

@@ -57,14 +57,14 @@ __device__ __forceinline__ uint32_t beam_to_pool(Beam<MAX_CAND, MAX_BEAM, DIMV>&
 }
 
 // stable compaction of the pool: entries [first, pool_size) that the latest head does not occlude
-template <int MAX_BEAM, class PL>
+template <int MAX_BEAM, int DIMV, class PL>
 __device__ __forceinline__ uint32_t compact_pool(PL* pl, uint32_t first, uint32_t pool_size, float relaxant, int metric, int lane) {
     uint32_t n = 0;
     for (uint32_t base = 0; base < pool_size; base += 64) {
         const uint32_t i = base + lane;
         const uint32_t id = i < pool_size ? pl->pool_id[i] : 0u;
         const float d = i < pool_size ? pl->pool_dist[i] : 0.f;
-        const bool ok = i >= first && i < pool_size && !(relaxant * finish_distance(pl->head_sq[i < pool_size ? i : 0u], metric) < d);
+        const bool ok = i >= first && i < pool_size && !(relaxant * finish_row_distance<DIMV>(pl->head_sq[i < pool_size ? i : 0u], metric) < d);
         const uint64_t m = ballot(ok);
         wave_sync();
         if (ok) {
@@ -97,7 +97,7 @@ __device__ __forceinline__ uint32_t prune_pool(PL* pl, uint32_t pool_size, row_d
                          [pl, segment_start](uint32_t idx) { return pl->pool_id[idx] + segment_start; },
                          [pl](uint32_t idx, float sq) { pl->head_sq[idx] = sq; });
         wave_sync();
-        pool_size = compact_pool<MAX_BEAM>(pl, 1, pool_size, relaxant, metric, lane);
+        pool_size = compact_pool<MAX_BEAM, DIMV>(pl, 1, pool_size, relaxant, metric, lane);
     }
     return nsize;
 }
@@ -141,7 +141,7 @@ __device__ __forceinline__ uint32_t prune_pool_refine(PL* pl, uint32_t pool_size
                          [pl](uint32_t idx) { return pl->pool_id[idx] & kClean; },
                          [pl](uint32_t idx, float sq) { pl->head_sq[idx] = sq; });
         wave_sync();
-        pool_size = compact_pool<MAX_BEAM>(pl, position, pool_size, relaxant, metric, lane);
+        pool_size = compact_pool<MAX_BEAM, DIMV>(pl, position, pool_size, relaxant, metric, lane);
     }
     return nsize;
 }

@@ -20,8 +20,8 @@ template <int MAX_CAND, int MAX_BEAM, int DIMV, bool WHOLE, bool LEFT>
 __device__ __forceinline__ void search_body(const SearchArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     auto* lds = reinterpret_cast<BeamLds<MAX_CAND>*>(smem);
-    float* cent = reinterpret_cast<float*>(smem + sizeof(BeamLds<MAX_CAND>));
-    uint32_t* hash = reinterpret_cast<uint32_t*>(cent + round_up32(a.centroid_num));
+    uint32_t* hash = reinterpret_cast<uint32_t*>(smem + sizeof(BeamLds<MAX_CAND>));   // at a constant offset: no addition a probe
+    float* cent = reinterpret_cast<float*>(hash + (1u << a.p.hash_bit));
     // one query a workgroup, as far as a launch has workgroups
     for (uint32_t qid = blockIdx.x; qid < a.query_num; qid += gridDim.x) {
         Beam<MAX_CAND, MAX_BEAM, DIMV, false, WHOLE> b;
@@ -92,10 +92,10 @@ __global__ __launch_bounds__(64 * kTeam) void search_team_kernel(SearchArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     using Shape = RowShape<DIMV>;
     auto* lds = reinterpret_cast<BeamLds<MAX_CAND>*>(smem);
-    float* cent = reinterpret_cast<float*>(smem + sizeof(BeamLds<MAX_CAND>));
-    float4* qlds = reinterpret_cast<float4*>(cent + round_up32(a.centroid_num));
+    float4* qlds = reinterpret_cast<float4*>(smem + sizeof(BeamLds<MAX_CAND>));
     uint32_t* ctl = reinterpret_cast<uint32_t*>(qlds + Shape::NV * Shape::LPR);   // [0] rows to score, [1] search over
     uint32_t* hash = ctl + 4;
+    float* cent = reinterpret_cast<float*>(hash + (1u << a.p.hash_bit));
     const uint32_t wave = threadIdx.x >> 6;
     const int lane = lane_id();
     for (uint32_t qid = blockIdx.x; qid < a.query_num; qid += gridDim.x) {
