@@ -20,6 +20,9 @@ struct BeamParams {
 
 constexpr uint32_t kCounterStripes = 256;
 
+// First result id of a query that a search over rows of bytes leaves to the fp32 kernel (result ids are below 2^31, or all ones).
+constexpr uint32_t kLeftOver = 0xfffffffeu;
+
 struct BeamCounters {  // wave-uniform tallies for traffic accounting
     uint32_t iterations = 0, rows_scored = 0, graph_rows = 0;
 };

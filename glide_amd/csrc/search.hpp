@@ -19,9 +19,6 @@ struct SearchArgs {
     const unsigned char* bytes;   // the rows as bytes, for the kernels for rows of bytes
 };
 
-// First result id of a query that the kernel for rows of bytes leaves to the fp32 kernel (result ids are below 2^31).
-constexpr uint32_t kLeftOver = 0xfffffffeu;
-
 // Wavefronts of a team (search_team_kernel) and what one needs.
 constexpr int kTeam = 4;
 

@@ -81,13 +81,29 @@ __global__ __launch_bounds__(64) void select_segments_kernel(SelectArgs a) {
 
 // Queries grouped by the partitions they selected: counts, then offsets, then the lists.  With them a partition's
 // search launches one wavefront per query that wants it instead of one per query of the batch.
-__global__ __launch_bounds__(256) void group_count_kernel(const uint32_t* segment_ids, uint32_t total, uint32_t centroid_num, uint32_t* counts) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+// RowProbe: workgroups behind the counting ones look whether the first rows are of bytes (a launch of its own for that cost
+// rows of fractions 3 % of a small batch).
+struct RowProbe {
+    const float* rows;      // null: nothing to look at
+    uint32_t num, dim, lanes;
+    uint32_t* other;        // set if some value is no whole number 0 .. 255
+};
+constexpr uint32_t kProbeBlocks = 64;
+__global__ __launch_bounds__(256) void group_count_kernel(const uint32_t* segment_ids, uint32_t total, uint32_t centroid_num, uint32_t* counts, RowProbe probe) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x, counting = ceil_div(total, 256);
+    if (blockIdx.x >= counting) {
+        const uint32_t piece = i - counting * 256, row = piece / probe.lanes;
+        uint4 unused;
+        const bool exact = row >= probe.num || pack_bytes(probe.rows + static_cast<size_t>(row) * probe.dim, 16 * (piece % probe.lanes), probe.dim, unused);
+        if (ballot(!exact) != 0 && lane_id() == 0) *probe.other = 1u;
+        return;
+    }
     if (i >= total) return;
     const uint32_t s = segment_ids[i];
     if (s < centroid_num) atomicAdd(&counts[s], 1u);
 }
-__global__ __launch_bounds__(256) void group_scan_kernel(uint32_t* counts, uint32_t centroid_num, uint32_t* offsets, uint32_t* cursor) {
+// other: nullable, passed on behind the offsets, so that both are read back together
+__global__ __launch_bounds__(256) void group_scan_kernel(uint32_t* counts, uint32_t centroid_num, uint32_t* offsets, uint32_t* cursor, const uint32_t* other) {
     if (threadIdx.x == 0) {
         uint32_t run = 0;
         for (uint32_t s = 0; s < centroid_num; s++) {
@@ -96,6 +112,7 @@ __global__ __launch_bounds__(256) void group_scan_kernel(uint32_t* counts, uint3
             run += counts[s];
         }
         offsets[centroid_num] = run;
+        if (other) offsets[centroid_num + 1] = *other;
     }
 }
 __global__ __launch_bounds__(256) void group_fill_kernel(const uint32_t* segment_ids, uint32_t total, uint32_t centroid_num, uint32_t* cursor,
@@ -223,6 +240,8 @@ int launch_search_sub(const float* segment_data, uint32_t dim, const uint32_t* s
     if (graph_degree > 256 || !beam_supported(beam) || dim % 4 != 0 || dim > 4096 || top_k > beam || top_k > 128 || hash_bit < 1 || hash_bit > 13)
         return GLIDE_ERR_UNSUPPORTED;   // top_k buckets: kernel_config.cuh:312-323
     SubArgs a;
+    a.bytes = nullptr;
+    a.other = nullptr;
     a.data = segment_data;
     a.graph = segment_graph;
     a.map = segment_map;
@@ -289,8 +308,8 @@ extern "C" int glide_hip_group_queries(const uint32_t* segment_ids, uint32_t que
     if (rc != GLIDE_OK) return rc;
     const uint32_t total = query_num * centroid_num;
     uint32_t* cursor = static_cast<uint32_t*>(workspace);
-    if (total) hipLaunchKernelGGL(group_count_kernel, dim3(ceil_div(total, 256)), dim3(256), 0, s, segment_ids, total, centroid_num, counts);
-    hipLaunchKernelGGL(group_scan_kernel, dim3(1), dim3(256), 0, s, counts, centroid_num, offsets, cursor);
+    if (total) hipLaunchKernelGGL(group_count_kernel, dim3(ceil_div(total, 256)), dim3(256), 0, s, segment_ids, total, centroid_num, counts, RowProbe{});
+    hipLaunchKernelGGL(group_scan_kernel, dim3(1), dim3(256), 0, s, counts, centroid_num, offsets, cursor, static_cast<const uint32_t*>(nullptr));
     if (total) hipLaunchKernelGGL(group_fill_kernel, dim3(ceil_div(total, 256)), dim3(256), 0, s, segment_ids, total, centroid_num, cursor, lists,
                                   static_cast<uint32_t*>(nullptr), static_cast<uint32_t*>(nullptr));
     return launch_status();
@@ -304,8 +323,8 @@ PartitionSearchLayout partition_search_layout(uint32_t query_num, uint32_t centr
     const size_t pairs = static_cast<size_t>(query_num) * centroid_num;   // every query could select every partition
     size_t off = 0;
     auto take = [&off](size_t bytes) { size_t o = off; off += align256(bytes); return o; };
-    l.counts = take(static_cast<size_t>(centroid_num) * 4);
-    l.offsets = take((static_cast<size_t>(centroid_num) + 1) * 4);
+    l.counts = take((static_cast<size_t>(centroid_num) + 1) * 4);    // the last word: whether some row is not of bytes
+    l.offsets = take((static_cast<size_t>(centroid_num) + 2) * 4);   // and here as well
     l.cursor = take(static_cast<size_t>(centroid_num) * 4);
     l.lists = take(pairs * 4);
     l.pair_segment = take(pairs * 4);
@@ -321,12 +340,39 @@ extern "C" size_t glide_hip_search_partitions_workspace_bytes(uint32_t query_num
     return partition_search_layout(query_num, centroid_num, top_k).total;
 }
 
+// As bytes for the duration of the call: where the searches score several times as many rows as there are, reading all of them
+// once to write a quarter is what they save many times over (fp32 : bytes, packing included, on 128 dims: 5 000 queries over
+// 500 000 rows, three partitions each, beam 96 2 284 : 1 262 us; over 200 000 rows 1 963 : 1 075, mixture rows, which come from
+// the caches, 1 072 : 900; at the line, 1 000 queries, 622 : 563 and 538 : 493).  Every query selects a partition at least, as a
+// rule two or three; half of an expansion's rows are new.
+static bool partitions_as_bytes_pay(uint32_t num, uint32_t dim, uint32_t degree, uint32_t query_num, uint32_t beam) {
+    return num != 0 && degree <= kMostByteDegree && glide_hip_byte_rows_bytes(1, dim) != 0 &&
+           static_cast<unsigned long long>(query_num) * beam * degree / 2 >= 4ull * num;
+}
+
+extern "C" size_t glide_hip_search_partitions_rows_workspace_bytes(uint32_t query_num, uint32_t centroid_num, uint32_t top_k, uint32_t num, uint32_t dim,
+                                                                   uint32_t graph_degree, uint32_t beam) {
+    return partition_search_layout(query_num, centroid_num, top_k).total +
+           (partitions_as_bytes_pay(num, dim, graph_degree, query_num, beam) ? glide_hip_byte_rows_bytes(num, dim) : 0);
+}
+
 extern "C" int glide_hip_search_partitions(const float* data, uint32_t dim, const uint32_t* graph, uint32_t graph_degree, const uint32_t* map,
                                            const uint32_t* segment_starts, const uint32_t* segment_start_points, uint32_t segment_num,
                                            const float* queries, uint32_t query_num, const uint32_t* segment_ids, uint32_t top_k, uint32_t beam,
                                            uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit, uint32_t hash_reset_interval,
                                            int metric, uint32_t* final_ids, float* final_dists, void* workspace, size_t workspace_bytes,
                                            unsigned long long* counters, void* stream) {
+    return glide_hip_search_partitions_rows(data, 0, dim, graph, graph_degree, map, segment_starts, segment_start_points, segment_num, queries, query_num,
+                                            segment_ids, top_k, beam, max_iterations, min_iterations, hash_bit, hash_reset_interval, metric, final_ids,
+                                            final_dists, workspace, workspace_bytes, counters, stream);
+}
+
+extern "C" int glide_hip_search_partitions_rows(const float* data, uint32_t num, uint32_t dim, const uint32_t* graph, uint32_t graph_degree,
+                                                const uint32_t* map, const uint32_t* segment_starts, const uint32_t* segment_start_points,
+                                                uint32_t segment_num, const float* queries, uint32_t query_num, const uint32_t* segment_ids,
+                                                uint32_t top_k, uint32_t beam, uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit,
+                                                uint32_t hash_reset_interval, int metric, uint32_t* final_ids, float* final_dists, void* workspace,
+                                                size_t workspace_bytes, unsigned long long* counters, void* stream) {
     if (!data || !graph || !map || !segment_starts || !segment_start_points || !queries || !segment_ids || !final_ids || !final_dists || !workspace)
         return GLIDE_ERR_BAD_ARGUMENT;
     if (dim == 0 || graph_degree == 0 || segment_num == 0 || beam == 0 || top_k == 0 || max_iterations == 0) return GLIDE_ERR_BAD_ARGUMENT;
@@ -336,9 +382,13 @@ extern "C" int glide_hip_search_partitions(const float* data, uint32_t dim, cons
         return GLIDE_ERR_UNSUPPORTED;
     if (static_cast<unsigned long long>(query_num) * segment_num >= 0xffffffffull) return GLIDE_ERR_UNSUPPORTED;   // pairs are numbered with 32 bits
     const PartitionSearchLayout l = partition_search_layout(query_num, segment_num, top_k);
-    if (workspace_bytes < l.total || reinterpret_cast<uintptr_t>(workspace) % 8) return GLIDE_ERR_BAD_ARGUMENT;
+    if (workspace_bytes < glide_hip_search_partitions_rows_workspace_bytes(query_num, segment_num, top_k, num, dim, graph_degree, beam))
+        return GLIDE_ERR_BAD_ARGUMENT;
+    const bool may_be_bytes = partitions_as_bytes_pay(num, dim, graph_degree, query_num, beam) && reinterpret_cast<uintptr_t>(data) % 16 == 0;
+    if ( reinterpret_cast<uintptr_t>(workspace) % (may_be_bytes ? 16 : 8)) return GLIDE_ERR_BAD_ARGUMENT;
     hipStream_t s = as_stream(stream);
     unsigned char* w = static_cast<unsigned char*>(workspace);
+    unsigned char* byte_rows = w + l.total;
     uint32_t* counts = reinterpret_cast<uint32_t*>(w + l.counts);
     uint32_t* offsets = reinterpret_cast<uint32_t*>(w + l.offsets);
     uint32_t* cursor = reinterpret_cast<uint32_t*>(w + l.cursor);
@@ -347,18 +397,24 @@ extern "C" int glide_hip_search_partitions(const float* data, uint32_t dim, cons
     uint32_t* pair_index = reinterpret_cast<uint32_t*>(w + l.pair_index);
     float* pair_dists = reinterpret_cast<float*>(w + l.pair_dists);
     uint32_t* pair_ids = reinterpret_cast<uint32_t*>(w + l.pair_ids);
-    int rc = glide_hip_fill_u32(counts, 0u, segment_num, stream);
+    uint32_t* other = counts + segment_num;
+    int rc = glide_hip_fill_u32(counts, 0u, static_cast<size_t>(segment_num) + 1, stream);
     if (rc != GLIDE_OK) return rc;
     const uint32_t total = query_num * segment_num;
-    hipLaunchKernelGGL(group_count_kernel, dim3(ceil_div(total, 256)), dim3(256), 0, s, segment_ids, total, segment_num, counts);
-    hipLaunchKernelGGL(group_scan_kernel, dim3(1), dim3(256), 0, s, counts, segment_num, offsets, cursor);
+    const RowProbe probe{data, num, dim, static_cast<uint32_t>(dim <= 128 ? RowShape<-1>::LPR : RowShape<-2>::LPR), other};
+    hipLaunchKernelGGL(group_count_kernel, dim3(ceil_div(total, 256) + (may_be_bytes ? kProbeBlocks : 0u)), dim3(256), 0, s, segment_ids, total, segment_num,
+                       counts, probe);
+    hipLaunchKernelGGL(group_scan_kernel, dim3(1), dim3(256), 0, s, counts, segment_num, offsets, cursor, other);
     hipLaunchKernelGGL(group_fill_kernel, dim3(ceil_div(total, 256)), dim3(256), 0, s, segment_ids, total, segment_num, cursor, lists, pair_segment,
                        pair_index);
-    uint32_t pairs = 0;   // the grid of the search: one wavefront per (query, selected partition)
-    GLIDE_HIP_TRY(hipMemcpyAsync(&pairs, offsets + segment_num, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    uint32_t back[2] = {0, 1};
+    GLIDE_HIP_TRY(hipMemcpyAsync(back, offsets + segment_num, (may_be_bytes ? 2 : 1) * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     GLIDE_HIP_TRY(hipStreamSynchronize(s));
+    const uint32_t pairs = back[0];   // the grid of the search: one wavefront per (query, selected partition)
     if (pairs) {
         SubArgs a;
+        a.bytes = nullptr;
+        a.other = nullptr;
         a.data = data;
         a.graph = graph;
         a.map = map;
@@ -381,10 +437,20 @@ extern "C" int glide_hip_search_partitions(const float* data, uint32_t dim, cons
         a.max_topk = top_k <= 32 ? 32 : (top_k <= 64 ? 64 : 128);
         a.list_len = pairs;
         a.p = BeamParams{beam, graph_degree, dim, hash_bit, hash_reset_interval ? hash_reset_interval : 1, max_iterations, min_iterations, metric};
-        sub_fn fn = pick_sub(graph_degree, beam, dim, pairs);
         const size_t lds_bytes = beam_lds_bytes(graph_degree) + 128 * 8 + (size_t{1} << hash_bit) * sizeof(uint32_t);
-        GLIDE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)));
-        hipLaunchKernelGGL(fn, dim3(pairs), dim3(64), lds_bytes, s, a);
+        auto launch = [&](sub_fn fn) {
+            GLIDE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)));
+            hipLaunchKernelGGL(fn, dim3(pairs), dim3(64), lds_bytes, s, a);
+            return GLIDE_OK;
+        };
+        if (back[1] == 0) {   // the rows that were looked at are of bytes; if others are not, every pair is left over
+            if ((rc = glide_hip_pack_byte_rows(data, num, dim, byte_rows, other, stream)) != GLIDE_OK) return rc;
+            a.bytes = byte_rows;
+            a.other = other;
+            if ((rc = launch(pick_sub_bytes(beam, dim))) != GLIDE_OK || (rc = launch(pick_sub_left_over(beam, dim))) != GLIDE_OK) return rc;
+        } else if ((rc = launch(pick_sub(graph_degree, beam, dim, pairs))) != GLIDE_OK) {
+            return rc;
+        }
     }
     hipLaunchKernelGGL(merge_pairs_kernel, dim3(query_num), dim3(64), 0, s, segment_ids, pair_index, pair_dists, pair_ids, query_num, segment_num, top_k,
                        top_k <= 32 ? 32u : (top_k <= 64 ? 64u : 128u), final_dists, final_ids);

@@ -23,6 +23,8 @@ struct SubArgs {
     unsigned long long* counters;
     uint32_t query_num, centroid_num, segment_id, start_point, top_k, max_topk, list_len;
     BeamParams p;
+    const unsigned char* bytes;   // pair mode: the rows as bytes, for the kernels for rows of bytes,
+    const uint32_t* other;        // and whether some row is not of bytes after all
 };
 
 using sub_fn = void (*)(SubArgs);
@@ -30,6 +32,11 @@ using sub_fn = void (*)(SubArgs);
 sub_fn pick_sub_64(uint32_t beam, uint32_t dim, bool six);
 sub_fn pick_sub_128(uint32_t beam, uint32_t dim, bool six);
 sub_fn pick_sub_256(uint32_t beam, uint32_t dim, bool six);
+
+// Rows of bytes, pair mode, up to 64 slots and kMostByteDims dims: the pairs whose query is of bytes, and the fp32 kernel for
+// those left over.
+sub_fn pick_sub_bytes(uint32_t beam, uint32_t dim);
+sub_fn pick_sub_left_over(uint32_t beam, uint32_t dim);
 
 size_t simd_count();   // of the current device; 0 if it cannot be told
 

@@ -40,8 +40,12 @@ __device__ __forceinline__ void merge_result(const float* beam_dist, const uint3
 // search_on_sub_kernel (search_kernel.cuh:653-765)
 // Up to 64 slots on rows of up to 512 dims: five wavefronts per SIMD, for beams up to 64 five or SIX (75 registers allow it;
 // which one is decided per launch, see six_resident).
-template <int MAX_CAND, int MAX_BEAM, int DIMV, bool WHOLE = false, bool SIX = false>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DIMV > 4 ? 1 : MAX_CAND <= 64 ? (SIX ? 6 : 5) : MAX_BEAM > 256 ? 4 : 1, DIMV > 4 || MAX_CAND > 64 ? 8 : (SIX ? 6 : 5))))
+// Over rows of bytes as many as the registers allow (eight up to beam 128).
+// LEFT: only the pairs that the kernel for rows of bytes has left over.
+constexpr int sub_waves_least(int cand, int beam, int dimv, bool six) { return dimv > 4 || dimv < 0 ? 1 : cand <= 64 ? (six ? 6 : 5) : beam > 256 ? 4 : 1; }
+constexpr int sub_waves_most(int cand, int dimv, bool six) { return dimv > 4 || dimv < 0 || cand > 64 ? 8 : six ? 6 : 5; }
+template <int MAX_CAND, int MAX_BEAM, int DIMV, bool WHOLE = false, bool SIX = false, bool LEFT = false>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sub_waves_least(MAX_CAND, MAX_BEAM, DIMV, SIX), sub_waves_most(MAX_CAND, DIMV, SIX))))
 void search_sub_kernel(SubArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     auto* lds = reinterpret_cast<BeamLds<MAX_CAND>*>(smem);
@@ -49,15 +53,18 @@ void search_sub_kernel(SubArgs a) {
     uint32_t* head_id = reinterpret_cast<uint32_t*>(head_dist + 128);
     uint32_t* hash = head_id + 128;
     uint32_t qid = blockIdx.x;
-    const float* data = a.data;
+    row_data<DIMV> data;
+    if constexpr (RowShape<DIMV>::BYTES) data = a.bytes;
+    else data = a.data;
     const uint32_t* graph = a.graph;
     const uint32_t* map = a.map;
     uint32_t start_point = a.start_point;
     if (a.pair_segment) {
         if (qid >= a.list_len) return;
+        if (LEFT && a.pair_ids[static_cast<size_t>(qid) * a.top_k] != kLeftOver) return;   // done on rows of bytes
         const uint32_t seg = a.pair_segment[qid];
         const size_t start = a.segment_starts[seg];
-        data += start * a.p.dim;
+        data = row_at<DIMV>(data, static_cast<uint32_t>(start), a.p.dim);
         graph += start * a.p.degree;
         map += start;
         start_point = a.segment_start_points[seg];
@@ -84,7 +91,15 @@ void search_sub_kernel(SubArgs a) {
     }
 
     Beam<MAX_CAND, MAX_BEAM, DIMV, false, WHOLE> b;
-    b.init(lds, hash, a.p, a.queries + static_cast<size_t>(qid) * a.p.dim);
+    const float* query = a.queries + static_cast<size_t>(qid) * a.p.dim;
+    if constexpr (RowShape<DIMV>::BYTES) {
+        if (*a.other != 0 || !b.init_packing(lds, hash, a.p, query)) {   // not of bytes: left to the fp32 kernel behind this one
+            if (lane_id() == 0) a.pair_ids[static_cast<size_t>(blockIdx.x) * a.top_k] = kLeftOver;
+            return;
+        }
+    } else {
+        b.init(lds, hash, a.p, query);
+    }
     b.expand(start_point, graph, data, kInvalid, kInvalid);   // get_init with point_id = 0xffffffff
     b.run(graph, data, kInvalid);
 
@@ -141,6 +156,19 @@ sub_fn pick_sub_beam(uint32_t beam, uint32_t dim, bool six) {
     if (beam == 512) return pick_sub_dim<MAX_CAND, 512, true>(dim);   // the whole of the widest beam: merged in the registers
     return pick_sub_dim<MAX_CAND, 512>(dim);
 }
+
+#if GLIDE_CAND == 64
+template <int DIMV, bool LEFT>
+sub_fn pick_sub_bytes_beam(uint32_t beam) {
+    if (beam <= 64) return search_sub_kernel<64, 64, DIMV, false, false, LEFT>;
+    if (beam <= 128) return search_sub_kernel<64, 128, DIMV, false, false, LEFT>;
+    if (beam <= 256) return search_sub_kernel<64, 256, DIMV, false, false, LEFT>;
+    if (beam == 512) return search_sub_kernel<64, 512, DIMV, true, false, LEFT>;
+    return search_sub_kernel<64, 512, DIMV, false, false, LEFT>;
+}
+sub_fn pick_sub_bytes(uint32_t beam, uint32_t dim) { return dim <= 128 ? pick_sub_bytes_beam<-1, false>(beam) : pick_sub_bytes_beam<-2, false>(beam); }
+sub_fn pick_sub_left_over(uint32_t beam, uint32_t dim) { return dim <= 128 ? pick_sub_bytes_beam<1, true>(beam) : pick_sub_bytes_beam<2, true>(beam); }
+#endif
 
 #define GLIDE_PICK_NAME(cand) pick_sub_##cand
 #define GLIDE_PICK(cand) GLIDE_PICK_NAME(cand)

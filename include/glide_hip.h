@@ -388,6 +388,20 @@ int glide_hip_search_partitions(const float *data, uint32_t dim, const uint32_t 
                                 uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit,
                                 uint32_t hash_reset_interval, int metric, uint32_t *final_ids, float *final_dists,
                                 void *workspace, size_t workspace_bytes, unsigned long long *counters, void *stream);
+/* The same with the number of rows in `data`, so that rows of bytes can be searched as bytes (see glide_hip_pack_byte_rows;
+ * they are packed into the workspace on each call, where the batch is large enough to gain by it).  Same results.
+ * workspace: glide_hip_search_partitions_rows_workspace_bytes(), 16-byte aligned. */
+size_t glide_hip_search_partitions_rows_workspace_bytes(uint32_t query_num, uint32_t centroid_num, uint32_t top_k,
+                                                        uint32_t num, uint32_t dim, uint32_t graph_degree,
+                                                        uint32_t beam);
+int glide_hip_search_partitions_rows(const float *data, uint32_t num, uint32_t dim, const uint32_t *graph,
+                                     uint32_t graph_degree, const uint32_t *map, const uint32_t *segment_starts,
+                                     const uint32_t *segment_start_points, uint32_t segment_num, const float *queries,
+                                     uint32_t query_num, const uint32_t *segment_ids, uint32_t top_k, uint32_t beam,
+                                     uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit,
+                                     uint32_t hash_reset_interval, int metric, uint32_t *final_ids, float *final_dists,
+                                     void *workspace, size_t workspace_bytes, unsigned long long *counters,
+                                     void *stream);
 
 /* ---- merged large build (GLIDE_large::build_with_merge, declared at glide_large.cuh:89-97 without a definition) --
  * The merged graph lives in device memory in reorder-id space: row r belongs to reorder row r (r < num) and holds

@@ -160,3 +160,37 @@ def test_index_follows_its_rows(hip):
     fractions = G.GLIDE(degree, first + 0.5, first[:2], G.Metric.Euclidean)
     fractions.load(knn, np.array([4, 9], np.uint32))
     assert fractions._byte_rows() is None
+
+
+@pytest.mark.parametrize("dim,degree,beam,top_k,bad_row", [(100, 16, 64, 10, None), (128, 32, 96, 30, None), (128, 32, 64, 10, 2500), (128, 32, 64, 10, 5),
+                                                            (256, 64, 256, 64, None), (132, 24, 512, 128, None)])
+def test_partitions(hip, dim, degree, beam, top_k, bad_row):
+    """Rows of a known number (a DeviceArray) are searched as bytes, the same rows by address as fp32."""
+    from oracle import oracle as O
+    rng = np.random.default_rng(dim + beam)
+    lengths = (1500, 0, 1300, 200)
+    n, c, nq = sum(lengths), len(lengths), 120
+    rows = rows_of(rng, n, dim)
+    if bad_row is not None:
+        rows[bad_row, 1] += 0.5
+    starts = np.concatenate([[0], np.cumsum(lengths)[:-1]]).astype(np.uint32)
+    graph = np.concatenate([O.bruteforce_knn(rows[s:s + m], rows[s:s + m], degree, exclude_self=True)[0] for s, m in zip(starts, lengths) if m])
+    entries = np.array([7, INV, 100, 0], np.uint32)
+    queries = rows_of(rng, nq, dim)
+    queries[3, 2], queries[nq - 1, 0], queries[40, 1] = 0.5, -1.0, np.nan
+    segments = np.full((nq, c), INV, np.uint32)
+    for q in range(nq):
+        pick = rng.permutation(c)[:rng.integers(1, c + 1)]
+        segments[q, :len(pick)] = pick
+    sp = O.search_params(beam, degree)
+    assert nq * beam * degree // 2 >= 4 * n
+    up = hip.DeviceArray.from_numpy
+    d, d_g, d_m, d_s, d_e, d_q, d_seg = up(rows), up(graph), up(rng.permutation(n).astype(np.uint32)), up(starts), up(entries), up(queries), up(segments)
+    got = []
+    for data in (d.ptr, d):
+        ids, dists, cnt = hip.DeviceArray.full((nq, top_k), 0xDEADBEEF), hip.DeviceArray.full((nq, top_k), 0xDEADBEEF), hip.new_counters()
+        hip.search_partitions(data, dim, d_g, degree, d_m, d_s, d_e, c, d_q, nq, d_seg, top_k, sp["beam"], sp["max_iterations"], sp["min_iterations"],
+                              sp["hash_bit"], sp["hash_reset_interval"], 0, ids, dists, cnt)
+        got.append((ids.numpy(), dists.numpy(), hip.read_counters(cnt)))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1]) and got[0][2] == got[1][2]
+    assert (got[0][0][:, 0] < n).sum() >= nq // 2          # some select the empty partition alone
