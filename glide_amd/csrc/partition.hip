@@ -621,6 +621,11 @@ __global__ __launch_bounds__(256) void row_norms_kernel(const float* rows, uint3
 // is reproducible and a CPU restatement can follow it.
 constexpr uint32_t kSeedTrials = 8;        // most candidates per step
 constexpr uint32_t kSeedPoints = 64;       // sample rows per workgroup of the trial kernel
+// The distances to a step's candidates are kept for the step after up to this many sample rows (1 MiB, in the L2).  For larger
+// samples the distance to the winner is computed a second time, by the trial kernel as one candidate more and for the 64 rows
+// that a draw ends in: the workspace stays at 5 bytes a row (a step of 33 000 rows of 96 dims 20 us, one of 200 000 of 200 dims
+// 102 us; with a pass of their own for the smallest distances 43 and 236).
+constexpr uint32_t kSeedKept = 32768;
 
 __host__ __device__ inline uint32_t seed_trials(uint32_t k) {
     uint32_t t = 2;
@@ -676,6 +681,37 @@ __device__ __forceinline__ uint32_t wave_locate(Load load, uint32_t len, double 
 // four values of a row, zeros in the lanes behind its end
 __device__ __forceinline__ float4 load4(const float* p, bool in) { return in ? *reinterpret_cast<const float4*>(p) : make_float4(0.f, 0.f, 0.f, 0.f); }
 
+// One wavefront: the squared distances of the rows [first, first + rows) to row c, a row a lane; summed as the trial kernel does.
+template <int LANES>
+__device__ __forceinline__ float block_distances(const float* sample, uint32_t dim, uint32_t first, uint32_t rows, uint32_t c, int lane) {
+    constexpr uint32_t kAtOnce = 64 / LANES, kUnder = 16;
+    const uint32_t t = static_cast<uint32_t>(lane) % LANES, part = static_cast<uint32_t>(lane) / LANES;
+    float mine = 0.f;
+    for (uint32_t r = 0; r < rows; r += kAtOnce * kUnder) {
+        float acc[kUnder] = {};
+        for (uint32_t d0 = t * 4; d0 < (LANES == 32 ? 128u : (dim + 255) / 256 * 256); d0 += LANES == 32 ? 128 : 256) {
+            const bool in = d0 < dim;
+            const float4 b = load4(sample + static_cast<size_t>(c) * dim + d0, in);
+#pragma unroll
+            for (uint32_t u = 0; u < kUnder; u++) {
+                const uint32_t i = r + u * kAtOnce + part;
+                const float4 x = load4(sample + static_cast<size_t>(first + (i < rows ? i : rows - 1)) * dim + d0, in);
+                if (LANES == 32 || in) acc[u] = sqdist4(x, b, acc[u]);
+            }
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kUnder; u++) {
+            const float d = LANES == 32 ? half_wave_sum(acc[u]) : wave_sum(acc[u]);
+#pragma unroll
+            for (uint32_t q = 0; q < kAtOnce; q++) {
+                const float of = read_lane(d, static_cast<int>(q * LANES));
+                if (static_cast<uint32_t>(lane) == r + u * kAtOnce + q) mine = of;
+            }
+        }
+    }
+    return mine;
+}
+
 // 64 sample rows per workgroup, LANES lanes a row: min_dist lowered by the distances to the last step's winner (`winner`, null
 // in the first step, says which of its candidates' trial_dist that are), the squared distance of every row to every candidate
 // (trial_dist, for the step after) and the candidates' potentials over these rows, in double, summed row after row in four runs of 16 whatever the layout.  Rows of up to 128 dims take half a wavefront and
@@ -684,12 +720,12 @@ __device__ __forceinline__ float4 load4(const float* p, bool in) { return in ? *
 // The candidates' ids are read before the first row, so that no row load waits for them, and the masked loads choose between
 // values: choosing between a row in memory and zeros held in a variable selects an address, which put the zeros into private
 // memory, made the loads flat ones and every wait for an id a wait for all rows (a step of 20 000 rows of 128 dims and 7
-// candidates, next kernel included: 28.8 -> 26.3 us; a sample of 200 rows 14.4 -> 13.5 us).  Rows of 129 to 256 dims go four at
-// a time (one at a time 2.5 % slower on 200 000 rows than a wavefront that keeps the sums of all candidates, four 4-15 %
-// faster); longer ones one at a time, so that a workgroup's rows stay in the L1 from candidate to candidate (960 dims, 50 000
-// rows: four at a time 1.36 times the time).
+// candidates, next kernel included: 28.8 -> 26.3 us; a sample of 200 rows 14.4 -> 13.5 us).  Rows of more than 128 dims
+// go four at a time, those of more than 256 past four candidates: eight rows and seven candidates of 960 dims do not fit an L1, and
+// one row at a time read 3.8 KB of candidate from the L2 for each distance (a step of 20 000 such rows 65.6 -> 42.7 us).
 constexpr uint32_t kTrialThreads = 512;
-template <int LANES, uint32_t TOGETHER = 1>   // TOGETHER: rows of more than 128 dims under way at once
+// TOGETHER, CANDS: rows and candidates that one pass over rows of more than 128 dims takes; !KEPT: no trial_dist, `winner` is its row.
+template <bool KEPT, int LANES, uint32_t TOGETHER = 1, uint32_t CANDS = 1>
 __global__ __launch_bounds__(kTrialThreads) void kmeanspp_trial_kernel(const float* sample, uint32_t n, uint32_t dim, float* min_dist,
                                                                       const uint32_t* candidates, uint32_t trials, const uint32_t* winner, double* partial,
                                                                       float* trial_dist) {
@@ -698,12 +734,13 @@ __global__ __launch_bounds__(kTrialThreads) void kmeanspp_trial_kernel(const flo
     __shared__ float dist[kSeedTrials][kSeedPoints];
     __shared__ double run_pot[4][kSeedTrials];
     __shared__ float lowered[kSeedPoints];
+    __shared__ float again[KEPT ? 1 : kSeedPoints];
     const uint32_t group = threadIdx.x / LANES, t = threadIdx.x % LANES, first = blockIdx.x * kSeedPoints;
-    const uint32_t last = threadIdx.x < kSeedPoints && winner ? *winner : 0u;
+    const uint32_t last = (!KEPT || threadIdx.x < kSeedPoints) && winner ? *winner : 0u;
     float so_far = 0.f, to_winner = 0.f;
     if (threadIdx.x < kSeedPoints && first + threadIdx.x < n) {
         so_far = min_dist[first + threadIdx.x];
-        to_winner = winner ? trial_dist[static_cast<size_t>(last) * n + first + threadIdx.x] : so_far;
+        to_winner = KEPT && winner ? trial_dist[static_cast<size_t>(last) * n + first + threadIdx.x] : so_far;
     }
     if constexpr (LANES == 32) {
         uint32_t id[kSeedTrials];
@@ -726,25 +763,53 @@ __global__ __launch_bounds__(kTrialThreads) void kmeanspp_trial_kernel(const flo
                 const float d = half_wave_sum(sqdist4(x[r], c[j], 0.f));
                 if (t == 0) dist[j][group * kRows + r] = d;
             }
+        if constexpr (!KEPT) {
+            const float4 w = load4(sample + static_cast<size_t>(last) * dim + t * 4, in);
+#pragma unroll
+            for (uint32_t r = 0; r < kRows; r++) {
+                const float d = half_wave_sum(sqdist4(x[r], w, 0.f));
+                if (t == 0) again[group * kRows + r] = d;
+            }
+        }
     } else {
         for (uint32_t r = 0; r < kRows; r += TOGETHER) {
             const uint32_t i = first + group * kRows + r;
-            for (uint32_t j = 0; j < trials; j++) {
-                const float* c = sample + static_cast<size_t>(candidates[j]) * dim;
-                float acc[TOGETHER] = {};
+            const uint32_t all = trials + (KEPT ? 0 : 1);
+            for (uint32_t j = 0; j < all; j += CANDS) {
+                const float* c[CANDS];
+#pragma unroll
+                for (uint32_t q = 0; q < CANDS; q++) {
+                    const uint32_t m = j + q < all ? j + q : j;
+                    c[q] = sample + static_cast<size_t>(m < trials ? candidates[m] : last) * dim;
+                }
+                float acc[CANDS][TOGETHER] = {};
                 for (uint32_t d0 = t * 4; d0 < dim; d0 += 256) {
-                    const float4 b = *reinterpret_cast<const float4*>(c + d0);
+                    float4 b[CANDS];
 #pragma unroll
-                    for (uint32_t p = 0; p < TOGETHER; p++)
-                        acc[p] = sqdist4(*reinterpret_cast<const float4*>(sample + static_cast<size_t>(i + p < n ? i + p : n - 1) * dim + d0), b, acc[p]);
+                    for (uint32_t q = 0; q < CANDS; q++) b[q] = *reinterpret_cast<const float4*>(c[q] + d0);
+#pragma unroll
+                    for (uint32_t p = 0; p < TOGETHER; p++) {
+                        const float4 x = *reinterpret_cast<const float4*>(sample + static_cast<size_t>(i + p < n ? i + p : n - 1) * dim + d0);
+#pragma unroll
+                        for (uint32_t q = 0; q < CANDS; q++) acc[q][p] = sqdist4(x, b[q], acc[q][p]);
+                    }
                 }
 #pragma unroll
-                for (uint32_t p = 0; p < TOGETHER; p++) {
-                    const float d = wave_sum(acc[p]);
-                    if (t == 0) dist[j][group * kRows + r + p] = d;
-                }
+                for (uint32_t q = 0; q < CANDS; q++)
+#pragma unroll
+                    for (uint32_t p = 0; p < TOGETHER; p++) {
+                        const float d = wave_sum(acc[q][p]);
+                        if (t == 0 && j + q < all) {
+                            if (KEPT || j + q < trials) dist[j + q][group * kRows + r + p] = d;
+                            else again[group * kRows + r + p] = d;
+                        }
+                    }
             }
         }
+    }
+    if constexpr (!KEPT) {
+        __syncthreads();
+        if (threadIdx.x < kSeedPoints && winner) to_winner = again[threadIdx.x];
     }
     if (threadIdx.x < kSeedPoints) {
         const float low = fminf(so_far, to_winner);
@@ -752,7 +817,7 @@ __global__ __launch_bounds__(kTrialThreads) void kmeanspp_trial_kernel(const flo
         if (winner && first + threadIdx.x < n) min_dist[first + threadIdx.x] = low;
     }
     __syncthreads();
-    {
+    if constexpr (KEPT) {
         const uint32_t j = threadIdx.x / kSeedPoints, i = first + threadIdx.x % kSeedPoints;
         if (j < trials && i < n) trial_dist[static_cast<size_t>(j) * n + i] = dist[j][threadIdx.x % kSeedPoints];
     }
@@ -815,6 +880,7 @@ __device__ __forceinline__ uint32_t choose_winner(const float* sample, uint32_t 
 // a workgroup's potential for the winner is the sum of its rows' min_dist once lowered, so a draw looks for its place among
 // the workgroups' sums and then among the 64 rows of one of them.  min_dist itself is lowered by the trial that follows, each
 // workgroup its own rows.  (Going through min_dist here, 20 000 rows took 18 us a step, most of them loads one after another.)
+template <int LANES, bool KEPT>
 __global__ __launch_bounds__(1024) void kmeanspp_next_kernel(const float* sample, uint32_t n, uint32_t dim, const double* partial, uint32_t blocks,
                                                              const float* min_dist, const float* trial_dist, uint32_t trials, uint32_t next_trials,
                                                              uint32_t seed, uint32_t step, uint32_t* candidates, uint32_t* winner, float* centroids,
@@ -822,7 +888,8 @@ __global__ __launch_bounds__(1024) void kmeanspp_next_kernel(const float* sample
     __shared__ double part[1024];   // sums of `chunk` workgroups each
     const uint32_t won = choose_winner(sample, dim, partial, blocks, candidates, trials, step, centroids, chosen_rows);
     if (next_trials == 0) return;   // that was the last one
-    if (threadIdx.x == 0) *winner = won;
+    const uint32_t won_row = candidates[won];
+    if (threadIdx.x == 0) *winner = KEPT ? won : won_row;
     const int lane = lane_id();
     const uint32_t wave = threadIdx.x >> 6, chunk = (blocks + 1023) / 1024, parts = (blocks + chunk - 1) / chunk;
     if (threadIdx.x < parts) {
@@ -847,8 +914,10 @@ __global__ __launch_bounds__(1024) void kmeanspp_next_kernel(const float* sample
         const uint32_t block = base + wave_locate([&](uint32_t i) { return sums[static_cast<size_t>(i) * kSeedTrials]; }, len, target - before, before_block, lane);
         const uint32_t first = block * kSeedPoints, rows = n - first < kSeedPoints ? n - first : kSeedPoints;
         const float* md = min_dist + first;
-        const float* td = trial_dist + static_cast<size_t>(won) * n + first;
-        const double value = static_cast<uint32_t>(lane) < rows ? static_cast<double>(fminf(md[lane], td[lane])) : 0.0;   // a row a lane
+        float to_won;
+        if constexpr (KEPT) to_won = static_cast<uint32_t>(lane) < rows ? trial_dist[static_cast<size_t>(won) * n + first + lane] : 0.f;
+        else to_won = block_distances<LANES>(sample, dim, first, rows, won_row, lane);
+        const double value = static_cast<uint32_t>(lane) < rows ? static_cast<double>(fminf(md[lane], to_won)) : 0.0;   // a row a lane
         cand = first + wave_locate([&](uint32_t) { return value; }, rows, target - before - before_block, unused, lane);
     }
     if (lane == 0) candidates[wave] = cand;
@@ -1319,9 +1388,9 @@ size_t glide_hip_kmeans_workspace_bytes(uint32_t cluster_num, uint32_t dim) {
 
 size_t glide_hip_kmeans_seed_workspace_bytes(uint32_t sample_num) {
     // min_dist (f32 per row) | candidates (8 u32), winner (u32) | per-workgroup potentials of the trial kernel (8 f64 each)
-    // | distances of every row to the candidates (8 f32 per row)
+    // | up to kSeedKept rows: their distances to the candidates (8 f32 per row)
     return align_up(static_cast<size_t>(sample_num) * 4, 256) + 256 + static_cast<size_t>(ceil_div(sample_num, kSeedPoints)) * kSeedTrials * 8 +
-           static_cast<size_t>(sample_num) * kSeedTrials * 4;
+           (sample_num <= kSeedKept ? static_cast<size_t>(sample_num) * kSeedTrials * 4 : 0);
 }
 
 int glide_hip_kmeans_seed(const float* sample, uint32_t sample_num, uint32_t dim, uint32_t cluster_num, uint32_t seed, float* centroids,
@@ -1339,13 +1408,17 @@ int glide_hip_kmeans_seed(const float* sample, uint32_t sample_num, uint32_t dim
     const uint32_t trials = seed_trials(cluster_num), blocks = ceil_div(sample_num, kSeedPoints);
     uint32_t* winner = candidates + kSeedTrials;
     float* trial_dist = reinterpret_cast<float*>(partial + static_cast<size_t>(blocks) * kSeedTrials);
-    auto trial = dim <= 128 ? kmeanspp_trial_kernel<32> : dim <= 256 ? kmeanspp_trial_kernel<64, 4> : kmeanspp_trial_kernel<64>;
+    const bool kept = sample_num <= kSeedKept;
+    auto trial = dim <= 128   ? (kept ? kmeanspp_trial_kernel<true, 32> : kmeanspp_trial_kernel<false, 32>)
+                 : dim <= 256 ? (kept ? kmeanspp_trial_kernel<true, 64, 4> : kmeanspp_trial_kernel<false, 64, 4>)
+                              : (kept ? kmeanspp_trial_kernel<true, 64, 4, 4> : kmeanspp_trial_kernel<false, 64, 4, 4>);
+    auto next_step = kept ? kmeanspp_next_kernel<64, true> : dim <= 128 ? kmeanspp_next_kernel<32, false> : kmeanspp_next_kernel<64, false>;
     hipLaunchKernelGGL(kmeanspp_begin_kernel, dim3(ceil_div(sample_num, 256)), dim3(256), 0, s, sample_num, seed, min_dist, candidates);
     for (uint32_t step = 0; step < cluster_num; step++) {
         const uint32_t now = step == 0 ? 1u : trials, next = step + 1 < cluster_num ? trials : 0u;
         hipLaunchKernelGGL(trial, dim3(blocks), dim3(kTrialThreads), 0, s, sample, sample_num, dim, min_dist, candidates, now,
                            step == 0 ? static_cast<const uint32_t*>(nullptr) : winner, partial, trial_dist);
-        hipLaunchKernelGGL(kmeanspp_next_kernel, dim3(1), dim3(1024), 0, s, sample, sample_num, dim, partial, blocks, min_dist, trial_dist, now, next, seed,
+        hipLaunchKernelGGL(next_step, dim3(1), dim3(1024), 0, s, sample, sample_num, dim, partial, blocks, min_dist, trial_dist, now, next, seed,
                            step, candidates, winner, centroids, chosen_rows);
     }
     return launch_status();
