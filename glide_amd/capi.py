@@ -225,8 +225,8 @@ def hashmap_insert_seq(table, bitlen, keys, n, flags, stream=None):
 
 def build_subgraph(reorder_data, num, dim, knn_graph, knn_degree, mp, segment_starts, segment_lengths, segment_num,
                    start_points, graph_degree, beam, max_iterations, min_iterations, hash_bit, hash_reset_interval,
-                   relaxant, metric, graph, counters=None, stream=None, byte_rows=None):
-    check(lib().glide_hip_build_subgraph_bytes(_ptr(reorder_data), _ptr(byte_rows), u32(num), u32(dim), _ptr(knn_graph), u32(knn_degree),
+                   relaxant, metric, graph, counters=None, stream=None, byte_rows=None, rough_rows=None):
+    check(lib().glide_hip_build_subgraph_rows(_ptr(reorder_data), _ptr(byte_rows), _ptr(rough_rows), u32(num), u32(dim), _ptr(knn_graph), u32(knn_degree),
                                                _ptr(mp), _ptr(segment_starts), _ptr(segment_lengths), u32(segment_num),
                                                _ptr(start_points), u32(graph_degree), u32(beam), u32(max_iterations),
                                                u32(min_iterations), u32(hash_bit), u32(hash_reset_interval), f32(relaxant),
@@ -236,8 +236,8 @@ def build_subgraph(reorder_data, num, dim, knn_graph, knn_degree, mp, segment_st
 
 def build_boundary(reorder_data, num, reorder_num, dim, knn_graph, knn_degree, mp, start_point, graph_degree, beam,
                    max_iterations, min_iterations, hash_bit, hash_reset_interval, relaxant, metric, graph,
-                   counters=None, stream=None, byte_rows=None):
-    check(lib().glide_hip_build_boundary_bytes(_ptr(reorder_data), _ptr(byte_rows), u32(num), u32(reorder_num), u32(dim), _ptr(knn_graph),
+                   counters=None, stream=None, byte_rows=None, rough_rows=None):
+    check(lib().glide_hip_build_boundary_rows(_ptr(reorder_data), _ptr(byte_rows), _ptr(rough_rows), u32(num), u32(reorder_num), u32(dim), _ptr(knn_graph),
                                                u32(knn_degree), _ptr(mp), u32(start_point), u32(graph_degree), u32(beam),
                                                u32(max_iterations), u32(min_iterations), u32(hash_bit),
                                                u32(hash_reset_interval), f32(relaxant), C.c_int(metric), _out(graph),
@@ -263,8 +263,8 @@ def insert_reverse(graph, reverse_graph, reverse_counts, num, graph_degree, stre
 
 def refine(data, num, dim, graph_in, graph_out, graph_degree, centroids, centroid_num, start_points, beam,
            max_iterations, min_iterations, hash_bit, hash_reset_interval, relaxant, metric, counters=None,
-           stream=None, order=None, byte_rows=None):
-    check(lib().glide_hip_refine_bytes(_ptr(data), _ptr(byte_rows), u32(num), u32(dim), _ptr(graph_in), _out(graph_out), u32(graph_degree),
+           stream=None, order=None, byte_rows=None, rough_rows=None):
+    check(lib().glide_hip_refine_rows(_ptr(data), _ptr(byte_rows), _ptr(rough_rows), u32(num), u32(dim), _ptr(graph_in), _out(graph_out), u32(graph_degree),
                                        _ptr(centroids), u32(centroid_num), _ptr(start_points), u32(beam),
                                        u32(max_iterations), u32(min_iterations), u32(hash_bit), u32(hash_reset_interval),
                                        f32(relaxant), C.c_int(metric), _ptr(order), _out(counters), vp(stream)), "glide_hip_refine")
@@ -444,6 +444,15 @@ def byte_rows_bytes(num, dim):
 def pack_byte_rows(rows, num, dim, byte_rows, other_values, stream=None):
     check(lib().glide_hip_pack_byte_rows(_ptr(rows), u32(num), u32(dim), _out(byte_rows), _out(other_values), vp(stream)),
           "glide_hip_pack_byte_rows")
+
+
+def rough_rows_bytes(num, dim):
+    f = _size_fn("glide_hip_rough_rows_bytes")
+    return int(f(u32(num), u32(dim)))
+
+
+def pack_rough_rows(rows, num, dim, rough_rows, stream=None):
+    check(lib().glide_hip_pack_rough_rows(_ptr(rows), u32(num), u32(dim), _out(rough_rows), vp(stream)), "glide_hip_pack_rough_rows")
 
 
 def copy_rows(src, num, src_dim, dst, dst_dim, stream=None):

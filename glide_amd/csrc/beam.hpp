@@ -154,11 +154,71 @@ __device__ __forceinline__ void score_list(const RowRegs<DIMV>& ref, row_data<DI
     score_share<DIMV, U>(RefInRegs<DIMV>{ref}, data, dim, first, count, lane, 0u, 1u, id_of, out);
 }
 
+// The same over the fp16 copy of long rows: out(idx, squared distance to the rounded row).  A lane owns the dims of a row that it
+// owns in score_step (eight bytes a load, so that the reference row serves as it is held), twice as many rows are under way.
+template <int DIMV, int U, class IdFn, class OutFn>
+__device__ __forceinline__ void rough_step(const RowRegs<DIMV>& ref, const RoughRows& rough, uint32_t dim, uint32_t base, uint32_t count, int g, int t,
+                                           IdFn id_of, OutFn out) {
+    using Shape = RowShape<DIMV>;
+    typedef _Float16 half4v __attribute__((ext_vector_type(4)));
+    half4v rows[U][Shape::NV];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const uint32_t idx = base + Shape::ROWS * u + g;
+        const _Float16* row = rough.rows + static_cast<size_t>(id_of(idx < count ? idx : count - 1)) * dim;
+#pragma unroll
+        for (int c = 0; c < Shape::NV; c++) {
+            const uint32_t d0 = (c * Shape::LPR + t) * 4;
+            rows[u][c] = d0 < dim ? *reinterpret_cast<const half4v*>(row + d0) : half4v{0, 0, 0, 0};
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const uint32_t idx = base + Shape::ROWS * u + g;
+        float acc = 0.f;
+#pragma unroll
+        for (int c = 0; c < Shape::NV; c++) {
+            const float4 q = ref.v[c];
+            const float dx = fmaf(-rough.unit, static_cast<float>(rows[u][c][0]), q.x), dy = fmaf(-rough.unit, static_cast<float>(rows[u][c][1]), q.y),
+                        dz = fmaf(-rough.unit, static_cast<float>(rows[u][c][2]), q.z), dw = fmaf(-rough.unit, static_cast<float>(rows[u][c][3]), q.w);
+            acc = fmaf(dx, dx, acc);
+            acc = fmaf(dy, dy, acc);
+            acc = fmaf(dz, dz, acc);
+            acc = fmaf(dw, dw, acc);
+        }
+        const float sq = row_sum<DIMV>(acc);
+        if (t == 0 && idx < count) out(idx, sq);
+    }
+}
+template <int DIMV, class IdFn, class OutFn>
+__device__ __forceinline__ void rough_list(const RowRegs<DIMV>& ref, const RoughRows& rough, uint32_t dim, uint32_t first, uint32_t count, int lane,
+                                           IdFn id_of, OutFn out) {
+    using Shape = RowShape<DIMV>;
+    constexpr int U = 8;
+    const int g = Shape::row_of_lane(lane), t = Shape::lane_in_row(lane);
+    for (uint32_t base = first; base < count; base += Shape::ROWS * U) {
+        if (count - base <= Shape::ROWS * (U / 2)) rough_step<DIMV, U / 2>(ref, rough, dim, base, count, g, t, id_of, out);
+        else rough_step<DIMV, U>(ref, rough, dim, base, count, g, t, id_of, out);
+    }
+}
+// the reference row's length, or a little more, for the bounds of the rough distances
+template <int DIMV>
+__device__ __forceinline__ float row_length(const RowRegs<DIMV>& r) {
+    float acc = 0.f;
+#pragma unroll
+    for (int c = 0; c < RowShape<DIMV>::NV; c++) acc = fmaf(r.v[c].x, r.v[c].x, fmaf(r.v[c].y, r.v[c].y, fmaf(r.v[c].z, r.v[c].z, fmaf(r.v[c].w, r.v[c].w, acc))));
+    return sqrtf(row_sum<DIMV>(acc)) * 1.001f;
+}
+
 // TEAM: the beam's wavefront is one of several in its workgroup (the others only score rows, see search_team_kernel).
 // WHOLE: the host promises beam == MAX_BEAM (asked for beams above 256 only, i.e. beam 512): the two-half merge of such a
 // beam needs no lane permutations and tracks no turning points (merge_beam_full).
-template <int MAX_CAND, int MAX_BEAM, int DIMV, bool TEAM = false, bool WHOLE = false>
+// ROUGH: rows are looked at in fp16 first (long rows, one candidate slot a lane).  The main loop over 120 000 rows of 960 values,
+// 46 of them scored an expansion, runs at 7.4 TB/s of row traffic; with nine tenths of that halved and the rest read after it,
+// the build of those rows (60 000, degree 64, beam 64) takes 224 ms instead of 355.
+template <int MAX_CAND, int MAX_BEAM, int DIMV, bool TEAM = false, bool WHOLE = false, bool ROUGH = false>
 struct Beam {
+    static_assert(!ROUGH || (MAX_CAND == 64 && MAX_BEAM <= 128), "the lists of entries to measure are sized for these");
     static_assert(!WHOLE || MAX_BEAM > 256, "beams up to 256 merge in the registers anyway");
     static __device__ __forceinline__ void wave_sync() { wave_sync_in<TEAM>(); }
     static constexpr int NB = MAX_BEAM / 64;
@@ -182,6 +242,9 @@ struct Beam {
     int rank_most;
     uint32_t cid;           // candidate id of this lane's slot (MAX_CAND == 64; larger buckets keep the ids in LDS)
     uint32_t place[NC];     // where in vlist each of this lane's slots is; kInvalid: not scored
+    RoughRows rough;        // ROUGH: the rows in fp16,
+    float q_length;         // the reference row's length,
+    uint64_t passed_over;   // and which entries of vlist a first look has found too far to enter (they count as infinitely far)
 
     __device__ __forceinline__ void begin(BeamLds<MAX_CAND>* lds_, uint32_t* hash_, const BeamParams& p_) {
         lds = lds_;
@@ -219,7 +282,7 @@ struct Beam {
     // One pass of the main loop up to the next expansion's candidate list (what `run` does between two score phases).
     // Returns false when the search is over; otherwise `nv` rows wait to be scored.
     __device__ __forceinline__ bool step_to_list(uint32_t& iter, bool& terminate, const uint32_t* graph, uint32_t self_id, uint32_t& nv) {
-        absorb(iter == 0);
+        absorb(iter == 0, nullptr);
         cnt.iterations++;
         const bool reset_now = count_down();
         if (reset_now) {
@@ -268,10 +331,44 @@ struct Beam {
         return nv;
     }
 
+    // exact squared distances of the entries of vlist named by a lane mask
+    __device__ __forceinline__ void measure(uint64_t which, row_data<DIMV> data) {
+        static_assert(!ROUGH || MAX_CAND == 64, "one entry a lane");
+        if (which == 0) {
+            wave_sync();
+            return;
+        }
+        BeamLds<MAX_CAND>* l = lds;
+        if ((which >> lane) & 1) l->cand_id[prefix_count(which)] = lane;   // the ids of a search with one slot a lane are in registers: the list is free
+        wave_sync();
+        score_list<DIMV>(q, data, p.dim, 0, __popcll(which), lane,
+                         [l](uint32_t idx) { return l->vlist[l->cand_id[idx]]; },
+                         [l](uint32_t idx, float sq) { l->cand_dist[l->cand_id[idx]] = sq; });
+        wave_sync();
+    }
+
+    // `entry`: the first expansion of a search, whose beam holds nothing yet
     __device__ __forceinline__ void expand(uint32_t parent, const uint32_t* graph, row_data<DIMV> data,
-                                           uint32_t exclude_insert, uint32_t exclude_score) {
+                                           uint32_t exclude_insert, uint32_t exclude_score, bool entry = true) {
         const uint32_t nv = expand_list(parent, graph, exclude_insert, exclude_score);
         BeamLds<MAX_CAND>* l = lds;
+        if constexpr (ROUGH) {
+            passed_over = 0;
+            const float tail = __uint_as_float(tail_key());
+            if (!entry && nv != 0 && tail < FLT_MAX) {   // a beam that is not full takes every row
+                rough_list<DIMV>(q, rough, p.dim, 0, nv, lane,
+                                 [l](uint32_t idx) { return l->vlist[idx]; },
+                                 [l](uint32_t idx, float sq) { l->cand_dist[idx] = sq; });
+                wave_sync();
+                const float least = rough_least(rough, l->cand_dist[lane], q_length);
+                const bool mine = static_cast<uint32_t>(lane) < nv;
+                const bool out = mine && least > 0.f && (p.metric == kEuclidean ? least : least * least * (1.f - rough.slack)) >= tail;
+                passed_over = ballot(out);
+                if (out) l->cand_dist[lane] = __builtin_inff();
+                measure(ballot(mine && !out), data);
+                return;
+            }
+        }
         score_list<DIMV>(q, data, p.dim, 0, nv, lane,
                          [l](uint32_t idx) { return l->vlist[idx]; },
                          [l](uint32_t idx, float sq) { l->cand_dist[idx] = sq; });
@@ -555,14 +652,8 @@ struct Beam {
         }
     }
 
-    // The candidates of the latest expansion that are below the last beam entry, as a lane mask (one candidate slot per
-    // lane).  None: the beam stays as it is -- the half-cleaner of the merge replaces an entry only by a strictly smaller
-    // candidate, entry `beam - 1 - k` by the k-th smallest, so if even the smallest candidate is not below the largest
-    // entry nothing is replaced, and the candidate sort in front of it only feeds that test.  Half of all iterations of
-    // a wide beam end here (the further a search has come, the fewer neighbours of its frontier are nearer than the worst
-    // entry it holds), for one comparison per lane.
-    __device__ __forceinline__ uint64_t entering(float ck) const {
-        static_assert(MAX_CAND == 64, "one candidate slot per lane");
+    // The last beam entry's key, as bits.
+    __device__ __forceinline__ uint32_t tail_key() const {
         // The beam is ascending, so its last entry is the largest key of the lane that holds it among that lane's entries
         // below `beam` (written as a maximum: a chain of selects between the registers becomes a run-time index, which
         // moves the beam out of the registers).  Keys are not negative, so they compare as their bits; what is not a number is
@@ -580,6 +671,18 @@ struct Beam {
             }
             tail = read_lane(mine, static_cast<int>(last / NB));
         }
+        return tail;
+    }
+
+    // The candidates of the latest expansion that are below the last beam entry, as a lane mask (one candidate slot per
+    // lane).  None: the beam stays as it is -- the half-cleaner of the merge replaces an entry only by a strictly smaller
+    // candidate, entry `beam - 1 - k` by the k-th smallest, so if even the smallest candidate is not below the largest
+    // entry nothing is replaced, and the candidate sort in front of it only feeds that test.  Half of all iterations of
+    // a wide beam end here (the further a search has come, the fewer neighbours of its frontier are nearer than the worst
+    // entry it holds), for one comparison per lane.
+    __device__ __forceinline__ uint64_t entering(float ck) const {
+        static_assert(MAX_CAND == 64, "one candidate slot per lane");
+        const uint32_t tail = tail_key();
         return ballot(__float_as_uint(ck) < tail);
     }
 
@@ -746,7 +849,7 @@ struct Beam {
     // meets one leaves its other keys unsorted.  They are no candidates, except while there are no others: the entry's
     // neighbours then make up the beam unsorted and are expanded like any entry (a query with a NaN ends with them), until an
     // expansion finds a row at a finite distance and a new beam starts with that expansion's candidates.
-    __device__ __forceinline__ void absorb(bool first) {
+    __device__ __forceinline__ void absorb(bool first, row_data<DIMV> data) {
         // No row scored: every candidate distance is FLT_MAX, the sort would not move anything (equal keys are never
         // exchanged) and no candidate can displace a beam entry, so the beam stays as it is.
         if (!first && last_scored == 0) return;
@@ -766,6 +869,12 @@ struct Beam {
                 }
                 wave_sync();
                 if (static_cast<int>(m) > rank_most || !rank_candidates(key, em)) {
+                    if constexpr (ROUGH) {   // the networks decide between equal keys by where all the others are
+                        if (passed_over != 0) {
+                            measure(passed_over, data);
+                            key = slot_distance(0);
+                        }
+                    }
                     // An unordered beam's keys are above all others and count as tied, so every candidate that enters one comes here
                     // (one that took none of its rows in has none to expand either, and no candidates follow).
                     if (rank_most == kUnordered) {
@@ -838,7 +947,7 @@ struct Beam {
         bool terminate = false;
         while (true) {
             asm volatile("" : "+v"(lane));   // a dozen addresses and masks made from the lane number are cheaper made anew in an iteration than held (and spilled) across it
-            absorb(iter == 0);
+            absorb(iter == 0, data);
             cnt.iterations++;
             const bool reset_now = count_down();
             if (reset_now) {
@@ -853,7 +962,7 @@ struct Beam {
                 wave_sync();
             }
             if (terminate && iter >= p.min_iterations) break;
-            expand(parent, graph, data, self_id, kInvalid);
+            expand(parent, graph, data, self_id, kInvalid, false);
             iter++;
         }
     }

@@ -257,6 +257,46 @@ __device__ __forceinline__ float partial_sqdist(const RowRegs<DIMV>& a, const Ro
     return acc;
 }
 
+// ---------------------------------------------------------------- long fp32 rows, a first look in fp16
+// Nine of ten rows that a search over long rows scores come in no nearer than the worst entry it holds, and of them only that
+// much has to be known.  A copy of the rows in fp16, scaled by one power of two for all of them, says it from half the bytes:
+// with s the distance to the rounded row, the distance as the exact pass would compute it lies in [rough_least, rough_most].
+// Rounding moves a row x by at most 2^-11 |x| + t (t: sqrt(dim) times half the smallest normal fp16 number, whatever becomes of
+// the numbers below it), |x| <= |q| + |q - x|, and the sums of either pass are off by (dim + 8) 2^-24 of themselves (`slack` is
+// four times that).  What the bounds leave open is measured exactly, so nothing but the traffic changes.
+struct RoughRows {
+    const _Float16* rows;   // num x dim
+    float unit;             // what a value of 1 stands for; NaN where some value is infinite or none: then nothing is decided
+    float tiny;             // t
+    float slack;
+};
+constexpr uint32_t kRoughHeader = 256;   // bytes before the rows: the largest |value| as bits
+// The largest value comes to lie in [2^14, 2^15).
+__device__ __forceinline__ float rough_unit(uint32_t max_bits) {
+    if (max_bits >= 0x7f800000u) return __builtin_nanf("");
+    const uint32_t e = max_bits >> 23;
+    return __uint_as_float((e < 15u ? 1u : e - 14u) << 23);
+}
+__device__ __forceinline__ RoughRows rough_rows(const unsigned char* held, uint32_t dim) {
+    RoughRows r;
+    r.rows = reinterpret_cast<const _Float16*>(held + kRoughHeader);
+    r.unit = rough_unit(*reinterpret_cast<const uint32_t*>(held));
+    r.tiny = sqrtf(static_cast<float>(dim)) * 6.2e-5f * r.unit;
+    r.slack = static_cast<float>(dim + 8) * 2.4e-7f;
+    return r;
+}
+constexpr float kRoughTurn = 4.93e-4f;   // 2^-11 and a little
+// sq: squared distance to the rounded row; norm: the reference's length, or more.  Not decided: minus infinity / infinity (also
+// where squares may have come out below the smallest normal number, whose rounding is no fraction of them).
+__device__ __forceinline__ float rough_least(const RoughRows& r, float sq, float norm) {
+    const float d = (sqrtf(sq) * (1.f - r.slack) - kRoughTurn * norm - r.tiny) * (1.f - kRoughTurn - r.slack);
+    return sq < 1e37f && sq > 1e-30f ? d : -__builtin_inff();
+}
+__device__ __forceinline__ float rough_most(const RoughRows& r, float sq, float norm) {
+    const float d = (sqrtf(sq) * (1.f + r.slack) + kRoughTurn * norm + r.tiny) * (1.f + 1.01f * kRoughTurn + r.slack);
+    return sq < 1e37f && sq > 1e-30f ? d : __builtin_inff();
+}
+
 // Sum over each group of LPR lanes; every lane of a group ends with the group's total.
 template <int DIMV>
 __device__ __forceinline__ float row_sum(float v) {

@@ -129,6 +129,40 @@ __global__ __launch_bounds__(256) void pack_bytes_kernel(const float* rows, uint
     if (ballot(!exact) != 0 && lane_id() == 0) *other = 1u;
 }
 
+// ------------------------------------------------------------------------------------------ long rows in fp16
+// The largest |value| as bits (what is no number orders last), then every value times the power of two that it fixes.
+__global__ __launch_bounds__(256) void rough_range_kernel(const float* rows, size_t quads, uint32_t* max_bits) {
+    uint32_t m = 0;
+    for (size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x; i < quads; i += static_cast<size_t>(gridDim.x) * 256) {
+        const uint4 q = reinterpret_cast<const uint4*>(rows)[i];
+        const uint32_t v[4] = {q.x & kClean, q.y & kClean, q.z & kClean, q.w & kClean};
+#pragma unroll
+        for (int e = 0; e < 4; e++) m = v[e] > m ? v[e] : m;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const uint32_t o = static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), off));
+        m = o > m ? o : m;
+    }
+    __shared__ uint32_t of_wave[4];
+    if (lane_id() == 0) of_wave[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int w = 1; w < 4; w++) m = of_wave[w] > m ? of_wave[w] : m;
+        if (m) atomicMax(max_bits, m);
+    }
+}
+__global__ __launch_bounds__(256) void rough_pack_kernel(const float* rows, size_t quads, const uint32_t* max_bits, _Float16* out) {
+    typedef _Float16 half4v __attribute__((ext_vector_type(4)));
+    const float scale = 1.f / rough_unit(*max_bits);   // a power of two: exact
+    for (size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x; i < quads; i += static_cast<size_t>(gridDim.x) * 256) {
+        const float4 x = reinterpret_cast<const float4*>(rows)[i];
+        reinterpret_cast<half4v*>(out)[i] = half4v{static_cast<_Float16>(x.x * scale), static_cast<_Float16>(x.y * scale), static_cast<_Float16>(x.z * scale),
+                                                   static_cast<_Float16>(x.w * scale)};
+    }
+}
+
 // ------------------------------------------------------------------------------------------ merged large build
 // A staged partition's sub-graph holds partition-local ids.  Its rows go to rows segment_start .. of the merged graph
 // with segment_start added to every id (what map_to_graph does through `map` on the small path,
@@ -178,9 +212,16 @@ int check_beam_sizes(uint32_t degree, uint32_t graph_degree, uint32_t beam, uint
 
 bool byte_rows_serve(const unsigned char* bytes, uint32_t degree, uint32_t dim) { return bytes && degree <= kMostByteDegree && dim <= kMostByteDims; }
 
+// the bounds of the prune want a factor that keeps their order
+bool rough_rows_serve(const unsigned char* rough, uint32_t degree, uint32_t beam, uint32_t dim, float relaxant) {
+    return rough && degree <= 64 && beam <= kMostRoughBeam && dim >= kLeastRoughDims && dim <= kMostRoughDims && relaxant > 0.f && relaxant < 1e18f;
+}
+
 int launch_build(BuildArgs& a, hipStream_t stream) {
-    if (reinterpret_cast<uintptr_t>(a.bytes) % 16) return GLIDE_ERR_BAD_ARGUMENT;
-    build_fn fn = byte_rows_serve(a.bytes, a.p.degree, a.p.dim) ? pick_build_bytes(a.p.beam, a.p.dim) : pick_build(a.p.degree, a.p.beam, a.p.dim);
+    if (reinterpret_cast<uintptr_t>(a.bytes) % 16 || reinterpret_cast<uintptr_t>(a.rough) % 16) return GLIDE_ERR_BAD_ARGUMENT;
+    build_fn fn = byte_rows_serve(a.bytes, a.p.degree, a.p.dim)                              ? pick_build_bytes(a.p.beam, a.p.dim)
+                  : rough_rows_serve(a.rough, a.p.degree, a.p.beam, a.p.dim, a.relaxant) ? pick_build_rough(a.p.beam)
+                                                                                             : pick_build(a.p.degree, a.p.beam, a.p.dim);
     const size_t lds_bytes = beam_lds_bytes(a.p.degree) + prune_lds_bytes(a.p.beam) + (size_t{1} << a.p.hash_bit) * sizeof(uint32_t);
     GLIDE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)));
     hipLaunchKernelGGL(fn, dim3(a.point_count), dim3(64), lds_bytes, stream, a);
@@ -198,16 +239,16 @@ int glide_hip_build_subgraph(const float* reorder_data, uint32_t num, uint32_t d
                              uint32_t segment_num, const uint32_t* start_points, uint32_t graph_degree, uint32_t beam,
                              uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit, uint32_t hash_reset_interval,
                              float relaxant, int metric, uint32_t* graph, unsigned long long* counters, void* stream) {
-    return glide_hip_build_subgraph_bytes(reorder_data, nullptr, num, dim, knn_graph, knn_degree, map, segment_starts, segment_lengths, segment_num,
-                                          start_points, graph_degree, beam, max_iterations, min_iterations, hash_bit, hash_reset_interval, relaxant,
-                                          metric, graph, counters, stream);
+    return glide_hip_build_subgraph_rows(reorder_data, nullptr, nullptr, num, dim, knn_graph, knn_degree, map, segment_starts, segment_lengths, segment_num,
+                                         start_points, graph_degree, beam, max_iterations, min_iterations, hash_bit, hash_reset_interval, relaxant,
+                                         metric, graph, counters, stream);
 }
 
-int glide_hip_build_subgraph_bytes(const float* reorder_data, const void* byte_rows, uint32_t num, uint32_t dim, const uint32_t* knn_graph,
-                                   uint32_t knn_degree, const uint32_t* map, const uint32_t* segment_starts, const uint32_t* segment_lengths,
-                                   uint32_t segment_num, const uint32_t* start_points, uint32_t graph_degree, uint32_t beam,
-                                   uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit, uint32_t hash_reset_interval,
-                                   float relaxant, int metric, uint32_t* graph, unsigned long long* counters, void* stream) {
+int glide_hip_build_subgraph_rows(const float* reorder_data, const void* byte_rows, const void* rough_rows, uint32_t num, uint32_t dim,
+                                  const uint32_t* knn_graph, uint32_t knn_degree, const uint32_t* map, const uint32_t* segment_starts, const uint32_t* segment_lengths,
+                                  uint32_t segment_num, const uint32_t* start_points, uint32_t graph_degree, uint32_t beam,
+                                  uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit, uint32_t hash_reset_interval,
+                                  float relaxant, int metric, uint32_t* graph, unsigned long long* counters, void* stream) {
     if (!reorder_data || !knn_graph || !map || !segment_starts || !segment_lengths || !start_points || !graph)
         return GLIDE_ERR_BAD_ARGUMENT;
     if (max_iterations == 0 || segment_num == 0) return GLIDE_ERR_BAD_ARGUMENT;
@@ -217,6 +258,7 @@ int glide_hip_build_subgraph_bytes(const float* reorder_data, const void* byte_r
     BuildArgs a;
     a.reorder_data = reorder_data;
     a.bytes = static_cast<const unsigned char*>(byte_rows);
+    a.rough = static_cast<const unsigned char*>(rough_rows);
     a.knn_graph = knn_graph;
     a.map = map;
     a.segment_starts = segment_starts;
@@ -239,15 +281,15 @@ int glide_hip_build_boundary(const float* reorder_data, uint32_t num, uint32_t r
                              uint32_t knn_degree, const uint32_t* map, uint32_t start_point, uint32_t graph_degree, uint32_t beam,
                              uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit, uint32_t hash_reset_interval,
                              float relaxant, int metric, uint32_t* graph, unsigned long long* counters, void* stream) {
-    return glide_hip_build_boundary_bytes(reorder_data, nullptr, num, reorder_num, dim, knn_graph, knn_degree, map, start_point, graph_degree, beam,
+    return glide_hip_build_boundary_rows(reorder_data, nullptr, nullptr, num, reorder_num, dim, knn_graph, knn_degree, map, start_point, graph_degree, beam,
                                           max_iterations, min_iterations, hash_bit, hash_reset_interval, relaxant, metric, graph, counters, stream);
 }
 
-int glide_hip_build_boundary_bytes(const float* reorder_data, const void* byte_rows, uint32_t num, uint32_t reorder_num, uint32_t dim,
-                                   const uint32_t* knn_graph, uint32_t knn_degree, const uint32_t* map, uint32_t start_point,
-                                   uint32_t graph_degree, uint32_t beam, uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit,
-                                   uint32_t hash_reset_interval, float relaxant, int metric, uint32_t* graph, unsigned long long* counters,
-                                   void* stream) {
+int glide_hip_build_boundary_rows(const float* reorder_data, const void* byte_rows, const void* rough_rows, uint32_t num, uint32_t reorder_num, uint32_t dim,
+                                  const uint32_t* knn_graph, uint32_t knn_degree, const uint32_t* map, uint32_t start_point,
+                                  uint32_t graph_degree, uint32_t beam, uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit,
+                                  uint32_t hash_reset_interval, float relaxant, int metric, uint32_t* graph, unsigned long long* counters,
+                                  void* stream) {
     if (!reorder_data || !knn_graph || !map || !graph) return GLIDE_ERR_BAD_ARGUMENT;
     if (max_iterations == 0 || reorder_num < num) return GLIDE_ERR_BAD_ARGUMENT;
     int rc = check_beam_sizes(knn_degree, graph_degree, beam, dim, hash_bit, metric);
@@ -257,6 +299,7 @@ int glide_hip_build_boundary_bytes(const float* reorder_data, const void* byte_r
     BuildArgs a;
     a.reorder_data = reorder_data;
     a.bytes = static_cast<const unsigned char*>(byte_rows);
+    a.rough = static_cast<const unsigned char*>(rough_rows);
     a.knn_graph = knn_graph;
     a.map = map;
     a.segment_starts = nullptr;
@@ -288,6 +331,7 @@ int glide_hip_build_segment(const float* segment_data, uint32_t num, uint32_t di
     BuildArgs a;
     a.reorder_data = segment_data;
     a.bytes = nullptr;
+    a.rough = nullptr;
     a.knn_graph = knn_graph;
     a.map = nullptr;
     a.segment_starts = nullptr;
@@ -320,6 +364,7 @@ int glide_hip_refine_segment(const float* segment_data, uint32_t num, uint32_t d
     a.order = nullptr;
     a.data = segment_data;
     a.bytes = nullptr;
+    a.rough = nullptr;
     a.graph_in = graph_in;
     a.graph_out = graph_out;
     a.centroids = nullptr;
@@ -405,6 +450,25 @@ int glide_hip_pack_byte_rows(const float* rows, uint32_t num, uint32_t dim, void
     return launch_status();
 }
 
+size_t glide_hip_rough_rows_bytes(uint32_t num, uint32_t dim) {
+    return dim >= kLeastRoughDims && dim <= kMostRoughDims && dim % 4 == 0 ? kRoughHeader + static_cast<size_t>(num) * dim * 2 : 0;
+}
+
+int glide_hip_pack_rough_rows(const float* rows, uint32_t num, uint32_t dim, void* rough_rows, void* stream) {
+    if (!rows || !rough_rows || dim == 0) return GLIDE_ERR_BAD_ARGUMENT;
+    if (glide_hip_rough_rows_bytes(1, dim) == 0) return GLIDE_ERR_UNSUPPORTED;
+    if (reinterpret_cast<uintptr_t>(rows) % 16 || reinterpret_cast<uintptr_t>(rough_rows) % 16) return GLIDE_ERR_BAD_ARGUMENT;
+    uint32_t* max_bits = static_cast<uint32_t*>(rough_rows);
+    const int rc = glide_hip_fill_u32(max_bits, 0u, kRoughHeader / 4, stream);
+    if (rc != GLIDE_OK || num == 0) return rc;
+    const size_t quads = static_cast<size_t>(num) * (dim / 4);
+    const uint32_t blocks = static_cast<uint32_t>(quads / 256 < 4096 ? quads / 256 + 1 : 4096);
+    hipLaunchKernelGGL(rough_range_kernel, dim3(blocks < 1024 ? blocks : 1024), dim3(256), 0, as_stream(stream), rows, quads, max_bits);
+    hipLaunchKernelGGL(rough_pack_kernel, dim3(blocks), dim3(256), 0, as_stream(stream), rows, quads, max_bits,
+                       reinterpret_cast<_Float16*>(static_cast<unsigned char*>(rough_rows) + kRoughHeader));
+    return launch_status();
+}
+
 int glide_hip_place_segment_graph(const uint32_t* segment_graph, uint32_t segment_length, uint32_t graph_degree, uint32_t segment_start,
                                   uint32_t* merged_graph, void* stream) {
     if (!segment_graph || !merged_graph || graph_degree == 0) return GLIDE_ERR_BAD_ARGUMENT;
@@ -429,7 +493,7 @@ int glide_hip_merge_boundary_graph(const uint32_t* boundary_graph, uint32_t boun
 }  // extern "C"
 
 namespace {
-int launch_refine(const float* data, const unsigned char* bytes, uint32_t num, uint32_t dim, const uint32_t* graph_in, uint32_t* graph_out, uint32_t graph_degree,
+int launch_refine(const float* data, const unsigned char* bytes, const unsigned char* rough, uint32_t num, uint32_t dim, const uint32_t* graph_in, uint32_t* graph_out, uint32_t graph_degree,
                   const float* centroids, uint32_t centroid_num, bool rank_all_centroids, const uint32_t* start_points, uint32_t beam,
                   uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit, uint32_t hash_reset_interval, float relaxant, int metric,
                   const uint32_t* order, unsigned long long* counters, void* stream) {
@@ -438,11 +502,12 @@ int launch_refine(const float* data, const unsigned char* bytes, uint32_t num, u
     int rc = check_beam_sizes(graph_degree, graph_degree, beam, dim, hash_bit, metric);
     if (rc != GLIDE_OK) return rc;
     if (centroid_num > 256) return GLIDE_ERR_UNSUPPORTED;
-    if (reinterpret_cast<uintptr_t>(bytes) % 16) return GLIDE_ERR_BAD_ARGUMENT;
+    if (reinterpret_cast<uintptr_t>(bytes) % 16 || reinterpret_cast<uintptr_t>(rough) % 16) return GLIDE_ERR_BAD_ARGUMENT;
     if (num == 0) return GLIDE_OK;
     RefineArgs a;
     a.data = data;
     a.bytes = bytes;
+    a.rough = rough;
     a.graph_in = graph_in;
     a.graph_out = graph_out;
     a.centroids = centroids;
@@ -456,7 +521,9 @@ int launch_refine(const float* data, const unsigned char* bytes, uint32_t num, u
     a.segment_start_point = 0;
     a.relaxant = relaxant;
     a.p = BeamParams{beam, graph_degree, dim, hash_bit, hash_reset_interval ? hash_reset_interval : 1, max_iterations, min_iterations, metric};
-    refine_fn fn = byte_rows_serve(bytes, graph_degree, dim) ? pick_refine_bytes(beam, dim) : pick_refine(graph_degree, beam, dim);
+    refine_fn fn = byte_rows_serve(bytes, graph_degree, dim)                           ? pick_refine_bytes(beam, dim)
+                   : rough_rows_serve(rough, graph_degree, beam, dim, relaxant) ? pick_refine_rough(beam)
+                                                                                 : pick_refine(graph_degree, beam, dim);
     const size_t lds_bytes = beam_lds_bytes(graph_degree) + prune_lds_bytes_refine(beam, graph_degree) + round_up32(centroid_num) * sizeof(float) +
                              (size_t{1} << hash_bit) * sizeof(uint32_t);
     GLIDE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)));
@@ -470,16 +537,16 @@ extern "C" int glide_hip_refine(const float* data, uint32_t num, uint32_t dim, c
                                 uint32_t beam, uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit,
                                 uint32_t hash_reset_interval, float relaxant, int metric, const uint32_t* order,
                                 unsigned long long* counters, void* stream) {
-    return launch_refine(data, nullptr, num, dim, graph_in, graph_out, graph_degree, centroids, centroid_num, false, start_points, beam, max_iterations,
+    return launch_refine(data, nullptr, nullptr, num, dim, graph_in, graph_out, graph_degree, centroids, centroid_num, false, start_points, beam, max_iterations,
                          min_iterations, hash_bit, hash_reset_interval, relaxant, metric, order, counters, stream);
 }
 
-extern "C" int glide_hip_refine_bytes(const float* data, const void* byte_rows, uint32_t num, uint32_t dim, const uint32_t* graph_in,
-                                      uint32_t* graph_out, uint32_t graph_degree, const float* centroids, uint32_t centroid_num,
+extern "C" int glide_hip_refine_rows(const float* data, const void* byte_rows, const void* rough_rows, uint32_t num, uint32_t dim,
+                                     const uint32_t* graph_in, uint32_t* graph_out, uint32_t graph_degree, const float* centroids, uint32_t centroid_num,
                                       const uint32_t* start_points, uint32_t beam, uint32_t max_iterations, uint32_t min_iterations,
                                       uint32_t hash_bit, uint32_t hash_reset_interval, float relaxant, int metric, const uint32_t* order,
                                       unsigned long long* counters, void* stream) {
-    return launch_refine(data, static_cast<const unsigned char*>(byte_rows), num, dim, graph_in, graph_out, graph_degree, centroids, centroid_num, false,
+    return launch_refine(data, static_cast<const unsigned char*>(byte_rows), static_cast<const unsigned char*>(rough_rows), num, dim, graph_in, graph_out, graph_degree, centroids, centroid_num, false,
                          start_points, beam, max_iterations, min_iterations, hash_bit, hash_reset_interval, relaxant, metric, order, counters, stream);
 }
 
@@ -488,6 +555,6 @@ extern "C" int glide_hip_refine_merged(const float* data, uint32_t num, uint32_t
                                        uint32_t beam, uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit,
                                        uint32_t hash_reset_interval, float relaxant, int metric, const uint32_t* order,
                                        unsigned long long* counters, void* stream) {
-    return launch_refine(data, nullptr, num, dim, graph_in, graph_out, graph_degree, centroids, centroid_num, true, start_points, beam, max_iterations,
+    return launch_refine(data, nullptr, nullptr, num, dim, graph_in, graph_out, graph_degree, centroids, centroid_num, true, start_points, beam, max_iterations,
                          min_iterations, hash_bit, hash_reset_interval, relaxant, metric, order, counters, stream);
 }

@@ -21,6 +21,7 @@ struct BuildArgs {
     float relaxant;
     BeamParams p;                         // p.degree = knn_degree
     const unsigned char* bytes;           // the same rows as bytes; the kernels for rows of bytes read nothing else
+    const unsigned char* rough;           // the same rows in fp16 (glide_hip_pack_rough_rows), for the kernels that look at them first
 };
 
 struct RefineArgs {
@@ -35,6 +36,7 @@ struct RefineArgs {
     float relaxant;
     BeamParams p;   // p.degree = graph_degree
     const unsigned char* bytes;   // the same rows as bytes, for the kernels for rows of bytes
+    const unsigned char* rough;   // the same rows in fp16, for the kernels that look at them first
 };
 
 using build_fn = void (*)(BuildArgs);
@@ -49,6 +51,10 @@ refine_fn pick_refine_256(uint32_t beam, uint32_t dim);
 // rows of bytes: up to 64 slots (kNN degree; graph degree) and kMostByteDims dims
 build_fn pick_build_bytes(uint32_t beam, uint32_t dim);
 refine_fn pick_refine_bytes(uint32_t beam, uint32_t dim);
+// rows of 513 to 1024 dims looked at in fp16 first: up to 64 slots, beams up to kMostRoughBeam
+constexpr uint32_t kLeastRoughDims = 513, kMostRoughDims = 1024, kMostRoughBeam = 128;
+build_fn pick_build_rough(uint32_t beam);
+refine_fn pick_refine_rough(uint32_t beam);
 inline build_fn pick_build(uint32_t degree, uint32_t beam, uint32_t dim) {
     return degree <= 64 ? pick_build_64(beam, dim) : degree <= 128 ? pick_build_128(beam, dim) : pick_build_256(beam, dim);
 }

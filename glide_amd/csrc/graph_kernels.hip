@@ -6,7 +6,7 @@ namespace glide {
 
 // Up to 64 slots on rows of up to 512 dims, here and in refine_kernel: six wavefronts per SIMD (80 registers; beams up to
 // 128 need no more anyway, beam 256 would take up to 84), five above beam 256 (96).
-template <int MAX_CAND, int MAX_BEAM, int DIMV>
+template <int MAX_CAND, int MAX_BEAM, int DIMV, bool ROUGH = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DIMV > 4 || MAX_CAND > 64 ? 1 : MAX_BEAM > 256 ? 5 : 6))) void build_kernel(BuildArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     auto* lds = reinterpret_cast<BeamLds<MAX_CAND>*>(smem);
@@ -37,15 +37,22 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DIMV > 4 || 
     const row_data<DIMV> sdata = row_at<DIMV>(rows, seg_start, a.p.dim);
     const uint32_t* sgraph = a.knn_graph + static_cast<size_t>(seg_start) * a.p.degree;
 
-    Beam<MAX_CAND, MAX_BEAM, DIMV> b;
+    Beam<MAX_CAND, MAX_BEAM, DIMV, false, false, ROUGH> b;
     b.init(lds, hash, a.p, row_at<DIMV>(rows, point, a.p.dim));
+    RoughPool look{};
+    if constexpr (ROUGH) {
+        look = RoughPool{rough_rows(a.rough, a.p.dim), lds->cand_id};
+        b.rough = look.rough;
+        b.rough.rows += static_cast<size_t>(seg_start) * a.p.dim;
+        b.q_length = row_length<DIMV>(b.q);
+    }
     // get_init (search_kernel.cuh:336-360): all neighbours of the entry are hashed; the one whose *local* id equals
     // this point's *reorder* id is left unscored (the reference compares across id spaces, graph_kernel.cuh:295-298)
     b.expand(entry, sgraph, sdata, kInvalid, point);
     b.run(sgraph, sdata, point - seg_start);
 
     uint32_t pool = beam_to_pool(b, pl);
-    prune_pool<MAX_BEAM, DIMV>(pl, pool, rows, a.p.dim, seg_start, a.graph_degree, a.relaxant, a.p.metric, b.lane,
+    prune_pool<MAX_BEAM, DIMV, ROUGH>(pl, look, pool, rows, a.p.dim, seg_start, a.graph_degree, a.relaxant, a.p.metric, b.lane,
                                b.cnt.rows_scored);
     wave_sync();
     if (segment_mode) {   // map_to_graph (graph_kernel.cuh:145-150)
@@ -79,7 +86,7 @@ __device__ __forceinline__ uint32_t pick_centroid_refine(uint32_t max_centroid, 
 
 // Rows are read from graph_in and written to graph_out (every row is written: copied, with its empty slots
 // filled).  The reference refines in place while other blocks still traverse the rows.
-template <int MAX_CAND, int MAX_BEAM, int DIMV>
+template <int MAX_CAND, int MAX_BEAM, int DIMV, bool ROUGH = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DIMV > 4 || MAX_CAND > 64 ? 1 : MAX_BEAM > 256 ? 5 : 6))) void refine_kernel(RefineArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     auto* lds = reinterpret_cast<BeamLds<MAX_CAND>*>(smem);
@@ -106,11 +113,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DIMV > 4 || 
     wave_sync();
     if (need == 0) return;
 
-    Beam<MAX_CAND, MAX_BEAM, DIMV> b;
+    Beam<MAX_CAND, MAX_BEAM, DIMV, false, false, ROUGH> b;
     row_data<DIMV> rows;
     if constexpr (RowShape<DIMV>::BYTES) rows = a.bytes;
     else rows = a.data;
     b.init(lds, hash, a.p, row_at<DIMV>(rows, point, a.p.dim));
+    RoughPool look{};
+    if constexpr (ROUGH) {
+        look = RoughPool{rough_rows(a.rough, a.p.dim), lds->cand_id};
+        b.rough = look.rough;
+        b.q_length = row_length<DIMV>(b.q);
+    }
     if (a.centroids != nullptr) {
         uint32_t c0;
         if constexpr (RowShape<DIMV>::BYTES) {
@@ -128,7 +141,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DIMV > 4 || 
     b.run(a.graph_in, rows, point);
 
     uint32_t pool = beam_to_pool(b, pl);
-    prune_pool_refine<MAX_BEAM, DIMV>(pl, pool, rows, a.p.dim, point, D, need, a.relaxant, a.p.metric, lane, b.cnt.rows_scored);
+    prune_pool_refine<MAX_BEAM, DIMV, ROUGH>(pl, look, pool, rows, a.p.dim, point, D, need, a.relaxant, a.p.metric, lane, b.cnt.rows_scored);
     wave_sync();
     uint32_t used = 0;
     for (uint32_t base = 0; base < round_up32(D); base += 64) {  // holes in slot order (graph_kernel.cuh:659-671)
@@ -190,6 +203,8 @@ refine_fn pick_refine_bytes_beam(uint32_t beam) {
     return refine_kernel<64, 512, DIMV>;
 }
 build_fn pick_build_bytes(uint32_t beam, uint32_t dim) { return dim <= 128 ? pick_build_bytes_beam<-1>(beam) : pick_build_bytes_beam<-2>(beam); }
+build_fn pick_build_rough(uint32_t beam) { return beam <= 64 ? build_kernel<64, 64, 8, true> : build_kernel<64, 128, 8, true>; }
+refine_fn pick_refine_rough(uint32_t beam) { return beam <= 64 ? refine_kernel<64, 64, 8, true> : refine_kernel<64, 128, 8, true>; }
 refine_fn pick_refine_bytes(uint32_t beam, uint32_t dim) { return dim <= 128 ? pick_refine_bytes_beam<-1>(beam) : pick_refine_bytes_beam<-2>(beam); }
 #endif
 

@@ -26,8 +26,8 @@ struct alignas(16) PruneLds {
 
 // Beam registers -> LDS pool in rank order with the explored bit stripped (graph_kernel.cuh:65-67), dropping
 // slots that never held a node (their id would be dereferenced by the reference).  Returns the pool size.
-template <int MAX_CAND, int MAX_BEAM, int DIMV, class PL>
-__device__ __forceinline__ uint32_t beam_to_pool(Beam<MAX_CAND, MAX_BEAM, DIMV>& b, PL* pl) {
+template <int MAX_CAND, int MAX_BEAM, int DIMV, bool ROUGH, class PL>
+__device__ __forceinline__ uint32_t beam_to_pool(Beam<MAX_CAND, MAX_BEAM, DIMV, false, false, ROUGH>& b, PL* pl) {
     constexpr int NB = MAX_BEAM / 64;
     // rank order is e = NB*lane + r; compact register by register would break the order, so stage then compact
 #pragma unroll
@@ -78,9 +78,53 @@ __device__ __forceinline__ uint32_t compact_pool(PL* pl, uint32_t first, uint32_
     return n;
 }
 
+// Where pool entries are looked at in fp16 first: the rows, and room for the entries that are left open (as many as a pool has).
+struct RoughPool {
+    RoughRows rough;
+    uint32_t* open;
+};
+
+// head_sq of the pool entries [first, pool_size): the squared distance to the latest head, or what makes compact_pool decide the
+// same -- 0 where even the largest distance the rough one allows is occluded, infinity where the smallest is not.
+// relaxant > 0.  id_of(idx) -> row id.
+template <bool ROUGH, int DIMV, class PL, class IdFn>
+__device__ __forceinline__ void score_against_head(PL* pl, const RowRegs<DIMV>& head, const RoughPool& look, row_data<DIMV> data, uint32_t dim, uint32_t first,
+                                                   uint32_t pool_size, float relaxant, int metric, int lane, IdFn id_of) {
+    auto out = [pl](uint32_t idx, float sq) { pl->head_sq[idx] = sq; };
+    if constexpr (!ROUGH) {
+        score_list<DIMV>(head, data, dim, first, pool_size, lane, id_of, out);
+    } else {
+        rough_list<DIMV>(head, look.rough, dim, first, pool_size, lane, id_of, out);
+        wave_sync();
+        const float length = row_length<DIMV>(head);
+        uint32_t n = 0;
+        for (uint32_t base = 0; base < pool_size; base += 64) {
+            const uint32_t i = base + lane;
+            const bool in = i >= first && i < pool_size;
+            const float sq = in ? pl->head_sq[i] : 0.f, d = in ? pl->pool_dist[i] : 0.f;
+            float least = rough_least(look.rough, sq, length), most = rough_most(look.rough, sq, length);
+            if (metric != kEuclidean) {
+                least = least > 0.f ? least * least * (1.f - look.rough.slack) : 0.f;
+                most = most * most * (1.f + look.rough.slack);
+            }
+            const bool occluded = relaxant * most < d, kept = !(relaxant * least < d);
+            if (in && (occluded || kept)) pl->head_sq[i] = occluded ? 0.f : __builtin_inff();
+            const uint64_t m = ballot(in && !occluded && !kept);
+            if ((m >> lane) & 1) look.open[n + prefix_count(m)] = i;
+            n += __popcll(m);
+        }
+        wave_sync();
+        const uint32_t* open = look.open;
+        if (n)
+            score_list<DIMV>(head, data, dim, 0, n, lane, [open, id_of](uint32_t k) { return id_of(open[k]); },
+                             [open, pl](uint32_t k, float sq) { pl->head_sq[open[k]] = sq; });
+    }
+    wave_sync();
+}
+
 // sync_prune: returns the neighbour count; pl->neighbor[0..round_up32(D)) holds ids (+segment_start) or invalid
-template <int MAX_BEAM, int DIMV, class PL>
-__device__ __forceinline__ uint32_t prune_pool(PL* pl, uint32_t pool_size, row_data<DIMV> data, uint32_t dim,
+template <int MAX_BEAM, int DIMV, bool ROUGH, class PL>
+__device__ __forceinline__ uint32_t prune_pool(PL* pl, const RoughPool& look, uint32_t pool_size, row_data<DIMV> data, uint32_t dim,
                                                uint32_t segment_start, uint32_t graph_degree, float relaxant, int metric,
                                                int lane, uint32_t& rows_scored) {
     for (uint32_t i = lane; i < PL::kCap; i += 64) pl->neighbor[i] = kInvalid;
@@ -93,18 +137,16 @@ __device__ __forceinline__ uint32_t prune_pool(PL* pl, uint32_t pool_size, row_d
         RowRegs<DIMV> hrow;
         load_reference<DIMV>(hrow, row_at<DIMV>(data, head, dim), dim, RowShape<DIMV>::lane_in_row(lane));
         rows_scored += pool_size - 1;
-        score_list<DIMV>(hrow, data, dim, 1, pool_size, lane,
-                         [pl, segment_start](uint32_t idx) { return pl->pool_id[idx] + segment_start; },
-                         [pl](uint32_t idx, float sq) { pl->head_sq[idx] = sq; });
-        wave_sync();
+        score_against_head<ROUGH, DIMV>(pl, hrow, look, data, dim, 1, pool_size, relaxant, metric, lane,
+                                        [pl, segment_start](uint32_t idx) { return pl->pool_id[idx] + segment_start; });
         pool_size = compact_pool<MAX_BEAM, DIMV>(pl, 1, pool_size, relaxant, metric, lane);
     }
     return nsize;
 }
 
 // sync_prune_refine: heads must be valid, differ from `self` and not already be in the row (pl->s_graph)
-template <int MAX_BEAM, int DIMV, class PL>
-__device__ __forceinline__ uint32_t prune_pool_refine(PL* pl, uint32_t pool_size, row_data<DIMV> data, uint32_t dim,
+template <int MAX_BEAM, int DIMV, bool ROUGH, class PL>
+__device__ __forceinline__ uint32_t prune_pool_refine(PL* pl, const RoughPool& look, uint32_t pool_size, row_data<DIMV> data, uint32_t dim,
                                                       uint32_t self, uint32_t graph_degree, uint32_t need, float relaxant,
                                                       int metric, int lane, uint32_t& rows_scored) {
     for (uint32_t i = lane; i < PL::kCap; i += 64) pl->neighbor[i] = kInvalid;
@@ -137,10 +179,8 @@ __device__ __forceinline__ uint32_t prune_pool_refine(PL* pl, uint32_t pool_size
         RowRegs<DIMV> hrow;
         load_reference<DIMV>(hrow, row_at<DIMV>(data, head, dim), dim, RowShape<DIMV>::lane_in_row(lane));
         rows_scored += pool_size - position;
-        score_list<DIMV>(hrow, data, dim, position, pool_size, lane,
-                         [pl](uint32_t idx) { return pl->pool_id[idx] & kClean; },
-                         [pl](uint32_t idx, float sq) { pl->head_sq[idx] = sq; });
-        wave_sync();
+        score_against_head<ROUGH, DIMV>(pl, hrow, look, data, dim, position, pool_size, relaxant, metric, lane,
+                                        [pl](uint32_t idx) { return pl->pool_id[idx] & kClean; });
         pool_size = compact_pool<MAX_BEAM, DIMV>(pl, position, pool_size, relaxant, metric, lane);
     }
     return nsize;

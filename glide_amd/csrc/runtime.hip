@@ -40,7 +40,10 @@ public:
             release();
             rc = hipMalloc(ptr, bytes);
         }
-        GLIDE_HIP_TRY(rc);
+        if (rc != hipSuccess) {
+            (void) hipGetLastError();   // reported here, not by the next launch
+            return static_cast<int>(rc);
+        }
         std::lock_guard<std::mutex> guard(mutex_);
         live_[*ptr] = Block{bytes, device};
         return GLIDE_OK;

@@ -19,6 +19,7 @@ from . import capi
 
 INVALID = 0xFFFFFFFF
 BYTE_ROWS_DEGREE = 64      # the searches over rows of bytes take graphs of up to this degree
+ROUGH_ROWS_DEGREE, ROUGH_ROWS_BEAM = 64, 128   # and the builds that look at long rows in fp16 first this degree and beam
 
 
 class Metric:
@@ -172,6 +173,11 @@ def cut_rows(d_rows, dim):
     return h
 
 
+def spare_array(nbytes):
+    """Memory for a copy that only makes things faster, or None: what is free must have room for two of it."""
+    return capi.DeviceArray(nbytes, np.uint8) if capi.mem_info()[0] // 2 >= nbytes else None
+
+
 def byte_rows(d_rows):
     """The rows of a DeviceArray once more as bytes, for the searches over rows of whole numbers 0..255, as a DeviceArray;
     None where a value is none of those or rows of that length are not held so."""
@@ -181,13 +187,26 @@ def byte_rows(d_rows):
         return None
     d_other = capi.DeviceArray(1, np.uint32)
     for rows in (min(num, 2048), num):      # the first ones alone: rows of fractions end there
-        d_bytes = capi.DeviceArray(capi.byte_rows_bytes(rows, dim), np.uint8)
+        d_bytes = spare_array(capi.byte_rows_bytes(rows, dim))
+        if d_bytes is None:
+            return None
         capi.pack_byte_rows(d_rows, rows, dim, d_bytes, d_other)
         if d_other.numpy()[0]:
             d_bytes.free()
             return None
         if rows == num:
             return d_bytes
+
+
+def rough_rows(d_rows):
+    """Long rows once more in fp16, for the builds that look at them before they measure (half the memory traffic, the same
+    results), as a DeviceArray; None where rows of that length are not looked at so."""
+    num, dim = d_rows.shape
+    nbytes = capi.rough_rows_bytes(num, dim)
+    d_rough = spare_array(nbytes) if nbytes else None
+    if d_rough is not None:
+        capi.pack_rough_rows(d_rows, num, dim, d_rough)
+    return d_rough
 
 
 def preprocess(param, d_data, result=None):
@@ -348,22 +367,23 @@ class GLIDE:
         p = search_param_knn
         with _Timer() as t:
             d_bytes = byte_rows(d_reorder_data) if knn_degree <= BYTE_ROWS_DEGREE else None
+            d_rough = rough_rows(d_reorder_data) if knn_degree <= ROUGH_ROWS_DEGREE and p.beam <= ROUGH_ROWS_BEAM else None
             capi.build_subgraph(d_reorder_data, num, dim, d_knn_graph, knn_degree, d_map, d_ss, d_sl, len(h_segment_start), d_rsp,
                                 deg, p.beam, p.max_iterations, p.min_iterations, p.hash_bit, p.hash_reset_interval,
-                                build_param.relaxant_factor, self.metric, self.d_graph, cnt, byte_rows=d_bytes)
+                                build_param.relaxant_factor, self.metric, self.d_graph, cnt, byte_rows=d_bytes, rough_rows=d_rough)
         times["subgraph"] = t.seconds
         with _Timer() as t:
             if reorder_num > num:
                 capi.build_boundary(d_reorder_data, num, reorder_num, dim, d_knn_graph, knn_degree, d_map,
                                     int(reorder_sp[self.centroid_num()]), deg, p.beam, p.max_iterations, p.min_iterations,
                                     p.hash_bit, p.hash_reset_interval, build_param.relaxant_factor, self.metric, self.d_graph, cnt,
-                                    byte_rows=d_bytes)
+                                    byte_rows=d_bytes, rough_rows=d_rough)
         times["boundary"] = t.seconds
         if counters and result is not None:
             capi.synchronize()
             result["build_counters"] = capi.read_counters(cnt)
         capi.synchronize()
-        for consumed in (d_knn_graph, d_reorder_data, d_bytes):     # d_map is kept until the refine stage, which uses it as its order
+        for consumed in (d_knn_graph, d_reorder_data, d_bytes, d_rough):     # d_map is kept until the refine stage, which uses it as its order
             if consumed is not None:
                 consumed.free()
         self.d_start_points = capi.DeviceArray.from_numpy(sp)
@@ -385,11 +405,14 @@ class GLIDE:
             cnt2 = capi.new_counters() if counters else None
             with _Timer() as t:
                 self._hold_byte_rows()
+                d_rough = rough_rows(self.d_data) if deg <= ROUGH_ROWS_DEGREE and p.beam <= ROUGH_ROWS_BEAM else None
                 capi.refine(self.d_data, num, dim, self.d_graph, d_rev, deg, self.d_centroids, self.centroid_num(),
                             self.d_start_points, p.beam, p.max_iterations, p.min_iterations, p.hash_bit, p.hash_reset_interval,
                             build_param.relaxant_factor, self.metric, cnt2, order=d_map,
-                            byte_rows=self._bytes[0] if self._bytes else None)
+                            byte_rows=self._bytes[0] if self._bytes else None, rough_rows=d_rough)
             times["refine"] = t.seconds
+            if d_rough is not None:
+                d_rough.free()
             self.d_graph, d_rev = d_rev, self.d_graph
             if counters and result is not None:
                 result["refine_counters"] = capi.read_counters(cnt2)

@@ -316,10 +316,17 @@ int glide_hip_refine(const float *data, uint32_t num, uint32_t dim, const uint32
  * values), 0 where rows of that length are not held so (more than 256 values).  glide_hip_pack_byte_rows writes them
  * (16-byte aligned) and sets *other_values (device) to 1 if some value is no whole number 0 .. 255, to 0 otherwise; the
  * byte rows are of use only in the second case.
- * The entry points that follow are those without `_bytes` with the same rows handed in a second time, as bytes: same
- * results to the bit, since the sums of squares of up to 256 such values are exact in fp32 and in integers alike.  With
+ * The entry points that follow are those without `_bytes` or `_rows` with the same rows handed in a second time: as bytes,
+ * same results to the bit, since the sums of squares of up to 256 such values are exact in fp32 and in integers alike.  With
  * byte_rows null, or a degree above 64, or rows of more than 256 values, they are those entry points; queries that are not
- * of bytes search the fp32 rows. */
+ * of bytes search the fp32 rows.
+ *
+ * Rows of 513 to 1024 values can be handed in as rough_rows, a copy in fp16 (glide_hip_rough_rows_bytes: its size, 0 for
+ * other lengths; 16-byte aligned): a point is measured exactly only where the distance to its rounded row, with bounds on
+ * what rounding can have done, leaves open whether it comes in.  Same results again; null, a degree above 64 or a beam
+ * above 128: not used. */
+size_t glide_hip_rough_rows_bytes(uint32_t num, uint32_t dim);
+int glide_hip_pack_rough_rows(const float *rows, uint32_t num, uint32_t dim, void *rough_rows, void *stream);
 size_t glide_hip_byte_rows_bytes(uint32_t num, uint32_t dim);
 int glide_hip_pack_byte_rows(const float *rows, uint32_t num, uint32_t dim, void *byte_rows, uint32_t *other_values,
                              void *stream);
@@ -329,21 +336,21 @@ int glide_hip_search_bytes(const float *data, const void *byte_rows, uint32_t nu
                            uint32_t beam, uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit,
                            uint32_t hash_reset_interval, int metric, uint32_t *result_ids, float *result_dists,
                            unsigned long long *counters, void *stream);
-int glide_hip_build_subgraph_bytes(const float *reorder_data, const void *byte_rows, uint32_t num, uint32_t dim,
-                                   const uint32_t *knn_graph, uint32_t knn_degree, const uint32_t *map,
+int glide_hip_build_subgraph_rows(const float *reorder_data, const void *byte_rows, const void *rough_rows,
+                                   uint32_t num, uint32_t dim, const uint32_t *knn_graph, uint32_t knn_degree, const uint32_t *map,
                                    const uint32_t *segment_starts, const uint32_t *segment_lengths, uint32_t segment_num,
                                    const uint32_t *start_points, uint32_t graph_degree, uint32_t beam,
                                    uint32_t max_iterations, uint32_t min_iterations, uint32_t hash_bit,
                                    uint32_t hash_reset_interval, float relaxant, int metric, uint32_t *graph,
                                    unsigned long long *counters, void *stream);
-int glide_hip_build_boundary_bytes(const float *reorder_data, const void *byte_rows, uint32_t num, uint32_t reorder_num,
-                                   uint32_t dim, const uint32_t *knn_graph, uint32_t knn_degree, const uint32_t *map,
+int glide_hip_build_boundary_rows(const float *reorder_data, const void *byte_rows, const void *rough_rows,
+                                   uint32_t num, uint32_t reorder_num, uint32_t dim, const uint32_t *knn_graph, uint32_t knn_degree, const uint32_t *map,
                                    uint32_t start_point, uint32_t graph_degree, uint32_t beam, uint32_t max_iterations,
                                    uint32_t min_iterations, uint32_t hash_bit, uint32_t hash_reset_interval,
                                    float relaxant, int metric, uint32_t *graph, unsigned long long *counters,
                                    void *stream);
-int glide_hip_refine_bytes(const float *data, const void *byte_rows, uint32_t num, uint32_t dim, const uint32_t *graph_in,
-                           uint32_t *graph_out, uint32_t graph_degree, const float *centroids, uint32_t centroid_num,
+int glide_hip_refine_rows(const float *data, const void *byte_rows, const void *rough_rows, uint32_t num, uint32_t dim,
+                           const uint32_t *graph_in, uint32_t *graph_out, uint32_t graph_degree, const float *centroids, uint32_t centroid_num,
                            const uint32_t *start_points, uint32_t beam, uint32_t max_iterations,
                            uint32_t min_iterations, uint32_t hash_bit, uint32_t hash_reset_interval, float relaxant,
                            int metric, const uint32_t *order, unsigned long long *counters, void *stream);

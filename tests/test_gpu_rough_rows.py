@@ -1,0 +1,107 @@
+"""Sub-graph builds and refinement that look at long rows in fp16 first, against the same calls without the fp16 copy: the copy
+only says which rows need not be measured, so graphs and counters must agree to the bit.  The rows include equal ones, near ties
+far below fp16's resolution, values at the ends of fp32's range, and values that are infinite or none."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+INV = 0xFFFFFFFF
+
+
+@pytest.fixture(scope="module")
+def hip():
+    from glide_amd import capi
+    capi.set_device(0)
+    return capi
+
+
+def rows_of(rng, n, dim, kind):
+    x = rng.standard_normal((6, dim))[rng.integers(0, 6, n)] * 0.5 + rng.standard_normal((n, dim)) * 0.3
+    if kind == "unit":
+        x /= np.linalg.norm(x, axis=1, keepdims=True)
+    elif kind == "whole":            # equal distances
+        x = np.rint(x * 2)
+    elif kind == "close":            # far from the origin: fp16 tells few of them apart
+        x = 40 + x * 0.01
+    elif kind == "spread":           # most values far below what fp16 holds next to the largest
+        x[:, 1:] *= 1e-4
+        x[:: 50, 0] = 3e4
+    elif kind == "tiny":
+        x *= 1e-21
+    elif kind == "huge":
+        x *= 3e17
+    x[n // 2: n // 2 + 8] = x[3]
+    x = x.astype(np.float32)
+    if kind == "infinite":
+        x[n // 3, 5] = np.inf
+    elif kind == "nan":
+        x[n // 3, dim - 1] = np.nan
+    return x
+
+
+def packed(hip, rows):
+    d = hip.DeviceArray.from_numpy(rows)
+    n, dim = rows.shape
+    d_rough = hip.DeviceArray(hip.rough_rows_bytes(n, dim), np.uint8)
+    hip.pack_rough_rows(d, n, dim, d_rough)
+    return d, d_rough
+
+
+@pytest.mark.parametrize("n,dim,kind", [(1, 516, "plain"), (300, 1024, "spread"), (77, 960, "tiny"), (77, 960, "huge"), (40, 600, "nan")])
+def test_packed_rows(hip, n, dim, kind):
+    rows = rows_of(np.random.default_rng(n), max(n, 16), dim, kind)[:n]
+    held = packed(hip, rows)[1].numpy()
+    most = held[:4].view(np.uint32)[0]
+    assert most == np.abs(rows).view(np.uint32).max()
+    if kind == "nan":
+        return
+    unit = np.float64(2.0) ** (max(int(most >> 23), 15) - 127 - 14)
+    rounded = held[256:].view(np.float16).reshape(n, dim).astype(np.float64) * unit
+    # half a unit in the eleventh place, or the smallest normal number where numbers below it are dropped
+    assert (np.abs(rounded - rows) <= np.maximum(np.abs(rows.astype(np.float64)) * 2.0 ** -11, 2.0 ** -14 * unit)).all()
+
+
+def test_lengths_that_are_not_held(hip):
+    assert hip.rough_rows_bytes(100, 512) == 0 and hip.rough_rows_bytes(100, 1028) == 0 and hip.rough_rows_bytes(100, 514) == 0
+    assert hip.rough_rows_bytes(100, 516) == 256 + 100 * 516 * 2
+    d = hip.DeviceArray((4, 512), np.float32)
+    with pytest.raises(hip.GlideHipError):
+        hip.pack_rough_rows(d, 4, 512, hip.DeviceArray(16384, np.uint8))
+
+
+@pytest.mark.parametrize("dim,knn_degree,degree,build_beam,refine_beam,metric,relaxant,kind", [
+    (516, 16, 8, 32, 64, 0, 1.05, "plain"), (960, 32, 32, 64, 128, 0, 1.05, "plain"), (960, 64, 32, 128, 96, 1, 1.05, "unit"), (1024, 32, 64, 96, 64, 1, 1.2, "unit"),
+    (768, 32, 32, 64, 128, 0, 1.0, "whole"), (640, 64, 24, 128, 128, 1, 0.9, "whole"), (960, 32, 32, 64, 64, 0, 1.05, "close"), (960, 32, 32, 128, 64, 1, 1.05, "close"),
+    (520, 32, 32, 64, 128, 0, 1.05, "spread"), (960, 32, 32, 64, 64, 0, 1.05, "tiny"), (960, 32, 32, 64, 64, 1, 1.05, "tiny"), (960, 32, 32, 64, 64, 0, 1.05, "huge"),
+    (960, 32, 32, 64, 64, 1, 1.05, "huge"), (800, 32, 32, 64, 64, 0, 1.05, "infinite"), (800, 32, 32, 64, 128, 1, 1.05, "nan"), (960, 32, 32, 64, 64, 0, 0.0, "plain")])
+def test_build_and_refine(hip, dim, knn_degree, degree, build_beam, refine_beam, metric, relaxant, kind):
+    from oracle import oracle as O
+    rng = np.random.default_rng(dim + degree + metric)
+    lengths, boundary = (400, 300), 120
+    n = sum(lengths)
+    rows = rows_of(rng, n, dim, kind)
+    reorder = np.concatenate([rows, rows[rng.permutation(n)[:boundary]]])
+    mp = np.concatenate([rng.permutation(n), rng.permutation(n)[:boundary]]).astype(np.uint32)
+    starts, lens = np.array([0, lengths[0], n], np.uint32), np.array([*lengths, boundary], np.uint32)
+    finite = np.nan_to_num(reorder, nan=0.0, posinf=0.0) * np.float32({"tiny": 1e21, "huge": 1e-17}.get(kind, 1))
+    knn = np.concatenate([O.bruteforce_knn(finite[s:s + m], finite[s:s + m], knn_degree, metric, exclude_self=True)[0] for s, m in zip(starts, lens)])
+    knn[:, knn_degree // 2:] = rng.integers(0, boundary, knn[:, knn_degree // 2:].shape)     # and rows that are far away
+    knn[rng.random(knn.shape) < 0.05] = INV
+    b, r = O.search_params(build_beam, knn_degree), O.search_params(refine_beam, max(knn_degree, degree))
+    d_re, d_re_rough = packed(hip, reorder)
+    d_rows, d_rows_rough = packed(hip, rows)
+    up = hip.DeviceArray.from_numpy
+    d_knn, d_map, d_s, d_l = up(knn), up(mp), up(starts), up(lens)
+    d_sp, d_c, d_gsp = up(np.array([5, 9, 2], np.uint32)), up(rows[[20, 600]] + np.float32(0.25)), up(np.array([3, 500], np.uint32))
+    got = []
+    for re_rough, row_rough in ((None, None), (d_re_rough, d_rows_rough)):
+        g, out, cnt = hip.DeviceArray.full((n, degree), INV), hip.DeviceArray.full((n, degree), 0xDEADBEEF), hip.new_counters()
+        args = (b["beam"], b["max_iterations"], b["min_iterations"], b["hash_bit"], b["hash_reset_interval"], relaxant, metric, g, cnt)
+        hip.build_subgraph(d_re, n, dim, d_knn, knn_degree, d_map, d_s, d_l, 3, d_sp, degree, *args, rough_rows=re_rough)
+        hip.build_boundary(d_re, n, n + boundary, dim, d_knn, knn_degree, d_map, 2, degree, *args, rough_rows=re_rough)
+        hip.refine(d_rows, n, dim, g, out, degree, d_c, 2, d_gsp, r["beam"], r["max_iterations"], r["min_iterations"], r["hash_bit"],
+                   r["hash_reset_interval"], relaxant, metric, cnt, order=d_map, rough_rows=row_rough)
+        hip.synchronize()
+        got.append((g.numpy(), out.numpy(), hip.read_counters(cnt)))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1]) and got[0][2] == got[1][2]
+    assert (got[0][1] != INV).any()
