@@ -154,52 +154,45 @@ __device__ __forceinline__ void score_list(const RowRegs<DIMV>& ref, row_data<DI
     score_share<DIMV, U>(RefInRegs<DIMV>{ref}, data, dim, first, count, lane, 0u, 1u, id_of, out);
 }
 
-// The same over the fp16 copy of long rows: out(idx, squared distance to the rounded row).  A lane owns the dims of a row that it
-// owns in score_step (eight bytes a load, so that the reference row serves as it is held), twice as many rows are under way.
-template <int DIMV, int U, class IdFn, class OutFn>
-__device__ __forceinline__ void rough_step(const RowRegs<DIMV>& ref, const RoughRows& rough, uint32_t dim, uint32_t base, uint32_t count, int g, int t,
+// The same over the fp16 copy of the rows: out(idx, squared distance of the rounded rows).
+template <int DIMV, int U, bool FULL, class IdFn, class OutFn>
+__device__ __forceinline__ void rough_step(const RoughRegs<DIMV>& ref, const RoughRows& rough, uint32_t dim, uint32_t base, uint32_t count, int g, int t,
                                            IdFn id_of, OutFn out) {
     using Shape = RowShape<DIMV>;
-    typedef _Float16 half4v __attribute__((ext_vector_type(4)));
-    half4v rows[U][Shape::NV];
+    RoughRegs<DIMV> rows[U];
 #pragma unroll
     for (int u = 0; u < U; u++) {
         const uint32_t idx = base + Shape::ROWS * u + g;
-        const _Float16* row = rough.rows + static_cast<size_t>(id_of(idx < count ? idx : count - 1)) * dim;
-#pragma unroll
-        for (int c = 0; c < Shape::NV; c++) {
-            const uint32_t d0 = (c * Shape::LPR + t) * 4;
-            rows[u][c] = d0 < dim ? *reinterpret_cast<const half4v*>(row + d0) : half4v{0, 0, 0, 0};
-        }
+        load_rough<DIMV, FULL>(rows[u], rough, id_of(idx < count ? idx : count - 1), dim, t);
     }
 #pragma unroll
     for (int u = 0; u < U; u++) {
         const uint32_t idx = base + Shape::ROWS * u + g;
-        float acc = 0.f;
-#pragma unroll
-        for (int c = 0; c < Shape::NV; c++) {
-            const float4 q = ref.v[c];
-            const float dx = fmaf(-rough.unit, static_cast<float>(rows[u][c][0]), q.x), dy = fmaf(-rough.unit, static_cast<float>(rows[u][c][1]), q.y),
-                        dz = fmaf(-rough.unit, static_cast<float>(rows[u][c][2]), q.z), dw = fmaf(-rough.unit, static_cast<float>(rows[u][c][3]), q.w);
-            acc = fmaf(dx, dx, acc);
-            acc = fmaf(dy, dy, acc);
-            acc = fmaf(dz, dz, acc);
-            acc = fmaf(dw, dw, acc);
-        }
-        const float sq = row_sum<DIMV>(acc);
+        const float sq = row_sum<DIMV>(rough_sqdist(ref, rows[u])) * rough.unit * rough.unit;
         if (t == 0 && idx < count) out(idx, sq);
     }
 }
-template <int DIMV, class IdFn, class OutFn>
-__device__ __forceinline__ void rough_list(const RowRegs<DIMV>& ref, const RoughRows& rough, uint32_t dim, uint32_t first, uint32_t count, int lane,
+template <int DIMV, bool FULL, class IdFn, class OutFn>
+__device__ __forceinline__ void rough_runs(const RoughRegs<DIMV>& ref, const RoughRows& rough, uint32_t dim, uint32_t first, uint32_t count, int lane,
                                            IdFn id_of, OutFn out) {
     using Shape = RowShape<DIMV>;
-    constexpr int U = 8;
+    constexpr int U = DIMV == 8 ? 8 : 4;   // twice the rows of the exact pass under way
     const int g = Shape::row_of_lane(lane), t = Shape::lane_in_row(lane);
     for (uint32_t base = first; base < count; base += Shape::ROWS * U) {
-        if (count - base <= Shape::ROWS * (U / 2)) rough_step<DIMV, U / 2>(ref, rough, dim, base, count, g, t, id_of, out);
-        else rough_step<DIMV, U>(ref, rough, dim, base, count, g, t, id_of, out);
+        if (count - base <= Shape::ROWS * (U / 2)) rough_step<DIMV, U / 2, FULL>(ref, rough, dim, base, count, g, t, id_of, out);
+        else rough_step<DIMV, U, FULL>(ref, rough, dim, base, count, g, t, id_of, out);
     }
+}
+template <int DIMV, class IdFn, class OutFn>
+__device__ __forceinline__ void rough_list(const RoughRegs<DIMV>& ref, const RoughRows& rough, uint32_t dim, uint32_t first, uint32_t count, int lane,
+                                           IdFn id_of, OutFn out) {
+    if constexpr (DIMV == 1 || DIMV == 2) {   // as in score_share
+        if (dim == RowShape<DIMV>::LPR * RowShape<DIMV>::NV * 4) {
+            rough_runs<DIMV, true>(ref, rough, dim, first, count, lane, id_of, out);
+            return;
+        }
+    }
+    rough_runs<DIMV, false>(ref, rough, dim, first, count, lane, id_of, out);
 }
 // the reference row's length, or a little more, for the bounds of the rough distances
 template <int DIMV>
@@ -213,9 +206,9 @@ __device__ __forceinline__ float row_length(const RowRegs<DIMV>& r) {
 // TEAM: the beam's wavefront is one of several in its workgroup (the others only score rows, see search_team_kernel).
 // WHOLE: the host promises beam == MAX_BEAM (asked for beams above 256 only, i.e. beam 512): the two-half merge of such a
 // beam needs no lane permutations and tracks no turning points (merge_beam_full).
-// ROUGH: rows are looked at in fp16 first (long rows, one candidate slot a lane).  The main loop over 120 000 rows of 960 values,
-// 46 of them scored an expansion, runs at 7.4 TB/s of row traffic; with nine tenths of that halved and the rest read after it,
-// the build of those rows (60 000, degree 64, beam 64) takes 224 ms instead of 355.
+// ROUGH: rows are looked at in fp16 first (one candidate slot a lane).  Sub-graph builds and refinement over rows that are not in
+// the caches run at the memory's rate: with nine tenths of the rows read in half the bytes, 120 000 rows of 512 values build in
+// 87 ms instead of 136, 250 000 of 128 in 59 instead of 75, 60 000 of 960 (degree 64) in 225 instead of 355.
 template <int MAX_CAND, int MAX_BEAM, int DIMV, bool TEAM = false, bool WHOLE = false, bool ROUGH = false>
 struct Beam {
     static_assert(!ROUGH || (MAX_CAND == 64 && MAX_BEAM <= 128), "the lists of entries to measure are sized for these");
@@ -243,6 +236,7 @@ struct Beam {
     uint32_t cid;           // candidate id of this lane's slot (MAX_CAND == 64; larger buckets keep the ids in LDS)
     uint32_t place[NC];     // where in vlist each of this lane's slots is; kInvalid: not scored
     RoughRows rough;        // ROUGH: the rows in fp16,
+    RoughRegs<ROUGH ? DIMV : 1> rough_q;
     float q_length;         // the reference row's length,
     uint64_t passed_over;   // and which entries of vlist a first look has found too far to enter (they count as infinitely far)
 
@@ -347,6 +341,15 @@ struct Beam {
         wave_sync();
     }
 
+    // `id`: the reference's row in `all`; the search's own ids start at `first`
+    __device__ __forceinline__ void look_first(const RoughRows& all, uint32_t id, uint32_t first) {
+        static_assert(ROUGH, "no fp16 rows");
+        load_rough<DIMV, false>(rough_q, all, id, p.dim, RowShape<DIMV>::lane_in_row(lane));
+        rough = all;
+        rough.rows += static_cast<size_t>(first) * all.stride;
+        q_length = row_length<DIMV>(q);
+    }
+
     // `entry`: the first expansion of a search, whose beam holds nothing yet
     __device__ __forceinline__ void expand(uint32_t parent, const uint32_t* graph, row_data<DIMV> data,
                                            uint32_t exclude_insert, uint32_t exclude_score, bool entry = true) {
@@ -356,7 +359,7 @@ struct Beam {
             passed_over = 0;
             const float tail = __uint_as_float(tail_key());
             if (!entry && nv != 0 && tail < FLT_MAX) {   // a beam that is not full takes every row
-                rough_list<DIMV>(q, rough, p.dim, 0, nv, lane,
+                rough_list<DIMV>(rough_q, rough, p.dim, 0, nv, lane,
                                  [l](uint32_t idx) { return l->vlist[idx]; },
                                  [l](uint32_t idx, float sq) { l->cand_dist[idx] = sq; });
                 wave_sync();

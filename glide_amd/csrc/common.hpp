@@ -257,43 +257,81 @@ __device__ __forceinline__ float partial_sqdist(const RowRegs<DIMV>& a, const Ro
     return acc;
 }
 
-// ---------------------------------------------------------------- long fp32 rows, a first look in fp16
-// Nine of ten rows that a search over long rows scores come in no nearer than the worst entry it holds, and of them only that
-// much has to be known.  A copy of the rows in fp16, scaled by one power of two for all of them, says it from half the bytes:
-// with s the distance to the rounded row, the distance as the exact pass would compute it lies in [rough_least, rough_most].
-// Rounding moves a row x by at most 2^-11 |x| + t (t: sqrt(dim) times half the smallest normal fp16 number, whatever becomes of
-// the numbers below it), |x| <= |q| + |q - x|, and the sums of either pass are off by (dim + 8) 2^-24 of themselves (`slack` is
-// four times that).  What the bounds leave open is measured exactly, so nothing but the traffic changes.
+// ---------------------------------------------------------------- fp32 rows, a first look in fp16
+// Nine of ten rows that a search scores come in no nearer than the worst entry it holds, and of them only that much has to be
+// known.  A copy of the rows in fp16, scaled by one power of two for all of them, says it from half the bytes and half the
+// instructions (a packed difference and a dot product for two values, in place of four): with s the distance of the rounded rows,
+// the distance as the exact pass would compute it lies in [rough_least, rough_most].  Rounding moves a row x by at most
+// r |x| + t (t: sqrt(dim) times the smallest normal fp16 number, whatever becomes of the numbers below it; r <= 2^-11, measured
+// over the rows when they are packed: some 0.4 of that), the reference q likewise, |x| <= |q| + |q - x|; the differences are off
+// by 2^-11 of themselves or t, and the sums of either pass by (dim + 8) 2^-24 of themselves (`slack` is four times that).  What the
+// bounds leave open is measured exactly, so nothing but the traffic changes.
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef _Float16 half8v __attribute__((ext_vector_type(8)));
 struct RoughRows {
-    const _Float16* rows;   // num x dim
+    const _Float16* rows;   // num x stride, zeros behind a row's dims
+    uint32_t stride;
     float unit;             // what a value of 1 stands for; NaN where some value is infinite or none: then nothing is decided
-    float tiny;             // t
+    float turn;             // r
+    float tiny;             // 3 t
     float slack;
 };
-constexpr uint32_t kRoughHeader = 256;   // bytes before the rows: the largest |value| as bits
-// The largest value comes to lie in [2^14, 2^15).
+template <int DIMV>
+struct RoughRegs {          // a lane's share of such a row: 8 (c LPR + t) .. + 7 for the c-th
+    static constexpr int NV = RowShape<DIMV>::NV / 2;
+    uint4 v[NV];
+};
+constexpr uint32_t kRoughHeader = 256;   // bytes before the rows: the largest |value| and r, as bits
+inline __host__ __device__ uint32_t rough_stride(uint32_t dim) { return (dim + 7) & ~7u; }
+// The largest value comes to lie in [2^13, 2^14): differences of two stay in range.
 __device__ __forceinline__ float rough_unit(uint32_t max_bits) {
     if (max_bits >= 0x7f800000u) return __builtin_nanf("");
     const uint32_t e = max_bits >> 23;
-    return __uint_as_float((e < 15u ? 1u : e - 14u) << 23);
+    return __uint_as_float((e < 14u ? 1u : e - 13u) << 23);
 }
 __device__ __forceinline__ RoughRows rough_rows(const unsigned char* held, uint32_t dim) {
     RoughRows r;
     r.rows = reinterpret_cast<const _Float16*>(held + kRoughHeader);
+    r.stride = rough_stride(dim);
     r.unit = rough_unit(*reinterpret_cast<const uint32_t*>(held));
-    r.tiny = sqrtf(static_cast<float>(dim)) * 6.2e-5f * r.unit;
+    r.turn = __uint_as_float(reinterpret_cast<const uint32_t*>(held)[1]);
+    r.tiny = sqrtf(static_cast<float>(dim)) * 3 * 6.2e-5f * r.unit;
     r.slack = static_cast<float>(dim + 8) * 2.4e-7f;
     return r;
 }
-constexpr float kRoughTurn = 4.93e-4f;   // 2^-11 and a little
-// sq: squared distance to the rounded row; norm: the reference's length, or more.  Not decided: minus infinity / infinity (also
+template <int DIMV, bool FULL>
+__device__ __forceinline__ void load_rough(RoughRegs<DIMV>& regs, const RoughRows& r, uint32_t id, uint32_t dim, int t) {
+    const _Float16* row = r.rows + static_cast<size_t>(id) * r.stride;
+#pragma unroll
+    for (int c = 0; c < RoughRegs<DIMV>::NV; c++) {
+        const uint32_t d0 = (c * RowShape<DIMV>::LPR + t) * 8;
+        regs.v[c] = FULL || d0 < dim ? *reinterpret_cast<const uint4*>(row + d0) : make_uint4(0u, 0u, 0u, 0u);
+    }
+}
+// a lane's part of the squared distance, in units
+template <int DIMV>
+__device__ __forceinline__ float rough_sqdist(const RoughRegs<DIMV>& a, const RoughRegs<DIMV>& b) {
+    float acc[4] = {};   // four chains: a product is not ready for the next instruction
+#pragma unroll
+    for (int c = 0; c < RoughRegs<DIMV>::NV; c++) {
+        const uint32_t of_a[4] = {a.v[c].x, a.v[c].y, a.v[c].z, a.v[c].w}, of_b[4] = {b.v[c].x, b.v[c].y, b.v[c].z, b.v[c].w};
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const half2v d = __builtin_bit_cast(half2v, of_a[e]) - __builtin_bit_cast(half2v, of_b[e]);
+            acc[e] = __builtin_amdgcn_fdot2(d, d, acc[e], false);
+        }
+    }
+    return (acc[0] + acc[1]) + (acc[2] + acc[3]);
+}
+constexpr float kRoughTurn = 4.93e-4f;   // 2^-11 and a little, the most that r is
+// sq: squared distance of the rounded rows; norm: the reference's length, or more.  Not decided: minus infinity / infinity (also
 // where squares may have come out below the smallest normal number, whose rounding is no fraction of them).
 __device__ __forceinline__ float rough_least(const RoughRows& r, float sq, float norm) {
-    const float d = (sqrtf(sq) * (1.f - r.slack) - kRoughTurn * norm - r.tiny) * (1.f - kRoughTurn - r.slack);
+    const float d = (sqrtf(sq) * (1.f - kRoughTurn - r.slack) - 2 * r.turn * norm - r.tiny) * (1.f - kRoughTurn - r.slack);
     return sq < 1e37f && sq > 1e-30f ? d : -__builtin_inff();
 }
 __device__ __forceinline__ float rough_most(const RoughRows& r, float sq, float norm) {
-    const float d = (sqrtf(sq) * (1.f + r.slack) + kRoughTurn * norm + r.tiny) * (1.f + 1.01f * kRoughTurn + r.slack);
+    const float d = (sqrtf(sq) * (1.f + 1.01f * kRoughTurn + r.slack) + 2 * r.turn * norm + r.tiny) * (1.f + 1.01f * kRoughTurn + r.slack);
     return sq < 1e37f && sq > 1e-30f ? d : __builtin_inff();
 }
 

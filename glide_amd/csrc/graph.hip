@@ -129,7 +129,7 @@ __global__ __launch_bounds__(256) void pack_bytes_kernel(const float* rows, uint
     if (ballot(!exact) != 0 && lane_id() == 0) *other = 1u;
 }
 
-// ------------------------------------------------------------------------------------------ long rows in fp16
+// ------------------------------------------------------------------------------------------ rows in fp16
 // The largest |value| as bits (what is no number orders last), then every value times the power of two that it fixes.
 __global__ __launch_bounds__(256) void rough_range_kernel(const float* rows, size_t quads, uint32_t* max_bits) {
     uint32_t m = 0;
@@ -153,14 +153,45 @@ __global__ __launch_bounds__(256) void rough_range_kernel(const float* rows, siz
         if (m) atomicMax(max_bits, m);
     }
 }
-__global__ __launch_bounds__(256) void rough_pack_kernel(const float* rows, size_t quads, const uint32_t* max_bits, _Float16* out) {
-    typedef _Float16 half4v __attribute__((ext_vector_type(4)));
-    const float scale = 1.f / rough_unit(*max_bits);   // a power of two: exact
-    for (size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x; i < quads; i += static_cast<size_t>(gridDim.x) * 256) {
-        const float4 x = reinterpret_cast<const float4*>(rows)[i];
-        reinterpret_cast<half4v*>(out)[i] = half4v{static_cast<_Float16>(x.x * scale), static_cast<_Float16>(x.y * scale), static_cast<_Float16>(x.z * scale),
-                                                   static_cast<_Float16>(x.w * scale)};
+// Sixteen lanes a row.
+__global__ __launch_bounds__(256) void rough_pack_kernel(const float* rows, uint32_t num, uint32_t dim, const uint32_t* max_bits, uint32_t* turn_bits,
+                                                         _Float16* out) {
+    const float unit = rough_unit(*max_bits), scale = 1.f / unit;   // powers of two: exact
+    const float t = sqrtf(static_cast<float>(dim)) * 6.2e-5f * unit;
+    const uint32_t stride = rough_stride(dim), lane = threadIdx.x % 16;
+    float most = 0.f;
+    for (size_t row = static_cast<size_t>(blockIdx.x) * 16 + threadIdx.x / 16; row < num; row += static_cast<size_t>(gridDim.x) * 16) {
+        float off = 0.f, length = 0.f;
+        for (uint32_t d0 = lane * 8; d0 < stride; d0 += 128) {
+            const float* from = rows + row * dim + d0;
+            const float4 x = *reinterpret_cast<const float4*>(from);
+            const float4 y = d0 + 4 < dim ? *reinterpret_cast<const float4*>(from + 4) : make_float4(0.f, 0.f, 0.f, 0.f);
+            const float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+            half8v h;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                h[e] = static_cast<_Float16>(v[e] * scale);
+                const float d = fmaf(-unit, static_cast<float>(h[e]), v[e]);
+                off = fmaf(d, d, off);
+                length = fmaf(v[e], v[e], length);
+            }
+            *reinterpret_cast<half8v*>(out + row * stride + d0) = h;
+        }
+#pragma unroll
+        for (int w = 8; w > 0; w >>= 1) {
+            off += __shfl_xor(off, w);
+            length += __shfl_xor(length, w);
+        }
+        float r = kRoughTurn;   // lengths whose squares leave the range say nothing
+        if (length > 1e-24f && length < 1e37f) r = fminf(fmaxf(sqrtf(off) * 1.001f - t, 0.f) / sqrtf(length) * 1.001f, kRoughTurn);
+        most = fmaxf(most, r);
     }
+#pragma unroll
+    for (int w = 32; w > 0; w >>= 1) most = fmaxf(most, __shfl_xor(most, w));
+    __shared__ float of_wave[4];
+    if (lane_id() == 0) of_wave[threadIdx.x >> 6] = most;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicMax(turn_bits, __float_as_uint(fmaxf(fmaxf(of_wave[0], of_wave[1]), fmaxf(of_wave[2], of_wave[3]))));
 }
 
 // ------------------------------------------------------------------------------------------ merged large build
@@ -214,13 +245,13 @@ bool byte_rows_serve(const unsigned char* bytes, uint32_t degree, uint32_t dim) 
 
 // the bounds of the prune want a factor that keeps their order
 bool rough_rows_serve(const unsigned char* rough, uint32_t degree, uint32_t beam, uint32_t dim, float relaxant) {
-    return rough && degree <= 64 && beam <= kMostRoughBeam && dim >= kLeastRoughDims && dim <= kMostRoughDims && relaxant > 0.f && relaxant < 1e18f;
+    return rough && degree <= 64 && beam <= kMostRoughBeam && dim <= kMostRoughDims && relaxant > 0.f && relaxant < 1e18f;
 }
 
 int launch_build(BuildArgs& a, hipStream_t stream) {
     if (reinterpret_cast<uintptr_t>(a.bytes) % 16 || reinterpret_cast<uintptr_t>(a.rough) % 16) return GLIDE_ERR_BAD_ARGUMENT;
     build_fn fn = byte_rows_serve(a.bytes, a.p.degree, a.p.dim)                              ? pick_build_bytes(a.p.beam, a.p.dim)
-                  : rough_rows_serve(a.rough, a.p.degree, a.p.beam, a.p.dim, a.relaxant) ? pick_build_rough(a.p.beam)
+                  : rough_rows_serve(a.rough, a.p.degree, a.p.beam, a.p.dim, a.relaxant) ? pick_build_rough(a.p.beam, a.p.dim)
                                                                                              : pick_build(a.p.degree, a.p.beam, a.p.dim);
     const size_t lds_bytes = beam_lds_bytes(a.p.degree) + prune_lds_bytes(a.p.beam) + (size_t{1} << a.p.hash_bit) * sizeof(uint32_t);
     GLIDE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)));
@@ -451,7 +482,7 @@ int glide_hip_pack_byte_rows(const float* rows, uint32_t num, uint32_t dim, void
 }
 
 size_t glide_hip_rough_rows_bytes(uint32_t num, uint32_t dim) {
-    return dim >= kLeastRoughDims && dim <= kMostRoughDims && dim % 4 == 0 ? kRoughHeader + static_cast<size_t>(num) * dim * 2 : 0;
+    return dim > 0 && dim <= kMostRoughDims && dim % 4 == 0 ? kRoughHeader + static_cast<size_t>(num) * rough_stride(dim) * 2 : 0;
 }
 
 int glide_hip_pack_rough_rows(const float* rows, uint32_t num, uint32_t dim, void* rough_rows, void* stream) {
@@ -462,9 +493,9 @@ int glide_hip_pack_rough_rows(const float* rows, uint32_t num, uint32_t dim, voi
     const int rc = glide_hip_fill_u32(max_bits, 0u, kRoughHeader / 4, stream);
     if (rc != GLIDE_OK || num == 0) return rc;
     const size_t quads = static_cast<size_t>(num) * (dim / 4);
-    const uint32_t blocks = static_cast<uint32_t>(quads / 256 < 4096 ? quads / 256 + 1 : 4096);
-    hipLaunchKernelGGL(rough_range_kernel, dim3(blocks < 1024 ? blocks : 1024), dim3(256), 0, as_stream(stream), rows, quads, max_bits);
-    hipLaunchKernelGGL(rough_pack_kernel, dim3(blocks), dim3(256), 0, as_stream(stream), rows, quads, max_bits,
+    const uint32_t blocks = static_cast<uint32_t>(quads / 256 < 1024 ? quads / 256 + 1 : 1024), row_blocks = num < 16 * 2048 ? ceil_div(num, 16u) : 2048u;
+    hipLaunchKernelGGL(rough_range_kernel, dim3(blocks), dim3(256), 0, as_stream(stream), rows, quads, max_bits);
+    hipLaunchKernelGGL(rough_pack_kernel, dim3(row_blocks), dim3(256), 0, as_stream(stream), rows, num, dim, max_bits, max_bits + 1,
                        reinterpret_cast<_Float16*>(static_cast<unsigned char*>(rough_rows) + kRoughHeader));
     return launch_status();
 }
@@ -522,7 +553,7 @@ int launch_refine(const float* data, const unsigned char* bytes, const unsigned 
     a.relaxant = relaxant;
     a.p = BeamParams{beam, graph_degree, dim, hash_bit, hash_reset_interval ? hash_reset_interval : 1, max_iterations, min_iterations, metric};
     refine_fn fn = byte_rows_serve(bytes, graph_degree, dim)                           ? pick_refine_bytes(beam, dim)
-                   : rough_rows_serve(rough, graph_degree, beam, dim, relaxant) ? pick_refine_rough(beam)
+                   : rough_rows_serve(rough, graph_degree, beam, dim, relaxant) ? pick_refine_rough(beam, dim)
                                                                                  : pick_refine(graph_degree, beam, dim);
     const size_t lds_bytes = beam_lds_bytes(graph_degree) + prune_lds_bytes_refine(beam, graph_degree) + round_up32(centroid_num) * sizeof(float) +
                              (size_t{1} << hash_bit) * sizeof(uint32_t);

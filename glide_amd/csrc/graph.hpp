@@ -51,10 +51,10 @@ refine_fn pick_refine_256(uint32_t beam, uint32_t dim);
 // rows of bytes: up to 64 slots (kNN degree; graph degree) and kMostByteDims dims
 build_fn pick_build_bytes(uint32_t beam, uint32_t dim);
 refine_fn pick_refine_bytes(uint32_t beam, uint32_t dim);
-// rows of 513 to 1024 dims looked at in fp16 first: up to 64 slots, beams up to kMostRoughBeam
-constexpr uint32_t kLeastRoughDims = 513, kMostRoughDims = 1024, kMostRoughBeam = 128;
-build_fn pick_build_rough(uint32_t beam);
-refine_fn pick_refine_rough(uint32_t beam);
+// rows looked at in fp16 first: up to 64 slots, beams up to kMostRoughBeam
+constexpr uint32_t kMostRoughDims = 1024, kMostRoughBeam = 128;
+build_fn pick_build_rough(uint32_t beam, uint32_t dim);
+refine_fn pick_refine_rough(uint32_t beam, uint32_t dim);
 inline build_fn pick_build(uint32_t degree, uint32_t beam, uint32_t dim) {
     return degree <= 64 ? pick_build_64(beam, dim) : degree <= 128 ? pick_build_128(beam, dim) : pick_build_256(beam, dim);
 }

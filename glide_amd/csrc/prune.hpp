@@ -88,13 +88,15 @@ struct RoughPool {
 // same -- 0 where even the largest distance the rough one allows is occluded, infinity where the smallest is not.
 // relaxant > 0.  id_of(idx) -> row id.
 template <bool ROUGH, int DIMV, class PL, class IdFn>
-__device__ __forceinline__ void score_against_head(PL* pl, const RowRegs<DIMV>& head, const RoughPool& look, row_data<DIMV> data, uint32_t dim, uint32_t first,
+__device__ __forceinline__ void score_against_head(PL* pl, const RowRegs<DIMV>& head, const RoughPool& look, uint32_t head_id, row_data<DIMV> data, uint32_t dim, uint32_t first,
                                                    uint32_t pool_size, float relaxant, int metric, int lane, IdFn id_of) {
     auto out = [pl](uint32_t idx, float sq) { pl->head_sq[idx] = sq; };
     if constexpr (!ROUGH) {
         score_list<DIMV>(head, data, dim, first, pool_size, lane, id_of, out);
     } else {
-        rough_list<DIMV>(head, look.rough, dim, first, pool_size, lane, id_of, out);
+        RoughRegs<DIMV> rough_head;
+        load_rough<DIMV, false>(rough_head, look.rough, head_id, dim, RowShape<DIMV>::lane_in_row(lane));
+        rough_list<DIMV>(rough_head, look.rough, dim, first, pool_size, lane, id_of, out);
         wave_sync();
         const float length = row_length<DIMV>(head);
         uint32_t n = 0;
@@ -137,7 +139,7 @@ __device__ __forceinline__ uint32_t prune_pool(PL* pl, const RoughPool& look, ui
         RowRegs<DIMV> hrow;
         load_reference<DIMV>(hrow, row_at<DIMV>(data, head, dim), dim, RowShape<DIMV>::lane_in_row(lane));
         rows_scored += pool_size - 1;
-        score_against_head<ROUGH, DIMV>(pl, hrow, look, data, dim, 1, pool_size, relaxant, metric, lane,
+        score_against_head<ROUGH, DIMV>(pl, hrow, look, head, data, dim, 1, pool_size, relaxant, metric, lane,
                                         [pl, segment_start](uint32_t idx) { return pl->pool_id[idx] + segment_start; });
         pool_size = compact_pool<MAX_BEAM, DIMV>(pl, 1, pool_size, relaxant, metric, lane);
     }
@@ -179,7 +181,7 @@ __device__ __forceinline__ uint32_t prune_pool_refine(PL* pl, const RoughPool& l
         RowRegs<DIMV> hrow;
         load_reference<DIMV>(hrow, row_at<DIMV>(data, head, dim), dim, RowShape<DIMV>::lane_in_row(lane));
         rows_scored += pool_size - position;
-        score_against_head<ROUGH, DIMV>(pl, hrow, look, data, dim, position, pool_size, relaxant, metric, lane,
+        score_against_head<ROUGH, DIMV>(pl, hrow, look, head, data, dim, position, pool_size, relaxant, metric, lane,
                                         [pl](uint32_t idx) { return pl->pool_id[idx] & kClean; });
         pool_size = compact_pool<MAX_BEAM, DIMV>(pl, position, pool_size, relaxant, metric, lane);
     }

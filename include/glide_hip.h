@@ -321,7 +321,7 @@ int glide_hip_refine(const float *data, uint32_t num, uint32_t dim, const uint32
  * byte_rows null, or a degree above 64, or rows of more than 256 values, they are those entry points; queries that are not
  * of bytes search the fp32 rows.
  *
- * Rows of 513 to 1024 values can be handed in as rough_rows, a copy in fp16 (glide_hip_rough_rows_bytes: its size, 0 for
+ * Rows of up to 1024 values can be handed in as rough_rows, a copy in fp16 (glide_hip_rough_rows_bytes: its size, 0 for
  * other lengths; 16-byte aligned): a point is measured exactly only where the distance to its rounded row, with bounds on
  * what rounding can have done, leaves open whether it comes in.  Same results again; null, a degree above 64 or a beam
  * above 128: not used. */

@@ -47,7 +47,7 @@ def packed(hip, rows):
     return d, d_rough
 
 
-@pytest.mark.parametrize("n,dim,kind", [(1, 516, "plain"), (300, 1024, "spread"), (77, 960, "tiny"), (77, 960, "huge"), (40, 600, "nan")])
+@pytest.mark.parametrize("n,dim,kind", [(1, 516, "plain"), (90, 4, "unit"), (65, 100, "close"), (300, 1024, "spread"), (77, 960, "tiny"), (77, 960, "huge"), (40, 600, "nan")])
 def test_packed_rows(hip, n, dim, kind):
     rows = rows_of(np.random.default_rng(n), max(n, 16), dim, kind)[:n]
     held = packed(hip, rows)[1].numpy()
@@ -55,21 +55,26 @@ def test_packed_rows(hip, n, dim, kind):
     assert most == np.abs(rows).view(np.uint32).max()
     if kind == "nan":
         return
-    unit = np.float64(2.0) ** (max(int(most >> 23), 15) - 127 - 14)
-    rounded = held[256:].view(np.float16).reshape(n, dim).astype(np.float64) * unit
+    unit = np.float64(2.0) ** (max(int(most >> 23), 14) - 127 - 13)
+    rounded = held[256:].view(np.float16).reshape(n, (dim + 7) // 8 * 8).astype(np.float64) * unit
+    assert not rounded[:, dim:].any()
+    rounded = rounded[:, :dim]
     # half a unit in the eleventh place, or the smallest normal number where numbers below it are dropped
     assert (np.abs(rounded - rows) <= np.maximum(np.abs(rows.astype(np.float64)) * 2.0 ** -11, 2.0 ** -14 * unit)).all()
 
 
 def test_lengths_that_are_not_held(hip):
-    assert hip.rough_rows_bytes(100, 512) == 0 and hip.rough_rows_bytes(100, 1028) == 0 and hip.rough_rows_bytes(100, 514) == 0
-    assert hip.rough_rows_bytes(100, 516) == 256 + 100 * 516 * 2
-    d = hip.DeviceArray((4, 512), np.float32)
+    assert hip.rough_rows_bytes(100, 1028) == 0 and hip.rough_rows_bytes(100, 514) == 0 and hip.rough_rows_bytes(100, 0) == 0
+    assert hip.rough_rows_bytes(100, 516) == 256 + 100 * 520 * 2
+    d = hip.DeviceArray((4, 1028), np.float32)
     with pytest.raises(hip.GlideHipError):
-        hip.pack_rough_rows(d, 4, 512, hip.DeviceArray(16384, np.uint8))
+        hip.pack_rough_rows(d, 4, 1028, hip.DeviceArray(16384, np.uint8))
 
 
 @pytest.mark.parametrize("dim,knn_degree,degree,build_beam,refine_beam,metric,relaxant,kind", [
+    (4, 16, 8, 32, 64, 0, 1.05, "plain"), (28, 32, 32, 64, 128, 0, 1.05, "unit"), (96, 32, 32, 128, 64, 1, 1.05, "unit"), (128, 64, 48, 64, 128, 0, 1.05, "plain"),
+    (128, 32, 32, 64, 64, 1, 1.05, "whole"), (132, 32, 32, 64, 64, 0, 1.05, "spread"), (200, 32, 24, 128, 128, 1, 1.05, "unit"), (256, 32, 32, 64, 64, 0, 1.05, "close"),
+    (260, 32, 64, 64, 128, 0, 1.05, "huge"), (384, 48, 48, 128, 64, 1, 1.05, "tiny"), (512, 32, 32, 64, 64, 0, 1.05, "nan"), (512, 64, 32, 64, 128, 0, 1.1, "plain"),
     (516, 16, 8, 32, 64, 0, 1.05, "plain"), (960, 32, 32, 64, 128, 0, 1.05, "plain"), (960, 64, 32, 128, 96, 1, 1.05, "unit"), (1024, 32, 64, 96, 64, 1, 1.2, "unit"),
     (768, 32, 32, 64, 128, 0, 1.0, "whole"), (640, 64, 24, 128, 128, 1, 0.9, "whole"), (960, 32, 32, 64, 64, 0, 1.05, "close"), (960, 32, 32, 128, 64, 1, 1.05, "close"),
     (520, 32, 32, 64, 128, 0, 1.05, "spread"), (960, 32, 32, 64, 64, 0, 1.05, "tiny"), (960, 32, 32, 64, 64, 1, 1.05, "tiny"), (960, 32, 32, 64, 64, 0, 1.05, "huge"),
@@ -105,3 +110,27 @@ def test_build_and_refine(hip, dim, knn_degree, degree, build_beam, refine_beam,
         got.append((g.numpy(), out.numpy(), hip.read_counters(cnt)))
     assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1]) and got[0][2] == got[1][2]
     assert (got[0][1] != INV).any()
+
+
+@pytest.mark.parametrize("dim,degree,knn_degree,metric", [(96, 32, 32, 1), (160, 48, 64, 0), (128, 24, 72, 0), (960, 64, 64, 0), (1028, 32, 32, 0)])
+def test_whole_build(hip, monkeypatch, dim, degree, knn_degree, metric):
+    """The same index with and without the copy, also where only one of its stages takes it or none does."""
+    from glide_amd import index as G
+    rows = rows_of(np.random.default_rng(dim), 3000, dim, "unit" if metric == 1 else "plain")
+    graphs = []
+    for pays in (False, True):
+        monkeypatch.setattr(G, "rough_rows_pay", lambda num, dim, pays=pays: pays)
+        d = hip.DeviceArray.from_numpy(rows)
+        d_reorder, d_map, starts, lengths, d_c = G.preprocess(G.PartitionParameter(centroid_num=3, boundary_factor=1.04, sample_factor=0.5, metric=metric), d)
+        d_knn = G.build_nnd(G.NNDescentParameter(graph_degree=knn_degree, max_iterations=6), d_reorder, starts, lengths)
+        index = G.GLIDE(degree, d, d_c, metric)
+        index.build(G.IndexParameter(graph_degree=degree, knn_degree=knn_degree, relaxant_factor=1.05, metric=metric),
+                    G.make_search_parameter(64, knn_degree), G.make_search_parameter(128, max(knn_degree, degree)), d_knn, starts, lengths, d_map, d_reorder)
+        graphs.append(index.d_graph.numpy())
+    assert np.array_equal(*graphs) and (graphs[0] != INV).mean() > 0.5
+
+
+def test_where_it_pays():
+    from glide_amd.index import rough_rows_pay as pays
+    assert pays(60_000, 960) and pays(250_000, 128) and pays(1_000_000, 96)
+    assert not pays(2_000, 512) and not pays(70_000, 128) and not pays(234_567, 96) and not pays(10_000_000, 64)
