@@ -163,9 +163,9 @@ struct RowShape {
 // traffic, and |x - q|^2 = x.x - 2 x.q + q.q takes eight dot products of four bytes for sixteen dims in place of 32 fp32
 // instructions.  All of it is integer arithmetic and exact; with at most kMostByteDims dims every sum the fp32 form makes
 // stays below 2^24 and is exact as well, so both give the same distances to the bit.  Measured on 128 dims, fp32 : bytes:
-// 10 000 searches of a million rows at beam 64 1 347 : 500 us (rows from memory; 1 query 124 : 110), at beam 256 on the mixture,
-// whose rows come from the caches, 2 320 : 1 710; refinement of a million points 71 : 55 ms (40.6 : 30.6 thousand vector
-// instructions a point, 0.95 of their issue rate), sub-graphs 44 : 33 ms.
+// 10 000 searches of a million rows at beam 64 1 347 : 479 us (rows from memory; 1 query 124 : 108), at beam 256 on the mixture,
+// whose rows come from the caches, 2 320 : 1 600; refinement of a million points 71 : 52 ms (0.95 of the vector issue rate),
+// sub-graphs 44 : 31 ms.
 constexpr uint32_t kMostByteDims = 256;   // 256 * 255^2 < 2^24
 constexpr uint32_t kMostByteDegree = 64;  // the searches over rows of bytes are built for one candidate slot a lane
 

@@ -1,4 +1,4 @@
-"""Sub-graph builds and refinement that look at long rows in fp16 first, against the same calls without the fp16 copy: the copy
+"""Sub-graph builds and refinement that look at rows in fp16 first, against the same calls without the fp16 copy: the copy
 only says which rows need not be measured, so graphs and counters must agree to the bit.  The rows include equal ones, near ties
 far below fp16's resolution, values at the ends of fp32's range, and values that are infinite or none."""
 import numpy as np
