@@ -234,17 +234,17 @@ def preprocess(param, d_data, result=None):
     d_ids = capi.DeviceArray(sample_num, np.uint32)
     d_sample = capi.DeviceArray((sample_num, dim), np.float32)
     d_centroids = capi.DeviceArray((c, dim), np.float32)
-    wb = capi.kmeans_workspace_bytes(c, dim)
-    ws = capi.DeviceArray(wb // 4 + 1, np.uint32)
-    sb = capi.kmeans_seed_workspace_bytes(sample_num)
-    seed_ws = capi.DeviceArray(sb // 8 + 1, np.uint64)
-    wb = capi.sample_ids_workspace_bytes(num)
-    ids_ws = capi.DeviceArray(wb // 16 + 1, np.dtype("V16"))
-    capi.sample_ids(num, sample_num, param.seed, d_ids, ids_ws, wb)
+    fit_bytes = capi.kmeans_workspace_bytes(c, dim)
+    fit_ws = capi.DeviceArray(fit_bytes // 4 + 1, np.uint32)
+    seed_bytes = capi.kmeans_seed_workspace_bytes(sample_num)
+    seed_ws = capi.DeviceArray(seed_bytes // 8 + 1, np.uint64)
+    ids_bytes = capi.sample_ids_workspace_bytes(num)
+    ids_ws = capi.DeviceArray(ids_bytes // 16 + 1, np.dtype("V16"))
+    capi.sample_ids(num, sample_num, param.seed, d_ids, ids_ws, ids_bytes)
     with _Timer() as t:
         capi.sample_rows(d_data, dim, d_ids, sample_num, d_sample)
-        capi.kmeans_seed(d_sample, sample_num, dim, c, param.seed, d_centroids, seed_ws, sb)
-        capi.kmeans_fit(d_sample, sample_num, dim, c, param.kmeans_iterations, d_centroids, ws, wb)
+        capi.kmeans_seed(d_sample, sample_num, dim, c, param.seed, d_centroids, seed_ws, seed_bytes)
+        capi.kmeans_fit(d_sample, sample_num, dim, c, param.kmeans_iterations, d_centroids, fit_ws, fit_bytes)
     times["centroids"] = t.seconds
     # define_partition (partition.cuh:61-116)
     d_seg_idx = capi.DeviceArray((num, 3), np.uint32)

@@ -66,3 +66,25 @@ def test_one_lloyd_step_by_either_kernel(n, dim, k):
     np.add.at(sums, nearest, x)
     expect = np.where(counts[:, None] > 0, sums / np.maximum(counts, 1)[:, None], start).astype(np.float32)
     assert np.array_equal(cent.numpy(), expect)
+
+
+# few points beside the size of the centroids, and many beside it: the scratch of the fit is larger than that of the draw of the sample, and smaller
+@pytest.mark.parametrize("num, dim, parts", [(1000, 960, 16), (3000, 128, 256), (10_000, 1000, 200), (60_000, 28, 5)])
+def test_partitioning_whatever_scratch_is_largest(num, dim, parts):
+    from glide_amd import capi as hip
+    from glide_amd import index as G
+    hip.set_device(0)
+    x = rows_of(num, dim, num)
+    param = G.PartitionParameter(centroid_num=parts, boundary_factor=1.04, sample_factor=0.1, metric=G.Metric.Euclidean)
+    d_reorder, d_map, starts, lengths, d_centroids = G.preprocess(param, hip.DeviceArray.from_numpy(x))
+    # the centroids: the steps one at a time, each with the scratch that it asks for
+    sample = x[np.random.default_rng(param.seed).permutation(num)[:max(num // 10, parts)]]
+    d_sample, cent = hip.DeviceArray.from_numpy(sample), hip.DeviceArray((parts, dim), np.float32)
+    size = hip.kmeans_seed_workspace_bytes(len(sample))
+    hip.kmeans_seed(d_sample, len(sample), dim, parts, param.seed, cent, hip.DeviceArray(size // 8 + 1, np.uint64), size)
+    size = hip.kmeans_workspace_bytes(parts, dim)
+    hip.kmeans_fit(d_sample, len(sample), dim, parts, param.kmeans_iterations, cent, hip.DeviceArray(size // 8 + 1, np.uint64), size)
+    hip.synchronize()
+    assert np.array_equal(d_centroids.numpy(), cent.numpy())
+    assert int(lengths[:parts].sum()) == num
+    assert np.array_equal(d_reorder.numpy(), x[d_map.numpy()])
