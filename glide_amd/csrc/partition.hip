@@ -624,7 +624,7 @@ constexpr uint32_t kSeedPoints = 64;       // sample rows per workgroup of the t
 // The distances to a step's candidates are kept for the step after up to this many sample rows (1 MiB, in the L2).  For larger
 // samples the distance to the winner is computed a second time, by the trial kernel as one candidate more and for the 64 rows
 // that a draw ends in: the workspace stays at 5 bytes a row (a step of 33 000 rows of 96 dims 20 us, one of 200 000 of 200 dims
-// 102 us; with a pass of their own for the smallest distances 43 and 236).
+// 102 us; with a pass of their own for the smallest distances 43 and 236; of 50 000 of 960 dims 129 and 158).
 constexpr uint32_t kSeedKept = 32768;
 
 __host__ __device__ inline uint32_t seed_trials(uint32_t k) {
@@ -899,28 +899,48 @@ __global__ __launch_bounds__(1024) void kmeanspp_next_kernel(const float* sample
         part[threadIdx.x] = acc;
     }
     __syncthreads();   // every thread has read the old candidates by now
-    if (wave >= next_trials) return;
+    // !KEPT: a candidate's 64 rows are shared by two wavefronts or more (of five candidates: by three), which all look for the place:
+    // with one a candidate half of the kernel's wavefronts idled through its longest part (50 000 rows of 960 dims, 64 clusters: a step
+    // 129 us, not 166; of 200 dims 43, not 55; of 128 dims 23 either way)
+    const uint32_t share = KEPT ? 1u : 16u / next_trials, draw = wave / share, member = wave % share;
+    const bool draws = draw < next_trials;
+    if (KEPT && !draws) return;
     double total = 0.0;
     for (uint32_t i = lane; i < parts; i += 64) total += part[i];
     for (int off = 32; off >= 1; off >>= 1) total += __shfl_xor(total, off);
     uint32_t cand = seed_hash(seed, 16 * (step + 1)) % n;      // every row already coincides with a centroid
-    if (total > 0.0) {
-        const uint32_t h = seed_hash(seed, 16 * (step + 1) + wave);
+    uint32_t first = 0, rows = 0;
+    double left = 0.0;
+    float to_won = 0.f;
+    if (total > 0.0 && draws) {
+        const uint32_t h = seed_hash(seed, 16 * (step + 1) + draw);
         const double target = static_cast<double>(h >> 8) * (1.0 / 16777216.0) * total;
-        double before = 0.0, before_block = 0.0, unused = 0.0;
+        double before = 0.0, before_block = 0.0;
         const uint32_t c = wave_locate([&](uint32_t i) { return part[i]; }, parts, target, before, lane);
         const uint32_t base = c * chunk, len = (base + chunk < blocks ? base + chunk : blocks) - base;
         const double* sums = partial + static_cast<size_t>(base) * kSeedTrials + won;
         const uint32_t block = base + wave_locate([&](uint32_t i) { return sums[static_cast<size_t>(i) * kSeedTrials]; }, len, target - before, before_block, lane);
-        const uint32_t first = block * kSeedPoints, rows = n - first < kSeedPoints ? n - first : kSeedPoints;
-        const float* md = min_dist + first;
-        float to_won;
+        first = block * kSeedPoints, rows = n - first < kSeedPoints ? n - first : kSeedPoints;
+        left = target - before - before_block;
         if constexpr (KEPT) to_won = static_cast<uint32_t>(lane) < rows ? trial_dist[static_cast<size_t>(won) * n + first + lane] : 0.f;
-        else to_won = block_distances<LANES>(sample, dim, first, rows, won_row, lane);
-        const double value = static_cast<uint32_t>(lane) < rows ? static_cast<double>(fminf(md[lane], to_won)) : 0.0;   // a row a lane
-        cand = first + wave_locate([&](uint32_t) { return value; }, rows, target - before - before_block, unused, lane);
     }
-    if (lane == 0) candidates[wave] = cand;
+    if constexpr (!KEPT) {
+        __shared__ float of_block[kSeedTrials][kSeedPoints];
+        const uint32_t each = (kSeedPoints + share - 1) / share, lo = member * each, mine = rows > lo ? (rows - lo < each ? rows - lo : each) : 0u;
+        if (mine != 0) {
+            const float d = block_distances<LANES>(sample, dim, first + lo, mine, won_row, lane);
+            if (static_cast<uint32_t>(lane) < mine) of_block[draw][lo + lane] = d;
+        }
+        __syncthreads();
+        if (!draws || member != 0) return;
+        to_won = of_block[draw][lane];
+    }
+    if (total > 0.0) {
+        const double value = static_cast<uint32_t>(lane) < rows ? static_cast<double>(fminf(min_dist[first + lane], to_won)) : 0.0;   // a row a lane
+        double unused = 0.0;
+        cand = first + wave_locate([&](uint32_t) { return value; }, rows, left, unused, lane);
+    }
+    if (lane == 0) candidates[draw] = cand;
 }
 
 // Before the first step: one candidate, drawn uniformly, and no distances yet (the smaller of NaN and a distance is the distance).

@@ -11,7 +11,7 @@ def rows_of(n, dim, seed):
     return np.random.default_rng(seed).integers(0, 16, (n, dim)).astype(np.float32)
 
 
-@pytest.mark.parametrize("n, dim, k", [(1, 4, 1), (63, 128, 3), (65, 132, 5), (1000, 256, 9), (200, 260, 4), (32768, 8, 3), (32769, 8, 3)])
+@pytest.mark.parametrize("n, dim, k", [(1, 4, 1), (63, 128, 3), (65, 132, 5), (1000, 256, 9), (200, 260, 4), (32768, 8, 3), (32769, 8, 3), (32770, 132, 40), (33000, 260, 12)])
 def test_seeding_rows(n, dim, k):
     from glide_amd import capi as hip
     from oracle import oracle as O
