@@ -13,6 +13,7 @@ LIB_PATH = os.environ.get("GLIDE_HIP_LIB", os.path.join(_HERE, "libglide_hip.so"
 _lib = None
 
 EUCLIDEAN, COSINE = 0, 1
+OUT_OF_MEMORY = 2          # hipErrorOutOfMemory, handed on as it is
 INVALID = 0xFFFFFFFF
 
 u32, f32, vp = C.c_uint32, C.c_float, C.c_void_p

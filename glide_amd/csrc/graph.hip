@@ -115,6 +115,7 @@ __global__ __launch_bounds__(256) void insert_reverse_kernel(uint32_t* graph, co
 // of fractions end there, and the others find the word set and leave (in one launch every wavefront reads its rows before
 // the word says anything, and all of them write it: 0.36 ms for 300k x 96 fractions).
 constexpr uint32_t kPackProbe = 64;
+constexpr size_t kMostPacked = size_t{16} << 32;   // bytes written at most: 2^32 threads (2^29 rows of up to 128 dims)
 __global__ __launch_bounds__(256) void pack_bytes_kernel(const float* rows, uint32_t num, uint32_t dim, uint32_t lanes, uint32_t first_block, uint4* bytes,
                                                          uint32_t* other) {
     if (*other != 0) return;
@@ -460,18 +461,18 @@ int glide_hip_insert_reverse(uint32_t* graph, const uint32_t* reverse_graph, con
 
 size_t glide_hip_byte_rows_bytes(uint32_t num, uint32_t dim) {
     if (dim == 0 || dim > kMostByteDims || dim % 4 != 0) return 0;
-    return static_cast<size_t>(num) * (dim <= 128 ? RowShape<-1>::STRIDE : RowShape<-2>::STRIDE);
+    const size_t bytes = static_cast<size_t>(num) * (dim <= 128 ? RowShape<-1>::STRIDE : RowShape<-2>::STRIDE);
+    return bytes <= kMostPacked ? bytes : 0;
 }
 
 int glide_hip_pack_byte_rows(const float* rows, uint32_t num, uint32_t dim, void* byte_rows, uint32_t* other_values, void* stream) {
     if (!rows || !byte_rows || !other_values || dim == 0) return GLIDE_ERR_BAD_ARGUMENT;
-    if (dim > kMostByteDims || dim % 4 != 0) return GLIDE_ERR_UNSUPPORTED;
+    if (glide_hip_byte_rows_bytes(1, dim) == 0 || (num != 0 && glide_hip_byte_rows_bytes(num, dim) == 0)) return GLIDE_ERR_UNSUPPORTED;
     if (reinterpret_cast<uintptr_t>(rows) % 16 || reinterpret_cast<uintptr_t>(byte_rows) % 16) return GLIDE_ERR_BAD_ARGUMENT;
     const int rc = glide_hip_fill_u32(other_values, 0u, 1, stream);
     if (rc != GLIDE_OK || num == 0) return rc;
     const uint32_t lanes = dim <= 128 ? RowShape<-1>::LPR : RowShape<-2>::LPR;   // sixteen dims each
     const size_t blocks = (static_cast<size_t>(num) * lanes + 255) / 256;
-    if (blocks > (1u << 24)) return GLIDE_ERR_UNSUPPORTED;   // 2^32 threads; over 2^28 rows
     const uint32_t probe = blocks < kPackProbe ? static_cast<uint32_t>(blocks) : kPackProbe;
     hipLaunchKernelGGL(pack_bytes_kernel, dim3(probe), dim3(256), 0, as_stream(stream), rows, num, dim, lanes, 0u, static_cast<uint4*>(byte_rows),
                        other_values);

@@ -346,7 +346,7 @@ extern "C" size_t glide_hip_search_partitions_workspace_bytes(uint32_t query_num
 // the caches, 1 072 : 900; at the line, 1 000 queries, 622 : 563 and 538 : 493).  Every query selects a partition at least, as a
 // rule two or three; half of an expansion's rows are new.
 static bool partitions_as_bytes_pay(uint32_t num, uint32_t dim, uint32_t degree, uint32_t query_num, uint32_t beam) {
-    return num != 0 && degree <= kMostByteDegree && glide_hip_byte_rows_bytes(1, dim) != 0 &&
+    return num != 0 && degree <= kMostByteDegree && glide_hip_byte_rows_bytes(num, dim) != 0 &&
            static_cast<unsigned long long>(query_num) * beam * degree / 2 >= 4ull * num;
 }
 

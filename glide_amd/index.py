@@ -174,13 +174,21 @@ def cut_rows(d_rows, dim):
 
 
 def spare_array(nbytes):
-    """Memory for a copy that only makes things faster, or None: what is free must have room for two of it."""
-    return capi.DeviceArray(nbytes, np.uint8) if capi.mem_info()[0] // 2 >= nbytes else None
+    """Memory for a copy that only makes things faster, or None: what is free must have room for two of it, and none is made
+    where the device has it in no one piece or another thread is faster."""
+    if capi.mem_info()[0] // 2 < nbytes:
+        return None
+    try:
+        return capi.DeviceArray(nbytes, np.uint8)
+    except capi.GlideHipError as e:
+        if e.code != capi.OUT_OF_MEMORY:
+            raise
+        return None
 
 
 def byte_rows(d_rows):
     """The rows of a DeviceArray once more as bytes, for the searches over rows of whole numbers 0..255, as a DeviceArray;
-    None where a value is none of those or rows of that length are not held so."""
+    None where a value is none of those, rows of that length or so many are not held so, or memory is short."""
     num, dim = d_rows.shape
     nbytes = capi.byte_rows_bytes(num, dim)
     if nbytes == 0:
@@ -208,7 +216,7 @@ def rough_rows_pay(num, dim):
 
 def rough_rows(d_rows):
     """Rows once more in fp16, for the builds that look at them before they measure (half the memory traffic, the same results), as
-    a DeviceArray; None where that does not pay or rows of that length are not looked at so."""
+    a DeviceArray; None where that does not pay, rows of that length are not looked at so, or memory is short."""
     num, dim = d_rows.shape
     nbytes = capi.rough_rows_bytes(num, dim) if rough_rows_pay(num, dim) else 0
     d_rough = spare_array(nbytes) if nbytes else None

@@ -313,7 +313,7 @@ int glide_hip_refine(const float *data, uint32_t num, uint32_t dim, const uint32
 /* ---- rows of whole numbers 0 .. 255 (image descriptors, quantised embeddings), held as bytes (no counterpart in the
  * reference, whose kernels read such rows as fp32 or cast every value as it is read) -----------------------------------
  * glide_hip_byte_rows_bytes: the size of `num` rows of `dim` values as bytes (rows of 128 or 256 bytes, zeros behind the
- * values), 0 where rows of that length are not held so (more than 256 values).  glide_hip_pack_byte_rows writes them
+ * values), 0 where rows of that length (more than 256 values) or that many (2^36 bytes of them) are not held so.  glide_hip_pack_byte_rows writes them
  * (16-byte aligned) and sets *other_values (device) to 1 if some value is no whole number 0 .. 255, to 0 otherwise; the
  * byte rows are of use only in the second case.
  * The entry points that follow are those without `_bytes` or `_rows` with the same rows handed in a second time: as bytes,

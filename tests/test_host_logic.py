@@ -74,3 +74,36 @@ def test_synthetic_generators_are_seeded_and_shaped():
     assert e.shape == (200, 960) and e.min() >= 0 and e.max() <= 1
     r = D.recall(np.array([[1, 2, 3]]), np.array([[3, 4, 1]]), 3)
     assert abs(r - 2 / 3) < 1e-9
+
+
+def test_copies_that_only_save_time_never_fail_a_call(monkeypatch):
+    """Short memory, memory that is gone when it is asked for, and more rows than are packed: no copy, no error."""
+    import pytest
+    from glide_amd import capi
+    asked = []
+
+    class NoMemory:
+        def __init__(self, shape, dtype):
+            if np.dtype(dtype) == np.uint8:
+                asked.append(shape)
+                raise capi.GlideHipError(code, "glide_hip_malloc")
+
+    class Rows:
+        shape = (100_000, 256)
+
+    code = 2                 # hipErrorOutOfMemory
+    monkeypatch.setattr(capi, "DeviceArray", NoMemory)
+    monkeypatch.setattr(capi, "mem_info", lambda: (1 << 40, 1 << 40))
+    assert G.spare_array(1 << 20) is None and G.byte_rows(Rows()) is None and G.rough_rows(Rows()) is None
+    assert len(asked) == 3
+    code = 719               # another error is none of memory
+    with pytest.raises(capi.GlideHipError):
+        G.spare_array(1 << 20)
+    monkeypatch.setattr(capi, "mem_info", lambda: (1 << 20, 1 << 40))
+    assert G.spare_array((1 << 19) + 1) is None
+    # 2^32 pieces of 16 bytes are packed at most
+    for dim, most in ((4, 2 ** 29), (128, 2 ** 29), (132, 2 ** 28), (256, 2 ** 28)):
+        assert capi.byte_rows_bytes(most, dim) == 2 ** 36 and capi.byte_rows_bytes(most + 1, dim) == 0
+        plain = capi._size_fn("glide_hip_search_partitions_workspace_bytes")(64, 8, 10)
+        size = capi._size_fn("glide_hip_search_partitions_rows_workspace_bytes")
+        assert size(64, 8, 10, 100, dim, 32, 64) > plain and size(2 ** 31, 8, 10, most + 1, dim, 64, 512) == capi._size_fn("glide_hip_search_partitions_workspace_bytes")(2 ** 31, 8, 10)
