@@ -214,6 +214,7 @@ using namespace glide;
 extern "C" {
 
 namespace {
+constexpr uint32_t kMostIds = 1u << 30;   // threads of the stream are counted with 32 bits
 struct SampleLayout { size_t stream, settled, heads, links, steps, total; uint32_t chunks; };
 SampleLayout sample_layout(uint32_t num) {
     SampleLayout l;
@@ -230,11 +231,11 @@ SampleLayout sample_layout(uint32_t num) {
 }
 }  // namespace
 
-size_t glide_hip_sample_ids_workspace_bytes(uint32_t num) { return sample_layout(num).total; }
+size_t glide_hip_sample_ids_workspace_bytes(uint32_t num) { return num <= kMostIds ? sample_layout(num).total : 0; }
 
 int glide_hip_sample_ids(uint32_t num, uint32_t count, const uint64_t* generator, uint32_t* ids, void* workspace, size_t workspace_bytes, void* stream) {
     if (!generator || !ids || !workspace || num == 0 || count > num) return GLIDE_ERR_BAD_ARGUMENT;
-    if (num > (1u << 30)) return GLIDE_ERR_UNSUPPORTED;
+    if (num > kMostIds) return GLIDE_ERR_UNSUPPORTED;
     const SampleLayout l = sample_layout(num);
     if (workspace_bytes < l.total || reinterpret_cast<uintptr_t>(workspace) % 16) return GLIDE_ERR_BAD_ARGUMENT;
     if (count == 0) return GLIDE_OK;

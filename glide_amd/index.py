@@ -173,17 +173,20 @@ def cut_rows(d_rows, dim):
     return h
 
 
-def spare_array(nbytes):
-    """Memory for a copy that only makes things faster, or None: what is free must have room for two of it, and none is made
-    where the device has it in no one piece or another thread is faster."""
-    if capi.mem_info()[0] // 2 < nbytes:
-        return None
+def try_array(nbytes):
+    """nbytes on the device, or None where it has them not."""
     try:
         return capi.DeviceArray(nbytes, np.uint8)
     except capi.GlideHipError as e:
         if e.code != capi.OUT_OF_MEMORY:
             raise
         return None
+
+
+def spare_array(nbytes):
+    """Memory for a copy that only makes things faster, or None: what is free must have room for two of it, and none is made
+    where the device has it in no one piece or another thread is faster."""
+    return try_array(nbytes) if capi.mem_info()[0] // 2 >= nbytes else None
 
 
 def byte_rows(d_rows):
@@ -225,6 +228,19 @@ def rough_rows(d_rows):
     return d_rough
 
 
+def draw_ids(num, count, seed, d_ids):
+    """The first `count` entries of np.random.default_rng(seed).permutation(num) into a DeviceArray.  Returns the scratch of the
+    device's draw (some 21 bytes a row; it may go once the draw is done), or None where the host has drawn: more rows than the
+    device draws from, or no memory for it."""
+    nbytes = capi.sample_ids_workspace_bytes(num)
+    workspace = try_array(nbytes) if nbytes else None
+    if workspace is None:
+        d_ids.upload(np.random.default_rng(seed).permutation(num)[:count].astype(np.uint32))
+    else:
+        capi.sample_ids(num, count, seed, d_ids, workspace, nbytes)
+    return workspace
+
+
 def preprocess(param, d_data, result=None):
     """partition.cuh:159-193.  d_data: DeviceArray (num, dim) float32; rows of a length that is no multiple of four are
     padded (pad_rows), and the reordered rows and centroids returned then have the padded length (cut_rows gives them
@@ -246,14 +262,15 @@ def preprocess(param, d_data, result=None):
     fit_ws = capi.DeviceArray(fit_bytes // 4 + 1, np.uint32)
     seed_bytes = capi.kmeans_seed_workspace_bytes(sample_num)
     seed_ws = capi.DeviceArray(seed_bytes // 8 + 1, np.uint64)
-    ids_bytes = capi.sample_ids_workspace_bytes(num)
-    ids_ws = capi.DeviceArray(ids_bytes // 16 + 1, np.dtype("V16"))
-    capi.sample_ids(num, sample_num, param.seed, d_ids, ids_ws, ids_bytes)
+    ids_ws = draw_ids(num, sample_num, param.seed, d_ids)
     with _Timer() as t:
         capi.sample_rows(d_data, dim, d_ids, sample_num, d_sample)
         capi.kmeans_seed(d_sample, sample_num, dim, c, param.seed, d_centroids, seed_ws, seed_bytes)
         capi.kmeans_fit(d_sample, sample_num, dim, c, param.kmeans_iterations, d_centroids, fit_ws, fit_bytes)
     times["centroids"] = t.seconds
+    for used in (ids_ws, d_ids, d_sample, seed_ws, fit_ws):     # before the reordered rows need their room
+        if used is not None:
+            used.free()
     # define_partition (partition.cuh:61-116)
     d_seg_idx = capi.DeviceArray((num, 3), np.uint32)
     d_seg_len = capi.DeviceArray(c + 1, np.uint32)

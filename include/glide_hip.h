@@ -126,7 +126,7 @@ int glide_hip_reorder_batch(const float *data, uint32_t num, uint32_t dim, const
 /* Replaces the iota + std::shuffle of get_centroids (partition.cuh:30-44): ids (device, `count` of them) = the first `count`
  * places of a random permutation of 0 .. num-1.  generator (host, 4 words) is a PCG64 generator's state before its first
  * output and its increment, upper halves first; the permutation is the one numpy's Generator.permutation(num) makes with
- * that generator.  workspace: glide_hip_sample_ids_workspace_bytes(), 16-byte aligned. */
+ * that generator.  workspace: glide_hip_sample_ids_workspace_bytes(), 16-byte aligned; num is at most 2^30, the size is 0 beyond. */
 size_t glide_hip_sample_ids_workspace_bytes(uint32_t num);
 int glide_hip_sample_ids(uint32_t num, uint32_t count, const uint64_t *generator, uint32_t *ids, void *workspace,
                          size_t workspace_bytes, void *stream);
