@@ -356,18 +356,25 @@ class GLIDE:
         d_bytes = byte_rows(self.d_data) if self._graph_degree <= BYTE_ROWS_DEGREE else None
         if d_bytes is not None:
             self._bytes = d_bytes, self.d_data, writes
+        return d_bytes
 
     def _byte_rows(self):
-        """The rows as bytes, or None: there are none, or the rows may have been written since (a search then reads the rows)."""
+        """The rows as bytes, or None: there are none, or the rows may have been written since.  A search then reads the rows,
+        and so do all that follow: the copy goes."""
         if self._bytes is None:
             return None
         d_bytes, made_from, writes = self._bytes
-        return d_bytes if made_from is self.d_data and writes == made_from.writes and not made_from.shared else None
+        if made_from is self.d_data and writes == made_from.writes and not made_from.shared:
+            return d_bytes
+        self._bytes = None
+        return None
 
     def load(self, h_graph, h_start_points):                                   # glide_impl.cuh:32-41
         self.d_graph.upload(np.ascontiguousarray(h_graph, dtype=np.uint32))
         self.d_start_points = capi.DeviceArray.from_numpy(np.ascontiguousarray(h_start_points, dtype=np.uint32))
-        self._hold_byte_rows()
+        self._bytes = None
+        if not self.d_data.shared:
+            self._hold_byte_rows()
 
     def start_point_select(self, h_segment_start, h_segment_length, h_map, seed):   # glide_impl.cuh:43-75
         rng = np.random.default_rng(seed)
@@ -437,19 +444,21 @@ class GLIDE:
             p = search_param_refine
             cnt2 = capi.new_counters() if counters else None
             with _Timer() as t:
-                self._hold_byte_rows()
-                d_rough = rough_rows(self.d_data) if self._bytes is None and deg <= ROUGH_ROWS_DEGREE and p.beam <= ROUGH_ROWS_BEAM else None
+                d_bytes = self._hold_byte_rows()
+                d_rough = rough_rows(self.d_data) if d_bytes is None and deg <= ROUGH_ROWS_DEGREE and p.beam <= ROUGH_ROWS_BEAM else None
                 capi.refine(self.d_data, num, dim, self.d_graph, d_rev, deg, self.d_centroids, self.centroid_num(),
                             self.d_start_points, p.beam, p.max_iterations, p.min_iterations, p.hash_bit, p.hash_reset_interval,
                             build_param.relaxant_factor, self.metric, cnt2, order=d_map,
-                            byte_rows=self._bytes[0] if self._bytes else None, rough_rows=d_rough)
+                            byte_rows=d_bytes, rough_rows=d_rough)
             times["refine"] = t.seconds
+            del d_bytes
+            self._byte_rows()      # the searches may not use them: rows whose address is known to others
             if d_rough is not None:
                 d_rough.free()
             self.d_graph, d_rev = d_rev, self.d_graph
             if counters and result is not None:
                 result["refine_counters"] = capi.read_counters(cnt2)
-        else:
+        elif not self.d_data.shared:
             self._hold_byte_rows()
         d_rev.free()
         d_map.free()

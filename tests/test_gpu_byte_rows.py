@@ -194,3 +194,33 @@ def test_partitions(hip, dim, degree, beam, top_k, bad_row):
         got.append((ids.numpy(), dists.numpy(), hip.read_counters(cnt)))
     assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1]) and got[0][2] == got[1][2]
     assert (got[0][0][:, 0] < n).sum() >= nq // 2          # some select the empty partition alone
+
+
+@pytest.mark.parametrize("refine_beam", [0, 128])
+def test_bytes_that_no_search_may_use_are_not_kept(hip, refine_beam):
+    """Once the address of the rows has been handed out an index searches its fp32 rows: it then holds no copy of them."""
+    from glide_amd import index as G
+    rng = np.random.default_rng(5)
+    n, dim, degree = 3000, 64, 32
+    rows = rows_of(rng, n, dim)
+    sp, queries = G.make_search_parameter(64, degree), hip.DeviceArray.from_numpy(rows_of(rng, 50, dim))
+
+    def build(d):
+        d_reorder, d_map, starts, lengths, d_c = G.preprocess(G.PartitionParameter(centroid_num=3, boundary_factor=1.04, sample_factor=0.5), d)
+        d_knn = G.build_nnd(G.NNDescentParameter(graph_degree=degree, max_iterations=6), d_reorder, starts, lengths)
+        index = G.GLIDE(degree, d, d_c, G.Metric.Euclidean)
+        index.build(G.IndexParameter(graph_degree=degree, knn_degree=degree, relaxant_factor=1.05), G.make_search_parameter(64, degree),
+                    G.make_search_parameter(refine_beam, degree) if refine_beam else G.SearchParameter(beam=0), d_knn, starts, lengths, d_map, d_reorder)
+        return index
+
+    own, known = build(hip.DeviceArray.from_numpy(rows)), hip.DeviceArray.from_numpy(rows)
+    assert known.ptr
+    other = build(known)
+    assert own._bytes is not None and other._bytes is None
+    assert np.array_equal(own.d_graph.numpy(), other.d_graph.numpy())
+    expect = own.search(sp, queries)
+    assert all(np.array_equal(a, b) for a, b in zip(expect, other.search(sp, queries)))
+    other.load(own.d_graph.numpy(), own.d_start_points.numpy())
+    assert other._bytes is None and all(np.array_equal(a, b) for a, b in zip(expect, other.search(sp, queries)))
+    assert own.d_data.ptr and own._bytes is not None       # handed out later: gone with the next search
+    assert all(np.array_equal(a, b) for a, b in zip(expect, own.search(sp, queries))) and own._bytes is None
