@@ -517,9 +517,16 @@ def search_partitions(data, dim, graph, graph_degree, mp, segment_starts, segmen
                       final_dists, counters=None, stream=None):
     known = isinstance(data, DeviceArray) and len(data.shape) == 2 and data.shape[1] == dim and data.dtype == np.float32
     num = data.shape[0] if known else 0
-    wb = int(_size_fn("glide_hip_search_partitions_rows_workspace_bytes")(u32(query_num), u32(segment_num), u32(top_k), u32(num), u32(dim), u32(graph_degree),
-                                                                          u32(beam)))
-    ws = DeviceArray(wb // 16 + 1, np.dtype("V16"))
+    while True:
+        wb = int(_size_fn("glide_hip_search_partitions_rows_workspace_bytes")(u32(query_num), u32(segment_num), u32(top_k), u32(num), u32(dim), u32(graph_degree),
+                                                                              u32(beam)))
+        try:
+            ws = DeviceArray(wb // 16 + 1, np.dtype("V16"))
+            break
+        except GlideHipError as e:
+            if e.code != OUT_OF_MEMORY or num == 0:
+                raise
+            num = 0      # no room for the rows as bytes: they are searched as they are
     check(lib().glide_hip_search_partitions_rows(_ptr(data), u32(num), u32(dim), _ptr(graph), u32(graph_degree), _ptr(mp),
                                                  _ptr(segment_starts), _ptr(segment_start_points), u32(segment_num), _ptr(queries), u32(query_num),
                                                  _ptr(segment_ids), u32(top_k), u32(beam), u32(max_iterations), u32(min_iterations), u32(hash_bit),

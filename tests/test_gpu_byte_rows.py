@@ -224,3 +224,33 @@ def test_bytes_that_no_search_may_use_are_not_kept(hip, refine_beam):
     assert other._bytes is None and all(np.array_equal(a, b) for a, b in zip(expect, other.search(sp, queries)))
     assert own.d_data.ptr and own._bytes is not None       # handed out later: gone with the next search
     assert all(np.array_equal(a, b) for a, b in zip(expect, own.search(sp, queries))) and own._bytes is None
+
+
+def test_partitions_without_room_for_the_bytes(hip, monkeypatch):
+    """Rows as bytes are a copy in the workspace: where there is no memory for it the search takes the rows as they are."""
+    from oracle import oracle as O
+    rng = np.random.default_rng(9)
+    n, dim, degree, nq, top_k = 4000, 64, 32, 200, 10
+    rows = rows_of(rng, n, dim)
+    graph = O.bruteforce_knn(rows, rows, degree, exclude_self=True)[0]
+    up = hip.DeviceArray.from_numpy
+    sp, d, d_q = O.search_params(64, degree), up(rows), up(rows_of(rng, nq, dim))
+    rest = up(graph), up(np.arange(n, dtype=np.uint32)), up(np.zeros(1, np.uint32)), up(np.array([5], np.uint32)), up(np.zeros((nq, 1), np.uint32))
+
+    def search():
+        ids, dists = hip.DeviceArray((nq, top_k), np.uint32), hip.DeviceArray((nq, top_k), np.float32)
+        hip.search_partitions(d, dim, rest[0], degree, rest[1], rest[2], rest[3], 1, d_q, nq, rest[4], top_k, sp["beam"], sp["max_iterations"],
+                              sp["min_iterations"], sp["hash_bit"], sp["hash_reset_interval"], 0, ids, dists)
+        return ids.numpy(), dists.numpy()
+
+    expect, make, refused = search(), hip.DeviceArray.__init__, []
+
+    def short(self, shape, dtype):
+        if np.dtype(dtype).itemsize * np.prod(shape) > n * 128:
+            refused.append(shape)
+            raise hip.GlideHipError(2, "glide_hip_malloc")
+        make(self, shape, dtype)
+
+    monkeypatch.setattr(hip.DeviceArray, "__init__", short)
+    got = search()
+    assert len(refused) == 1 and all(np.array_equal(a, b) for a, b in zip(expect, got))
