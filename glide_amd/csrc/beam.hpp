@@ -29,8 +29,13 @@ struct BeamCounters {  // wave-uniform tallies for traffic accounting
 
 template <int MAX_CAND>
 struct alignas(16) BeamLds {  // per-wave LDS (the hash table follows, 1 << hash_bit words)
-    uint32_t cand_id[MAX_CAND];
-    float cand_dist[MAX_CAND];   // squared distances of vlist's rows while an expansion is scored, then distances by slot or rank
+    union {
+        struct {
+            uint32_t cand_id[MAX_CAND];
+            float cand_dist[MAX_CAND];   // squared distances of vlist's rows while an expansion is scored, then distances by slot or rank
+        };
+        uint32_t pool_open[2 * MAX_CAND];   // once the search is over: see RoughPool
+    };
     uint32_t vlist[MAX_CAND];    // row ids to score, compacted
 };
 

@@ -42,7 +42,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DIMV > 4 || 
     b.init(lds, hash, a.p, row_at<DIMV>(rows, point, a.p.dim));
     RoughPool look{};
     if constexpr (ROUGH) {
-        look = RoughPool{rough_rows(a.rough, a.p.dim), lds->cand_id};
+        static_assert(sizeof(lds->pool_open) / 4 >= MAX_BEAM, "room for every entry of a pool");
+        look = RoughPool{rough_rows(a.rough, a.p.dim), lds->pool_open};
         b.look_first(look.rough, point, seg_start);
     }
     // get_init (search_kernel.cuh:336-360): all neighbours of the entry are hashed; the one whose *local* id equals
@@ -119,7 +120,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DIMV > 4 || 
     b.init(lds, hash, a.p, row_at<DIMV>(rows, point, a.p.dim));
     RoughPool look{};
     if constexpr (ROUGH) {
-        look = RoughPool{rough_rows(a.rough, a.p.dim), lds->cand_id};
+        static_assert(sizeof(lds->pool_open) / 4 >= MAX_BEAM, "room for every entry of a pool");
+        look = RoughPool{rough_rows(a.rough, a.p.dim), lds->pool_open};
         b.look_first(look.rough, point, 0u);
     }
     if (a.centroids != nullptr) {
