@@ -456,6 +456,12 @@ def pack_rough_rows(rows, num, dim, rough_rows, stream=None):
     check(lib().glide_hip_pack_rough_rows(_ptr(rows), u32(num), u32(dim), _out(rough_rows), vp(stream)), "glide_hip_pack_rough_rows")
 
 
+def survey_rough_rows(rows, rough_rows, num, dim, graph, degree, segment_starts, segment_lengths, segment_num, start_points, counts, stream=None):
+    check(lib().glide_hip_survey_rough_rows(_ptr(rows), _ptr(rough_rows), u32(num), u32(dim), _ptr(graph), u32(degree), _ptr(segment_starts),
+                                            _ptr(segment_lengths), u32(segment_num), _ptr(start_points), _out(counts), vp(stream)),
+          "glide_hip_survey_rough_rows")
+
+
 def copy_rows(src, num, src_dim, dst, dst_dim, stream=None):
     check(lib().glide_hip_copy_rows(_ptr(src), C.c_uint64(num), C.c_uint32(src_dim), _out(dst, stream), C.c_uint32(dst_dim), vp(stream)),
           "glide_hip_copy_rows")

@@ -195,6 +195,83 @@ __global__ __launch_bounds__(256) void rough_pack_kernel(const float* rows, uint
     if (threadIdx.x == 0) atomicMax(turn_bits, __float_as_uint(fmaxf(fmaxf(of_wave[0], of_wave[1]), fmaxf(of_wave[2], of_wave[3]))));
 }
 
+// Whether a first look in fp16 will settle anything, from some rows and the graph that their searches will go through; one
+// wavefront a row.  counts[0] / counts[1]: neighbours of a neighbour that are farther than the row's own farthest one, and how many
+// of them the look's bounds would tell to be so.  counts[2] / counts[3]: rows, and those that a greedy walk from their segment's
+// start ends one and a half times that far from, or more: searches that do not get to where they should stay among few rows, the caches
+// serve those, and the look has no traffic to save.  One wavefront's round trips: with the counts read back 70 us on rows of 128
+// values, 90 on 256, 110 on 512, 190 on 960 at degree 64 (builds of 40, 50, 35 and 158 ms).
+struct SurveyArgs {
+    const float* rows;
+    const unsigned char* rough;
+    const uint32_t *graph, *starts, *lengths, *start_points;
+    uint32_t num, dim, degree, segment_num;
+    uint32_t* counts;
+};
+constexpr uint32_t kSurveyed = 512, kMostHops = 64;
+template <int DIMV>
+__global__ __launch_bounds__(64) void rough_survey_kernel(SurveyArgs a) {
+    __shared__ uint32_t own[64], list[64];
+    __shared__ float sq[64];
+    const int lane = lane_id();
+    const uint32_t row = static_cast<uint32_t>(static_cast<unsigned long long>(blockIdx.x) * a.num / gridDim.x);
+    uint32_t seg = kInvalid;
+    for (uint32_t s0 = 0; s0 < a.segment_num && seg == kInvalid; s0 += 64) {
+        const uint32_t s = s0 + lane;
+        const uint64_t m = ballot(s < a.segment_num && row - a.starts[s] < a.lengths[s]);   // below the start it wraps
+        if (m != 0) seg = s0 + __builtin_ctzll(m);
+    }
+    if (seg == kInvalid) return;
+    const uint32_t first = a.starts[seg], length = a.lengths[seg], self = row - first, degree = a.degree < 64 ? a.degree : 64;
+    const float* data = a.rows + static_cast<size_t>(first) * a.dim;
+    RowRegs<DIMV> q;
+    load_row<DIMV>(q, a.rows + static_cast<size_t>(row) * a.dim, a.dim, RowShape<DIMV>::lane_in_row(lane));
+    // this lane's neighbour of a row of the segment, kInvalid if none or the row itself, and its squared distance
+    auto look_at = [&](uint32_t of, float& d) {
+        uint32_t id = static_cast<uint32_t>(lane) < degree ? a.graph[static_cast<size_t>(first + of) * a.degree + lane] : kInvalid;
+        if (id >= length || id == self) id = kInvalid;
+        list[lane] = id != kInvalid ? id : self;
+        wave_sync();
+        score_list<DIMV>(q, data, a.dim, 0, degree, lane, [](uint32_t i) { return list[i]; }, [](uint32_t i, float v) { sq[i] = v; });
+        wave_sync();
+        d = id != kInvalid ? sq[lane] : __builtin_inff();
+        return id;
+    };
+    float d;
+    const uint32_t id = look_at(self, d);
+    own[lane] = id;
+    uint64_t some = ballot(id != kInvalid);
+    if (some == 0) return;
+    float farthest = id != kInvalid ? d : 0.f;
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) farthest = fmaxf(farthest, __shfl_xor(farthest, m));
+    for (int drop = __popcll(some) / 2; drop > 0; drop--) some &= some - 1;
+    const uint32_t of_middle = look_at(read_lane(id, __builtin_ctzll(some)), d);
+    bool far = of_middle != kInvalid && d >= farthest;
+    for (uint32_t j = 0; j < degree; j++) far &= own[j] != of_middle;
+    const RoughRows look = rough_rows(a.rough, a.dim);
+    const float off = 2 * look.turn * row_length<DIMV>(q) + look.tiny;   // a sum over lanes: every lane takes part
+    const bool settled = far && sqrtf(d) * (1.f - 2 * kRoughTurn) - off >= sqrtf(farthest);
+    const uint32_t fars = __popcll(ballot(far)), settleds = __popcll(ballot(settled));
+    float nearest = __builtin_inff();
+    uint32_t at = a.start_points[seg] < length ? a.start_points[seg] : 0u;
+    for (uint32_t hop = 0; hop < kMostHops; hop++) {
+        const uint32_t next = look_at(at, d);
+        float least = d;
+#pragma unroll
+        for (int m = 32; m >= 1; m >>= 1) least = fminf(least, __shfl_xor(least, m));
+        if (!(least < nearest)) break;
+        nearest = least;
+        at = read_lane(next, __builtin_ctzll(ballot(d == least)));
+    }
+    if (lane == 0) {
+        atomicAdd(&a.counts[0], fars);
+        atomicAdd(&a.counts[1], settleds);
+        atomicAdd(&a.counts[2], 1u);
+        if (!(nearest <= 2.25f * farthest)) atomicAdd(&a.counts[3], 1u);
+    }
+}
+
 // ------------------------------------------------------------------------------------------ merged large build
 // A staged partition's sub-graph holds partition-local ids.  Its rows go to rows segment_start .. of the merged graph
 // with segment_start added to every id (what map_to_graph does through `map` on the small path,
@@ -498,6 +575,22 @@ int glide_hip_pack_rough_rows(const float* rows, uint32_t num, uint32_t dim, voi
     hipLaunchKernelGGL(rough_range_kernel, dim3(blocks), dim3(256), 0, as_stream(stream), rows, quads, max_bits);
     hipLaunchKernelGGL(rough_pack_kernel, dim3(row_blocks), dim3(256), 0, as_stream(stream), rows, num, dim, max_bits, max_bits + 1,
                        reinterpret_cast<_Float16*>(static_cast<unsigned char*>(rough_rows) + kRoughHeader));
+    return launch_status();
+}
+
+int glide_hip_survey_rough_rows(const float* rows, const void* rough_rows, uint32_t num, uint32_t dim, const uint32_t* graph, uint32_t degree,
+                                const uint32_t* segment_starts, const uint32_t* segment_lengths, uint32_t segment_num, const uint32_t* start_points,
+                                uint32_t* counts, void* stream) {
+    if (!rows || !rough_rows || !graph || !segment_starts || !segment_lengths || !start_points || !counts || dim == 0 || degree == 0)
+        return GLIDE_ERR_BAD_ARGUMENT;
+    if (glide_hip_rough_rows_bytes(1, dim) == 0) return GLIDE_ERR_UNSUPPORTED;
+    if (reinterpret_cast<uintptr_t>(rows) % 16 || reinterpret_cast<uintptr_t>(rough_rows) % 16) return GLIDE_ERR_BAD_ARGUMENT;
+    const int rc = glide_hip_fill_u32(counts, 0u, 4, stream);
+    if (rc != GLIDE_OK || num == 0) return rc;
+    const SurveyArgs a{rows, static_cast<const unsigned char*>(rough_rows), graph, segment_starts, segment_lengths, start_points, num, dim, degree,
+                       segment_num, counts};
+    const auto kernel = dim <= 128 ? rough_survey_kernel<1> : dim <= 256 ? rough_survey_kernel<2> : dim <= 512 ? rough_survey_kernel<4> : rough_survey_kernel<8>;
+    hipLaunchKernelGGL(kernel, dim3(num < kSurveyed ? num : kSurveyed), dim3(64), 0, as_stream(stream), a);
     return launch_status();
 }
 

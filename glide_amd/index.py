@@ -228,6 +228,21 @@ def rough_rows(d_rows):
     return d_rough
 
 
+def rough_rows_help(d_rows, d_rough, d_graph, d_starts, d_lengths, d_start_points):
+    """Whether the rows' distances are such that a look at them in fp16 tells most of those that need no measuring, and the searches
+    such that the look saves traffic: from some rows and the graph that is there (see glide_hip_survey_rough_rows).
+    Share told of the far ones, share of walks that arrive, and index with the copy against without, in ms: unit rows 250 000 x 128
+    1.00, 1.0, 39 : 64; the same 16 standard deviations from the origin 0.97, 1.0, 41 : 64, 64 off 0.88, 39 : 45, 128 off 0.73,
+    38 : 28.  60 000 x 960 at degree 64 0.97, 1.0, 158 : 258; 32 off 0.67, 180 : 210; 64 off 0.2, 221 : 219.  Dense clusters,
+    60 000 x 384, 0.1, 0.1, 16.8 : 11.8.  Clusters far from each other, whose searches end in the wrong one, 200 000 x 128 0.99, 0.1,
+    27 : 24, 60 000 x 384 0.98, 0.1, 18.7 : 18.9."""
+    num, dim = d_rows.shape
+    d_counts = capi.DeviceArray(4, np.uint32)
+    capi.survey_rough_rows(d_rows, d_rough, num, dim, d_graph, d_graph.shape[1], d_starts, d_lengths, d_starts.shape[0], d_start_points, d_counts)
+    far, told, rows, astray = (int(v) for v in d_counts.numpy())
+    return far > 0 and told >= 0.6 * far and 2 * astray < rows
+
+
 def draw_ids(num, count, seed, d_ids):
     """The first `count` entries of np.random.default_rng(seed).permutation(num) into a DeviceArray.  Returns the scratch of the
     device's draw (some 21 bytes a row; it may go once the draw is done), or None where the host has drawn: more rows than the
@@ -408,6 +423,12 @@ class GLIDE:
         with _Timer() as t:
             d_bytes = byte_rows(d_reorder_data) if knn_degree <= BYTE_ROWS_DEGREE else None
             d_rough = rough_rows(d_reorder_data) if d_bytes is None and knn_degree <= ROUGH_ROWS_DEGREE and p.beam <= ROUGH_ROWS_BEAM else None
+            helps = None      # whether a look in fp16 helps; not known yet
+            if d_rough is not None:
+                helps = rough_rows_help(d_reorder_data, d_rough, d_knn_graph, d_ss, d_sl, d_rsp)
+                if not helps:
+                    d_rough.free()
+                    d_rough = None
             capi.build_subgraph(d_reorder_data, num, dim, d_knn_graph, knn_degree, d_map, d_ss, d_sl, len(h_segment_start), d_rsp,
                                 deg, p.beam, p.max_iterations, p.min_iterations, p.hash_bit, p.hash_reset_interval,
                                 build_param.relaxant_factor, self.metric, self.d_graph, cnt, byte_rows=d_bytes, rough_rows=d_rough)
@@ -445,7 +466,11 @@ class GLIDE:
             cnt2 = capi.new_counters() if counters else None
             with _Timer() as t:
                 d_bytes = self._hold_byte_rows()
-                d_rough = rough_rows(self.d_data) if d_bytes is None and deg <= ROUGH_ROWS_DEGREE and p.beam <= ROUGH_ROWS_BEAM else None
+                may = d_bytes is None and helps is not False and deg <= ROUGH_ROWS_DEGREE and p.beam <= ROUGH_ROWS_BEAM
+                d_rough = rough_rows(self.d_data) if may else None
+                if d_rough is not None and helps is None and not rough_rows_help(self.d_data, d_rough, self.d_graph, *self._one_segment()):
+                    d_rough.free()
+                    d_rough = None
                 capi.refine(self.d_data, num, dim, self.d_graph, d_rev, deg, self.d_centroids, self.centroid_num(),
                             self.d_start_points, p.beam, p.max_iterations, p.min_iterations, p.hash_bit, p.hash_reset_interval,
                             build_param.relaxant_factor, self.metric, cnt2, order=d_map,
@@ -466,6 +491,10 @@ class GLIDE:
             result["index_time"] = times["subgraph"] + times["boundary"] + times["reverse"]
             result["refine_time"] = times["refine"]
             result["build_stages"] = times
+
+    def _one_segment(self):
+        """Start, length and start point of all rows taken as one segment."""
+        return (capi.DeviceArray.from_numpy(np.array([v], dtype=np.uint32)) for v in (0, self.num(), self.d_start_points.numpy()[0]))
 
     def search(self, param, d_query, result=None, counters=None, stream=None, out=None):
         """glide_impl.cuh:370-454.  d_query: DeviceArray (query_num, dim), in the data's own row length or padded as

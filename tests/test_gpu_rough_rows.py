@@ -134,3 +134,95 @@ def test_where_it_pays():
     from glide_amd.index import rough_rows_pay as pays
     assert pays(60_000, 960) and pays(250_000, 128) and pays(1_000_000, 96)
     assert not pays(2_000, 512) and not pays(70_000, 128) and not pays(234_567, 96) and not pays(10_000_000, 64)
+
+
+def survey(rows, turn, tiny, graph, starts, lengths, start_points):
+    """glide_hip_survey_rough_rows in numpy: [far neighbours of neighbours, those told, rows, rows whose walk goes astray]."""
+    n, counts = len(rows), [0, 0, 0, 0]
+    x = rows.astype(np.float64)
+    for row in np.arange(min(n, 512)) * n // min(n, 512):
+        seg = np.flatnonzero((row >= starts) & (row < starts + lengths.astype(np.int64)))
+        if len(seg) == 0:
+            continue
+        first, length = int(starts[seg[0]]), int(lengths[seg[0]])
+
+        def neighbours(of):
+            ids = graph[first + of, :64].astype(np.int64)
+            ids = ids[(ids < length) & (ids != row - first)]
+            return ids, np.linalg.norm(x[first + ids] - x[row], axis=1)
+
+        ids, d = neighbours(row - first)
+        if len(ids) == 0:
+            continue
+        other, e = neighbours(ids[len(ids) // 2])
+        far = ~np.isin(other, ids) & (e >= d.max())
+        told = far & (e * (1 - 2 * 4.93e-4) - 2 * turn * np.linalg.norm(x[row]) - tiny >= d.max())
+        at, nearest = int(start_points[seg[0]]) if start_points[seg[0]] < length else 0, np.inf
+        while True:
+            there, f = neighbours(at)
+            if len(there) == 0 or f.min() >= nearest:
+                break
+            at, nearest = int(there[f.argmin()]), f.min()
+        counts = [counts[0] + far.sum(), counts[1] + told.sum(), counts[2] + 1, counts[3] + (not nearest <= 1.5 * d.max())]
+    return [int(c) for c in counts]
+
+
+@pytest.mark.parametrize("n,dim,degree,kind", [(1, 8, 4, "plain"), (40, 4, 3, "plain"), (700, 128, 32, "unit"), (600, 132, 64, "close"), (513, 260, 20, "plain"),
+                                               (900, 512, 72, "unit"), (511, 960, 40, "plain"), (640, 1024, 16, "close")])
+def test_survey(hip, n, dim, degree, kind):
+    from oracle import oracle as O
+    rng = np.random.default_rng(n)
+    rows = rows_of(rng, max(n, 16), dim, kind)[:n]
+    starts, lengths = np.array([0, n // 3, n // 3], np.uint32), np.array([n // 3, 0, n - n // 3], np.uint32)
+    graph = np.full((n, degree), INV, np.uint32)
+    for s, m in zip(starts, lengths):
+        k = min(degree, m - 1) if m else 0
+        if k > 0:
+            graph[s:s + m, :k] = O.bruteforce_knn(rows[s:s + m], rows[s:s + m], k, exclude_self=True)[0]
+    graph[rng.random(graph.shape) < 0.1] = INV
+    start_points = np.array([max(n // 3 - 1, 0), 0, 1 << 30], np.uint32)
+    d, d_rough = packed(hip, rows)
+    head = d_rough.numpy()[:8]
+    unit = np.float64(2.0) ** (max(int(head[:4].view(np.uint32)[0] >> 23), 14) - 127 - 13)
+    d_counts = hip.DeviceArray(4, np.uint32)
+    hip.survey_rough_rows(d, d_rough, n, dim, hip.DeviceArray.from_numpy(graph), degree, hip.DeviceArray.from_numpy(starts),
+                          hip.DeviceArray.from_numpy(lengths), 3, hip.DeviceArray.from_numpy(start_points), d_counts)
+    got, expect = [int(v) for v in d_counts.numpy()], survey(rows, float(head[4:].view(np.float32)[0]), np.sqrt(dim) * 3 * 6.2e-5 * unit, graph, starts, lengths, start_points)
+    # a comparison of two sums of squares can go the other way where they agree to (dim + 8) 2^-24: less than one in ten thousand here
+    assert got[2] == expect[2] and all(abs(g - e) <= 2 + 1e-3 * expect[0] for g, e in zip(got, expect)), (got, expect)
+
+
+@pytest.mark.parametrize("metric,degree,knn_degree", [(0, 32, 32), (1, 32, 32), (0, 32, 72)])
+@pytest.mark.parametrize("kind", ["plain", "dense", "apart"])
+def test_a_copy_that_tells_nothing_is_not_used(hip, monkeypatch, kind, metric, degree, knn_degree):
+    """Clusters so dense that rounding blurs them, and clusters so far apart that searches end in the wrong one: the builds do without the
+    copy.  Rows of low intrinsic dimension: they take it.  (72 neighbours a row: the sub-graphs never take it, refinement decides by itself.)"""
+    from glide_amd import index as G
+    rng = np.random.default_rng(8)
+    n, dim = 6000, 96
+    if kind == "plain":
+        rows = rng.standard_normal((n, 6)) @ rng.standard_normal((6, dim)) + rng.standard_normal((n, dim)) * 0.1
+    else:
+        rows = rng.random((12, dim))[rng.integers(0, 12, n)] * 160 + rng.standard_normal((n, dim)) * (0.05 if kind == "dense" else 8)
+    rows = rows.astype(np.float32)
+    taken, graphs = [], []
+    for name in ("build_subgraph", "build_boundary", "refine"):
+        def spy(*args, call=getattr(hip, name), **kw):
+            taken.append(kw["rough_rows"] is not None)
+            return call(*args, **kw)
+        monkeypatch.setattr(hip, name, spy)
+    for pays in (True, False):
+        monkeypatch.setattr(G, "rough_rows_pay", lambda num, dim, pays=pays: pays)
+        d = hip.DeviceArray.from_numpy(rows)
+        d_reorder, d_map, starts, lengths, d_c = G.preprocess(G.PartitionParameter(centroid_num=3, boundary_factor=1.04, sample_factor=0.5, metric=metric), d)
+        d_knn = G.build_nnd(G.NNDescentParameter(graph_degree=knn_degree, max_iterations=8), d_reorder, starts, lengths)
+        index = G.GLIDE(degree, d, d_c, metric)
+        index.build(G.IndexParameter(graph_degree=degree, knn_degree=knn_degree, relaxant_factor=1.05, metric=metric),
+                    G.make_search_parameter(64, knn_degree), G.make_search_parameter(128, knn_degree), d_knn, starts, lengths, d_map, d_reorder)
+        graphs.append(index.d_graph.numpy())
+        if pays:
+            assert taken[-1] == (kind == "plain") and not any(taken[:-1]) == (kind != "plain" or knn_degree > 64), taken
+        else:
+            assert not any(taken)
+        taken.clear()
+    assert np.array_equal(*graphs)
