@@ -81,28 +81,41 @@ __global__ __launch_bounds__(64) void select_segments_kernel(SelectArgs a) {
 
 // Queries grouped by the partitions they selected: counts, then offsets, then the lists.  With them a partition's
 // search launches one wavefront per query that wants it instead of one per query of the batch.
-// RowProbe: workgroups behind the counting ones look whether the first rows are of bytes (a launch of its own for that cost
-// rows of fractions 3 % of a small batch).
+// RowProbe: workgroups behind the counting ones look whether the first rows are of bytes, others how many of the first queries
+// are not (a launch of its own for that cost rows of fractions 3 % of a small batch).
 struct RowProbe {
-    const float* rows;      // null: nothing to look at
-    uint32_t num, dim, lanes;
-    uint32_t* other;        // set if some value is no whole number 0 .. 255
+    const float *rows, *queries;   // null: nothing to look at
+    uint32_t num, query_num, dim, lanes;   // lanes: pieces of 16 values a row
+    uint32_t *other, *queries_other;       // set if some value of the rows is no whole number 0 .. 255; queries with such a value
+    __host__ __device__ uint32_t queries_seen() const { return query_num < kProbeBlocks * 256 / lanes ? query_num : kProbeBlocks * 256 / lanes; }
+    static constexpr uint32_t kProbeBlocks = 64;   // of each kind
 };
-constexpr uint32_t kProbeBlocks = 64;
 __global__ __launch_bounds__(256) void group_count_kernel(const uint32_t* segment_ids, uint32_t total, uint32_t centroid_num, uint32_t* counts, RowProbe probe) {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x, counting = ceil_div(total, 256);
     if (blockIdx.x >= counting) {
-        const uint32_t piece = i - counting * 256, row = piece / probe.lanes;
+        const bool of_queries = blockIdx.x - counting >= RowProbe::kProbeBlocks;
+        const uint32_t piece = i - counting * 256 - (of_queries ? RowProbe::kProbeBlocks * 256 : 0), row = piece / probe.lanes;
+        const float* from = of_queries ? probe.queries : probe.rows;
         uint4 unused;
-        const bool exact = row >= probe.num || pack_bytes(probe.rows + static_cast<size_t>(row) * probe.dim, 16 * (piece % probe.lanes), probe.dim, unused);
-        if (ballot(!exact) != 0 && lane_id() == 0) *probe.other = 1u;
+        const bool exact = row >= (of_queries ? probe.query_num : probe.num) ||
+                           pack_bytes(from + static_cast<size_t>(row) * probe.dim, 16 * (piece % probe.lanes), probe.dim, unused);
+        const uint64_t others = ballot(!exact);
+        if (others == 0) return;
+        if (!of_queries) {
+            if (lane_id() == 0) *probe.other = 1u;
+            return;
+        }
+        const uint32_t t = piece % probe.lanes;   // 8 or 16 lanes a query
+        const uint64_t mine = others >> (lane_id() - t) & ((1ull << probe.lanes) - 1);
+        const uint64_t queries = ballot(t == 0 && mine != 0);
+        if (lane_id() == 0) atomicAdd(probe.queries_other, static_cast<uint32_t>(__popcll(queries)));
         return;
     }
     if (i >= total) return;
     const uint32_t s = segment_ids[i];
     if (s < centroid_num) atomicAdd(&counts[s], 1u);
 }
-// other: nullable, passed on behind the offsets, so that both are read back together
+// other: nullable, what the probes have found (two words), passed on behind the offsets, so that all are read back together
 __global__ __launch_bounds__(256) void group_scan_kernel(uint32_t* counts, uint32_t centroid_num, uint32_t* offsets, uint32_t* cursor, const uint32_t* other) {
     if (threadIdx.x == 0) {
         uint32_t run = 0;
@@ -112,7 +125,10 @@ __global__ __launch_bounds__(256) void group_scan_kernel(uint32_t* counts, uint3
             run += counts[s];
         }
         offsets[centroid_num] = run;
-        if (other) offsets[centroid_num + 1] = *other;
+        if (other) {
+            offsets[centroid_num + 1] = other[0];
+            offsets[centroid_num + 2] = other[1];
+        }
     }
 }
 __global__ __launch_bounds__(256) void group_fill_kernel(const uint32_t* segment_ids, uint32_t total, uint32_t centroid_num, uint32_t* cursor,
@@ -323,8 +339,8 @@ PartitionSearchLayout partition_search_layout(uint32_t query_num, uint32_t centr
     const size_t pairs = static_cast<size_t>(query_num) * centroid_num;   // every query could select every partition
     size_t off = 0;
     auto take = [&off](size_t bytes) { size_t o = off; off += align256(bytes); return o; };
-    l.counts = take((static_cast<size_t>(centroid_num) + 1) * 4);    // the last word: whether some row is not of bytes
-    l.offsets = take((static_cast<size_t>(centroid_num) + 2) * 4);   // and here as well
+    l.counts = take((static_cast<size_t>(centroid_num) + 2) * 4);    // the last words: whether some row is not of bytes, how many queries are not
+    l.offsets = take((static_cast<size_t>(centroid_num) + 3) * 4);   // and here as well
     l.cursor = take(static_cast<size_t>(centroid_num) * 4);
     l.lists = take(pairs * 4);
     l.pair_segment = take(pairs * 4);
@@ -344,7 +360,9 @@ extern "C" size_t glide_hip_search_partitions_workspace_bytes(uint32_t query_num
 // once to write a quarter is what they save many times over (fp32 : bytes, packing included, on 128 dims: 5 000 queries over
 // 500 000 rows, three partitions each, beam 96 2 284 : 1 262 us; over 200 000 rows 1 963 : 1 075, mixture rows, which come from
 // the caches, 1 072 : 900; at the line, 1 000 queries, 622 : 563 and 538 : 493).  Every query selects a partition at least, as a
-// rule two or three; half of an expansion's rows are new.
+// rule two or three; half of an expansion's rows are new.  Not where most of the first queries (1 024 or 2 048) are of fractions:
+// those search the fp32 rows, for them packing is for nothing (5 000 queries at beam 96 over 500 000 rows 2 288 : 2 362 us, 2 000 over
+// 200 000 of 256 dims 1 309 : 1 459).
 static bool partitions_as_bytes_pay(uint32_t num, uint32_t dim, uint32_t degree, uint32_t query_num, uint32_t beam) {
     return num != 0 && degree <= kMostByteDegree && glide_hip_byte_rows_bytes(num, dim) != 0 &&
            static_cast<unsigned long long>(query_num) * beam * degree / 2 >= 4ull * num;
@@ -385,7 +403,7 @@ extern "C" int glide_hip_search_partitions_rows(const float* data, uint32_t num,
     if (workspace_bytes < glide_hip_search_partitions_rows_workspace_bytes(query_num, segment_num, top_k, num, dim, graph_degree, beam))
         return GLIDE_ERR_BAD_ARGUMENT;
     const bool may_be_bytes = partitions_as_bytes_pay(num, dim, graph_degree, query_num, beam) && reinterpret_cast<uintptr_t>(data) % 16 == 0;
-    if ( reinterpret_cast<uintptr_t>(workspace) % (may_be_bytes ? 16 : 8)) return GLIDE_ERR_BAD_ARGUMENT;
+    if (reinterpret_cast<uintptr_t>(workspace) % (may_be_bytes ? 16 : 8)) return GLIDE_ERR_BAD_ARGUMENT;
     hipStream_t s = as_stream(stream);
     unsigned char* w = static_cast<unsigned char*>(workspace);
     unsigned char* byte_rows = w + l.total;
@@ -398,17 +416,17 @@ extern "C" int glide_hip_search_partitions_rows(const float* data, uint32_t num,
     float* pair_dists = reinterpret_cast<float*>(w + l.pair_dists);
     uint32_t* pair_ids = reinterpret_cast<uint32_t*>(w + l.pair_ids);
     uint32_t* other = counts + segment_num;
-    int rc = glide_hip_fill_u32(counts, 0u, static_cast<size_t>(segment_num) + 1, stream);
+    int rc = glide_hip_fill_u32(counts, 0u, static_cast<size_t>(segment_num) + 2, stream);
     if (rc != GLIDE_OK) return rc;
     const uint32_t total = query_num * segment_num;
-    const RowProbe probe{data, num, dim, static_cast<uint32_t>(dim <= 128 ? RowShape<-1>::LPR : RowShape<-2>::LPR), other};
-    hipLaunchKernelGGL(group_count_kernel, dim3(ceil_div(total, 256) + (may_be_bytes ? kProbeBlocks : 0u)), dim3(256), 0, s, segment_ids, total, segment_num,
-                       counts, probe);
+    const RowProbe probe{data, queries, num, query_num, dim, static_cast<uint32_t>(dim <= 128 ? RowShape<-1>::LPR : RowShape<-2>::LPR), other, other + 1};
+    hipLaunchKernelGGL(group_count_kernel, dim3(ceil_div(total, 256) + (may_be_bytes ? 2 * RowProbe::kProbeBlocks : 0u)), dim3(256), 0, s, segment_ids, total,
+                       segment_num, counts, probe);
     hipLaunchKernelGGL(group_scan_kernel, dim3(1), dim3(256), 0, s, counts, segment_num, offsets, cursor, other);
     hipLaunchKernelGGL(group_fill_kernel, dim3(ceil_div(total, 256)), dim3(256), 0, s, segment_ids, total, segment_num, cursor, lists, pair_segment,
                        pair_index);
-    uint32_t back[2] = {0, 1};
-    GLIDE_HIP_TRY(hipMemcpyAsync(back, offsets + segment_num, (may_be_bytes ? 2 : 1) * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    uint32_t back[3] = {0, 1, 0};
+    GLIDE_HIP_TRY(hipMemcpyAsync(back, offsets + segment_num, (may_be_bytes ? 3 : 1) * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     GLIDE_HIP_TRY(hipStreamSynchronize(s));
     const uint32_t pairs = back[0];   // the grid of the search: one wavefront per (query, selected partition)
     if (pairs) {
@@ -443,7 +461,7 @@ extern "C" int glide_hip_search_partitions_rows(const float* data, uint32_t num,
             hipLaunchKernelGGL(fn, dim3(pairs), dim3(64), lds_bytes, s, a);
             return GLIDE_OK;
         };
-        if (back[1] == 0) {   // the rows that were looked at are of bytes; if others are not, every pair is left over
+        if (back[1] == 0 && 2 * back[2] <= probe.queries_seen()) {   // the rows that were looked at are of bytes; if others are not, every pair is left over
             if ((rc = glide_hip_pack_byte_rows(data, num, dim, byte_rows, other, stream)) != GLIDE_OK) return rc;
             a.bytes = byte_rows;
             a.other = other;

@@ -404,7 +404,8 @@ int glide_hip_search_partitions(const float *data, uint32_t dim, const uint32_t 
                                 uint32_t hash_reset_interval, int metric, uint32_t *final_ids, float *final_dists,
                                 void *workspace, size_t workspace_bytes, unsigned long long *counters, void *stream);
 /* The same with the number of rows in `data`, so that rows of bytes can be searched as bytes (see glide_hip_pack_byte_rows;
- * they are packed into the workspace on each call, where the batch is large enough to gain by it).  Same results.
+ * they are packed into the workspace on each call, where the batch is large enough to gain by it and at least half of its
+ * first queries are of bytes too).  Same results.
  * workspace: glide_hip_search_partitions_rows_workspace_bytes(), 16-byte aligned. */
 size_t glide_hip_search_partitions_rows_workspace_bytes(uint32_t query_num, uint32_t centroid_num, uint32_t top_k,
                                                         uint32_t num, uint32_t dim, uint32_t graph_degree,

@@ -254,3 +254,35 @@ def test_partitions_without_room_for_the_bytes(hip, monkeypatch):
     monkeypatch.setattr(hip.DeviceArray, "__init__", short)
     got = search()
     assert len(refused) == 1 and all(np.array_equal(a, b) for a, b in zip(expect, got))
+
+
+@pytest.mark.parametrize("dim,nq,fractions,packs", [(64, 120, 0.0, True), (128, 200, 0.45, True), (128, 200, 0.55, False), (160, 130, 1.0, False), (256, 1300, 0.4, True),
+                                                    (100, 2500, 0.6, False), (4, 300, 1.0, False)])
+def test_partitions_for_queries_of_fractions(hip, dim, nq, fractions, packs):
+    """Rows are packed for queries that search them: not where most of the first queries have other values.  Same results either way."""
+    import ctypes as C
+    from oracle import oracle as O
+    rng = np.random.default_rng(nq)
+    n, degree, top_k = 1500, 32, 10
+    rows, queries = rows_of(rng, n, dim), rows_of(rng, nq, dim)
+    queries[rng.permutation(nq)[:round(fractions * nq)], rng.integers(dim)] += 0.5
+    graph = O.bruteforce_knn(rows, rows, degree, exclude_self=True)[0]
+    up = hip.DeviceArray.from_numpy
+    sp, d, d_q = O.search_params(64, degree), up(rows), up(queries)
+    rest = up(graph), up(rng.permutation(n).astype(np.uint32)), up(np.zeros(1, np.uint32)), up(np.array([5], np.uint32)), up(np.zeros((nq, 1), np.uint32))
+    u32 = C.c_uint32
+    plain = hip._size_fn("glide_hip_search_partitions_workspace_bytes")(u32(nq), u32(1), u32(top_k))
+    got = []
+    for num in (0, n):
+        size = hip._size_fn("glide_hip_search_partitions_rows_workspace_bytes")(u32(nq), u32(1), u32(top_k), u32(num), u32(dim), u32(degree), u32(sp["beam"]))
+        assert (size > plain) == (num > 0)
+        ws = hip.DeviceArray.full(size // 4, 0xA5A5A5A5)
+        ids, dists, cnt = hip.DeviceArray((nq, top_k), np.uint32), hip.DeviceArray((nq, top_k), np.float32), hip.new_counters()
+        hip.check(hip.lib().glide_hip_search_partitions_rows(
+            *(hip._ptr(v) if not isinstance(v, int) else u32(v) for v in (d, num, dim, rest[0], degree, *rest[1:4], 1, d_q, nq, rest[4], top_k, sp["beam"],
+              sp["max_iterations"], sp["min_iterations"], sp["hash_bit"], sp["hash_reset_interval"])), C.c_int(0), hip._ptr(ids), hip._ptr(dists), hip._ptr(ws),
+            C.c_size_t(size), hip._ptr(cnt), None), "search")
+        hip.synchronize()
+        got.append((ids.numpy(), dists.numpy(), hip.read_counters(cnt)))
+    assert all(np.array_equal(a, b) for a, b in zip(got[0], got[1]))
+    assert (ws.numpy()[plain // 4:] != 0xA5A5A5A5).any() == packs
