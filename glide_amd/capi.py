@@ -209,6 +209,10 @@ def distance_batch(a, b, n, dim, metric, out, stream=None):
           "glide_hip_distance_batch")
 
 
+def byte_distances(first, n, metric, out, stream=None):
+    check(lib().glide_hip_byte_distances(u32(first), u32(n), C.c_int(metric), _out(out), vp(stream)), "glide_hip_byte_distances")
+
+
 def bitonic_sort_kv(keys, vals, m, batch, stream=None):
     check(lib().glide_hip_bitonic_sort_kv(_out(keys), _out(vals), u32(m), u32(batch), vp(stream)),
           "glide_hip_bitonic_sort_kv")

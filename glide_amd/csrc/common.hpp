@@ -367,7 +367,8 @@ __device__ __forceinline__ float finish_distance(float sq, int metric) { return 
 // The same for a whole number below 2^24, the squared distance of rows of bytes: sqrtf without the scaling it needs for very
 // small arguments and without the cases of infinity and NaN, half of its fourteen instructions.  The hardware root is off by
 // one place at most; with neighbours l and h of it, l * root >= sq says that it is too large, h * root < sq that it is too small
-// (both exact in the sign of one rounded multiply-add).
+// (both exact in the sign of one rounded multiply-add): Tuckerman's test, from Agarwal, Cooley, Gustavson, Shearer, Slishman and
+// Tuckerman, "New scalar and vector elementary functions for the IBM System/370", IBM J. Res. Dev. 30 (1986) 126.
 __device__ __forceinline__ float finish_byte_distance(float sq, int metric) {
     if (metric != kEuclidean) return sq;
     const float root = __builtin_amdgcn_sqrtf(sq);

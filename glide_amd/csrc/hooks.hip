@@ -45,6 +45,12 @@ __global__ __launch_bounds__(64) void distance_batch_kernel(const float* a, cons
     if (i < n && t == 0) out[i] = d;
 }
 
+// out[i]: what searches over rows of bytes report for the squared distance first + i
+__global__ __launch_bounds__(256) void byte_distance_kernel(uint32_t first, uint32_t n, int metric, float* out) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) out[i] = finish_byte_distance(static_cast<float>(first + i), metric);
+}
+
 template <int M, bool MERGE_ONLY>
 __global__ __launch_bounds__(64) void bitonic_kernel(float* keys, uint32_t* vals, uint32_t batch) {
     constexpr int NR = WaveNet<M>::NR;
@@ -121,6 +127,14 @@ int launch_bitonic(float* keys, uint32_t* vals, uint32_t m, uint32_t batch, hipS
 using namespace glide;
 
 extern "C" {
+
+int glide_hip_byte_distances(uint32_t first, uint32_t n, int metric, float* out, void* stream) {
+    if (!out) return GLIDE_ERR_BAD_ARGUMENT;
+    if (first >= (1u << 24) || n > (1u << 24) - first) return GLIDE_ERR_UNSUPPORTED;
+    if (n == 0) return GLIDE_OK;
+    hipLaunchKernelGGL(byte_distance_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, as_stream(stream), first, n, metric, out);
+    return launch_status();
+}
 
 int glide_hip_distance_batch(const float* a, const float* b, uint32_t n, uint32_t dim, int metric, float* out, void* stream) {
     if (!a || !b || !out || dim == 0) return GLIDE_ERR_BAD_ARGUMENT;

@@ -66,7 +66,8 @@ int launch_search(const float* data, const unsigned char* bytes, uint32_t num, u
     a.p.metric = metric;
 
     // Rows of bytes: a first launch takes the queries that are of bytes themselves and marks the others, which a second one
-    // searches on the fp32 rows (on a batch without any it costs 3 us).
+    // searches on the fp32 rows (on a batch without any it costs 3 us).  A batch of fractions pays for the first one: on a million rows of
+    // 128 values, with it and without, 1 query at beam 32 85 : 83 us, 60 queries 112 : 109, 10 000 at beam 64 1 325 : 1 318.
     if (bytes && graph_degree <= kMostByteDegree && dim <= kMostByteDims) {
         if (reinterpret_cast<uintptr_t>(bytes) % 16) return GLIDE_ERR_BAD_ARGUMENT;
         a.bytes = bytes;

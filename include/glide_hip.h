@@ -506,6 +506,8 @@ int glide_hip_copy_rows(const float *src, uint64_t num, uint32_t src_dim, float 
 /* compute_similarity_warp (distance.cuh:9-27): out[i] = dist(a[i], b[i]) for n row pairs */
 int glide_hip_distance_batch(const float *a, const float *b, uint32_t n, uint32_t dim, int metric, float *out,
                              void *stream);
+/* the distance that a search over rows of bytes reports for the squared distance first + i, a whole number below 2^24 */
+int glide_hip_byte_distances(uint32_t first, uint32_t n, int metric, float *out, void *stream);
 /* bitonic::warp_sort (bitonic.cuh:207-212): each of `batch` arrays of m (32..512, power of two) pairs is
  * sorted by one wavefront; arrays are in network element order */
 int glide_hip_bitonic_sort_kv(float *keys, uint32_t *vals, uint32_t m, uint32_t batch, void *stream);

@@ -286,3 +286,24 @@ def test_partitions_for_queries_of_fractions(hip, dim, nq, fractions, packs):
         got.append((ids.numpy(), dists.numpy(), hip.read_counters(cnt)))
     assert all(np.array_equal(a, b) for a, b in zip(got[0], got[1]))
     assert (ws.numpy()[plain // 4:] != 0xA5A5A5A5).any() == packs
+
+
+def test_every_distance(hip):
+    """Rows of bytes have whole squared distances below 2^24: the root of every one of them, correctly rounded (as the fp32 kernels'
+    sqrtf and numpy's are), and the number itself for the cosine metric."""
+    n = 1 << 24
+    out, whole = hip.DeviceArray(n, np.float32), np.arange(n, dtype=np.float32)
+    for metric, expect in ((0, np.sqrt(whole)), (1, whole)):
+        hip.byte_distances(0, n, metric, out)
+        hip.synchronize()
+        assert np.array_equal(out.numpy(), expect)
+    some = np.random.default_rng(1).integers(0, 4096, 4096)
+    rows = np.zeros((4096, 4), np.float32)      # and the fp32 kernels' own distances, of some
+    rows[:, 0] = some
+    dists = hip.DeviceArray(4096, np.float32)
+    hip.distance_batch(hip.DeviceArray.from_numpy(rows), hip.DeviceArray.from_numpy(np.zeros_like(rows)), 4096, 4, 0, dists)
+    hip.byte_distances(0, n, 0, out)
+    hip.synchronize()
+    assert np.array_equal(dists.numpy(), out.numpy()[some * some])
+    with pytest.raises(hip.GlideHipError):
+        hip.byte_distances(1, n, 0, out)
