@@ -105,15 +105,16 @@ def measured_knn(workload):
     return None
 
 
-def search_kernel_name(dim, degree, beam, queries, compute_units):
-    """The kernel glide_hip_search launches for this shape, as a profiler names it (search.hip: launch_search)."""
-    shape = "%d,%d,%d" % (64 if degree <= 64 else 128 if degree <= 128 else 256,
-                          64 if beam <= 64 else 128 if beam <= 128 else 256 if beam <= 256 else 512,
-                          1 if dim <= 128 else 2 if dim <= 256 else 4 if dim <= 512 else 8 if dim <= 1024 else 16)
+def search_kernel_name(dim, degree, beam, queries, compute_units, of_bytes=False):
+    """The kernel glide_hip_search launches for this shape, as a profiler names it (search.hip: launch_search).  of_bytes: rows and
+    queries are whole numbers 0..255 and searched as bytes (a second launch finds no query left over)."""
+    shape = "%d, %d, %d" % (64 if degree <= 64 else 128 if degree <= 128 else 256,
+                            64 if beam <= 64 else 128 if beam <= 128 else 256 if beam <= 256 else 512,
+                            (-1 if dim <= 128 else -2) if of_bytes else 1 if dim <= 128 else 2 if dim <= 256 else 4 if dim <= 512 else 8 if dim <= 1024 else 16)
     whole = "true" if beam == 512 else "false"      # the whole of the widest beam: merged in the registers
     if dim > 256 and queries * 4 <= 2 * 4 * compute_units:
-        return "search_team_kernel<%s,%s>" % (shape, whole)
-    return "search_kernel<%s,%s>" % (shape, whole)
+        return "search_team_kernel<%s, %s>" % (shape, whole)
+    return "search_kernel<%s, %s, false>" % (shape, whole)
 
 
 def measured_knn_bytes(workload):
@@ -258,6 +259,8 @@ def run_workload(args, workload, torch, want_cpu):
     index.build(bp, sp_knn, sp_ref, d_knn, h_start, h_len, d_map, d_re, res, counters=True)
     build_sec = res["pre_time"] + res["knn_time"] + res["index_time"] + res["refine_time"]
     graph = index.d_graph.numpy()
+    d_bytes = index._byte_rows()       # rows of whole numbers 0..255 are searched as bytes, with the same ids and distances
+    row_bytes = capi.byte_rows_bytes(1, dim) if d_bytes is not None else dim * 4
     holes = float((graph == 0xFFFFFFFF).mean())
 
     # ---- search sweep
@@ -275,8 +278,8 @@ def run_workload(args, workload, torch, want_cpu):
         r = {}
         index.search(sp, d_q, result=r, out=(d_ids, d_dists))
         rec = D.recall(d_ids.numpy(), gt, top_k)
-        # algorithmic bytes of one launch: query rows + centroid table once + graph rows + scored data rows + results
-        alg = nq * dim * 4 + parts * dim * 4 + int(c[2]) * degree * 4 + int(c[1]) * dim * 4 + nq * top_k * 8
+        # algorithmic bytes of one launch: query rows + centroid table once + graph rows + scored data rows (as they are read) + results
+        alg = nq * dim * 4 + parts * dim * 4 + int(c[2]) * degree * 4 + int(c[1]) * row_bytes + nq * top_k * 8
         sweep.append(dict(beam=beam, recall_at_10=rec, qps=r["QPS"], ms=r["search_time"] * 1e3, iterations_per_query=c[0] / nq,
                           rows_per_query=c[1] / nq, algorithmic_bytes=alg))
         return rec
@@ -309,7 +312,7 @@ def run_workload(args, workload, torch, want_cpu):
     e0.record()
     for _ in range(args.steps):
         capi.search(index.d_data, num, dim, index.d_graph, degree, index.d_centroids, parts, index.d_start_points, d_q, nq, top_k,
-                    sp.beam, sp.max_iterations, sp.min_iterations, sp.hash_bit, sp.hash_reset_interval, metric, d_ids, d_dists)
+                    sp.beam, sp.max_iterations, sp.min_iterations, sp.hash_bit, sp.hash_reset_interval, metric, d_ids, d_dists, byte_rows=d_bytes)
     e1.record()
     gpu_ms = e0.elapsed_ms(e1)
     capi.synchronize()
@@ -347,6 +350,9 @@ def run_workload(args, workload, torch, want_cpu):
             out.update(achieved=None, frac=None, note="no counters committed for this stage on this workload")
         return out
 
+    # a row as the kernels of a stage read it; looked at in fp16 first: without the few that are then read in fp32 as well
+    read = {k: {"bytes": row_bytes, "fp16 first": dim * 2, "fp32": dim * 4}[v] for k, v in res["rows_read"].items()}
+
     stage_rooflines = {}
     assign_flops = 2.0 * num * parts * dim
     a = hbm_stage(det["assign"], num * dim * 4 + num * 12)
@@ -376,16 +382,16 @@ def run_workload(args, workload, torch, want_cpu):
     if "build_counters" in res:
         _, rows, grows = res["build_counters"]
         stage_rooflines["subgraph+boundary"] = graph_stage(det["subgraph"] + det["boundary"],
-                                                           reorder_rows * dim * 4 + grows * knn_degree * 4 + rows * dim * 4 + reorder_rows * degree * 4,
+                                                           reorder_rows * dim * 4 + grows * knn_degree * 4 + rows * read["subgraph"] + reorder_rows * degree * 4,
                                                            "subgraph+boundary")
     if "refine_counters" in res:
         _, rows, grows = res["refine_counters"]
-        stage_rooflines["refine"] = graph_stage(det["refine"], num * dim * 4 + 2 * num * degree * 4 + grows * degree * 4 + rows * dim * 4, "refine")
+        stage_rooflines["refine"] = graph_stage(det["refine"], num * dim * 4 + 2 * num * degree * 4 + grows * degree * 4 + rows * read["refine"], "refine")
 
     bound = D.reachable_recall_bound(graph, d_cent.numpy(), index.d_start_points.numpy(), queries, gt, metric)
 
     out = dict(
-        workload=desc, gen_sec=gen_s, build_sec=build_sec, stage_rooflines=stage_rooflines,
+        workload=desc, rows_read=dict(res["rows_read"], search="bytes" if d_bytes is not None else "fp32"), gen_sec=gen_s, build_sec=build_sec, stage_rooflines=stage_rooflines,
         build_stages=dict(pre=res["pre_time"], knn=res["knn_time"], index=res["index_time"], refine=res["refine_time"],
                           detail={**res["pre_stages"], **res["build_stages"]}),
         nnd_iterations=nnd_iters, nnd_offers=res["nnd_stats"][0], nnd_offers_declined_by_threshold=res["nnd_stats"][1],
@@ -398,11 +404,11 @@ def run_workload(args, workload, torch, want_cpu):
         roofline=dict(bound="hbm", achieved=achieved, peak=HBM_PEAK_GBS, unit="GB/s", frac=achieved / HBM_PEAK_GBS,
                       traffic=(measured_traffic(workload, chosen["beam"]) or {}).get("bytes"),
                       traffic_source=(measured_traffic(workload, chosen["beam"]) or {}).get("source"),
-                      kernel=search_kernel_name(dim, degree, chosen["beam"], nq, info_cus),
+                      kernel=search_kernel_name(dim, degree, chosen["beam"], nq, info_cus, d_bytes is not None),
                       algorithmic_bytes_per_launch=chosen["algorithmic_bytes"]),
     )
     # what scattered rows of this length can be read at on this GPU at all (a probe kernel that only gathers rows)
-    ceiling = scattered_row_ceiling(dim * 4)
+    ceiling = scattered_row_ceiling(row_bytes)
     if ceiling:
         out["roofline"].update(scattered_row_ceiling_GBps=ceiling["GBps"], scattered_row_ceiling_frac=ceiling["GBps"] / HBM_PEAK_GBS,
                                scattered_row_ceiling_source=ceiling["source"])
@@ -524,7 +530,9 @@ def main():
         out = capi.DeviceArray(4, np.float32)
         res = {}
         # (label, row bytes, row stride, rows per wave-wide step, table rows)
-        for label, row_bytes, stride, rps, rows in (("512-byte rows (128 dims), 8 lanes a row, 16 rows in flight per wavefront", 512, 512, 8, 1 << 20),
+        for label, row_bytes, stride, rps, rows in (("128-byte rows (up to 128 dims as bytes), 8 lanes a row, 16 rows in flight per wavefront", 128, 128, 8, 1 << 20),
+                                                    ("128-byte rows of a table of 4M, 8 lanes a row, 16 rows in flight per wavefront", 128, 128, 8, 1 << 22),
+                                                    ("512-byte rows (128 dims), 8 lanes a row, 16 rows in flight per wavefront", 512, 512, 8, 1 << 20),
                                                     ("3840-byte rows (960 dims), 32 lanes a row, 8 rows in flight per wavefront", 3840, 3840, 2, 1 << 20),
                                                     ("3840-byte rows (960 dims), 64 lanes a row, 8 rows in flight per wavefront", 3840, 3840, 1, 1 << 20),
                                                     ("3840-byte rows 4096 bytes apart, 32 lanes a row, 8 rows in flight per wavefront", 3840, 4096, 2, 1 << 20),
@@ -612,7 +620,7 @@ def main():
     print(json.dumps(headline(args, args.workload, details, info["name"], args.details_file), default=float), flush=True)
 
 
-DETAIL_KEYS = ("workload", "build_sec", "build_stages", "graph_recall_at_32", "graph_recall_at_32_global", "empty_slots_fraction", "beam",
+DETAIL_KEYS = ("workload", "rows_read", "build_sec", "build_stages", "graph_recall_at_32", "graph_recall_at_32_global", "empty_slots_fraction", "beam",
                "recall_at_10", "recall_target_met", "reachable_recall_bound", "reachable_fraction_of_points", "qps", "ms_per_step", "kernel_ms",
                "nnd_iterations", "nnd_offers", "nnd_offers_declined_by_threshold", "sweep", "stage_rooflines", "roofline", "cpu_baseline", "wall_sec")
 
@@ -643,7 +651,7 @@ def headline(args, workload, details, device, details_file="the details file"):
         "config": {"workload": r["workload"], "graph_degree": WORKLOADS[workload][8], "top_k": 10, "beam": r["beam"], "build_beam": 64,
                    "refine_beam": 128, "relaxant": 1.05, "boundary_factor": 1.04, "sample_factor": 0.01, "nnd_iterations": r["nnd_iterations"],
                    "nnd_termination_threshold": 1e-4},
-        "device": device, "beam": r["beam"], "recall_at_10": r3(r["recall_at_10"]), "recall_target_met": met,
+        "rows_read": r.get("rows_read"), "device": device, "beam": r["beam"], "recall_at_10": r3(r["recall_at_10"]), "recall_target_met": met,
         "reachable_recall_bound": r3(r["reachable_recall_bound"]),
         "qps_at_recall_target": r["qps"] if met else None, "qps_at_max_beam": None if met else r["qps"],
         "build_sec": r3(r["build_sec"]), "build_stages": {k: r3(v) for k, v in r["build_stages"].items() if k != "detail"},

@@ -243,6 +243,10 @@ def rough_rows_help(d_rows, d_rough, d_graph, d_starts, d_lengths, d_start_point
     return far > 0 and told >= 0.6 * far and 2 * astray < rows
 
 
+def _rows_read(d_bytes, d_rough):
+    return "bytes" if d_bytes is not None else "fp16 first" if d_rough is not None else "fp32"
+
+
 def draw_ids(num, count, seed, d_ids):
     """The first `count` entries of np.random.default_rng(seed).permutation(num) into a DeviceArray.  Returns the scratch of the
     device's draw (some 21 bytes a row; it may go once the draw is done), or None where the host has drawn: more rows than the
@@ -429,6 +433,7 @@ class GLIDE:
                 if not helps:
                     d_rough.free()
                     d_rough = None
+            rows_read = dict(subgraph=_rows_read(d_bytes, d_rough))
             capi.build_subgraph(d_reorder_data, num, dim, d_knn_graph, knn_degree, d_map, d_ss, d_sl, len(h_segment_start), d_rsp,
                                 deg, p.beam, p.max_iterations, p.min_iterations, p.hash_bit, p.hash_reset_interval,
                                 build_param.relaxant_factor, self.metric, self.d_graph, cnt, byte_rows=d_bytes, rough_rows=d_rough)
@@ -471,6 +476,7 @@ class GLIDE:
                 if d_rough is not None and helps is None and not rough_rows_help(self.d_data, d_rough, self.d_graph, *self._one_segment()):
                     d_rough.free()
                     d_rough = None
+                rows_read["refine"] = _rows_read(d_bytes, d_rough)
                 capi.refine(self.d_data, num, dim, self.d_graph, d_rev, deg, self.d_centroids, self.centroid_num(),
                             self.d_start_points, p.beam, p.max_iterations, p.min_iterations, p.hash_bit, p.hash_reset_interval,
                             build_param.relaxant_factor, self.metric, cnt2, order=d_map,
@@ -488,6 +494,7 @@ class GLIDE:
         d_rev.free()
         d_map.free()
         if result is not None:
+            result["rows_read"] = rows_read
             result["index_time"] = times["subgraph"] + times["boundary"] + times["reverse"]
             result["refine_time"] = times["refine"]
             result["build_stages"] = times
