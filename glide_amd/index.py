@@ -380,9 +380,10 @@ class GLIDE:
     def _byte_rows(self):
         """The rows as bytes, or None: there are none, or the rows may have been written since.  A search then reads the rows,
         and so do all that follow: the copy goes."""
-        if self._bytes is None:
+        held = self._bytes      # read once: another thread's search may let the copy go
+        if held is None:
             return None
-        d_bytes, made_from, writes = self._bytes
+        d_bytes, made_from, writes = held
         if made_from is self.d_data and writes == made_from.writes and not made_from.shared:
             return d_bytes
         self._bytes = None

@@ -107,3 +107,25 @@ def test_copies_that_only_save_time_never_fail_a_call(monkeypatch):
         plain = capi._size_fn("glide_hip_search_partitions_workspace_bytes")(64, 8, 10)
         size = capi._size_fn("glide_hip_search_partitions_rows_workspace_bytes")
         assert size(64, 8, 10, 100, dim, 32, 64) > plain and size(2 ** 31, 8, 10, most + 1, dim, 64, 512) == capi._size_fn("glide_hip_search_partitions_workspace_bytes")(2 ** 31, 8, 10)
+
+
+def test_a_search_beside_one_that_lets_the_byte_rows_go():
+    """Two threads search an index whose rows have become known to others: both find that the copy may not be used."""
+    class Rows:
+        writes, shared = 3, True
+
+    class Index(G.GLIDE):
+        reads = 0
+
+        @property
+        def _bytes(self):      # held when this thread looks, gone a moment later
+            self.reads += 1
+            return (object(), self.d_data, 3) if self.reads == 1 else None
+
+        @_bytes.setter
+        def _bytes(self, value):
+            assert value is None
+
+    index = Index.__new__(Index)
+    index.d_data = Rows()
+    assert index._byte_rows() is None
