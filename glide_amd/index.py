@@ -213,7 +213,10 @@ def rough_rows_pay(num, dim):
     """Whether a build over `num` rows of `dim` values gains from a copy of them in fp16: the first look saves memory traffic and
     costs instructions and a second round of loads for the rows it leaves open.  Short rows leave lanes idle and gain later.
     Build with against without, in ms: 20 000 x 384 10.0 : 13.6, 20 000 x 200 7.5 : 7.8, 5 000 x 300 3.8 : 3.7; 120 000 x 128
-    28.8 : 30.9, 70 000 x 128 17.4 : 17.2; 1 000 000 x 96 257 : 304, 234 567 x 96 56 : 53, 1 000 000 x 64 236 : 212."""
+    28.8 : 30.9, 70 000 x 128 17.4 : 17.2; 1 000 000 x 96 257 : 304, 234 567 x 96 56 : 53, 1 000 000 x 64 236 : 212.
+    Sub-graphs to refinement alone: unit rows 200 000 x 112 34 : 46, 300 000 x 96 49 : 59, 600 000 x 96 100 : 138, 120 000 x 128 19 : 25;
+    Beta-like rows, which share more of what they read, 200 000 x 112 42 : 43, 300 000 x 96 60 : 56, 700 000 x 96 145 : 156, 120 000 x 128
+    23 : 22: the lines lie where neither loses."""
     return dim > 64 and 4 * num * dim >= (16 << 20 if dim >= 192 else 64 << 20 if dim >= 112 else 256 << 20)
 
 
