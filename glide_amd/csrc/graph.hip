@@ -195,12 +195,13 @@ __global__ __launch_bounds__(256) void rough_pack_kernel(const float* rows, uint
     if (threadIdx.x == 0) atomicMax(turn_bits, __float_as_uint(fmaxf(fmaxf(of_wave[0], of_wave[1]), fmaxf(of_wave[2], of_wave[3]))));
 }
 
-// Whether a first look in fp16 will settle anything, from some rows and the graph that their searches will go through; one
-// wavefront a row.  counts[0] / counts[1]: neighbours of a neighbour that are farther than the row's own farthest one, and how many
-// of them the look's bounds would tell to be so.  counts[2] / counts[3]: rows, and those that a greedy walk from their segment's
-// start ends one and a half times that far from, or more: searches that do not get to where they should stay among few rows, the caches
-// serve those, and the look has no traffic to save.  One wavefront's round trips: with the counts read back 70 us on rows of 128
-// values, 90 on 256, 110 on 512, 190 on 960 at degree 64 (builds of 40, 50, 35 and 158 ms).
+// Whether a first look in fp16 will settle anything, from some rows and the graph that their searches will go through; four
+// wavefronts a row, which have all rows of a list under way at once.  counts[0] / counts[1]: neighbours of a neighbour that are
+// farther than the row's own farthest one, and how many of them the look's bounds would tell to be so.  counts[2] / counts[3]: rows,
+// and those that a greedy walk from their segment's start ends one and a half times that far from, or more: searches that do not get to
+// where they should stay among few rows, the caches serve those, and the look has no traffic to save.  A chain of two round trips a
+// list: with the counts read back 50 to 60 us on rows of 128 to 512 values, 72 on 960 (one wavefront a row, 512 rows and all of up to 64
+// neighbours: 70 to 110, and 190 at degree 64; 1.3 % of a build of 13 000 x 512).
 struct SurveyArgs {
     const float* rows;
     const unsigned char* rough;
@@ -208,12 +209,13 @@ struct SurveyArgs {
     uint32_t num, dim, degree, segment_num;
     uint32_t* counts;
 };
-constexpr uint32_t kSurveyed = 512, kMostHops = 64;
+constexpr uint32_t kSurveyed = 256, kSurveyWaves = 4, kSurveyDegree = 32, kMostHops = 64;
 template <int DIMV>
-__global__ __launch_bounds__(64) void rough_survey_kernel(SurveyArgs a) {
-    __shared__ uint32_t own[64], list[64];
-    __shared__ float sq[64];
+__global__ __launch_bounds__(64 * kSurveyWaves) void rough_survey_kernel(SurveyArgs a) {
+    __shared__ uint32_t own[kSurveyDegree], list[kSurveyDegree];
+    __shared__ float sq[kSurveyDegree];
     const int lane = lane_id();
+    const uint32_t wave = threadIdx.x >> 6;
     const uint32_t row = static_cast<uint32_t>(static_cast<unsigned long long>(blockIdx.x) * a.num / gridDim.x);
     uint32_t seg = kInvalid;
     for (uint32_t s0 = 0; s0 < a.segment_num && seg == kInvalid; s0 += 64) {
@@ -222,7 +224,7 @@ __global__ __launch_bounds__(64) void rough_survey_kernel(SurveyArgs a) {
         if (m != 0) seg = s0 + __builtin_ctzll(m);
     }
     if (seg == kInvalid) return;
-    const uint32_t first = a.starts[seg], length = a.lengths[seg], self = row - first, degree = a.degree < 64 ? a.degree : 64;
+    const uint32_t first = a.starts[seg], length = a.lengths[seg], self = row - first, degree = a.degree < kSurveyDegree ? a.degree : kSurveyDegree;
     const float* data = a.rows + static_cast<size_t>(first) * a.dim;
     RowRegs<DIMV> q;
     load_row<DIMV>(q, a.rows + static_cast<size_t>(row) * a.dim, a.dim, RowShape<DIMV>::lane_in_row(lane));
@@ -230,16 +232,17 @@ __global__ __launch_bounds__(64) void rough_survey_kernel(SurveyArgs a) {
     auto look_at = [&](uint32_t of, float& d) {
         uint32_t id = static_cast<uint32_t>(lane) < degree ? a.graph[static_cast<size_t>(first + of) * a.degree + lane] : kInvalid;
         if (id >= length || id == self) id = kInvalid;
-        list[lane] = id != kInvalid ? id : self;
-        wave_sync();
-        score_list<DIMV>(q, data, a.dim, 0, degree, lane, [](uint32_t i) { return list[i]; }, [](uint32_t i, float v) { sq[i] = v; });
-        wave_sync();
+        if (wave == 0 && static_cast<uint32_t>(lane) < degree) list[lane] = id != kInvalid ? id : self;
+        __syncthreads();
+        score_share<DIMV, DIMV < 4 ? DIMV : 4>(RefInRegs<DIMV>{q}, data, a.dim, 0, degree, lane, wave, kSurveyWaves, [](uint32_t i) { return list[i]; },
+                             [](uint32_t i, float v) { sq[i] = v; });
+        __syncthreads();   // the next list is written behind the reads below: by wavefront 0, which has made them; sq behind a barrier more
         d = id != kInvalid ? sq[lane] : __builtin_inff();
         return id;
     };
     float d;
     const uint32_t id = look_at(self, d);
-    own[lane] = id;
+    if (wave == 0 && static_cast<uint32_t>(lane) < degree) own[lane] = id;   // read behind the barriers of the next list
     uint64_t some = ballot(id != kInvalid);
     if (some == 0) return;
     float farthest = id != kInvalid ? d : 0.f;
@@ -264,7 +267,7 @@ __global__ __launch_bounds__(64) void rough_survey_kernel(SurveyArgs a) {
         nearest = least;
         at = read_lane(next, __builtin_ctzll(ballot(d == least)));
     }
-    if (lane == 0) {
+    if (threadIdx.x == 0) {
         atomicAdd(&a.counts[0], fars);
         atomicAdd(&a.counts[1], settleds);
         atomicAdd(&a.counts[2], 1u);
@@ -590,7 +593,7 @@ int glide_hip_survey_rough_rows(const float* rows, const void* rough_rows, uint3
     const SurveyArgs a{rows, static_cast<const unsigned char*>(rough_rows), graph, segment_starts, segment_lengths, start_points, num, dim, degree,
                        segment_num, counts};
     const auto kernel = dim <= 128 ? rough_survey_kernel<1> : dim <= 256 ? rough_survey_kernel<2> : dim <= 512 ? rough_survey_kernel<4> : rough_survey_kernel<8>;
-    hipLaunchKernelGGL(kernel, dim3(num < kSurveyed ? num : kSurveyed), dim3(64), 0, as_stream(stream), a);
+    hipLaunchKernelGGL(kernel, dim3(num < kSurveyed ? num : kSurveyed), dim3(64 * kSurveyWaves), 0, as_stream(stream), a);
     return launch_status();
 }
 

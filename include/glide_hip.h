@@ -327,9 +327,9 @@ int glide_hip_refine(const float *data, uint32_t num, uint32_t dim, const uint32
  * above 128: not used. */
 size_t glide_hip_rough_rows_bytes(uint32_t num, uint32_t dim);
 int glide_hip_pack_rough_rows(const float *rows, uint32_t num, uint32_t dim, void *rough_rows, void *stream);
-/* Whether rough_rows will be of use to a build: counts (device, 4 words) = over some 500 of the rows, neighbours of neighbours
+/* Whether rough_rows will be of use to a build: counts (device, 4 words) = over 256 of the rows, neighbours of neighbours
  * in the graph that lie farther than a row's own; those of them that rough_rows tells to be so; the rows; those that a greedy
- * walk from their segment's start point does not come near.  The graph (`degree` ids a row, the first 64 are looked at) and the
+ * walk from their segment's start point does not come near.  The graph (`degree` ids a row, the first 32 are looked at) and the
  * start points are relative to segments, as for glide_hip_build_subgraph; a graph over all rows is one segment.  A look pays
  * where most of the far ones are told and most walks arrive. */
 int glide_hip_survey_rough_rows(const float *rows, const void *rough_rows, uint32_t num, uint32_t dim, const uint32_t *graph,

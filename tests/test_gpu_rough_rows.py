@@ -140,14 +140,14 @@ def survey(rows, turn, tiny, graph, starts, lengths, start_points):
     """glide_hip_survey_rough_rows in numpy: [far neighbours of neighbours, those told, rows, rows whose walk goes astray]."""
     n, counts = len(rows), [0, 0, 0, 0]
     x = rows.astype(np.float64)
-    for row in np.arange(min(n, 512)) * n // min(n, 512):
+    for row in np.arange(min(n, 256)) * n // min(n, 256):
         seg = np.flatnonzero((row >= starts) & (row < starts + lengths.astype(np.int64)))
         if len(seg) == 0:
             continue
         first, length = int(starts[seg[0]]), int(lengths[seg[0]])
 
         def neighbours(of):
-            ids = graph[first + of, :64].astype(np.int64)
+            ids = graph[first + of, :32].astype(np.int64)
             ids = ids[(ids < length) & (ids != row - first)]
             return ids, np.linalg.norm(x[first + ids] - x[row], axis=1)
 
